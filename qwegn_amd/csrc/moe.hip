@@ -1,153 +1,10 @@
-// MoE plumbing around the grouped GEMM: router logits, softmax top-k routing, the expert-major pair sort
+// MoE plumbing around the grouped GEMM: softmax top-k routing, the expert-major pair sort
 // with its tile list, and the weighted combine.
 #include <algorithm>
 #include <atomic>
 
 #include "qwhip_common.h"
 #include "qwhip_route.h"
-
-// ------------------------------------------------------------------------------------------------
-// Router logits: logits[t, e] = sum_h x[t, h] * Wr[e, h], fp32 accumulate.
-// A workgroup owns TT token rows (staged as fp32 in LDS; 8 rows up to hidden = 2048, fewer on wider rows so the tile
-// stays within 64 KiB, and no more than the call has) so each router row is read once per TT tokens; blockIdx.y owns a band of `eb` weight rows
-// (a multiple of 4, so that few token rows still spread over the chip), a wavefront the band's rows wave, wave+4, ...;
-// lanes stride the hidden dimension, so an output's summation order does not depend on the band size.  With a shared-expert gate row (fp32 [hidden]) the workgroup also writes
-// sh_out[t] = sigmoid(x[t] . sh_w), the extra output column of the reference's router kernels
-// (Sources/QWMetal/subsystems/qwrouter.metal:467-483,566-574,587-633).
-// ------------------------------------------------------------------------------------------------
-// The scalar epilogues of the dense f32 GEMV door (qwg_f32_gemv, Sources/QWMetal/gemm/qwgemm_f32.metal:120-143):
-// 0 none, 1 silu(y / scale), 2 sigmoid(y), 3 2 sigmoid(y / scale).
-__device__ __forceinline__ float qw_f32_gemv_epilogue(float y, uint32_t epi, float scale) {
-    if (epi == 1u) {
-        const float z = y / scale;
-        return z / (1.0f + expf(-z));
-    }
-    if (epi == 2u) return 1.0f / (1.0f + expf(-y));
-    if (epi == 3u) return 2.0f / (1.0f + expf(-(y / scale)));
-    return y;
-}
-
-template <int XDT, int WDT, int TT>
-__global__ __launch_bounds__(256) void qw_router_gemm_kernel(const void* __restrict__ x, const void* __restrict__ wr,
-                                                              float* __restrict__ logits, uint32_t T, uint32_t E, uint32_t H,
-                                                              const float* __restrict__ sh_w, float* __restrict__ sh_out,
-                                                              uint32_t epi, float scale, uint32_t eb) {
-    extern __shared__ float xs[];  // [TT][H]
-    const uint32_t t0 = blockIdx.x * TT;
-    const uint32_t nt = min((uint32_t)TT, T - t0);
-#pragma unroll
-    for (uint32_t r = 0; r < (uint32_t)TT; ++r)
-        for (uint32_t h = threadIdx.x; h < H; h += 256) xs[r * H + h] = r < nt ? qw_load_f32<XDT>(x, (uint64_t)(t0 + r) * H + h) : 0.0f;
-    __syncthreads();
-    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    const uint32_t rows = min(E + (sh_w ? 1u : 0u), (blockIdx.y + 1u) * eb);
-    for (uint32_t e = blockIdx.y * eb + wave; e < rows; e += 4) {
-        const bool gate_row = e == E;   // wave-uniform
-        float acc[TT];
-#pragma unroll
-        for (int r = 0; r < TT; ++r) acc[r] = 0.0f;
-        // eight weight loads in flight per lane, consumed in the order h = lane, lane + 64, ... so the sums do not depend on it
-        uint32_t h = lane;
-        if (!gate_row) {
-            const uint64_t row = (uint64_t)e * H;
-            for (; h + 7u * 64u < H; h += 8u * 64u) {
-                float w[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) w[u] = qw_load_f32<WDT>(wr, row + h + (uint32_t)u * 64u);
-#pragma unroll
-                for (int u = 0; u < 8; ++u)
-#pragma unroll
-                    for (int r = 0; r < TT; ++r) acc[r] = fmaf(w[u], xs[r * H + h + (uint32_t)u * 64u], acc[r]);
-            }
-        }
-        for (; h < H; h += 64) {
-            const float w = gate_row ? sh_w[h] : qw_load_f32<WDT>(wr, (uint64_t)e * H + h);
-#pragma unroll
-            for (int r = 0; r < TT; ++r) acc[r] = fmaf(w, xs[r * H + h], acc[r]);
-        }
-#pragma unroll
-        for (int r = 0; r < TT; ++r) {
-            const float v = qw_reduce64(acc[r]);
-            if (lane == 0 && (uint32_t)r < nt) {
-                if (gate_row) sh_out[t0 + r] = 1.0f / (1.0f + expf(-v));
-                else logits[(uint64_t)(t0 + r) * E + e] = qw_f32_gemv_epilogue(v, epi, scale);
-            }
-        }
-    }
-}
-
-static qwhip_status qw_router_gemm_impl(qwhip_stream_t s, const void* x, uint32_t x_dtype, const void* wr, uint32_t w_dtype, uint32_t t,
-                                        uint32_t experts, uint32_t hidden, float* logits, const float* sh_gate_w, float* sh_gate_out,
-                                        uint32_t epi, float scale) {
-    QWHIP_REQUIRE(s);
-    if (t == 0) return QWHIP_OK;
-    QWHIP_REQUIRE(x);
-    QWHIP_REQUIRE(wr);
-    QWHIP_REQUIRE(logits);
-    if ((sh_gate_w != nullptr) != (sh_gate_out != nullptr))
-        return qwhip_fail(QWHIP_E_NULL, "router gemm: the shared-expert gate needs both its weight row and its output");
-    if (experts == 0 || hidden == 0) return qwhip_fail(QWHIP_E_BAD_SHAPE, "router gemm: empty experts or hidden");
-    // token rows per workgroup: the fp32 tile stays within 64 KiB
-    uint32_t tt = 8;
-    while (tt > 1u && ((size_t)tt * hidden * 4u > 64u * 1024u || tt >= 2u * t)) tt >>= 1;
-    const size_t lds = (size_t)tt * hidden * 4u;
-    if (lds > 64u * 1024u) return qwhip_fail(QWHIP_E_BAD_SHAPE, "router gemm: hidden %u exceeds the staged row (<= 16384)", hidden);
-    // weight rows per workgroup: about 1024 workgroups over the launch, at least one row per wavefront
-    const uint32_t gx = qwhip_cdiv(t, tt), rows_total = experts + (sh_gate_w ? 1u : 0u);
-    const uint32_t gy_want = std::min(qwhip_cdiv(rows_total, 4u), std::max(1u, 1024u / gx));
-    const uint32_t eb = (qwhip_cdiv(rows_total, gy_want) + 3u) & ~3u;
-    const dim3 grid(gx, qwhip_cdiv(rows_total, eb)), block(256);
-    if (grid.y > 65535u) return qwhip_fail(QWHIP_E_BAD_SHAPE, "router gemm: %u weight rows exceed the launch grid", rows_total);
-#define QW_RG(XD, WD, TT) \
-    hipLaunchKernelGGL((qw_router_gemm_kernel<XD, WD, TT>), grid, block, lds, s->stream, x, wr, logits, t, experts, hidden, sh_gate_w, sh_gate_out, epi, scale, eb)
-#define QW_RG_T(XD, WD)                       \
-    switch (tt) {                             \
-        case 8: QW_RG(XD, WD, 8); break;      \
-        case 4: QW_RG(XD, WD, 4); break;      \
-        case 2: QW_RG(XD, WD, 2); break;      \
-        default: QW_RG(XD, WD, 1); break;     \
-    }
-#define QW_RG_W(XD)                                                   \
-    switch (w_dtype) {                                                \
-        case QWHIP_F32: QW_RG_T(XD, QWHIP_F32) break;                 \
-        case QWHIP_F16: QW_RG_T(XD, QWHIP_F16) break;                 \
-        case QWHIP_BF16: QW_RG_T(XD, QWHIP_BF16) break;               \
-        default: return qwhip_fail(QWHIP_E_BAD_SHAPE, "router gemm: unsupported weight dtype %u", w_dtype); \
-    }
-    switch (x_dtype) {
-        case QWHIP_F32: QW_RG_W(QWHIP_F32) break;
-        case QWHIP_F16: QW_RG_W(QWHIP_F16) break;
-        case QWHIP_BF16: QW_RG_W(QWHIP_BF16) break;
-        default: return qwhip_fail(QWHIP_E_BAD_SHAPE, "router gemm: unsupported activation dtype %u", x_dtype);
-    }
-#undef QW_RG_W
-#undef QW_RG_T
-#undef QW_RG
-    QWHIP_TRY_HIP(hipGetLastError());
-    return QWHIP_OK;
-}
-
-extern "C" qwhip_status qwhip_router_gemm_shared_gate(qwhip_stream_t s, const void* x, uint32_t x_dtype, const void* wr, uint32_t w_dtype,
-                                                      uint32_t t, uint32_t experts, uint32_t hidden, float* logits,
-                                                      const float* sh_gate_w, float* sh_gate_out) {
-    return qw_router_gemm_impl(s, x, x_dtype, wr, w_dtype, t, experts, hidden, logits, sh_gate_w, sh_gate_out, 0u, 1.0f);
-}
-
-extern "C" qwhip_status qwhip_router_gemm(qwhip_stream_t s, const void* x, uint32_t x_dtype, const void* wr, uint32_t w_dtype,
-                                          uint32_t t, uint32_t experts, uint32_t hidden, float* logits) {
-    return qw_router_gemm_impl(s, x, x_dtype, wr, w_dtype, t, experts, hidden, logits, nullptr, nullptr, 0u, 1.0f);
-}
-
-// Dense fp32-weight GEMV with the scalar epilogues (QWGemm.encodeF32Gemv, Sources/Operators/QWGEMM/QWGemmF32.swift:117-141 ->
-// qwg_f32_gemv / qwg_f32_gemv_bm): y[t, n] = epilogue(sum_k W[n, k] x[t, k]) on the router kernel (every weight row read once
-// per eight activation rows).
-extern "C" qwhip_status qwhip_f32_gemv(qwhip_stream_t s, const float* w, const float* x, uint32_t rows, uint32_t n, uint32_t k,
-                                       uint32_t epi, float scale, float* y) {
-    if (epi > 3u) return qwhip_fail(QWHIP_E_BAD_SHAPE, "epilogue %u is not one of 0 none, 1 silu(y/scale), 2 sigmoid, 3 2 sigmoid(y/scale)", epi);
-    if ((epi == 1u || epi == 3u) && !(scale != 0.0f && scale == scale))
-        return qwhip_fail(QWHIP_E_BAD_SHAPE, "epilogue %u divides by its scale, which must be a non-zero number", epi);
-    return qw_router_gemm_impl(s, x, QWHIP_F32, w, QWHIP_F32, rows, n, k, y, nullptr, nullptr, epi, scale);
-}
 
 // ------------------------------------------------------------------------------------------------
 // Routing: one wavefront per token row; lane l holds experts l, l+64, ... (E <= 512 -> <= 8 each).

@@ -102,6 +102,30 @@ def test_router_gemm_shared_gate_and_wide_rows(dev, t, e, h, wdt):
     assert lib.qwhip_router_gemm(st, xb.ptr, qwhip.F32, wb.ptr, wcode, t, e, 16388, l1.ptr) == qwhip.E_BAD_SHAPE
 
 
+@pytest.mark.parametrize("xdt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("wdt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("t,e,h", [(1, 1, 32), (1, 65, 2080), (2, 16, 64), (16, 17, 2048), (17, 33, 1056), (300, 130, 544), (1025, 257, 96)])
+def test_router_gemm_tiles(dev, t, e, h, xdt, wdt):
+    """One row, the edges of the 16-row tiles, both tile widths and hidden sizes that leave a wave without a chunk, with the gate
+    column.  Every product and sum is fp32 (bf16 products hold all bits of the activations): h sums of relative size 2^-24 stay
+    below h 2^-24 of the sum of magnitudes, which for signs as they fall is sqrt(h) times the result - 2e-5 at h = 2080 at most,
+    2e-6 where the roundings fall either way."""
+    rng = np.random.default_rng(t + e + h)
+    cast = {"f32": (lambda v: (v, qwhip.F32, v)), "f16": (lambda v: (v.astype(np.float16), qwhip.F16, v.astype(np.float16).astype(np.float32))),
+            "bf16": (lambda v: (qo.f32_to_bf16_bits(v), qwhip.BF16, qo.round_bf16(v)))}
+    xh, xcode, xv = cast[xdt](rng.standard_normal((t, h)).astype(np.float32))
+    wh, wcode, wv = cast[wdt]((rng.standard_normal((e, h)) * 0.05).astype(np.float32))
+    shw = (rng.standard_normal(h) * 0.03).astype(np.float32)
+    xb, wb, sb = dev.put(xh), dev.put(wh), dev.put(shw)
+    lb, go = dev.alloc(t * e * 4), dev.alloc(t * 4)
+    qwhip.check(dev.lib.qwhip_router_gemm_shared_gate(dev.stream.handle, xb.ptr, xcode, wb.ptr, wcode, t, e, h, lb.ptr, sb.ptr, go.ptr))
+    got, gate = lb.download(np.float32, (t, e)), go.download(np.float32, (t,))
+    assert qo.normalized_error(got, xv.astype(np.float64) @ wv.astype(np.float64).T) <= 2e-6
+    np.testing.assert_allclose(gate, qo.router_shared_gate_f64(xv, shw), rtol=0, atol=2e-6)
+    for b in (xb, wb, sb, lb, go):
+        b.free()
+
+
 @pytest.mark.parametrize("t,e,k", [(33, 128, 8), (5, 40, 4), (9, 512, 16), (7, 100, 3)])
 @pytest.mark.parametrize("mode", ["bias", "split", "bias+split", "softmax+scale"])
 @pytest.mark.parametrize("norm", [0, 1])
