@@ -3,23 +3,15 @@
 #include "qwhip_common.h"
 
 // ---- FWHT-32 over consecutive 32-groups: src (f16 | bf16 | f32) -> dst f16 ----------------------
-// One lane owns one group: 64/128 bytes in, 64 bytes out, all butterflies in registers.
+// Four lanes a group (qw_fwht32_quad).
 template <int DT>
-__global__ __launch_bounds__(256) void qw_fwht32_kernel(const void* __restrict__ src, h1_t* __restrict__ dst,
-                                                         uint64_t groups) {
-    const uint64_t g = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (g >= groups) return;
-    float v[32];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) qw_load8_f32<DT>(src, g * 32 + 8 * j, v + 8 * j);
-    qw_fwht32(v);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        h8_t o;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = (h1_t)v[8 * j + e];
-        *(h8_t*)(dst + g * 32 + 8 * j) = o;
-    }
+__global__ __launch_bounds__(256) void qw_fwht32_kernel(const void* __restrict__ src, h1_t* __restrict__ dst, uint64_t octets) {
+    const uint64_t o = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (o >= octets) return;   // whole groups of four lanes leave together
+    float v[8];
+    qw_load8_f32<DT>(src, o * 8, v);
+    qw_fwht32_quad(v, threadIdx.x);
+    qw_store8_f16(dst + o * 8, v);
 }
 
 extern "C" qwhip_status qwhip_fwht32(qwhip_stream_t s, const void* src, uint32_t src_dtype, void* dst_f16, uint64_t n) {
@@ -30,12 +22,12 @@ extern "C" qwhip_status qwhip_fwht32(qwhip_stream_t s, const void* src, uint32_t
     if (n % 32 != 0) return qwhip_fail(QWHIP_E_BAD_SHAPE, "fwht32: n=%llu is not a multiple of 32", (unsigned long long)n);
     if (((uintptr_t)src & 15u) || ((uintptr_t)dst_f16 & 15u))
         return qwhip_fail(QWHIP_E_BAD_SHAPE, "fwht32: buffers must be 16-byte aligned");
-    const uint64_t groups = n / 32;
-    const dim3 grid((unsigned)((groups + 255) / 256)), block(256);
+    const uint64_t octets = n / 8;
+    const dim3 grid((unsigned)((octets + 255) / 256)), block(256);
     switch (src_dtype) {
-        case QWHIP_F16: hipLaunchKernelGGL(qw_fwht32_kernel<QWHIP_F16>, grid, block, 0, s->stream, src, (h1_t*)dst_f16, groups); break;
-        case QWHIP_BF16: hipLaunchKernelGGL(qw_fwht32_kernel<QWHIP_BF16>, grid, block, 0, s->stream, src, (h1_t*)dst_f16, groups); break;
-        case QWHIP_F32: hipLaunchKernelGGL(qw_fwht32_kernel<QWHIP_F32>, grid, block, 0, s->stream, src, (h1_t*)dst_f16, groups); break;
+        case QWHIP_F16: hipLaunchKernelGGL(qw_fwht32_kernel<QWHIP_F16>, grid, block, 0, s->stream, src, (h1_t*)dst_f16, octets); break;
+        case QWHIP_BF16: hipLaunchKernelGGL(qw_fwht32_kernel<QWHIP_BF16>, grid, block, 0, s->stream, src, (h1_t*)dst_f16, octets); break;
+        case QWHIP_F32: hipLaunchKernelGGL(qw_fwht32_kernel<QWHIP_F32>, grid, block, 0, s->stream, src, (h1_t*)dst_f16, octets); break;
         default: return qwhip_fail(QWHIP_E_BAD_SHAPE, "fwht32: unsupported source dtype %u", src_dtype);
     }
     QWHIP_TRY_HIP(hipGetLastError());
@@ -101,31 +93,22 @@ extern "C" qwhip_status qwhip_cast_f32_to_f16(qwhip_stream_t s, const float* src
 // SwiGLU runs in fp32 on the values as stored (f16 inputs are the rounded values the fused prefill
 // path also sees, Sources/QWMetal/include/qw_gemm_nax_swiglu.metalh:132-152); rotation in fp32, one
 // f16 rounding on store.
+// Four lanes a 32-group, a row of act per blockIdx.y: with one lane a group and a 64-bit division by the row length, 4 x 17408
+// fp32 pairs (2176 lanes of long serial work) took 5.7 us where an empty launch takes 1.7; now 2.4.
 template <int DT, bool ROT>
 __global__ __launch_bounds__(256) void qw_swiglu_fwht_kernel(const void* __restrict__ gu, h1_t* __restrict__ act,
                                                               uint32_t rows, uint32_t inter, const qw_act ga) {
-    const uint32_t gpr = inter / 32;  // groups per row
-    const uint64_t gid = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (gid >= (uint64_t)rows * gpr) return;
-    const uint32_t r = (uint32_t)(gid / gpr), g = (uint32_t)(gid % gpr);
-    const uint64_t gbase = (uint64_t)r * 2 * inter + 32 * g;
-    float v[32];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    const uint32_t c = (blockIdx.x * 256u + threadIdx.x) * 8u;
+    if (c >= inter) return;   // whole groups of four lanes leave together
+    for (uint32_t r = blockIdx.y; r < rows; r += gridDim.y) {
+        const uint64_t at = (uint64_t)r * 2 * inter + c;
         float a[8], b[8];
-        qw_load8_f32<DT>(gu, gbase + 8 * j, a);
-        qw_load8_f32<DT>(gu, gbase + inter + 8 * j, b);
+        qw_load8_f32<DT>(gu, at, a);
+        qw_load8_f32<DT>(gu, at + inter, b);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[8 * j + e] = qw_gated(a[e], b[e], ga);
-    }
-    if (ROT) qw_fwht32(v);
-    h1_t* o = act + (uint64_t)r * inter + 32 * g;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        h8_t t;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) t[e] = (h1_t)v[8 * j + e];
-        *(h8_t*)(o + 8 * j) = t;
+        for (int e = 0; e < 8; ++e) a[e] = qw_gated(a[e], b[e], ga);
+        if (ROT) qw_fwht32_quad(a, threadIdx.x);
+        qw_store8_f16(act + (uint64_t)r * inter + c, a);
     }
 }
 
@@ -158,8 +141,7 @@ extern "C" qwhip_status qwhip_swiglu_fwht(qwhip_stream_t s, const void* gu, uint
         if (gu_dtype == QWHIP_F16) hipLaunchKernelGGL(qw_swiglu_scalar_kernel<QWHIP_F16>, grid, block, 0, s->stream, gu, act, rows, inter, s->dev->act);
         else hipLaunchKernelGGL(qw_swiglu_scalar_kernel<QWHIP_F32>, grid, block, 0, s->stream, gu, act, rows, inter, s->dev->act);
     } else {
-        const uint64_t groups = (uint64_t)rows * (inter / 32);
-        const dim3 grid((unsigned)((groups + 255) / 256)), block(256);
+        const dim3 grid(qwhip_cdiv(inter, 2048u), min(rows, 65535u)), block(256);
         if (gu_dtype == QWHIP_F16) {
             if (rotate) hipLaunchKernelGGL((qw_swiglu_fwht_kernel<QWHIP_F16, true>), grid, block, 0, s->stream, gu, act, rows, inter, s->dev->act);
             else hipLaunchKernelGGL((qw_swiglu_fwht_kernel<QWHIP_F16, false>), grid, block, 0, s->stream, gu, act, rows, inter, s->dev->act);
@@ -231,30 +213,25 @@ extern "C" qwhip_status qwhip_dequant_f16(qwhip_stream_t s, const qwhip_weight_v
 }
 
 // ---- fp32 seams of the MoE operator chain ----------------------------------------------------------
-// One thread per 32-group, the group in registers, the fp32 butterfly of qw_fwht32 (strides 1, 2, 4, 8, 16, then one
+// Four lanes per 32-group, the fp32 butterfly of qw_fwht32 (strides 1, 2, 4, 8, 16, then one
 // multiply by 1/sqrt(32): the order of fwht32_f32_inplace, Sources/QWMetal/include/qw_dequant.metalh:442-478).
 
 // silu(gate) * up in fp32, then the 32-point transform, fp32 out (qwg_silu_mul_f32, Sources/QWMetal/gemm/qwgemm_f32.metal:291-317;
 // door QWGemm.encodeSiluMulF32, Sources/Operators/QWGEMM/QWGemmF32.swift:83-94).  gu fp32 [rows, 2 inter], inter % 32 == 0.
 __global__ __launch_bounds__(256) void qw_silu_mul_f32_kernel(const float* __restrict__ gu, float* __restrict__ act, uint32_t rows,
                                                                uint32_t inter, const qw_act ga) {
-    const uint64_t gi = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    const uint32_t gpr = inter / 32u;
-    if (gi >= (uint64_t)rows * gpr) return;
-    const uint32_t r = (uint32_t)(gi / gpr), g = (uint32_t)(gi % gpr);
-    const f4_t* gp = (const f4_t*)(gu + (uint64_t)r * 2u * inter + 32u * g);
-    const f4_t* up = (const f4_t*)(gu + (uint64_t)r * 2u * inter + inter + 32u * g);
-    float v[32];
+    const uint32_t c = (blockIdx.x * 256u + threadIdx.x) * 8u;
+    if (c >= inter) return;
+    for (uint32_t r = blockIdx.y; r < rows; r += gridDim.y) {
+        const uint64_t at = (uint64_t)r * 2u * inter + c;
+        float a[8], b[8];
+        qw_load8_f32<QWHIP_F32>(gu, at, a);
+        qw_load8_f32<QWHIP_F32>(gu, at + inter, b);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const f4_t a = gp[j], b = up[j];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[4 * j + e] = qw_gated(a[e], b[e], ga);
+        for (int e = 0; e < 8; ++e) a[e] = qw_gated(a[e], b[e], ga);
+        qw_fwht32_quad(a, threadIdx.x);
+        qw_store8_f32(act + (uint64_t)r * inter + c, a);
     }
-    qw_fwht32(v);
-    f4_t* o = (f4_t*)(act + (uint64_t)r * inter + 32u * g);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = f4_t{v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]};
 }
 
 extern "C" qwhip_status qwhip_silu_mul_f32(qwhip_stream_t s, const float* gu, float* act, uint32_t rows, uint32_t inter) {
@@ -264,8 +241,7 @@ extern "C" qwhip_status qwhip_silu_mul_f32(qwhip_stream_t s, const float* gu, fl
     QWHIP_REQUIRE(act);
     if (inter == 0 || inter % 32u != 0) return qwhip_fail(QWHIP_E_BAD_SHAPE, "f32 silu-mul needs intermediate %% 32 == 0, got %u", inter);
     if (((uintptr_t)gu | (uintptr_t)act) & 15u) return qwhip_fail(QWHIP_E_BAD_SHAPE, "f32 silu-mul needs 16-byte aligned buffers");
-    const uint64_t groups = (uint64_t)rows * (inter / 32u);
-    hipLaunchKernelGGL(qw_silu_mul_f32_kernel, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s->stream, gu, act, rows, inter, s->dev->act);
+    hipLaunchKernelGGL(qw_silu_mul_f32_kernel, dim3(qwhip_cdiv(inter, 2048u), min(rows, 65535u)), dim3(256), 0, s->stream, gu, act, rows, inter, s->dev->act);
     QWHIP_TRY_HIP(hipGetLastError());
     return QWHIP_OK;
 }
@@ -276,32 +252,20 @@ extern "C" qwhip_status qwhip_silu_mul_f32(qwhip_stream_t s, const float* gu, fl
 // router reads - the transform again (it is its own inverse) in fp32, taken through the f16 hi/lo split of the reference's
 // helper: plain = f32(hi) + f32(lo), hi = f16(v), lo = f16(v - f32(hi)).
 __global__ __launch_bounds__(256) void qw_moe_bridge_kernel(const h1_t* __restrict__ x, float* __restrict__ rot32, float* __restrict__ plain32,
-                                                             uint64_t groups) {
-    const uint64_t gi = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (gi >= groups) return;
-    const h8_t* xp = (const h8_t*)(x + 32u * gi);
-    float v[32];
+                                                             uint64_t octets) {
+    const uint64_t o = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (o >= octets) return;
+    float v[8];
+    qw_load8_f32<QWHIP_F16>(x, 8u * o, v);
+    if (rot32) qw_store8_f32(rot32 + 8u * o, v);
+    qw_fwht32_quad(v, threadIdx.x);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const h8_t a = xp[j];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[8 * j + e] = (float)a[e];
-    }
-    if (rot32) {
-        f4_t* o = (f4_t*)(rot32 + 32u * gi);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] = f4_t{v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]};
-    }
-    qw_fwht32(v);
-#pragma unroll
-    for (int i = 0; i < 32; ++i) {
+    for (int i = 0; i < 8; ++i) {
         const h1_t hi = (h1_t)v[i];
         const h1_t lo = (h1_t)(v[i] - (float)hi);
         v[i] = (float)hi + (float)lo;
     }
-    f4_t* o = (f4_t*)(plain32 + 32u * gi);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = f4_t{v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]};
+    qw_store8_f32(plain32 + 8u * o, v);
 }
 
 extern "C" qwhip_status qwhip_moe_bridge_f16_to_f32(qwhip_stream_t s, const void* x_f16, float* x_rot32, float* x_plain32, uint32_t rows,
@@ -313,9 +277,9 @@ extern "C" qwhip_status qwhip_moe_bridge_f16_to_f32(qwhip_stream_t s, const void
     QWHIP_REQUIRE(x_plain32);
     if (((uintptr_t)x_f16 | (uintptr_t)x_rot32 | (uintptr_t)x_plain32) & 15u)
         return qwhip_fail(QWHIP_E_BAD_SHAPE, "moe bridge needs 16-byte aligned buffers");
-    const uint64_t groups = (uint64_t)rows * (hidden / 32u);
-    hipLaunchKernelGGL(qw_moe_bridge_kernel, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s->stream, (const h1_t*)x_f16, x_rot32,
-                       x_plain32, groups);
+    const uint64_t octets = (uint64_t)rows * (hidden / 8u);
+    hipLaunchKernelGGL(qw_moe_bridge_kernel, dim3((unsigned)((octets + 255) / 256)), dim3(256), 0, s->stream, (const h1_t*)x_f16, x_rot32,
+                       x_plain32, octets);
     QWHIP_TRY_HIP(hipGetLastError());
     return QWHIP_OK;
 }
@@ -344,33 +308,17 @@ __global__ __launch_bounds__(256) void qw_latent_norm_kernel(const float* __rest
         __syncthreads();
         rstd = rsqrtf(((wsum[0] + wsum[1]) + (wsum[2] + wsum[3])) / (float)latent + eps);
     }
-    for (uint32_t g = tid; g < latent / 32u; g += 256u) {
-        float v[32];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const f4_t a = *(const f4_t*)(xr + 32u * g + 4 * j);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[4 * j + e] = a[e];
-        }
+    for (uint32_t c = tid * 8u; c < latent; c += 2048u) {   // four lanes a group
+        float v[8];
+        qw_load8_f32<QWHIP_F32>(xr, c, v);
         if (gamma) {
 #pragma unroll
-            for (int i = 0; i < 32; ++i) v[i] = (v[i] * rstd) * (1.0f + (float)gamma[32u * g + i]);
+            for (int i = 0; i < 8; ++i) v[i] = (v[i] * rstd) * (1.0f + (float)gamma[c + i]);
         }
-        qw_fwht32(v);
-        const uint64_t at = (uint64_t)blockIdx.x * latent + 32u * g;
-        if (out32) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) *(f4_t*)(out32 + at + 4 * j) = f4_t{v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]};
-        }
-        if (out16) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                h8_t o;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) o[e] = (h1_t)v[8 * j + e];
-                *(h8_t*)(out16 + at + 8 * j) = o;
-            }
-        }
+        qw_fwht32_quad(v, tid);
+        const uint64_t at = (uint64_t)blockIdx.x * latent + c;
+        if (out32) qw_store8_f32(out32 + at, v);
+        if (out16) qw_store8_f16(out16 + at, v);
     }
 }
 
@@ -415,7 +363,7 @@ extern "C" qwhip_status qwhip_add_f32(qwhip_stream_t s, const float* a, const fl
 template <bool M5>
 __global__ __launch_bounds__(256) void qw_embed_kernel(const uint8_t* __restrict__ bank, const int32_t* __restrict__ tokens,
                                                         float* __restrict__ out, uint32_t vocab, uint32_t hidden, uint32_t hc,
-                                                        uint32_t bits, uint32_t group, uint32_t row_bytes) {
+                                                        uint32_t bits, uint32_t group, uint32_t gshift8, uint32_t row_bytes) {
     const uint32_t oi = blockIdx.x * 256u + threadIdx.x;   // octet of the row
     if (oi * 8u >= hidden) return;
     const uint32_t r = blockIdx.y;
@@ -433,13 +381,16 @@ __global__ __launch_bounds__(256) void qw_embed_kernel(const uint8_t* __restrict
             v[e] = __fadd_rn(__fmul_rn(code, sc), bi);
         }
     } else {
-        const uint32_t opg = group / 8u;
-        const uint8_t* p = rowp + (uint64_t)(oi / opg) * (4u + group * bits / 8u);
-        const uint32_t o = oi % opg;
-        const float sc = (float)__builtin_bit_cast(h1_t, (uint16_t)(p[0] | (p[1] << 8)));
-        const float bi = (float)__builtin_bit_cast(h1_t, (uint16_t)(p[2] | (p[3] << 8)));
-        uint64_t stream = 0;
-        for (uint32_t b = 0; b < bits; ++b) stream |= (uint64_t)p[4 + o * bits + b] << (8 * b);
+        // the octet's `bits` bytes lie in at most two words of the block (blocks are whole words); the second is read only where
+        // the octet reaches it
+        const uint32_t at = (oi & (group / 8u - 1u)) * bits;
+        const uint32_t* p = (const uint32_t*)(rowp + (uint64_t)(oi >> gshift8) * (4u + group * bits / 8u));
+        const h2_t hd = __builtin_bit_cast(h2_t, p[0]);
+        const float sc = (float)hd[0], bi = (float)hd[1];
+        const uint32_t* q = p + 1 + (at >> 2);
+        uint64_t stream = q[0];
+        if ((at & 3u) + bits > 4u) stream |= (uint64_t)q[1] << 32;
+        stream >>= 8u * (at & 3u);
         const uint32_t mask = (1u << bits) - 1u;
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = __fadd_rn(__fmul_rn((float)((uint32_t)(stream >> (e * bits)) & mask), sc), bi);
@@ -467,13 +418,15 @@ extern "C" qwhip_status qwhip_embed_aq_f32(qwhip_stream_t s, const qwhip_weight_
     const uint32_t bb = qwhip_block_bytes(table->kind, table->bits, table->group);
     const uint64_t row_bytes = (uint64_t)(hidden / table->group) * bb;
     if (row_bytes >= (1ull << 32)) return qwhip_fail(QWHIP_E_BAD_SHAPE, "embedding rows of %llu bytes are not addressable", (unsigned long long)row_bytes);
+    uint32_t gshift8 = 2;   // log2 of the octets in a group
+    while ((8u << gshift8) < table->group) ++gshift8;
     const dim3 grid(qwhip_cdiv(hidden / 8u, 256u), rows), block(256);
     if (table->kind == QWHIP_KIND_HQ4_G32_M5)
         hipLaunchKernelGGL(qw_embed_kernel<true>, grid, block, 0, s->stream, (const uint8_t*)table->blocks, tokens, out, table->n, hidden, hc,
-                           table->bits, table->group, (uint32_t)row_bytes);
+                           table->bits, table->group, gshift8, (uint32_t)row_bytes);
     else
         hipLaunchKernelGGL(qw_embed_kernel<false>, grid, block, 0, s->stream, (const uint8_t*)table->blocks, tokens, out, table->n, hidden, hc,
-                           table->bits, table->group, (uint32_t)row_bytes);
+                           table->bits, table->group, gshift8, (uint32_t)row_bytes);
     QWHIP_TRY_HIP(hipGetLastError());
     return QWHIP_OK;
 }
@@ -514,88 +467,66 @@ extern "C" qwhip_status qwhip_embed_bf16_f32(qwhip_stream_t s, const void* table
 // Plus-one law: gamma is stored raw and applied as (1 + gamma) in fp32; sum of squares in fp32; the 32-point
 // transform in fp32 in the butterfly order of fwht32_f32_inplace (qw_dequant.metalh:442-478: strides 1, 2, 4 inside a
 // lane's 8 values, 8 and 16 across 4 lanes, times 1/sqrt(32)); one f16 rounding at the store.
-// One workgroup per row; a thread owns 8 consecutive values per 2048-column sweep (16-byte loads, the row stays in
-// registers up to 16384 columns); four neighbouring lanes hold one 32-group.
+// One workgroup per row, a thread to 8 consecutive values (16-byte loads) in SW sweeps, the row in registers (16384 columns at
+// most); four neighbouring lanes hold one 32-group.  A few rows are their own latency: one sweep, gamma asked for together with
+// the row, before the sum's barrier (1 x 5120 in a chain of such launches 3.2 -> 2.4 us, 1 x 2048 2.2 -> 1.9; an empty launch 1.7).
+// Many rows want more bytes in flight per wave: two sweeps (4096 x 5120: 15.5 us, 19.1 in one sweep).  The sum does not depend
+// on that choice: 64 octets are summed across the lanes that hold them, those sums across 16 or 32 lanes, in one order for a row length.
 // ------------------------------------------------------------------------------------------------
-template <bool RESIDUAL>
-__global__ __launch_bounds__(256) void qw_rmsnorm_kernel(const h1_t* __restrict__ x, const h1_t* __restrict__ gamma,
-                                                         h1_t* __restrict__ residual, h1_t* __restrict__ y, uint32_t hidden,
-                                                         float eps, uint32_t rotate) {
-    constexpr int SW = 8;   // sweeps held in registers
-    __shared__ float wsum[4];
-    const uint32_t tid = threadIdx.x;
+template <bool RESIDUAL, int SW>
+__global__ __launch_bounds__(1024) void qw_rmsnorm_kernel(const h1_t* __restrict__ x, const h1_t* __restrict__ gamma,
+                                                          h1_t* __restrict__ residual, h1_t* __restrict__ y, uint32_t hidden,
+                                                          float eps, uint32_t rotate) {
+    __shared__ float wsum[32];
+    const uint32_t tid = threadIdx.x, nw = blockDim.x >> 6;
     const uint64_t row = (uint64_t)blockIdx.x * hidden;
-    h8_t v[SW];
-    float acc = 0.f;
+    h8_t v[SW], gv[SW], rv[SW];
 #pragma unroll
     for (int k = 0; k < SW; ++k) {
-        const uint32_t c = (k * 256u + tid) * 8u;
+        const uint32_t c = (k * blockDim.x + tid) * 8u;
         if (c < hidden) {
-            h8_t xv = *(const h8_t*)(x + row + c);
-            if constexpr (RESIDUAL) {
-                const h8_t rv = *(const h8_t*)(residual + row + c);
+            v[k] = *(const h8_t*)(x + row + c);
+            if constexpr (RESIDUAL) rv[k] = *(const h8_t*)(residual + row + c);
+            gv[k] = *(const h8_t*)(gamma + c);
+        }
+    }
 #pragma unroll
-                for (int i = 0; i < 8; ++i) xv[i] = (h1_t)((float)xv[i] + (float)rv[i]);
-                *(h8_t*)(residual + row + c) = xv;
+    for (int k = 0; k < SW; ++k) {
+        const uint32_t c = (k * blockDim.x + tid) * 8u;
+        float acc = 0.f;
+        if (c < hidden) {
+            if constexpr (RESIDUAL) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[k][i] = (h1_t)((float)v[k][i] + (float)rv[k][i]);
+                *(h8_t*)(residual + row + c) = v[k];
             }
-            v[k] = xv;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const float t = (float)xv[i];
+                const float t = (float)v[k][i];
                 acc = fmaf(t, t, acc);
             }
         }
+        acc = qw_reduce64(acc);
+        if ((tid & 63u) == 0u) wsum[k * nw + (tid >> 6)] = acc;
     }
-    acc = qw_reduce64(acc);
-    if ((tid & 63u) == 0u) wsum[tid >> 6] = acc;
     __syncthreads();
-    const float total = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+    const uint32_t unit = tid & (hidden > 8192u ? 31u : 15u);   // 512 columns each; a row of 16384 has 32
+    float total = unit * 512u < hidden ? wsum[unit] : 0.0f;
+    total += QW_DPP_F32(total, 0xB1);    // lane ^ 1
+    total += QW_DPP_F32(total, 0x4E);    // lane ^ 2
+    total += QW_DPP_F32(total, 0x141);   // row_half_mirror
+    total += QW_DPP_F32(total, 0x140);   // row_mirror
+    if (hidden > 8192u) total += __shfl_xor(total, 16, 64);
     const float rstd = 1.0f / sqrtf(total / (float)hidden + eps);
 #pragma unroll
     for (int k = 0; k < SW; ++k) {
-        const uint32_t c = (k * 256u + tid) * 8u;
+        const uint32_t c = (k * blockDim.x + tid) * 8u;
         if (c >= hidden) continue;   // whole quads of lanes leave together: hidden is a multiple of 32
-        const h8_t gv = *(const h8_t*)(gamma + c);
         float f[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) f[i] = (float)v[k][i] * rstd * ((float)gv[i] + 1.0f);
-        if (rotate) {
-#pragma unroll
-            for (int i = 0; i < 8; i += 2) {
-                const float a = f[i], b = f[i + 1];
-                f[i] = a + b;
-                f[i + 1] = a - b;
-            }
-#pragma unroll
-            for (int i = 0; i < 8; i += 4) {
-                const float a0 = f[i], a1 = f[i + 1], b0 = f[i + 2], b1 = f[i + 3];
-                f[i] = a0 + b0;
-                f[i + 1] = a1 + b1;
-                f[i + 2] = a0 - b0;
-                f[i + 3] = a1 - b1;
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float a = f[i], b = f[i + 4];
-                f[i] = a + b;
-                f[i + 4] = a - b;
-            }
-            const bool neg1 = (tid & 1u) != 0u, neg2 = (tid & 2u) != 0u;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float p = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, f[i]), 0xB1, 0xF, 0xF, true));
-                f[i] = neg1 ? (p - f[i]) : (f[i] + p);
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float p = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, f[i]), 0x4E, 0xF, 0xF, true));
-                f[i] = (neg2 ? (p - f[i]) : (f[i] + p)) * QW_INV_SQRT32;
-            }
-        }
-        h8_t o;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = (h1_t)f[i];
-        *(h8_t*)(y + row + c) = o;
+        for (int i = 0; i < 8; ++i) f[i] = (float)v[k][i] * rstd * ((float)gv[k][i] + 1.0f);
+        if (rotate) qw_fwht32_quad(f, tid);
+        qw_store8_f16(y + row + c, f);
     }
 }
 
@@ -611,12 +542,17 @@ extern "C" qwhip_status qwhip_rmsnorm(qwhip_stream_t s, const void* x_f16, const
     if (hidden > 16384u) return qwhip_fail(QWHIP_E_BAD_GEOMETRY, "the norm kernel holds rows of at most 16384 columns, got %u", hidden);
     if (((uintptr_t)x_f16 | (uintptr_t)gamma_f16 | (uintptr_t)y_f16 | (uintptr_t)residual_f16) & 15u)
         return qwhip_fail(QWHIP_E_BAD_SHAPE, "the norm kernel needs 16-byte aligned rows");
-    if (residual_f16)
-        hipLaunchKernelGGL(qw_rmsnorm_kernel<true>, dim3(rows), dim3(256), 0, s->stream, (const h1_t*)x_f16, (const h1_t*)gamma_f16,
-                           (h1_t*)residual_f16, (h1_t*)y_f16, hidden, eps, rotate ? 1u : 0u);
-    else
-        hipLaunchKernelGGL(qw_rmsnorm_kernel<false>, dim3(rows), dim3(256), 0, s->stream, (const h1_t*)x_f16, (const h1_t*)gamma_f16,
-                           (h1_t*)nullptr, (h1_t*)y_f16, hidden, eps, rotate ? 1u : 0u);
+    const uint32_t sweeps = (hidden > 8192u ? 2u : 1u) * (rows > 512u && hidden > 4096u ? 2u : 1u);
+    const dim3 grid(rows), block((hidden / 8u / sweeps + 63u) & ~63u);
+#define QW_NORM(R, SW)                                                                                                                \
+    hipLaunchKernelGGL((qw_rmsnorm_kernel<R, SW>), grid, block, 0, s->stream, (const h1_t*)x_f16, (const h1_t*)gamma_f16,             \
+                       (h1_t*)residual_f16, (h1_t*)y_f16, hidden, eps, rotate ? 1u : 0u)
+    if (residual_f16) {
+        if (sweeps == 1u) QW_NORM(true, 1); else if (sweeps == 2u) QW_NORM(true, 2); else QW_NORM(true, 4);
+    } else {
+        if (sweeps == 1u) QW_NORM(false, 1); else if (sweeps == 2u) QW_NORM(false, 2); else QW_NORM(false, 4);
+    }
+#undef QW_NORM
     QWHIP_TRY_HIP(hipGetLastError());
     return QWHIP_OK;
 }

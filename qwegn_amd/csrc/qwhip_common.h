@@ -212,6 +212,48 @@ __device__ __forceinline__ float qw_fwht32_lanes(float v, const qw_fwht32_signs&
     return v;
 }
 
+// FWHT-32 with four neighbouring lanes to a group, lane j & 3 holding elements 8 (j & 3) .. + 7: strides 1, 2, 4 inside a lane,
+// 8 and 16 by DPP, then the 1/sqrt(32).  Additions and order are those of qw_fwht32, so the bits are too, but a group takes
+// consecutive 16- or 32-byte pieces of four lanes (whole lines per load, where a lane per group reads 64 to 128 bytes apart)
+// and four times the threads.  All four lanes of a group must be active.
+__device__ __forceinline__ void qw_fwht32_quad(float* f, uint32_t lane) {
+#pragma unroll
+    for (int h = 1; h < 8; h <<= 1) {
+#pragma unroll
+        for (int i0 = 0; i0 < 8; i0 += 2 * h) {
+#pragma unroll
+            for (int j = i0; j < i0 + h; ++j) {
+                const float a = f[j], b = f[j + h];
+                f[j] = a + b;
+                f[j + h] = a - b;
+            }
+        }
+    }
+    const bool neg1 = (lane & 1u) != 0u, neg2 = (lane & 2u) != 0u;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float p = QW_DPP_F32(f[i], 0xB1);   // quad_perm [1,0,3,2]
+        f[i] = neg1 ? (p - f[i]) : (f[i] + p);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float p = QW_DPP_F32(f[i], 0x4E);   // quad_perm [2,3,0,1]
+        f[i] = (neg2 ? (p - f[i]) : (f[i] + p)) * QW_INV_SQRT32;
+    }
+}
+
+// Eight floats as one 16-byte store of f16, or as two of fp32.
+__device__ __forceinline__ void qw_store8_f16(h1_t* dst, const float* f) {
+    h8_t o;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o[i] = (h1_t)f[i];
+    *(h8_t*)dst = o;
+}
+__device__ __forceinline__ void qw_store8_f32(float* dst, const float* f) {
+    ((f4_t*)dst)[0] = f4_t{f[0], f[1], f[2], f[3]};
+    ((f4_t*)dst)[1] = f4_t{f[4], f[5], f[6], f[7]};
+}
+
 // A constant pinned in a VGPR (v_and_or_b32 is VOP3: on gfx9 it takes no literal and one scalar operand,
 // so one of mask / magic has to live in a vector register to get the single-instruction form).
 __device__ __forceinline__ uint32_t qw_vgpr_const(uint32_t c) {

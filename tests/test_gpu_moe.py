@@ -479,6 +479,16 @@ def test_online_quantizer_writes_the_packers_bytes(dev):
             assert np.array_equal(got, qo.quant_hq4_blocks(val, rotate=bool(rotate)))
 
 
+def test_swiglu_fwht_more_rows_than_a_grid_dimension(dev):
+    """65,600 rows of one rotation group: the rows past the grid's 65,535 are taken by its second step."""
+    rows, inter = 65600, 32
+    gu = np.random.default_rng(5).standard_normal((rows, 2 * inter)).astype(np.float32)
+    gb, ab = dev.put(gu), dev.alloc(rows * inter * 2)
+    qwhip.check(dev.lib.qwhip_swiglu_fwht(dev.stream.handle, gb.ptr, qwhip.F32, ab.ptr, rows, inter, 1))
+    want = qo.swiglu_fwht_f16(gu[:, :inter], gu[:, inter:], rotate=True).astype(np.float32)
+    assert qo.normalized_error(ab.download(np.float16, (rows, inter)), want) <= 2e-3
+
+
 def test_swiglu_fwht_matches_oracle(dev):
     rng = np.random.default_rng(2)
     rows, inter = 9, 160

@@ -282,6 +282,28 @@ def test_rmsnorm_with_rotation_matches_oracle(dev, rows, hidden, residual, rotat
         assert np.array_equal(rb.download(np.float16, (rows, hidden)).view(np.uint16), want_res.view(np.uint16))
 
 
+@pytest.mark.parametrize("hidden", [256, 4352, 5376, 8192, 8448, 16384])
+@pytest.mark.parametrize("residual", [0, 1])
+def test_rmsnorm_rows_do_not_depend_on_the_row_count(dev, hidden, residual):
+    """Many rows run in more sweeps of fewer threads: the same bits as one row alone, at row lengths that fill the last 512 columns
+    of the sum or leave them part empty."""
+    rows = 600
+    rng = np.random.default_rng(hidden)
+    x16 = (rng.standard_normal((rows, hidden)) * 1.5).astype(np.float16)
+    gam = (rng.standard_normal(hidden) * 0.1).astype(np.float16)
+    res = (rng.standard_normal((rows, hidden)) * 2.0).astype(np.float16)
+    xb, gb, rb, yb = dev.put(x16), dev.put(gam), dev.put(res), dev.alloc(rows * hidden * 2)
+    qwhip.check(dev.lib.qwhip_rmsnorm(dev.stream.handle, xb.ptr, gb.ptr, rb.ptr if residual else None, rows, hidden, 1e-6, 1, yb.ptr))
+    got = yb.download(np.uint16, (rows, hidden))
+    rb.upload(res)
+    for r in (0, rows - 1):
+        at = r * hidden * 2
+        qwhip.check(dev.lib.qwhip_rmsnorm(dev.stream.handle, xb.ptr + at, gb.ptr, rb.ptr + at if residual else None, 1, hidden, 1e-6, 1, yb.ptr))
+        assert np.array_equal(yb.download(np.uint16, (hidden,)), got[r])
+    for b in (xb, gb, rb, yb):
+        b.free()
+
+
 def test_rmsnorm_refuses_the_geometries_the_reference_driver_refuses(dev):
     z = dev.put(np.zeros(4096, np.float16))
     st = dev.stream.handle
