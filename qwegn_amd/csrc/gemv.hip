@@ -982,11 +982,11 @@ bool qw_stream_gemv(hipStream_t st, const qwhip_weight_view* w, const void* x, u
                     void* y16, float* y32, uint32_t kw_override, hipError_t* err);
 
 // moe_col.hip
-bool qw_moe_gateup_col(hipStream_t st, const qwhip_weight_view* w, uint32_t experts, const void* x, uint32_t x_dtype, bool rotate,
+bool qw_moe_gateup_col(hipStream_t st, const qwhip_weight_view* w, int fmt, uint32_t experts, const void* x, uint32_t x_dtype, bool rotate,
                        bool rot_out, const int32_t* idx, uint32_t pairs, uint32_t top_k, void* act16, hipError_t* err,
                        const qw_act act, const float* logits = nullptr, int32_t* idx_out = nullptr, float* wts_out = nullptr, uint32_t norm_topk = 0,
                        float routed_scale = 1.0f, const int32_t* x_rows = nullptr, uint32_t reuse_tokens = 0);
-bool qw_moe_down_col(hipStream_t st, const qwhip_weight_view* w, uint32_t experts, const void* act16, const int32_t* idx,
+bool qw_moe_down_col(hipStream_t st, const qwhip_weight_view* w, int fmt, uint32_t experts, const void* act16, const int32_t* idx,
                      const float* wts, uint32_t t, uint32_t top_k, const float* shared, const float* shared_gate, void* out,
                      uint32_t out_dtype, hipError_t* err, uint32_t x_div = 1, const int32_t* labels = nullptr,
                      uint32_t num_groups = 0);
@@ -1301,7 +1301,7 @@ extern "C" qwhip_status qwhip_gemv_silu_pair(qwhip_stream_t s, const qwhip_weigh
     // decode path, as one dense bank with one "route" per activation row
     if (fmt == QW_FMT_M5 && ((flags >> 8) & 0xFu) != 2u) {
         hipError_t e = hipSuccess;
-        if (qw_moe_gateup_col(s->stream, w, 1, x, x_dtype, rotate, rotate_out && inter % 32 == 0, nullptr, m, 1, act16, &e, s->dev->act)) {
+        if (qw_moe_gateup_col(s->stream, w, fmt, 1, x, x_dtype, rotate, rotate_out && inter % 32 == 0, nullptr, m, 1, act16, &e, s->dev->act)) {
             QWHIP_TRY_HIP(e);
             return QWHIP_OK;
         }
@@ -1356,11 +1356,11 @@ extern "C" qwhip_status qwhip_moe_route_gateup_decode(qwhip_stream_t s, const qw
     if (experts == 0 || experts > 512) return qwhip_fail(QWHIP_E_BAD_SHAPE, "moe route: experts must be 1..512, got %u", experts);
     if (top_k > 16) return qwhip_fail(QWHIP_E_BAD_SHAPE, "moe route: top_k must be 1..16, got %u", top_k);
     const float scale = routed_scale > 0.0f ? routed_scale : 1.0f;
-    if (fmt == QW_FMT_M5 && w_gate_up->n % (2 * experts) == 0 && (uint64_t)t * top_k <= 65535u) {
+    if (w_gate_up->n % (2 * experts) == 0 && (uint64_t)t * top_k <= 65535u) {
         const uint32_t inter = w_gate_up->n / (2 * experts);
         const bool rotate = qwhip_view_rotated(w_gate_up) && !(flags & QWHIP_X_PREROTATED);
         hipError_t e = hipSuccess;
-        if (qw_moe_gateup_col(s->stream, w_gate_up, experts, x, x_dtype, rotate, qwhip_view_rotated(w_gate_up) && inter % 32 == 0, nullptr,
+        if (qw_moe_gateup_col(s->stream, w_gate_up, fmt, experts, x, x_dtype, rotate, qwhip_view_rotated(w_gate_up) && inter % 32 == 0, nullptr,
                               t * top_k, top_k, act16, &e, s->dev->act, logits, idx, wts, norm_topk ? 1u : 0u, scale, nullptr,
                               (flags & QWHIP_MOE_REUSE_EXPERTS) ? t : 0u)) {
             QWHIP_TRY_HIP(e);
@@ -1389,10 +1389,10 @@ static qwhip_status qw_moe_gateup_decode_impl(qwhip_stream_t s, const qwhip_weig
     if ((uint64_t)t * top_k > 65535u) return qwhip_fail(QWHIP_E_BAD_SHAPE, "decode path holds at most 65535 (token, route) pairs");
     const uint32_t inter = w_gate_up->n / (2 * experts);
     const bool rotate = qwhip_view_rotated(w_gate_up) && !(flags & QWHIP_X_PREROTATED);
-    // HQ4_G32_M5 banks take the column-stationary kernel (flags bits 8..11 = 2 keep the general one, for tests)
-    if (fmt == QW_FMT_M5 && ((flags >> 8) & 0xFu) != 2u) {
+    // the column-stationary kernel (flags bits 8..11 = 2 keep the general one, for tests)
+    if (((flags >> 8) & 0xFu) != 2u) {
         hipError_t e = hipSuccess;
-        if (qw_moe_gateup_col(s->stream, w_gate_up, experts, x, x_dtype, rotate, qwhip_view_rotated(w_gate_up) && inter % 32 == 0,
+        if (qw_moe_gateup_col(s->stream, w_gate_up, fmt, experts, x, x_dtype, rotate, qwhip_view_rotated(w_gate_up) && inter % 32 == 0,
                               idx, t * top_k, top_k, act16, &e, s->dev->act, nullptr, nullptr, nullptr, 0, 1.0f, x_rows,
                               (flags & QWHIP_MOE_REUSE_EXPERTS) ? t : 0u)) {
             QWHIP_TRY_HIP(e);
@@ -1464,9 +1464,9 @@ static qwhip_status qw_moe_down_decode_impl(qwhip_stream_t s, const qwhip_weight
     if (out_rows > 65535u) return qwhip_fail(QWHIP_E_BAD_SHAPE, "decode path holds at most 65535 output rows");
     if ((w_down->k * 2u) % 16u != 0) return qwhip_fail(QWHIP_E_BAD_SHAPE, "activation rows must be 16-byte multiples");
     const uint32_t hidden = w_down->n / experts;
-    if (fmt == QW_FMT_M5) {
+    {
         hipError_t e = hipSuccess;
-        if (qw_moe_down_col(s->stream, w_down, experts, act16, idx, wts, t, top_k, shared, shared_gate, out, out_dtype, &e, x_div, labels,
+        if (qw_moe_down_col(s->stream, w_down, fmt, experts, act16, idx, wts, t, top_k, shared, shared_gate, out, out_dtype, &e, x_div, labels,
                             num_groups)) {
             QWHIP_TRY_HIP(e);
             return QWHIP_OK;

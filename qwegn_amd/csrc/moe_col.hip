@@ -1,4 +1,4 @@
-// MoE decode (a handful of tokens) over HQ4_G32_M5 expert banks, column-stationary form.
+// MoE decode (a handful of tokens) over the expert banks of any container, column-stationary form.
 //
 // Both routed projections of the decode path (encodeMoEGateUpF32R1 / encodeMoEDownSharedCombineF32,
 // Sources/Operators/QWGEMM/QWGemmMoE.swift:120-199) read a few short rows from each routed expert: the launch is
@@ -8,7 +8,15 @@
 //     sum_i w_i x_i = s * (sum_i q_i x_i + 1024 S) + b * S,   S = sum_i x_i      (w = (1024 + q) s + b,
 // unpack_hq4_word8, Sources/QWMetal/include/qw_dequant.metalh:42-62).  A half-wavefront covers 32 block columns of a
 // row and reduces with DPP; the per-chunk partial sums meet in LDS and are added in chunk order.
-#include "qwhip_common.h"
+// The bit-stream containers differ in the slice alone (header and code words at two addresses, the operand order and
+// masks of qw_colx_slice.h).
+// Bound by the latency of one chain (route, expert id, first weight rows), not by bandwidth; all rows of a lane are asked for
+// at once.  Against the general kernels these containers took before (matrix tiles of 16 rows, a route launch in front):
+// 4 rows x top-8 of 256 experts, 4-bit affine, 2048 x 512: route 4.5 + gate|up 17 + down 9.4 us -> 13.8 (routing inside) + 5.5 us,
+// the layer 52 -> 40 us.
+#include <type_traits>
+
+#include "qw_colx_slice.h"
 #include "qwhip_route.h"
 
 namespace {
@@ -48,6 +56,46 @@ __device__ __forceinline__ float qmc_block_dot(const qw_hq4_block& b, const h2_t
     return __builtin_fmaf((float)hd[0], q, (float)hd[1] * S);
 }
 
+// A slice as the lane holds it, and what the two kernels do with it: HQ4_G32_M5 blocks in one piece, bit-stream slices by
+// their header and code offsets inside a row.
+template <int FMT>
+using qmc_slice = std::conditional_t<FMT == QW_FMT_M5, qw_hq4_block, qcx_slice<FMT>>;
+
+template <int FMT>
+__device__ __forceinline__ void qmc_offsets(uint32_t g, uint32_t gshift, uint32_t bb, uint32_t& hdr_off, uint32_t& pay_off) {
+    if constexpr (FMT == QW_FMT_M5) {
+        hdr_off = g * 20u;
+        pay_off = 0u;
+    } else {
+        hdr_off = (g >> gshift) * bb;
+        pay_off = hdr_off + 4u + (g & ((1u << gshift) - 1u)) * (4u * qcx_fmt<FMT>::PW);
+    }
+}
+
+template <int FMT>
+__device__ __forceinline__ void qmc_load(const uint8_t* bank, uint32_t row, uint32_t hdr_off, uint32_t pay_off, qmc_slice<FMT>& b) {
+    if constexpr (FMT == QW_FMT_M5) b = *(const qw_hq4_block*)(bank + (row + hdr_off));
+    else qcx_load<FMT>(bank, row + hdr_off, row + pay_off, b);
+}
+
+template <int FMT>
+__device__ __forceinline__ float qmc_operands_of(const h8_t* v, h2_t* xo) {
+    if constexpr (FMT == QW_FMT_M5) return qmc_operands(v, xo);
+    else return qcx_operands<FMT>(v, xo);
+}
+
+template <int FMT>
+__device__ __forceinline__ float qmc_dot(const qmc_slice<FMT>& b, const h2_t* xo, float S, float c1) {
+    if constexpr (FMT == QW_FMT_M5) {
+        return qmc_block_dot(b, xo, S, c1);
+    } else {
+        uint32_t ow[16];
+        qcx_mask<FMT>(b, ow);
+        const h2_t hd = __builtin_bit_cast(h2_t, b.hdr);
+        return __builtin_fmaf((float)hd[0], qcx_code_dot<FMT>(ow, xo, S), (float)hd[1] * S);
+    }
+}
+
 // ------------------------------------------------------------------------------------------------
 // gate|up: grid (ceil(I / 32), pairs).  A workgroup owns 32 gate rows and the 32 matching up rows of the pair's expert
 // (row slot s: up = s >> 5, n = n0 + (s & 31)); set j of SETS takes slots j * R .. j * R + R - 1, R = 64 / SETS.
@@ -63,7 +111,7 @@ __device__ __forceinline__ float qmc_block_dot(const qw_hq4_block& b, const h2_t
     X(const uint8_t*, bank) X(const void*, x) X(h1_t*, act) X(const int32_t*, idx) X(const float*, logits) X(uint32_t, top_k)    \
     X(uint32_t, nb) X(uint32_t, cpr) X(uint32_t, I) X(uint32_t, rotate) X(uint32_t, rot_out) X(uint64_t, expert_bytes)           \
     X(const int32_t*, x_rows) X(uint32_t, experts) X(int32_t*, idx_out) X(float*, wts_out) X(uint32_t, norm)                     \
-    X(float, routed_scale) X(qw_act, ga)
+    X(float, routed_scale) X(qw_act, ga) X(uint32_t, gshift) X(uint32_t, bb) X(uint32_t, row_bytes)
 QW_ARG_BLOCK(qmc_gu_params, QMC_GU_FIELDS)
 
 // MT > 1 (a verify window of 2 .. MT tokens, at most 64 pairs): an expert that several tokens route to is read once
@@ -73,10 +121,11 @@ QW_ARG_BLOCK(qmc_gu_params, QMC_GU_FIELDS)
 // first token's primary pair gathers the primary pairs of the later tokens and runs every row block against all of their
 // activation rows.  A token's second route to one expert runs alone.  Every pair's outputs come from the same operations
 // in the same order as in a launch of its own.  Dynamic LDS = MT * (nb * 80 + 64 * cpr * 4) bytes, blockDim.x <= 512.
-template <int XDT, int SETS, int JN = 0, int MT = 1>
+template <int FMT, int XDT, int SETS, int JN = 0, int MT = 1>
 struct qw_moe_gateup_col_kernel {
 static constexpr int kLaunchBound = MT > 1 ? 512 : 1024;
 static __device__ __forceinline__ void run(const qmc_gu_params& p) {
+    static_assert(MT == 1 || FMT == QW_FMT_M5, "shared experts are gathered for HQ4_G32_M5 banks");
     constexpr int R = 64 / SETS;
     constexpr int D = R < 8 ? R : 8;             // rows in flight per lane
     constexpr int XT = SETS == 2 ? 2 : 1;        // 16-group activation tiles per wave: ceil(2 cpr / (cpr * SETS / 2))
@@ -93,7 +142,9 @@ static __device__ __forceinline__ void run(const qmc_gu_params& p) {
     const bool gvalid = g0 < nb;
     const uint32_t g = gvalid ? g0 : nb - 1u;
     const uint32_t pair = blockIdx.y, n0 = blockIdx.x * 32u;
-    const uint32_t row_bytes = nb * 20u;
+    const uint32_t row_bytes = FMT == QW_FMT_M5 ? nb * 20u : p.row_bytes;
+    uint32_t hdr_off, pay_off;
+    qmc_offsets<FMT>(g, p.gshift, p.bb, hdr_off, pay_off);
 
     // memory order: the route's expert id, the token's activations, the first weight rows; the rotation runs under them
     int32_t e = 0;                               // no route list: one dense gate|up bank
@@ -203,11 +254,11 @@ static __device__ __forceinline__ void run(const qmc_gu_params& p) {
     auto row_off = [&](uint32_t r) {   // r-th row of this set
         const uint32_t s = set * R + min(r, (uint32_t)R - 1u);
         const uint32_t n = min(n0 + (s & 31u), I - 1u);
-        return ((s >> 5) * I + n) * row_bytes + g * 20u;
+        return ((s >> 5) * I + n) * row_bytes;
     };
-    qw_hq4_block buf[D];
+    qmc_slice<FMT> buf[D];
 #pragma unroll
-    for (int j = 0; j < D; ++j) buf[j] = *(const qw_hq4_block*)(bank + row_off(j));
+    for (int j = 0; j < D; ++j) qmc_load<FMT>(bank, row_off(j), hdr_off, pay_off, buf[j]);
     __builtin_amdgcn_sched_barrier(0);
     {
         h8_t h_lo, h_hi;
@@ -222,16 +273,16 @@ static __device__ __forceinline__ void run(const qmc_gu_params& p) {
     // The lane's blocks stay in registers while the slots pass over them: slot 0 consumes each block as it lands, the
     // further slots of a shared expert take their operands from LDS one after the other.
     h2_t xo[16];
-    const float S = qmc_operands(xs + g * 5, xo);
+    const float S = qmc_operands_of<FMT>(xs + g * 5, xo);
     const float c1 = 1024.0f * S;
 #pragma unroll
     for (int r0 = 0; r0 < R; r0 += D) {
-        qw_hq4_block blk[D];
+        qmc_slice<FMT> blk[D];
 #pragma unroll
         for (int j = 0; j < D; ++j) {
             blk[j] = buf[j];
-            if (r0 + D + j < R) buf[j] = *(const qw_hq4_block*)(bank + row_off(r0 + D + j));
-            float v = qmc_block_dot(blk[j], xo, S, c1);
+            if (r0 + D + j < R) qmc_load<FMT>(bank, row_off(r0 + D + j), hdr_off, pay_off, buf[j]);
+            float v = qmc_dot<FMT>(blk[j], xo, S, c1);
             v = gvalid ? v : 0.0f;
             v = qw_reduce32_dpp(v);
             if (lane == 31u) part[(set * R + r0 + j) * cpr + chunk] = v;
@@ -290,10 +341,11 @@ static __device__ __forceinline__ void run(const qmc_gu_params& p) {
 #define QMC_DN_FIELDS(X)                                                                                                     \
     X(const uint8_t*, bank) X(const h1_t*, act) X(const int32_t*, idx) X(const float*, wts) X(void*, out) X(uint32_t, top_k)     \
     X(uint32_t, nbI) X(uint32_t, nbv) X(uint32_t, cprv) X(uint32_t, H) X(uint32_t, sets) X(uint64_t, expert_bytes)               \
-    X(const float*, shared) X(const float*, shared_gate) X(const int32_t*, labels) X(uint32_t, num_groups) X(uint32_t, x_div)
+    X(const float*, shared) X(const float*, shared_gate) X(const int32_t*, labels) X(uint32_t, num_groups) X(uint32_t, x_div)    \
+    X(uint32_t, gshift) X(uint32_t, bb) X(uint32_t, row_bytes)
 QW_ARG_BLOCK(qmc_dn_params, QMC_DN_FIELDS)
 
-template <int ODT, int D, bool GRP = false>   // GRP: one output row per (token, latent group)
+template <int FMT, int ODT, int D, bool GRP = false>   // GRP: one output row per (token, latent group)
 struct qw_moe_down_col_kernel {
 static constexpr int kLaunchBound = 1024;
 static __device__ __forceinline__ void run(const qmc_dn_params& p) {
@@ -319,30 +371,32 @@ static __device__ __forceinline__ void run(const qmc_dn_params& p) {
         valid = valid && ((uint32_t)e & 0xFFFFu) < n_experts;       // an id past the labels is no route
         valid = valid && p.labels[valid ? ((uint32_t)e & 0xFFFFu) : 0u] == grp;
     }
-    const uint32_t row_bytes = p.nbI * 20u;
+    const uint32_t row_bytes = FMT == QW_FMT_M5 ? p.nbI * 20u : p.row_bytes;
+    uint32_t hdr_off, pay_off;
+    qmc_offsets<FMT>(b, p.gshift, p.bb, hdr_off, pay_off);
     // activations do not wait for the expert id; the weight rows follow as soon as it is known
     h8_t xr[4];
     const h8_t* xsrc = (const h8_t*)(p.act + ((uint64_t)(p.x_div > 1u ? pair / p.x_div : pair) * p.nbI + b) * 32u);
 #pragma unroll
     for (int j = 0; j < 4; ++j) xr[j] = xsrc[j];
-    const uint8_t* base = p.bank + (uint64_t)(valid ? ((uint32_t)e & 0xFFFFu) : 0u) * p.expert_bytes + b * 20u;
-    qw_hq4_block buf[D];
+    const uint8_t* base = p.bank + (uint64_t)(valid ? ((uint32_t)e & 0xFFFFu) : 0u) * p.expert_bytes;
+    qmc_slice<FMT> buf[D];
 #pragma unroll
     for (int j = 0; j < D; ++j) {
         const uint32_t n = min(n0 + set * D + j, H - 1u);
         if constexpr (GRP) {   // lanes of other groups' routes read nothing
-            buf[j] = qw_hq4_block{};
-            if (valid) buf[j] = *(const qw_hq4_block*)(base + (uint64_t)n * row_bytes);
+            buf[j] = qmc_slice<FMT>{};
+            if (valid) qmc_load<FMT>(base + (uint64_t)n * row_bytes, 0u, hdr_off, pay_off, buf[j]);
         } else {
-            buf[j] = *(const qw_hq4_block*)(base + (uint64_t)n * row_bytes);
+            qmc_load<FMT>(base + (uint64_t)n * row_bytes, 0u, hdr_off, pay_off, buf[j]);
         }
     }
     h2_t xo[16];
-    const float S = qmc_operands(xr, xo);
+    const float S = qmc_operands_of<FMT>(xr, xo);
     const float c1 = 1024.0f * S;
 #pragma unroll
     for (int j = 0; j < D; ++j) {
-        float r = qmc_block_dot(buf[j], xo, S, c1) * wk;
+        float r = qmc_dot<FMT>(buf[j], xo, S, c1) * wk;
         r = valid ? r : 0.0f;
         r = qw_reduce32_dpp(r);
         if (lane == 31u) part[(set * D + j) * cprv + chunk] = r;
@@ -365,21 +419,21 @@ static __device__ __forceinline__ void run(const qmc_dn_params& p) {
 
 }  // namespace
 
-// Routed gate|up projection with the SwiGLU (+ rotation) epilogue for a validated HQ4_G32_M5 bank; false when the shape
+// Routed gate|up projection with the SwiGLU (+ rotation) epilogue for a validated bank; false when the shape
 // is outside the kernel's envelope (the caller then takes the general kernel).
-bool qw_moe_gateup_col(hipStream_t st, const qwhip_weight_view* w, uint32_t experts, const void* x, uint32_t x_dtype, bool rotate,
+bool qw_moe_gateup_col(hipStream_t st, const qwhip_weight_view* w, int fmt, uint32_t experts, const void* x, uint32_t x_dtype, bool rotate,
                        bool rot_out, const int32_t* idx, uint32_t pairs, uint32_t top_k, void* act16, hipError_t* err,
                        const qw_act act, const float* logits, int32_t* idx_out, float* wts_out, uint32_t norm_topk, float routed_scale,
                        const int32_t* x_rows, uint32_t reuse_tokens) {
-    if (w->kind != QWHIP_KIND_HQ4_G32_M5) return false;
+    const uint64_t row_bytes = qwhip_view_row_bytes(w);
     const uint32_t inter = w->n / (2u * experts);
     const uint32_t nb = w->k / 32u, cpr = (nb + 31u) / 32u;
     if (cpr > 16u || pairs > 65535u) return false;
-    if ((uint64_t)2u * inter * nb * 20u >= (1ull << 32)) return false;   // 32-bit offsets inside an expert's sub-bank
+    if (2ull * inter * row_bytes >= (1ull << 32)) return false;   // 32-bit offsets inside an expert's sub-bank
     // experts shared by the 2..4 tokens of a verify window are read once when the window's route table fits one wavefront
     // and four activation rows fit the workgroup's LDS; the workgroup is then at most 512 threads wide
     constexpr uint32_t kReuseRows = 4;
-    const bool reuse = reuse_tokens >= 2u && reuse_tokens <= kReuseRows && (idx || logits) && top_k >= 1u && top_k <= 16u &&
+    const bool reuse = fmt == QW_FMT_M5 && reuse_tokens >= 2u && reuse_tokens <= kReuseRows && (idx || logits) && top_k >= 1u && top_k <= 16u &&
                        pairs == reuse_tokens * top_k && pairs <= 64u && cpr <= 8u &&
                        kReuseRows * ((size_t)nb * 80u + (size_t)64u * cpr * 4u) <= 60u * 1024u;
     const uint32_t sets = reuse ? (cpr <= 2u ? 8u : (cpr <= 4u ? 4u : 2u)) : (cpr <= 4u ? 8u : (cpr <= 8u ? 4u : 2u));
@@ -398,7 +452,10 @@ bool qw_moe_gateup_col(hipStream_t st, const qwhip_weight_view* w, uint32_t expe
     p.top_k = top_k;
     p.rotate = rotate ? 1u : 0u;
     p.rot_out = rot_out ? 1u : 0u;
-    p.expert_bytes = (uint64_t)2u * inter * nb * 20u;
+    p.expert_bytes = 2ull * inter * row_bytes;
+    p.gshift = (uint32_t)__builtin_ctz(w->group / 32u);
+    p.bb = (uint32_t)qwhip_view_block_bytes(w);
+    p.row_bytes = (uint32_t)row_bytes;
     p.logits = logits;
     p.idx_out = idx_out;
     p.wts_out = wts_out;
@@ -406,14 +463,20 @@ bool qw_moe_gateup_col(hipStream_t st, const qwhip_weight_view* w, uint32_t expe
     p.norm = norm_topk;
     p.routed_scale = routed_scale;
     const dim3 grid(qwhip_cdiv(inter, 32u), pairs), block(32u * cpr * sets);
-#define QMC_GU(DT, S, J, M) qw_launch_scalar<qw_moe_gateup_col_kernel<DT, S, J, M>>(grid, block, lds, st, p)
-#define QMC_GU_M(DT, J, M)                                                                                              \
-    do {                                                                                                                \
-        if (sets == 8u) QMC_GU(DT, 8, J, M); else if (sets == 4u) QMC_GU(DT, 4, J, M); else QMC_GU(DT, 2, J, M);        \
+#define QMC_GU(F, DT, S, J, M) qw_launch_scalar<qw_moe_gateup_col_kernel<F, DT, S, J, M>>(grid, block, lds, st, p)
+#define QMC_GU_M(F, DT, J, M)                                                                                                          \
+    do {                                                                                                                               \
+        if (sets == 8u) QMC_GU(F, DT, 8, J, M); else if (sets == 4u) QMC_GU(F, DT, 4, J, M); else QMC_GU(F, DT, 2, J, M);              \
     } while (0)
-#define QMC_GU_S(DT, J)                                                            \
-    do {                                                                           \
-        if (reuse) QMC_GU_M(DT, J, (int)kReuseRows); else QMC_GU_M(DT, J, 1);      \
+#define QMC_GU_S(DT, J)                                                                                                                \
+    do {                                                                                                                               \
+        if (reuse) QMC_GU_M(QW_FMT_M5, DT, J, (int)kReuseRows);                                                                        \
+        else if (fmt == QW_FMT_M5) QMC_GU_M(QW_FMT_M5, DT, J, 1);                                                                      \
+        else if (fmt == QW_FMT_B4) QMC_GU_M(QW_FMT_B4, DT, J, 1);                                                                      \
+        else if (fmt == QW_FMT_B8) QMC_GU_M(QW_FMT_B8, DT, J, 1);                                                                      \
+        else if (fmt == QW_FMT_B2) QMC_GU_M(QW_FMT_B2, DT, J, 1);                                                                      \
+        else if (fmt == QW_FMT_B3) QMC_GU_M(QW_FMT_B3, DT, J, 1);                                                                      \
+        else QMC_GU_M(QW_FMT_B6, DT, J, 1);                                                                                            \
     } while (0)
     if (!logits) {
         if (x_dtype == QWHIP_F16) QMC_GU_S(QWHIP_F16, 0); else QMC_GU_S(QWHIP_BF16, 0);
@@ -429,12 +492,12 @@ bool qw_moe_gateup_col(hipStream_t st, const qwhip_weight_view* w, uint32_t expe
     return true;
 }
 
-// Routed down projection + weighted combine (+ gated shared expert) for a validated HQ4_G32_M5 bank; false when the
+// Routed down projection + weighted combine (+ gated shared expert) for a validated bank; false when the
 // shape is outside the kernel's envelope.
-bool qw_moe_down_col(hipStream_t st, const qwhip_weight_view* w, uint32_t experts, const void* act16, const int32_t* idx,
+bool qw_moe_down_col(hipStream_t st, const qwhip_weight_view* w, int fmt, uint32_t experts, const void* act16, const int32_t* idx,
                      const float* wts, uint32_t t, uint32_t top_k, const float* shared, const float* shared_gate, void* out,
                      uint32_t out_dtype, hipError_t* err, uint32_t x_div, const int32_t* labels, uint32_t num_groups) {
-    if (w->kind != QWHIP_KIND_HQ4_G32_M5) return false;
+    const uint64_t row_bytes = qwhip_view_row_bytes(w);
     const uint32_t hidden = w->n / experts;
     const uint32_t nbI = w->k / 32u;
     const uint32_t nbv = top_k * nbI, cprv = (nbv + 31u) / 32u;
@@ -458,21 +521,34 @@ bool qw_moe_down_col(hipStream_t st, const qwhip_weight_view* w, uint32_t expert
     p.cprv = cprv;
     p.top_k = top_k;
     p.sets = sets;
-    p.expert_bytes = (uint64_t)hidden * nbI * 20u;
+    p.expert_bytes = (uint64_t)hidden * row_bytes;
+    p.gshift = (uint32_t)__builtin_ctz(w->group / 32u);
+    p.bb = (uint32_t)qwhip_view_block_bytes(w);
+    p.row_bytes = (uint32_t)row_bytes;
     p.x_div = x_div;
     p.labels = labels;
     p.num_groups = num_groups ? (num_groups | (experts << 8)) : 0u;
     const dim3 grid(qwhip_cdiv(hidden, sets * D), out_rows), block(32u * cprv * sets);
+#define QMC_DN_F(F, OD)                                                                                       \
+    do {                                                                                                      \
+        if (num_groups) qw_launch_scalar<qw_moe_down_col_kernel<F, OD, D, true>>(grid, block, 0, st, p);      \
+        else qw_launch_scalar<qw_moe_down_col_kernel<F, OD, D, false>>(grid, block, 0, st, p);                \
+    } while (0)
 #define QMC_DN(OD)                                                                                            \
     do {                                                                                                      \
-        if (num_groups) qw_launch_scalar<qw_moe_down_col_kernel<OD, D, true>>(grid, block, 0, st, p);         \
-        else qw_launch_scalar<qw_moe_down_col_kernel<OD, D, false>>(grid, block, 0, st, p);                   \
+        if (fmt == QW_FMT_M5) QMC_DN_F(QW_FMT_M5, OD);                                                        \
+        else if (fmt == QW_FMT_B4) QMC_DN_F(QW_FMT_B4, OD);                                                   \
+        else if (fmt == QW_FMT_B8) QMC_DN_F(QW_FMT_B8, OD);                                                   \
+        else if (fmt == QW_FMT_B2) QMC_DN_F(QW_FMT_B2, OD);                                                   \
+        else if (fmt == QW_FMT_B3) QMC_DN_F(QW_FMT_B3, OD);                                                   \
+        else QMC_DN_F(QW_FMT_B6, OD);                                                                         \
     } while (0)
     if (out_dtype == QWHIP_F32) QMC_DN(QWHIP_F32);
     else if (out_dtype == QWHIP_F16) QMC_DN(QWHIP_F16);
     else if (out_dtype == QWHIP_BF16) QMC_DN(QWHIP_BF16);
     else return false;
 #undef QMC_DN
+#undef QMC_DN_F
     *err = hipGetLastError();
     return true;
 }

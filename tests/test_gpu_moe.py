@@ -304,8 +304,8 @@ def test_grouped_gemm_refuses_expert_of_4gib(dev):
     assert lib.qwhip_moe_grouped_gemm_swiglu(st, C.byref(v), 1, xb.ptr, qwhip.F16, 0, None, *tiles, 1, out.ptr, 0) == qwhip.E_BAD_GEOMETRY
 
 
-# (format, gate_up kernel override): HQ4_G32_M5 runs the column-stationary kernels, override 2 keeps its gate_up on the
-# general kernel; the bit-stream container runs the general kernels for both projections.
+# (format, gate_up kernel override): every container runs the column-stationary kernels, override 2 keeps gate_up on the
+# general kernel.
 @pytest.mark.parametrize("fmt,gu_flags", [("hq4_g32_m5", 0), ("hq4_g32_m5", 2 << 8), ("hq4_g32", 0), ("hq3_g32", 0), ("hq6_g32", 0)])
 @pytest.mark.parametrize("experts,hidden,inter,k", [(16, 512, 192, 4), (8, 1280, 96, 3), (4, 2048, 768, 4)])
 @pytest.mark.parametrize("t", [1, 3, 8])
@@ -340,6 +340,31 @@ def test_moe_decode_chain_matches_oracle(dev, t, xdt, experts, hidden, inter, k,
     assert qo.normalized_error(got, ref) <= TOL
     a = act.download(np.float16, (t, k, inter))
     assert np.all(a[0, k - 1] == 0)
+
+
+# Group widths of several slices and every code width, at rows that end inside a 32-slice chunk and at one slice row per expert;
+# the general kernel's f16 weights and the column form's factored sum differ by the weights' f16 rounding, 2^-11 of a product.
+@pytest.mark.parametrize("fmt", ["aq4_g32", "hq4_g128", "hq8_g64", "aq8_g256", "aq2_g64", "aq6_g128", "hq3_g32"])
+@pytest.mark.parametrize("t,experts,hidden,inter,k", [(2, 4, 1280, 256, 3), (1, 3, 256, 512, 2), (3, 2, 4352, 256, 1)])
+def test_moe_decode_column_form_of_every_container(dev, fmt, t, experts, hidden, inter, k):
+    rot = H.FORMATS[fmt][4]
+    gu_blocks, gu16, dn_blocks, dn16 = _moe_banks(experts, hidden, inter, seed=33, fmt=fmt)
+    rng = np.random.default_rng(34)
+    x = rng.standard_normal((t, hidden)).astype(np.float16)
+    idx, wts = _route(dev, rng.standard_normal((t, experts)).astype(np.float32), k)
+    lib, st = dev.lib, dev.stream.handle
+    gub, dnb, xb, ib, wb = dev.put(gu_blocks), dev.put(dn_blocks), dev.put(x), dev.put(idx), dev.put(wts)
+    act, act2, out = dev.alloc(t * k * inter * 2), dev.alloc(t * k * inter * 2), dev.alloc(t * hidden * 4)
+    vgu = H.view_of(dev, gub, fmt, experts * 2 * inter, hidden)
+    vdn = H.view_of(dev, dnb, fmt, experts * hidden, inter)
+    for flags, a in ((0, act), (2 << 8, act2)):
+        qwhip.check(lib.qwhip_moe_gateup_decode(st, C.byref(vgu), experts, xb.ptr, qwhip.F16, flags, ib.ptr, t, k, a.ptr))
+    qwhip.check(lib.qwhip_moe_down_decode(st, C.byref(vdn), experts, act.ptr, ib.ptr, wb.ptr, t, k, None, None, out.ptr, qwhip.F32))
+    dev.stream.sync()
+    col, general = (a.download(np.float16, (t, k, inter)).astype(np.float64) for a in (act, act2))
+    assert qo.normalized_error(col, general) <= TOL
+    ref = qo.moe_forward_f64(H.x_in_basis(x, fmt), idx, wts, gu16, dn16, act_f16=True, rotate_act=rot)
+    assert qo.normalized_error(out.download(np.float32, (t, hidden)), ref) <= TOL
 
 
 @pytest.mark.parametrize("xdt", ["f16", "bf16"])
