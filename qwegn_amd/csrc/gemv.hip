@@ -1546,7 +1546,7 @@ bool qw_f32_gemm(hipStream_t st, const qwhip_weight_view* w, int fmt, uint32_t g
 
 // fp32 activations in the container's basis -> fp32 outputs with the scalar epilogues of the reference's f32 family
 // (QWGemm.encodeHQ4F32V4 / encodeHQ4F32BM, Sources/Operators/QWGEMM/QWGemmF32.swift:178-199,311-350): the rows go through
-// the column-stationary fp32 kernel four (long rows: two, one) at a time, as the reference's v4 door walks them; from 32
+// the fp32 matrix kernel of gemv_f32.hip eight at a time, where the reference's v4 door walks them four by four; from 32
 // rows on (where the reference switches to its batched kernels) the matrix-core form of gemm_f32.hip reads the bank once
 // per 64 rows.
 extern "C" qwhip_status qwhip_gemv_f32(qwhip_stream_t s, const qwhip_weight_view* w, const float* x, uint32_t m, uint32_t epi,

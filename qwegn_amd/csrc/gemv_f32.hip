@@ -2,23 +2,33 @@
 // (qwg_gemv_*_f32_v4 / qwg_gemm_*_f32_bm, Sources/QWMetal/include/qw_gemm_f32_common.metalh:15-19,152-225;
 // doors QWGemm.encodeHQ4F32V4 / encodeHQ4F32BM, Sources/Operators/QWGEMM/QWGemmF32.swift:178-199,311-350).
 //
-// Launch shape: the column-stationary persistent form of gemv_colx.hip - a fixed population of workgroups walks the bank
-// once (row slot s of workgroup w is bank row s * gridDim.x + w); a 32-lane half-wavefront (set, chunk) owns slice
-// columns 32 * chunk .. + 31 (a slice = 32 columns) of the rows set, set + sets, ...; a lane keeps its 32 fp32
-// activations of each of the MR activation rows in registers.
+// Launch shape: the 16-block form of gemv_quad.hip with the fp32 matrix instruction v_mfma_f32_4x4x1_16B_f32, which multiplies
+// 16 independent 4x1 by 1x4 blocks: block b (lanes 4b .. 4b + 3) is one 32-column slice, lane (b, i) converts the codes of
+// bank row i, lane (b, j) keeps the 32 fp32 activations of row j, and 32 instructions contract the slice for four bank rows
+// and four activation rows.  A fixed population of workgroups walks row quads; wave wv of a row set owns slice chunk
+// kr * wpr + wv (16 slices) in K range kr.  One and two rows take vector FMAs
+// in the same layout.  Bound by issue, not by the bank's bytes, from three rows on: the 4x4 instruction takes as long as the
+// four vector FMAs it stands for, but a lane holds 32 activations instead of 128 (those spilled into the accumulator file),
+// so three times the waves fit and eight rows share one pass over the bank.  Against a lane per slice with 32 activations
+// of every row: 17408 x 5120, HQ4_G32_M5, 1 / 2 / 3 / 8 rows 18.6 / 21.6 / 29.9 / 57.0 -> 16.1 / 19.3 / 25.9 / 39.1 us;
+// 5120 x 1024, 4-bit, 5.7 / 8.3 / 10.6 / 21.4 -> 4.6 / 5.4 / 6.2 / 10.0 us.
 //
 // Arithmetic: all in fp32.  The reference dequantises one weight as fma(float(code [+ 1024]), scale, bias) in fp32 and
 // feeds an fp32 FMA chain (qwg_unpack_hq4_word8_f32 / qwg_dot_hq4_block_f32_reg, qw_dequant_f32.metalh:10-58); here the
 // affine part is applied once per slice, sum_i w_i x_i = scale * sum_i code_i x_i + bias * sum_i x_i (HQ4_G32_M5: bias stands
 // for fma(1024, scale, bias), rounded once), codes converted to fp32 exactly.  Both differ from the exact sum only by
 // fp32 rounding.
+#include <atomic>
+#include <type_traits>
+
 #include "qwhip_common.h"
 
 namespace {
 
 #define QF_FIELDS(X)                                                                                                        \
     X(const uint8_t*, bank) X(const float*, x) X(float*, y) X(uint32_t, N) X(uint32_t, K) X(uint32_t, M) X(uint32_t, nsl)       \
-    X(uint32_t, cpr) X(uint32_t, sets) X(uint32_t, gshift) X(uint32_t, bb) X(uint32_t, row_bytes) X(uint32_t, epi) X(float, scale)
+    X(uint32_t, wpr) X(uint32_t, sets) X(uint32_t, nkr) X(uint32_t, gshift) X(uint32_t, bb) X(uint32_t, row_bytes)              \
+    X(uint32_t, epi) X(float, scale)
 QW_ARG_BLOCK(qf_params, QF_FIELDS)
 
 template <int FMT>
@@ -43,15 +53,11 @@ __device__ __forceinline__ uint32_t qf_code(const uint32_t* q, int e) {
     }
 }
 
-// Byte B of a word as a float, one instruction.
-template <int B>
-__device__ __forceinline__ float qf_ubyte(uint32_t v) {
-    float r;
-    if constexpr (B == 0) asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(r) : "v"(v));
-    else if constexpr (B == 1) asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(r) : "v"(v));
-    else if constexpr (B == 2) asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(r) : "v"(v));
-    else asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(r) : "v"(v));
-    return r;
+// The four bytes of a word as floats, one conversion each (the barrier keeps the compiler from folding the shift into the
+// mask in front, which would cost a second instruction a byte).
+__device__ __forceinline__ f4_t qf_bytes(uint32_t v) {
+    asm("" : "+v"(v));
+    return f4_t{(float)(v & 255u), (float)((v >> 8) & 255u), (float)((v >> 16) & 255u), (float)(v >> 24)};
 }
 
 __device__ __forceinline__ float qf_epilogue(float v, uint32_t epi, float scale) {
@@ -63,132 +69,239 @@ __device__ __forceinline__ float qf_epilogue(float v, uint32_t epi, float scale)
     return v;
 }
 
-// MR activation rows, three (MR = 4: four) slices in flight per lane.  blockDim.x = 32 * cpr * sets;
-// dynamic LDS = rows-per-workgroup * cpr * MR * 4 bytes.
-template <int FMT, int MR, int LB>
+#define QF_DPP(v, ctrl) __builtin_amdgcn_update_dpp(0, (int)(v), ctrl, 0xF, 0xF, true)
+#define QF_DPP_F32(v, ctrl) __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xF, 0xF, true))
+
+// MG groups of four activation rows on the matrix pipe, or (MV > 0, MG = 1) one or two rows by vector FMAs: every lane of a
+// block then holds the same activations and contracts its own bank row, product by product in the matrix form's order, so a
+// row's bits are the same from either.  D row quads in flight per lane.  blockDim.x = 64 * wpr * sets;
+// dynamic LDS = quad slots per workgroup * (4 wpr) * (4 MG) * 16 bytes.  A row's sums do not depend on M, MG or the grid.
+template <int FMT, int MG, int MV, int D, int LB>
 struct qw_gemv_f32_kernel {
 static constexpr int kLaunchBound = LB;
 static __device__ __forceinline__ void run(const qf_params& p) {
-    constexpr int D = MR == 4 ? 4 : 3, PW = qf_fmt<FMT>::PW;
-    extern __shared__ float qf_part[];   // [row slot][chunk][MR]
-    const uint32_t cpr = p.cpr, N = p.N, sets = p.sets;
+    static_assert(MV == 0 || MG == 1, "the vector form takes one or two rows");
+    constexpr int PW = qf_fmt<FMT>::PW, XR = MV ? MV : MG;   // XR: activation rows a lane holds
+    extern __shared__ f4_t qf_part[];   // [quad slot][wave of the set * 4 + 16-lane row][activation row] -> 4 bank rows
+    const uint32_t N = p.N, wpr = p.wpr, sets = p.sets;
     const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 31u, hw = tid >> 5;
-    const uint32_t set = hw / cpr, chunk = hw - set * cpr;
-    const uint32_t g0 = chunk * 32u + lane;
-    const bool gvalid = g0 < p.nsl;
-    const uint32_t g = gvalid ? g0 : p.nsl - 1u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), l64 = tid & 63u;
+    const uint32_t b = l64 >> 2, j = l64 & 3u;
+    const uint32_t set = wave / wpr, wv = wave - set * wpr;
     const uint32_t G = gridDim.x;
-    if (blockIdx.x >= N) return;
-    const uint32_t nrows = (N - blockIdx.x + G - 1u) / G;   // row slots of this workgroup
-    const uint32_t nmax = (nrows + sets - 1u) / sets;       // trip count, uniform over the workgroup
-    const uint32_t step = G * sets * p.row_bytes;
-    const uint32_t mine = nrows > set ? (nrows - set + sets - 1u) / sets : 0u;
-    uint32_t hdr_off, pay_off;
-    if constexpr (FMT == QW_FMT_M5) {
-        hdr_off = g * 20u;
-        pay_off = hdr_off + 4u;
-    } else {
-        hdr_off = (g >> p.gshift) * p.bb;
-        pay_off = hdr_off + 4u + (g & ((1u << p.gshift) - 1u)) * (4u * PW);
-    }
-    uint32_t off = ((mine ? set : 0u) * G + blockIdx.x) * p.row_bytes;
-    const uint32_t off_max = off + (mine ? mine - 1u : 0u) * step;   // loads past the set's last row re-read it
+    const uint32_t NQ = (N + 3u) >> 2;
+    if (blockIdx.x >= NQ) return;
+    const uint32_t nq = (NQ - blockIdx.x + G - 1u) / G;    // quad slots of this workgroup
+    const uint32_t nmax = (nq + sets - 1u) / sets;          // trip count, uniform over the workgroup
+    const uint32_t mine = nq > set ? (nq - set + sets - 1u) / sets : 0u;
+    const uint32_t W16 = wpr * 4u;
+    const uint32_t step = G * sets * 4u * p.row_bytes;      // bytes between consecutive quads of one set
 
-    // activations first; rows past M re-read row M - 1
-    f4_t xv[MR][8];
-#pragma unroll
-    for (int m = 0; m < MR; ++m) {
-        const float* xp = p.x + (uint64_t)min((uint32_t)m, p.M - 1u) * p.K + (uint64_t)g * 32u;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) xv[m][j] = *(const f4_t*)(xp + 4 * j);
-    }
-    __builtin_amdgcn_sched_barrier(0);
+    // this lane's bank row inside a quad is j (the A role); rows past the bank re-read its last row (never stored)
+    const uint32_t q_first = (mine ? set : 0u) * G + blockIdx.x;
+    const uint32_t off_first = min(4u * q_first + j, N - 1u) * p.row_bytes;
+    const uint32_t last_quad = q_first + (mine ? mine - 1u : 0u) * G * sets;
+    const uint32_t off_max = min(4u * last_quad + j, N - 1u) * p.row_bytes;   // loads past the set's last quad re-read it
+    // slice of this lane in K range kr (clamped into the row) and its byte offsets inside a bank row
+    auto slice_of = [&](uint32_t kr, uint32_t& hdr_off, uint32_t& pay_off) {
+        const uint32_t g = min((kr * wpr + wv) * 16u + b, p.nsl - 1u);
+        if constexpr (FMT == QW_FMT_M5) {
+            hdr_off = g * 20u;
+            pay_off = hdr_off + 4u;
+        } else {
+            hdr_off = (g >> p.gshift) * p.bb;
+            pay_off = hdr_off + 4u + (g & ((1u << p.gshift) - 1u)) * (4u * PW);
+        }
+        return g;
+    };
+    // the weight prefetch runs on across K ranges: after the last quad of a range comes the first one of the next
+    uint32_t i_kr = 0, i_left = nmax, i_off = off_first, i_hdr, i_pay;
+    slice_of(0, i_hdr, i_pay);
     uint32_t hdr[D], q[D][PW];
     auto issue = [&](int slot) {
-        const uint8_t* rp = p.bank + off;
-        hdr[slot] = *(const uint32_t*)(rp + hdr_off);
+        const uint32_t o_hdr = i_off + i_hdr, o_pay = i_off + i_pay;   // the bank is under 1 GiB
+        hdr[slot] = *(const uint32_t*)(p.bank + o_hdr);
 #pragma unroll
-        for (int j = 0; j < PW; ++j) q[slot][j] = *(const uint32_t*)(rp + pay_off + 4 * j);
-        off = min(off + step, off_max);
+        for (int t = 0; t < PW; ++t) q[slot][t] = *(const uint32_t*)(p.bank + o_pay + 4 * t);
+        i_off = min(i_off + step, off_max);
+        if (--i_left == 0u && i_kr + 1u < p.nkr) {   // uniform over the workgroup
+            ++i_kr;
+            slice_of(i_kr, i_hdr, i_pay);
+            i_off = off_first;
+            i_left = nmax;
+        }
     };
+    // activations of a K range, zero for slices past the row's end; rows past M re-read row M - 1
+    f4_t xv[XR][8];
+    auto load_x = [&](uint32_t kr) {
+        uint32_t ho, po;
+        const uint32_t g = slice_of(kr, ho, po);
 #pragma unroll
-    for (int j = 0; j < D; ++j) issue(j);
+        for (int mg = 0; mg < XR; ++mg) {
+            const float* xp = p.x + (uint64_t)min(MV ? (uint32_t)mg : 4u * mg + j, p.M - 1u) * p.K + (uint64_t)g * 32u;
+#pragma unroll
+            for (int t = 0; t < 8; ++t) xv[mg][t] = *(const f4_t*)(xp + 4 * t);
+        }
+    };
+    load_x(0);
     __builtin_amdgcn_sched_barrier(0);
-    float S[MR];
 #pragma unroll
-    for (int m = 0; m < MR; ++m) {
-        f4_t t = (xv[m][0] + xv[m][1]) + (xv[m][2] + xv[m][3]);
-        t += (xv[m][4] + xv[m][5]) + (xv[m][6] + xv[m][7]);
-        S[m] = (t[0] + t[1]) + (t[2] + t[3]);
-    }
+    for (int d = 0; d < D; ++d) issue(d);
+    __builtin_amdgcn_sched_barrier(0);
 
-    uint32_t rslot = set;
-    for (uint32_t ib = 0; ib < nmax; ib += D) {
+    for (uint32_t kr = 0; kr < p.nkr; ++kr) {
+        if (kr > 0u) load_x(kr);
+        const bool gvalid = (kr * wpr + wv) * 16u + b < p.nsl;
+        float S[XR];
 #pragma unroll
-        for (int j = 0; j < D; ++j) {
-            if (ib + j >= nmax) break;
-            uint32_t qq[PW];
+        for (int mg = 0; mg < XR; ++mg) {
+            if (!gvalid) {
 #pragma unroll
-            for (int t = 0; t < PW; ++t) qq[t] = q[j][t];
-            const h2_t hd = __builtin_bit_cast(h2_t, hdr[j]);
-            issue(j);
-            const float sc = (float)hd[0];
-            // HQ4_G32_M5: weight = (1024 + code) * scale + bias = code * scale + (1024 * scale + bias); the bracket is formed with
-            // one rounding, so the large terms cancel before they meet the activations
-            const float bi = FMT == QW_FMT_M5 ? __builtin_fmaf(1024.0f, sc, (float)hd[1]) : (float)hd[1];
-            float acc[MR][4];
+                for (int t = 0; t < 8; ++t) xv[mg][t] = f4_t{0.f, 0.f, 0.f, 0.f};
+            }
+            f4_t t4 = (xv[mg][0] + xv[mg][1]) + (xv[mg][2] + xv[mg][3]);
+            t4 += (xv[mg][4] + xv[mg][5]) + (xv[mg][6] + xv[mg][7]);
+            S[mg] = (t4[0] + t4[1]) + (t4[2] + t4[3]);
+        }
+        uint32_t qslot = set;   // quad slot being consumed
+        for (uint32_t ib = 0; ib < nmax; ib += D) {
 #pragma unroll
-            for (int m = 0; m < MR; ++m) acc[m][0] = acc[m][1] = acc[m][2] = acc[m][3] = 0.f;
-            auto contract = [&](float c, int e) {
+            for (int d = 0; d < D; ++d) {
+                if (ib + d >= nmax) break;
+                uint32_t qq[PW];
 #pragma unroll
-                for (int m = 0; m < MR; ++m) acc[m][e & 3] = __builtin_fmaf(c, xv[m][e >> 2][e & 3], acc[m][e & 3]);
-            };
-            if constexpr (FMT == QW_FMT_M5 || FMT == QW_FMT_B4 || FMT == QW_FMT_B8) {
-                // byte-aligned codes: one mask per four codes, then the byte-to-float conversions
+                for (int t = 0; t < PW; ++t) qq[t] = q[d][t];
+                const uint32_t hd0 = hdr[d];
+                issue(d);
+                using acc_t = std::conditional_t<MV != 0, float, f4_t>;
+                acc_t acc[XR][4];
 #pragma unroll
-                for (int w = 0; w < PW; ++w) {
-                    if constexpr (FMT == QW_FMT_B8) {
-                        contract(qf_ubyte<0>(qq[w]), 4 * w + 0);
-                        contract(qf_ubyte<1>(qq[w]), 4 * w + 1);
-                        contract(qf_ubyte<2>(qq[w]), 4 * w + 2);
-                        contract(qf_ubyte<3>(qq[w]), 4 * w + 3);
-                    } else {
+                for (int mg = 0; mg < XR; ++mg)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) acc[mg][c] = acc_t{};
+                auto contract = [&](float c, int e) {
+#pragma unroll
+                    for (int mg = 0; mg < XR; ++mg) {
+                        if constexpr (MV != 0) acc[mg][e & 3] = __builtin_fmaf(c, xv[mg][e >> 2][e & 3], acc[mg][e & 3]);
+                        else acc[mg][e & 3] = __builtin_amdgcn_mfma_f32_4x4x1f32(c, xv[mg][e >> 2][e & 3], acc[mg][e & 3], 0, 0, 0);
+                    }
+                };
+                if constexpr (FMT == QW_FMT_B8) {
+#pragma unroll
+                    for (int w = 0; w < 8; ++w) {
+                        const f4_t c = qf_bytes(qq[w]);
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) contract(c[t], 4 * w + t);
+                    }
+                } else if constexpr (FMT == QW_FMT_M5 || FMT == QW_FMT_B4) {
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
                         // HQ4_G32_M5: the nibble at bit 4 t + 16 u is element 2 t + u of the word; streams: nibble i is element i
-                        constexpr bool M5 = FMT == QW_FMT_M5;
-                        const uint32_t lo = qq[w] & 0x0F0F0F0Fu, hi = (qq[w] >> 4) & 0x0F0F0F0Fu;
-                        contract(qf_ubyte<0>(lo), 8 * w + 0);
-                        contract(qf_ubyte<1>(lo), 8 * w + (M5 ? 4 : 2));
-                        contract(qf_ubyte<2>(lo), 8 * w + (M5 ? 1 : 4));
-                        contract(qf_ubyte<3>(lo), 8 * w + (M5 ? 5 : 6));
-                        contract(qf_ubyte<0>(hi), 8 * w + (M5 ? 2 : 1));
-                        contract(qf_ubyte<1>(hi), 8 * w + (M5 ? 6 : 3));
-                        contract(qf_ubyte<2>(hi), 8 * w + (M5 ? 3 : 5));
-                        contract(qf_ubyte<3>(hi), 8 * w + (M5 ? 7 : 7));
+                        const f4_t lo = qf_bytes(qq[w] & 0x0F0F0F0Fu), hi = qf_bytes((qq[w] >> 4) & 0x0F0F0F0Fu);
+                        if constexpr (FMT == QW_FMT_M5) {
+                            const float c[8] = {lo[0], lo[2], hi[0], hi[2], lo[1], lo[3], hi[1], hi[3]};
+#pragma unroll
+                            for (int t = 0; t < 8; ++t) contract(c[t], 8 * w + t);
+                        } else {
+#pragma unroll
+                            for (int t = 0; t < 4; ++t) {
+                                contract(lo[t], 8 * w + 2 * t);
+                                contract(hi[t], 8 * w + 2 * t + 1);
+                            }
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 32; ++e) contract((float)qf_code<FMT>(qq, e), e);
+                }
+                float* const part = (float*)(qf_part + (size_t)(qslot * W16 + wv * 4u + (l64 >> 4)) * (4u * MG));
+                if constexpr (MV != 0) {
+                    const h2_t hd = __builtin_bit_cast(h2_t, hd0);
+                    const float sc = (float)hd[0];
+                    const float bi = FMT == QW_FMT_M5 ? __builtin_fmaf(1024.0f, sc, (float)hd[1]) : (float)hd[1];
+#pragma unroll
+                    for (int m = 0; m < MV; ++m) {
+                        const float qs = (acc[m][0] + acc[m][1]) + (acc[m][2] + acc[m][3]);
+                        float r = __builtin_fmaf(sc, qs, bi * S[m]);
+                        r += QF_DPP_F32(r, 0x114);
+                        r += QF_DPP_F32(r, 0x118);
+                        if ((l64 & 12u) == 12u && qslot < nq) {   // lane 12 + j: bank row j
+                            float* dst = part + 4 * m + j;
+                            if (kr == 0) *dst = r;
+                            else *dst += r;
+                        }
+                    }
+                } else {
+                    // the four headers of this block's rows
+                    float sc[4], bi[4];
+                    const uint32_t hq[4] = {(uint32_t)QF_DPP(hd0, 0x00), (uint32_t)QF_DPP(hd0, 0x55), (uint32_t)QF_DPP(hd0, 0xAA),
+                                            (uint32_t)QF_DPP(hd0, 0xFF)};   // quad_perm [i,i,i,i]
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const h2_t hd = __builtin_bit_cast(h2_t, hq[i]);
+                        sc[i] = (float)hd[0];
+                        // HQ4_G32_M5: weight = (1024 + code) * scale + bias = code * scale + (1024 * scale + bias); the bracket is
+                        // formed with one rounding, so the large terms cancel before they meet the activations
+                        bi[i] = FMT == QW_FMT_M5 ? __builtin_fmaf(1024.0f, sc[i], (float)hd[1]) : (float)hd[1];
+                    }
+#pragma unroll
+                    for (int mg = 0; mg < MG; ++mg) {
+                        f4_t v;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float qs = (acc[mg][0][i] + acc[mg][1][i]) + (acc[mg][2][i] + acc[mg][3][i]);
+                            float r = __builtin_fmaf(sc[i], qs, bi[i] * S[mg]);
+                            r += QF_DPP_F32(r, 0x114);   // row_shr:4
+                            r += QF_DPP_F32(r, 0x118);   // row_shr:8: lanes 12..15 of each 16-lane row hold its four blocks
+                            v[i] = r;
+                        }
+                        if ((l64 & 12u) == 12u && qslot < nq) {
+                            f4_t* dst = (f4_t*)part + 4u * mg + j;
+                            if (kr == 0) *dst = v;
+                            else *dst += v;
+                        }
                     }
                 }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 32; ++e) contract((float)qf_code<FMT>(qq, e), e);
+                qslot += sets;
             }
+        }
+        // the next range's first quads are already in flight, in the slots after the last one consumed: turn the window so
+        // that they sit in slots 0, 1, ... again
+        if (kr + 1u < p.nkr) {
+            for (uint32_t k = nmax % D; k > 0u; --k) {
+                const uint32_t h0 = hdr[0];
+                uint32_t q0[PW];
 #pragma unroll
-            for (int m = 0; m < MR; ++m) {
-                const float qs = (acc[m][0] + acc[m][1]) + (acc[m][2] + acc[m][3]);
-                float v = __builtin_fmaf(sc, qs, bi * S[m]);
-                v = gvalid ? v : 0.0f;
-                v = qw_reduce32_dpp(v);
-                if (lane == 31u && rslot < nrows) qf_part[(rslot * cpr + chunk) * MR + m] = v;
+                for (int t = 0; t < PW; ++t) q0[t] = q[0][t];
+#pragma unroll
+                for (int d = 0; d + 1 < D; ++d) {
+                    hdr[d] = hdr[d + 1];
+#pragma unroll
+                    for (int t = 0; t < PW; ++t) q[d][t] = q[d + 1][t];
+                }
+                hdr[D - 1] = h0;
+#pragma unroll
+                for (int t = 0; t < PW; ++t) q[D - 1][t] = q0[t];
             }
-            rslot += sets;
         }
     }
     __syncthreads();
-    // fixed-order sum of the chunk partials of each (row, activation row), then the scalar epilogue
-    for (uint32_t t = tid; t < nrows * p.M; t += blockDim.x) {
-        const uint32_t m = t / nrows, s = t - m * nrows;
+    // fixed-order sum of the partials of each (quad slot, activation row, bank row), then the scalar epilogue
+    for (uint32_t t = tid; t < nq * p.M * 4u; t += blockDim.x) {
+        const uint32_t i = t & 3u, sm = t >> 2;
+        const uint32_t s = sm / p.M, m = sm - s * p.M;
+        const uint32_t row = 4u * (s * G + blockIdx.x) + i;
+        if (row >= N) continue;
         float v = 0.f;
-        for (uint32_t c = 0; c < cpr; ++c) v += qf_part[(s * cpr + c) * MR + m];
-        p.y[(uint64_t)m * N + s * G + blockIdx.x] = qf_epilogue(v, p.epi, p.scale);
+        const float* part = (const float*)(qf_part + (size_t)s * W16 * (4u * MG) + m) + i;
+        for (uint32_t w = 0; w < W16; w += 4u) {   // W16 is a multiple of four: four partials on their way at a time
+            float t4[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) t4[u] = part[(size_t)(w + u) * (16u * MG)];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) v += t4[u];
+        }
+        p.y[(uint64_t)m * N + row] = qf_epilogue(v, p.epi, p.scale);
     }
 }
 };
@@ -205,11 +318,23 @@ __global__ __launch_bounds__(256) void qw_h32_f32_kernel(const float* x, float* 
     if (col < hidden) out[at] = v * 0.17677669529663689f;
 }
 
+template <int FMT, int MG, int MV>
+void qf_launch1(hipStream_t st, const qf_params& p, uint32_t wgs, uint32_t threads, size_t lds) {
+    using kern = qw_gemv_f32_kernel<FMT, MG, MV, FMT == QW_FMT_B8 || FMT == QW_FMT_B6 ? 2 : 3, 768>;
+    static std::atomic<bool> attr_done{false};   // per instantiation
+    if (!attr_done.load(std::memory_order_acquire)) {
+        (void)hipFuncSetAttribute(qw_scalar_kernel_ptr<kern>((const qf_params*)nullptr), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+        attr_done.store(true, std::memory_order_release);
+    }
+    qw_launch_scalar<kern>(dim3(wgs), dim3(threads), lds, st, p);
+}
+
 template <int FMT>
-void qf_launch(hipStream_t st, const qf_params& p, uint32_t mr, uint32_t wgs, uint32_t threads, size_t lds) {
-    if (mr == 1) qw_launch_scalar<qw_gemv_f32_kernel<FMT, 1, 1024>>(dim3(wgs), dim3(threads), lds, st, p);
-    else if (mr == 2) qw_launch_scalar<qw_gemv_f32_kernel<FMT, 2, 768>>(dim3(wgs), dim3(threads), lds, st, p);
-    else qw_launch_scalar<qw_gemv_f32_kernel<FMT, 4, 512>>(dim3(wgs), dim3(threads), lds, st, p);
+void qf_launch(hipStream_t st, const qf_params& p, uint32_t mg, uint32_t wgs, uint32_t threads, size_t lds) {
+    if (p.M == 1) qf_launch1<FMT, 1, 1>(st, p, wgs, threads, lds);
+    else if (p.M == 2) qf_launch1<FMT, 1, 2>(st, p, wgs, threads, lds);
+    else if (mg == 1) qf_launch1<FMT, 1, 0>(st, p, wgs, threads, lds);
+    else qf_launch1<FMT, 2, 0>(st, p, wgs, threads, lds);
 }
 
 }  // namespace
@@ -219,30 +344,29 @@ void qw_h32_f32_launch(hipStream_t st, const float* x, float* out, uint32_t rows
     hipLaunchKernelGGL(qw_h32_f32_kernel, dim3((padded + 255u) / 256u, rows), dim3(256), 0, st, x, out, hidden, padded);
 }
 
-// Largest number of activation rows (4, 2, 1 or 0 = none) the kernel takes per launch on this bank.
+// Largest number of activation rows (8, or 0 = none) the kernel takes per launch on this bank.
 uint32_t qw_f32_gemv_rows(const qwhip_weight_view* w, uint64_t row_bytes) {
-    if ((uint64_t)w->n * row_bytes >= (1ull << 30)) return 0;   // 32-bit offsets inside the bank, one row step past its end included
-    const uint32_t cpr = (w->k / 32u + 31u) / 32u;
-    if (32u * cpr <= 512u) return 4;
-    if (32u * cpr <= 768u) return 2;
-    return 32u * cpr <= 1024u ? 1u : 0u;
+    if ((uint64_t)w->n * row_bytes >= (1ull << 30)) return 0;   // 32-bit offsets inside the bank, one quad step past its end included
+    return w->k <= 32768u ? 8u : 0u;
 }
 
 // One launch over m <= qw_f32_gemv_rows() activation rows already in the container's basis; epilogue 3's rotation is the
 // caller's second launch.
 void qw_f32_gemv(hipStream_t st, const qwhip_weight_view* w, int fmt, uint32_t gshift, uint32_t bb, uint64_t row_bytes,
                  const float* x, uint32_t m, uint32_t epi, float scale, float* y) {
-    const uint32_t mr = m <= 1 ? 1u : (m <= 2 ? 2u : 4u);
-    const uint32_t nsl = w->k / 32u, cpr = (nsl + 31u) / 32u;
-    const uint32_t lb = mr == 1 ? 1024u : (mr == 2 ? 768u : 512u);
-    const uint32_t waves_cu = lb / 64u;
-    const uint32_t sets = min(lb / (32u * cpr), 8u);
-    const uint32_t threads = 32u * cpr * sets;
-    const uint32_t waves = (threads + 63u) / 64u;
-    uint32_t wgs = min(256u * max(1u, waves_cu / waves), max(1u, w->n / sets));
+    const uint32_t mr = (m + 3u) / 4u;   // groups of four activation rows
+    const uint32_t nsl = w->k / 32u, nch = (nsl + 15u) / 16u;
+    // at most 12 waves per row set (768 threads); longer rows take several K ranges
+    const uint32_t nkr = (nch + 11u) / 12u;
+    const uint32_t wpr = (nch + nkr - 1u) / nkr;
+    const uint32_t sets = max(1u, 12u / wpr);
+    const uint32_t threads = 64u * wpr * sets;
+    const uint32_t nquads = (w->n + 3u) / 4u;
+    uint32_t wgs = max(1u, min(256u * max(1u, 12u / (wpr * sets)), nquads / sets));
     // the partial sums of a workgroup's rows stay in LDS: more, smaller workgroups when the bank has very many rows
-    while ((size_t)qwhip_cdiv(w->n, wgs) * cpr * mr * 4u > 60u * 1024u) wgs *= 2u;
-    const size_t lds = (size_t)qwhip_cdiv(w->n, wgs) * cpr * mr * 4u;
+    auto lds_of = [&](uint32_t g) { return (size_t)qwhip_cdiv(nquads, g) * (wpr * 4u) * (4u * mr) * 16u; };
+    while (lds_of(wgs) > 96u * 1024u) wgs *= 2u;
+    const size_t lds = lds_of(wgs);
     qf_params p;
     p.bank = (const uint8_t*)w->blocks;
     p.x = x;
@@ -251,8 +375,9 @@ void qw_f32_gemv(hipStream_t st, const qwhip_weight_view* w, int fmt, uint32_t g
     p.K = w->k;
     p.M = m;
     p.nsl = nsl;
-    p.cpr = cpr;
+    p.wpr = wpr;
     p.sets = sets;
+    p.nkr = nkr;
     p.gshift = gshift;
     p.bb = bb;
     p.row_bytes = (uint32_t)row_bytes;

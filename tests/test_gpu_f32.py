@@ -146,6 +146,14 @@ def test_epilogue3_rows_together_equal_rows_alone(dev, fmt):
         assert qo.normalized_error(a, qo.gemv_f32(blocks, x[:rows], bits, group, is_m5, 3, 2.0)) <= TOL
 
 
+# two groups of four rows, one to three K ranges of 12 x 16 slices with a ragged last one, row quads cut by N, a bank of one quad
+@pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq4_g64", "hq8_g32", "hq6_g32"])
+@pytest.mark.parametrize("n,k,m", [(77, 6400, 5), (130, 12352, 8), (3, 32768, 2), (1025, 64, 9), (4100, 1088, 7)])
+def test_f32_row_quads_and_k_ranges(dev, fmt, n, k, m):
+    got, want, _ = _run(dev, fmt, n, k, m, 0, 1.0, seed=17)
+    assert qo.normalized_error(got, want) <= TOL
+
+
 def test_h32_f32_is_the_reference_butterfly(dev):
     """qwhip_h32_f32 against the golden-pinned fp32 FWHT (same butterfly order: equal bits), out of place and in place."""
     x = H.make_x(9, 1280, 5)
