@@ -480,8 +480,10 @@ bool qw_moe_gateup_col(hipStream_t st, const qwhip_weight_view* w, int fmt, uint
     } while (0)
     if (!logits) {
         if (x_dtype == QWHIP_F16) QMC_GU_S(QWHIP_F16, 0); else QMC_GU_S(QWHIP_BF16, 0);
-    } else if (experts <= 128u) {   // routing in the kernel: two experts per lane cover the usual 64 / 128, eight cover up to 512
+    } else if (experts <= 128u) {   // routing in the kernel: two experts per lane cover the usual 64 / 128, four 256, eight up to 512
         if (x_dtype == QWHIP_F16) QMC_GU_S(QWHIP_F16, 2); else QMC_GU_S(QWHIP_BF16, 2);
+    } else if (experts <= 256u) {
+        if (x_dtype == QWHIP_F16) QMC_GU_S(QWHIP_F16, 4); else QMC_GU_S(QWHIP_BF16, 4);
     } else {
         if (x_dtype == QWHIP_F16) QMC_GU_S(QWHIP_F16, 8); else QMC_GU_S(QWHIP_BF16, 8);
     }
