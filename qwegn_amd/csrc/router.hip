@@ -46,7 +46,7 @@ struct qw_raw8 {
 };
 
 // The upper halves of eight floats as bf16, and what they leave: taken one to three times this writes a float as a sum of
-// bf16 numbers without loss (8 significant bits each: 3 for fp32, 2 for the 11 bits of f16).  A non-finite value leaves NaN.
+// bf16 numbers without loss (8 significant bits each: 3 for fp32, 2 for the 11 bits of f16).  An infinite value leaves NaN.
 __device__ __forceinline__ qw_bf8_t qw_take_bf16(float* f) {
     u4_t w;
 #pragma unroll
@@ -159,7 +159,17 @@ __global__ __launch_bounds__(64 * W) void qw_router_mfma_kernel(const void* __re
         float v = 0.0f;
 #pragma unroll
         for (int w = 0; w < W; ++w) v += part[w][row * PITCH + col];
-        if (t0 + row < T && e0 + col < E) out[(uint64_t)(t0 + row) * E + e0 + col] = qw_f32_gemv_epilogue(v, epi, scale);
+        if (t0 + row >= T || e0 + col >= E) continue;
+        if constexpr (WDT == QWHIP_BF16 && XDT != QWHIP_BF16) {
+            // the bf16 terms of an infinity, and zero terms against an infinite weight, make NaN of what may be an infinity:
+            // such an output is summed again from the operands as they are
+            if (v != v) {
+                v = 0.0f;
+                for (uint32_t h = 0; h < H; ++h)
+                    v = fmaf(qw_load_f32<WDT>(wr, (uint64_t)(e0 + col) * H + h), qw_load_f32<XDT>(x, (uint64_t)(t0 + row) * H + h), v);
+            }
+        }
+        out[(uint64_t)(t0 + row) * E + e0 + col] = qw_f32_gemv_epilogue(v, epi, scale);
     }
 }
 

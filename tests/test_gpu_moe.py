@@ -304,6 +304,32 @@ def test_grouped_gemm_refuses_expert_of_4gib(dev):
     assert lib.qwhip_moe_grouped_gemm_swiglu(st, C.byref(v), 1, xb.ptr, qwhip.F16, 0, None, *tiles, 1, out.ptr, 0) == qwhip.E_BAD_GEOMETRY
 
 
+@pytest.mark.parametrize("xdt", ["f32", "f16"])
+@pytest.mark.parametrize("t,e,h", [(1, 20, 96), (3, 20, 96), (300, 1040, 96)])
+def test_router_gemm_keeps_infinities(dev, t, e, h, xdt):
+    """An infinite activation or weight gives the infinity, or the NaN, that the plain sum of the products gives."""
+    rng = np.random.default_rng(e)
+    x = rng.standard_normal((t, h)).astype(np.float16).astype(np.float32)
+    w = qo.round_bf16(rng.standard_normal((e, h)).astype(np.float32))
+    x[:, 5] = 1.0                                     # one bf16 term, the others zero
+    x[0, 7], x[t - 1, 40] = np.inf, -np.inf
+    w[2, 5], w[e - 1, 5], w[4, 7], w[6, 9] = np.inf, -np.inf, 0.0, np.nan
+    xb = dev.put(x if xdt == "f32" else x.astype(np.float16))
+    wb, lb = dev.put(qo.f32_to_bf16_bits(w)), dev.alloc(t * e * 4)
+    qwhip.check(dev.lib.qwhip_router_gemm(dev.stream.handle, xb.ptr, qwhip.F32 if xdt == "f32" else qwhip.F16, wb.ptr, qwhip.BF16, t, e, h, lb.ptr))
+    dev.stream.sync()
+    got = lb.download(np.float32, (t, e))
+    with np.errstate(invalid="ignore"):
+        want = np.stack([(w.astype(np.float64) * r).sum(axis=1) for r in x.astype(np.float64)])
+    odd = ~np.isfinite(want)
+    assert odd.any() and np.array_equal(got[odd], want[odd].astype(np.float32), equal_nan=True)
+    assert np.isfinite(got[~odd]).all()
+    if (~odd).any():
+        assert np.abs(got[~odd] - want[~odd]).max() <= 1e-4
+    for b in (xb, wb, lb):
+        b.free()
+
+
 # (format, gate_up kernel override): every container runs the column-stationary kernels, override 2 keeps gate_up on the
 # general kernel.
 @pytest.mark.parametrize("fmt,gu_flags", [("hq4_g32_m5", 0), ("hq4_g32_m5", 2 << 8), ("hq4_g32", 0), ("hq3_g32", 0), ("hq6_g32", 0)])
