@@ -2,7 +2,20 @@
 // packer (quant_hq4_blocks, Scripts/quantize/hq4.py:54-123; GPU twin qwg_quantize_bf16_to_hq4_g32_m5,
 // Sources/QWMetal/quant/qw_online_quant.metal:17-55).  One lane owns one 32-weight group; every
 // operation is a single IEEE fp32 operation in the packer's order (no contraction).
+//
+// Bound by vector instructions, not by memory: an IEEE division per weight was half of them.  The divisor is an f16 value that
+// 32 weights share, so its reciprocal is divided once and a weight takes three instructions (qw_div_exact) with the same
+// bits.  17408 x 5120 bf16 (234 MB): HQ4_G32_M5 57.1 -> 40.8 us (5.7 TB/s), 4-bit group 64 61.5 -> 48.3,
+// 8-bit group 32 62.5 -> 49.6; the 2- and 3-bit search, ten divisions a weight, 535 -> 253 and 546 -> 273 us.
 #include "qwhip_common.h"
+
+// d / s for s an f16 value > 0 and r = 1 / s correctly rounded: the product is within an ulp or so, its remainder is exact in
+// an fma, and the corrected quotient is the correctly rounded one (Markstein's final step; compared with the division over all
+// 2^23 mantissas of d times all 1024 of s: none differs).  d finite, no overflow; quotients under 2^-92 may be off by an ulp.
+__device__ __forceinline__ float qw_div_exact(float d, float s, float r) {
+    const float q = d * r;
+    return __builtin_fmaf(__builtin_fmaf(-q, s, d), r, q);
+}
 
 template <int DT>
 __global__ __launch_bounds__(256) void qw_quantize_hq4_kernel(const void* __restrict__ src, uint8_t* __restrict__ out,
@@ -21,7 +34,12 @@ __global__ __launch_bounds__(256) void qw_quantize_hq4_kernel(const void* __rest
     const h1_t bias16 = (h1_t)(-1032.0f * s);
     const float b = (float)bias16;
     uint32_t q[32];
-    if (s > 0.0f) {
+    if (s > 0.0f && amax < 1e30f) {
+        const float r = 1.0f / s;
+#pragma unroll
+        for (int i = 0; i < 32; ++i)   // the clamp to 0 leaves the conversion's truncation as the floor
+            q[i] = (uint32_t)fminf(fmaxf(qw_div_exact(v[i] - b, s, r) - 1023.5f, 0.0f), 15.0f);
+    } else if (s > 0.0f) {             // infinities divide as they are
 #pragma unroll
         for (int i = 0; i < 32; ++i) {
             const float t = floorf((v[i] - b) / s - 1023.5f);
@@ -70,27 +88,11 @@ extern "C" qwhip_status qwhip_quantize_hq4_g32(qwhip_stream_t s, const void* src
 // packer's array library (eight running sums over the group's elements in order, 128 elements at a time, combined pairwise),
 // which the lanes of a group reproduce by passing the running sums from lane to lane.
 // ------------------------------------------------------------------------------------------------
-template <int DT, int BITS>
-__global__ __launch_bounds__(256) void qw_quantize_blocks_kernel(const void* __restrict__ src, uint8_t* __restrict__ out,
-                                                                  uint64_t subgroups, uint32_t lshift, uint32_t rotate, uint32_t mse) {
-    const uint64_t sg0 = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    const bool live = sg0 < subgroups;                 // a quant group's lanes are live or idle together
-    const uint64_t sg = live ? sg0 : subgroups - 1u;
+// FAST: divisions as qw_div_exact, for groups whose scale and bias stay inside f16.
+template <int BITS, bool FAST>
+__device__ __forceinline__ void qw_quantize_blocks_group(const float* v, float mn, float mx, bool live, uint64_t sg, uint32_t lshift, uint32_t mse,
+                                                         uint8_t* __restrict__ out) {
     const uint32_t L = 1u << lshift, lig = threadIdx.x & (L - 1u);
-    float v[32];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) qw_load8_f32<DT>(src, sg * 32 + 8 * j, v + 8 * j);
-    if (rotate) qw_fwht32(v);
-    float mn = v[0], mx = v[0];
-#pragma unroll
-    for (int i = 1; i < 32; ++i) {
-        mn = fminf(mn, v[i]);
-        mx = fmaxf(mx, v[i]);
-    }
-    for (uint32_t off = 1; off < L; off <<= 1) {
-        mn = fminf(mn, __shfl_xor(mn, (int)off, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, (int)off, 64));
-    }
     constexpr float qmax = (float)((1 << BITS) - 1);
     h1_t sc16 = (h1_t)((mx - mn) / qmax), bi16 = (h1_t)mn;
     if (mse) {
@@ -103,11 +105,12 @@ __global__ __launch_bounds__(256) void qw_quantize_blocks_kernel(const void* __r
             const float c_min = mid - shrinks[c] * half_span, c_max = mid + shrinks[c] * half_span;
             const h1_t s16 = (h1_t)((c_max - c_min) / qmax), b16 = (h1_t)c_min;
             const float s = (float)s16, b = (float)b16;
-            const float safe = s > 0.0f ? s : 1.0f;
+            const float safe = s > 0.0f ? s : 1.0f, rs = 1.0f / safe;
             float dd[32];
 #pragma unroll
             for (int i = 0; i < 32; ++i) {
-                float q = fminf(fmaxf(__builtin_rintf((v[i] - b) / safe), 0.0f), qmax);
+                const float t = FAST ? qw_div_exact(v[i] - b, safe, rs) : (v[i] - b) / safe;
+                float q = fminf(fmaxf(__builtin_rintf(t), 0.0f), qmax);
                 q = s > 0.0f ? q : 0.0f;
                 const float d = v[i] - (q * s + b);
                 dd[i] = d * d;
@@ -142,13 +145,14 @@ __global__ __launch_bounds__(256) void qw_quantize_blocks_kernel(const void* __r
         }
     }
     const float s = (float)sc16, b = (float)bi16;
-    const float safe = s > 0.0f ? s : 1.0f;
+    const float safe = s > 0.0f ? s : 1.0f, rs = 1.0f / safe;
     uint32_t words[BITS];
 #pragma unroll
     for (int w = 0; w < BITS; ++w) words[w] = 0u;
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
-        float qf = fminf(fmaxf(__builtin_rintf((v[i] - b) / safe), 0.0f), qmax);
+        const float t = FAST ? qw_div_exact(v[i] - b, safe, rs) : (v[i] - b) / safe;
+        const float qf = fminf(fmaxf(__builtin_rintf(t), 0.0f), qmax);
         const uint32_t q = s > 0.0f ? (uint32_t)qf : 0u;
         constexpr int dummy = 0;
         (void)dummy;
@@ -162,6 +166,32 @@ __global__ __launch_bounds__(256) void qw_quantize_blocks_kernel(const void* __r
     if (lig == 0u) dst[0] = (uint32_t)__builtin_bit_cast(uint16_t, sc16) | ((uint32_t)__builtin_bit_cast(uint16_t, bi16) << 16);
 #pragma unroll
     for (int w = 0; w < BITS; ++w) dst[1 + lig * BITS + w] = words[w];
+}
+
+template <int DT, int BITS>
+__global__ __launch_bounds__(256) void qw_quantize_blocks_kernel(const void* __restrict__ src, uint8_t* __restrict__ out,
+                                                                  uint64_t subgroups, uint32_t lshift, uint32_t rotate, uint32_t mse) {
+    const uint64_t sg0 = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    const bool live = sg0 < subgroups;                 // a quant group's lanes are live or idle together
+    const uint64_t sg = live ? sg0 : subgroups - 1u;
+    const uint32_t L = 1u << lshift, lig = threadIdx.x & (L - 1u);
+    float v[32];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) qw_load8_f32<DT>(src, sg * 32 + 8 * j, v + 8 * j);
+    if (rotate) qw_fwht32(v);
+    float mn = v[0], mx = v[0];
+#pragma unroll
+    for (int i = 1; i < 32; ++i) {
+        mn = fminf(mn, v[i]);
+        mx = fmaxf(mx, v[i]);
+    }
+    for (uint32_t off = 1; off < L; off <<= 1) {
+        mn = fminf(mn, __shfl_xor(mn, (int)off, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, (int)off, 64));
+    }
+    // scales reach at most 2 x 60000 / 3
+    if (__all(fmaxf(fabsf(mn), fabsf(mx)) < 60000.0f)) qw_quantize_blocks_group<BITS, true>(v, mn, mx, live, sg, lshift, mse, out);
+    else qw_quantize_blocks_group<BITS, false>(v, mn, mx, live, sg, lshift, mse, out);
 }
 
 extern "C" qwhip_status qwhip_quantize_blocks(qwhip_stream_t s, const void* src, uint32_t src_dtype, uint32_t n, uint32_t k,

@@ -547,6 +547,39 @@ def test_device_block_quantizer_matches_the_oracle_on_seeded_weights(dev, fmt, s
         b.free()
 
 
+def _spread_weights(n, k, top):
+    """Rows of magnitudes from 1e-9 (scales that are f16 subnormals or zero) to `top`, full fp32 mantissas."""
+    w = np.random.default_rng(n).standard_normal((n, k)) * 0.3
+    w = np.clip(w, -1.0, 1.0)
+    w[:, 0] = 1.0
+    return (w * np.logspace(-9, np.log10(top), n)[:, None]).astype(np.float32)
+
+
+@pytest.mark.parametrize("fmt", ["hq4_g64", "aq8_g256", "aq6_g128", "aq2_g64", "hq3_g32"])
+def test_device_block_quantizer_over_all_magnitudes(dev, fmt):
+    """Division by the shared scale: same bytes as the oracle's division up to and past 60,000, where the kernel divides."""
+    kind, bits, group, is_m5, rotate = H.FORMATS[fmt]
+    w = _spread_weights(300, 768, 64000.0 if not rotate else 11000.0)   # rotated values reach sqrt(32) times a weight
+    want, _ = qo.quant_hq_blocks(w, bits=bits, group=group, is_m5=False, rotate=rotate)
+    src, out = dev.put(w), dev.alloc(want.nbytes)
+    qwhip.check(dev.lib.qwhip_quantize_blocks(dev.stream.handle, src.ptr, qwhip.F32, *w.shape, bits, group, int(rotate), 2, out.ptr))
+    assert np.array_equal(out.download(np.uint8, want.shape), want)
+    for b in (src, out):
+        b.free()
+
+
+@pytest.mark.parametrize("rotate", [0, 1])
+@pytest.mark.parametrize("top", [400.0, 1e6, 1e33])
+def test_hq4_quantizer_over_all_magnitudes(dev, top, rotate):
+    """The same for HQ4_G32_M5; the scale is capped, so weights past its reach take the end codes."""
+    w = _spread_weights(300, 768, top)
+    src, out = dev.put(w), dev.alloc(300 * 24 * 20)
+    qwhip.check(dev.lib.qwhip_quantize_hq4_g32(dev.stream.handle, src.ptr, qwhip.F32, 300, 768, rotate, out.ptr))
+    assert np.array_equal(out.download(np.uint8, (300, 24, 20)), qo.quant_hq4_blocks(w, rotate=bool(rotate)))
+    for b in (src, out):
+        b.free()
+
+
 def test_block_quantizer_rejects_bad_calls(dev):
     src, out = dev.put(np.zeros((4, 96), np.float32)), dev.alloc(4096)
     lib, st = dev.lib, dev.stream.handle
