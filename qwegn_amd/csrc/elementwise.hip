@@ -6,12 +6,19 @@
 // Four lanes a group (qw_fwht32_quad).
 template <int DT>
 __global__ __launch_bounds__(256) void qw_fwht32_kernel(const void* __restrict__ src, h1_t* __restrict__ dst, uint64_t octets) {
-    const uint64_t o = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (o >= octets) return;   // whole groups of four lanes leave together
-    float v[8];
-    qw_load8_f32<DT>(src, o * 8, v);
-    qw_fwht32_quad(v, threadIdx.x);
-    qw_store8_f16(dst + o * 8, v);
+    // whole groups of four lanes leave together
+    for (uint64_t o = (uint64_t)blockIdx.x * 256 + threadIdx.x; o < octets; o += (uint64_t)gridDim.x * 256) {
+        float v[8];
+        qw_load8_f32<DT>(src, o * 8, v);
+        qw_fwht32_quad(v, threadIdx.x);
+        qw_store8_f16(dst + o * 8, v);
+    }
+}
+
+// Workgroups of 256 lanes over `octets`: one step, up to 2^31 lanes (a launch holds under 2^32); past that the kernels take further steps.
+static dim3 qw_octet_grid(uint64_t octets) {
+    const uint64_t blocks = (octets + 255u) / 256u;
+    return dim3((unsigned)(blocks < (1u << 23) ? blocks : (1u << 23)));
 }
 
 extern "C" qwhip_status qwhip_fwht32(qwhip_stream_t s, const void* src, uint32_t src_dtype, void* dst_f16, uint64_t n) {
@@ -23,7 +30,7 @@ extern "C" qwhip_status qwhip_fwht32(qwhip_stream_t s, const void* src, uint32_t
     if (((uintptr_t)src & 15u) || ((uintptr_t)dst_f16 & 15u))
         return qwhip_fail(QWHIP_E_BAD_SHAPE, "fwht32: buffers must be 16-byte aligned");
     const uint64_t octets = n / 8;
-    const dim3 grid((unsigned)((octets + 255) / 256)), block(256);
+    const dim3 grid = qw_octet_grid(octets), block(256);
     switch (src_dtype) {
         case QWHIP_F16: hipLaunchKernelGGL(qw_fwht32_kernel<QWHIP_F16>, grid, block, 0, s->stream, src, (h1_t*)dst_f16, octets); break;
         case QWHIP_BF16: hipLaunchKernelGGL(qw_fwht32_kernel<QWHIP_BF16>, grid, block, 0, s->stream, src, (h1_t*)dst_f16, octets); break;
@@ -253,19 +260,19 @@ extern "C" qwhip_status qwhip_silu_mul_f32(qwhip_stream_t s, const float* gu, fl
 // helper: plain = f32(hi) + f32(lo), hi = f16(v), lo = f16(v - f32(hi)).
 __global__ __launch_bounds__(256) void qw_moe_bridge_kernel(const h1_t* __restrict__ x, float* __restrict__ rot32, float* __restrict__ plain32,
                                                              uint64_t octets) {
-    const uint64_t o = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (o >= octets) return;
-    float v[8];
-    qw_load8_f32<QWHIP_F16>(x, 8u * o, v);
-    if (rot32) qw_store8_f32(rot32 + 8u * o, v);
-    qw_fwht32_quad(v, threadIdx.x);
+    for (uint64_t o = (uint64_t)blockIdx.x * 256 + threadIdx.x; o < octets; o += (uint64_t)gridDim.x * 256) {
+        float v[8];
+        qw_load8_f32<QWHIP_F16>(x, 8u * o, v);
+        if (rot32) qw_store8_f32(rot32 + 8u * o, v);
+        qw_fwht32_quad(v, threadIdx.x);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const h1_t hi = (h1_t)v[i];
-        const h1_t lo = (h1_t)(v[i] - (float)hi);
-        v[i] = (float)hi + (float)lo;
+        for (int i = 0; i < 8; ++i) {
+            const h1_t hi = (h1_t)v[i];
+            const h1_t lo = (h1_t)(v[i] - (float)hi);
+            v[i] = (float)hi + (float)lo;
+        }
+        qw_store8_f32(plain32 + 8u * o, v);
     }
-    qw_store8_f32(plain32 + 8u * o, v);
 }
 
 extern "C" qwhip_status qwhip_moe_bridge_f16_to_f32(qwhip_stream_t s, const void* x_f16, float* x_rot32, float* x_plain32, uint32_t rows,
@@ -278,7 +285,7 @@ extern "C" qwhip_status qwhip_moe_bridge_f16_to_f32(qwhip_stream_t s, const void
     if (((uintptr_t)x_f16 | (uintptr_t)x_rot32 | (uintptr_t)x_plain32) & 15u)
         return qwhip_fail(QWHIP_E_BAD_SHAPE, "moe bridge needs 16-byte aligned buffers");
     const uint64_t octets = (uint64_t)rows * (hidden / 8u);
-    hipLaunchKernelGGL(qw_moe_bridge_kernel, dim3((unsigned)((octets + 255) / 256)), dim3(256), 0, s->stream, (const h1_t*)x_f16, x_rot32,
+    hipLaunchKernelGGL(qw_moe_bridge_kernel, qw_octet_grid(octets), dim3(256), 0, s->stream, (const h1_t*)x_f16, x_rot32,
                        x_plain32, octets);
     QWHIP_TRY_HIP(hipGetLastError());
     return QWHIP_OK;
