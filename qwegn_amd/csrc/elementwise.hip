@@ -474,60 +474,68 @@ extern "C" qwhip_status qwhip_embed_bf16_f32(qwhip_stream_t s, const void* table
 // Plus-one law: gamma is stored raw and applied as (1 + gamma) in fp32; sum of squares in fp32; the 32-point
 // transform in fp32 in the butterfly order of fwht32_f32_inplace (qw_dequant.metalh:442-478: strides 1, 2, 4 inside a
 // lane's 8 values, 8 and 16 across 4 lanes, times 1/sqrt(32)); one f16 rounding at the store.
-// One workgroup per row, a thread to 8 consecutive values (16-byte loads) in SW sweeps, the row in registers (16384 columns at
-// most); four neighbouring lanes hold one 32-group.  A few rows are their own latency: one sweep, gamma asked for together with
-// the row, before the sum's barrier (1 x 5120 in a chain of such launches 3.2 -> 2.4 us, 1 x 2048 2.2 -> 1.9; an empty launch 1.7).
-// Many rows want more bytes in flight per wave: two sweeps (4096 x 5120: 15.5 us, 19.1 in one sweep).  The sum does not depend
-// on that choice: 64 octets are summed across the lanes that hold them, those sums across 16 or 32 lanes, in one order for a row length.
+// The row stays in registers (16384 columns at most), 8 consecutive values a thread and step; four neighbouring lanes hold one
+// 32-group.  The squares are summed in one order for a row length, whatever the launch: 256 threads, thread t over the octets t,
+// t + 256, ..., then across each wave, then (w0 + w1) + (w2 + w3).  Every load of the row, gamma's too, is asked for before the
+// first sum (gamma behind the barrier: 1 x 5120 3.3 us, 1 x 2048 2.3, now 2.7 and 2.0; an empty launch 1.7).  Many rows are bound
+// by memory: 4096 x 5120 with a residual 25.6 us, 6.5 TB/s.
 // ------------------------------------------------------------------------------------------------
-template <bool RESIDUAL, int SW>
-__global__ __launch_bounds__(1024) void qw_rmsnorm_kernel(const h1_t* __restrict__ x, const h1_t* __restrict__ gamma,
-                                                          h1_t* __restrict__ residual, h1_t* __restrict__ y, uint32_t hidden,
-                                                          float eps, uint32_t rotate) {
-    __shared__ float wsum[32];
-    const uint32_t tid = threadIdx.x, nw = blockDim.x >> 6;
+__device__ __forceinline__ float qw_squares8(const h8_t& v, float acc) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float t = (float)v[i];
+        acc = fmaf(t, t, acc);
+    }
+    return acc;
+}
+
+// The row is spread over T threads in SW steps.  T = 256: a thread holds the octets it sums.  SPREAD (T > 256, a multiple of 64):
+// the octets pass through LDS (2 bytes a column) to the 256 threads that sum them.
+template <bool RESIDUAL, int SW, bool SPREAD>
+__global__ __launch_bounds__(SPREAD ? 1024 : 256) void qw_rmsnorm_kernel(const h1_t* __restrict__ x, const h1_t* __restrict__ gamma,
+                                                                         h1_t* __restrict__ residual, h1_t* __restrict__ y,
+                                                                         uint32_t hidden, float eps, uint32_t rotate) {
+    __shared__ float wsum[4];
+    extern __shared__ h8_t octets[];
+    const uint32_t tid = threadIdx.x, T = SPREAD ? blockDim.x : 256u;
     const uint64_t row = (uint64_t)blockIdx.x * hidden;
     h8_t v[SW], gv[SW], rv[SW];
 #pragma unroll
     for (int k = 0; k < SW; ++k) {
-        const uint32_t c = (k * blockDim.x + tid) * 8u;
+        const uint32_t c = (k * T + tid) * 8u;
         if (c < hidden) {
             v[k] = *(const h8_t*)(x + row + c);
             if constexpr (RESIDUAL) rv[k] = *(const h8_t*)(residual + row + c);
             gv[k] = *(const h8_t*)(gamma + c);
         }
     }
+    float acc = 0.f;
 #pragma unroll
     for (int k = 0; k < SW; ++k) {
-        const uint32_t c = (k * blockDim.x + tid) * 8u;
-        float acc = 0.f;
+        const uint32_t c = (k * T + tid) * 8u;
         if (c < hidden) {
             if constexpr (RESIDUAL) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) v[k][i] = (h1_t)((float)v[k][i] + (float)rv[k][i]);
                 *(h8_t*)(residual + row + c) = v[k];
             }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float t = (float)v[k][i];
-                acc = fmaf(t, t, acc);
-            }
+            if constexpr (SPREAD) octets[k * T + tid] = v[k];
+            else acc = qw_squares8(v[k], acc);
         }
+    }
+    if constexpr (SPREAD) __syncthreads();
+    if (tid < 256u) {
+        if constexpr (SPREAD)
+            for (uint32_t o = tid; o * 8u < hidden; o += 256u) acc = qw_squares8(octets[o], acc);
         acc = qw_reduce64(acc);
-        if ((tid & 63u) == 0u) wsum[k * nw + (tid >> 6)] = acc;
+        if ((tid & 63u) == 0u) wsum[tid >> 6] = acc;
     }
     __syncthreads();
-    const uint32_t unit = tid & (hidden > 8192u ? 31u : 15u);   // 512 columns each; a row of 16384 has 32
-    float total = unit * 512u < hidden ? wsum[unit] : 0.0f;
-    total += QW_DPP_F32(total, 0xB1);    // lane ^ 1
-    total += QW_DPP_F32(total, 0x4E);    // lane ^ 2
-    total += QW_DPP_F32(total, 0x141);   // row_half_mirror
-    total += QW_DPP_F32(total, 0x140);   // row_mirror
-    if (hidden > 8192u) total += __shfl_xor(total, 16, 64);
+    const float total = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
     const float rstd = 1.0f / sqrtf(total / (float)hidden + eps);
 #pragma unroll
     for (int k = 0; k < SW; ++k) {
-        const uint32_t c = (k * blockDim.x + tid) * 8u;
+        const uint32_t c = (k * T + tid) * 8u;
         if (c >= hidden) continue;   // whole quads of lanes leave together: hidden is a multiple of 32
         float f[8];
 #pragma unroll
@@ -549,16 +557,25 @@ extern "C" qwhip_status qwhip_rmsnorm(qwhip_stream_t s, const void* x_f16, const
     if (hidden > 16384u) return qwhip_fail(QWHIP_E_BAD_GEOMETRY, "the norm kernel holds rows of at most 16384 columns, got %u", hidden);
     if (((uintptr_t)x_f16 | (uintptr_t)gamma_f16 | (uintptr_t)y_f16 | (uintptr_t)residual_f16) & 15u)
         return qwhip_fail(QWHIP_E_BAD_SHAPE, "the norm kernel needs 16-byte aligned rows");
-    const uint32_t sweeps = (hidden > 8192u ? 2u : 1u) * (rows > 512u && hidden > 4096u ? 2u : 1u);
-    const dim3 grid(rows), block((hidden / 8u / sweeps + 63u) & ~63u);
-#define QW_NORM(R, SW)                                                                                                                \
-    hipLaunchKernelGGL((qw_rmsnorm_kernel<R, SW>), grid, block, 0, s->stream, (const h1_t*)x_f16, (const h1_t*)gamma_f16,             \
-                       (h1_t*)residual_f16, (h1_t*)y_f16, hidden, eps, rotate ? 1u : 0u)
-    if (residual_f16) {
-        if (sweeps == 1u) QW_NORM(true, 1); else if (sweeps == 2u) QW_NORM(true, 2); else QW_NORM(true, 4);
-    } else {
-        if (sweeps == 1u) QW_NORM(false, 1); else if (sweeps == 2u) QW_NORM(false, 2); else QW_NORM(false, 4);
-    }
+    // up to a row per compute unit the row is its own latency and spreads over up to 1024 threads (with a residual, 1 x 5120 2.7 us
+    // against 3.1 in 256 threads, 128 x 5120 3.2 / 3.6, 1 x 16384 4.8 / 5.8); past that 256 threads keep more rows in flight
+    // (333 x 5120 4.7 us spread / 4.6, 512 x 5120 5.3 / 5.1, 512 x 6144 5.7 / 5.6); both give the same bits
+    const bool spread = rows <= 256u && hidden > 2048u;
+    const uint32_t steps = spread ? (hidden > 8192u ? 2u : 1u) : qwhip_cdiv(hidden, 2048u);
+    const uint32_t threads = spread ? (hidden / 8u / steps + 63u) & ~63u : 256u;
+#define QW_NORM(R, SW, SP)                                                                                                            \
+    hipLaunchKernelGGL((qw_rmsnorm_kernel<R, SW, SP>), dim3(rows), dim3(threads), SP ? hidden * 2u : 0u, s->stream,                   \
+                       (const h1_t*)x_f16, (const h1_t*)gamma_f16, (h1_t*)residual_f16, (h1_t*)y_f16, hidden, eps, rotate ? 1u : 0u)
+#define QW_NORM_SW(R)                                                                                                                 \
+    do {                                                                                                                              \
+        if (spread) {                                                                                                                 \
+            if (steps == 1u) QW_NORM(R, 1, true); else QW_NORM(R, 2, true);                                                           \
+        } else if (steps == 1u) QW_NORM(R, 1, false); else if (steps == 2u) QW_NORM(R, 2, false); else if (steps == 3u) QW_NORM(R, 3, false); \
+        else if (steps == 4u) QW_NORM(R, 4, false); else QW_NORM(R, 8, false);                                                        \
+    } while (0)
+    if (residual_f16) QW_NORM_SW(true);
+    else QW_NORM_SW(false);
+#undef QW_NORM_SW
 #undef QW_NORM
     QWHIP_TRY_HIP(hipGetLastError());
     return QWHIP_OK;

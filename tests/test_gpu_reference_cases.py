@@ -304,6 +304,50 @@ def test_rmsnorm_rows_do_not_depend_on_the_row_count(dev, hidden, residual):
         b.free()
 
 
+def _rmsnorm_in_order(x16, gam, eps, rotate):
+    """The norm with every fp32 operation in its place: a thread's squares in sweep order (f16 squares are exact in fp32, so a sum
+    is the fused sum), the wave's sums 32, 16, .. 1 lanes apart, then (w0 + w1) + (w2 + w3)."""
+    f32 = np.float32
+    rows, hidden = x16.shape
+    x = x16.astype(f32)
+    sweeps = -(-hidden // 2048)
+    p = np.zeros((rows, sweeps * 2048), f32)
+    p[:, :hidden] = x
+    p = p.reshape(rows, sweeps, 4, 64, 8)
+    acc = np.zeros((rows, 4, 64), f32)
+    for k in range(sweeps):
+        for i in range(8):
+            acc = acc + p[:, k, :, :, i] * p[:, k, :, :, i]
+    for off in (32, 16, 8, 4, 2, 1):
+        acc = acc + acc[:, :, np.arange(64) ^ off]
+    w = acc[:, :, 0]
+    total = (w[:, 0] + w[:, 1]) + (w[:, 2] + w[:, 3])
+    rstd = f32(1.0) / np.sqrt(total / f32(hidden) + f32(eps))
+    f = (x * rstd[:, None]) * (gam.astype(f32) + f32(1.0))
+    return (qo.fwht32_ortho(f) if rotate else f).astype(np.float16)
+
+
+@pytest.mark.parametrize("hidden", [256, 2048, 2304, 4096, 5120, 8192, 16384])
+@pytest.mark.parametrize("residual", [0, 1])
+@pytest.mark.parametrize("rotate", [1, 0])
+@pytest.mark.parametrize("rows", [3, 256, 257])
+def test_rmsnorm_sums_in_its_documented_order(dev, rows, hidden, residual, rotate):
+    """Bit for bit, on both sides of the row count that changes the launch, rows of one to eight sweeps, full and part empty."""
+    rng = np.random.default_rng(hidden + residual + rows)
+    x16 = (rng.standard_normal((rows, hidden)) * 1.5).astype(np.float16)
+    gam = (rng.standard_normal(hidden) * 0.1).astype(np.float16)
+    res = (rng.standard_normal((rows, hidden)) * 2.0).astype(np.float16)
+    xb, gb, rb, yb = dev.put(x16), dev.put(gam), dev.put(res), dev.alloc(rows * hidden * 2)
+    qwhip.check(dev.lib.qwhip_rmsnorm(dev.stream.handle, xb.ptr, gb.ptr, rb.ptr if residual else None, rows, hidden, 1e-6, rotate, yb.ptr))
+    got = yb.download(np.float16, (rows, hidden))
+    row = (x16.astype(np.float32) + res.astype(np.float32)).astype(np.float16) if residual else x16
+    want = _rmsnorm_in_order(row, gam, 1e-6, rotate)
+    # equal values: a zero's sign may differ where the transform cancels
+    assert np.array_equal(got + np.float16(0), want + np.float16(0))
+    for b in (xb, gb, rb, yb):
+        b.free()
+
+
 def test_rmsnorm_refuses_the_geometries_the_reference_driver_refuses(dev):
     z = dev.put(np.zeros(4096, np.float16))
     st = dev.stream.handle
