@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "qw_colx_slice.h"
+#include "qw_slice.h"
 #include "qwhip_route.h"
 
 namespace {
@@ -94,6 +95,28 @@ __device__ __forceinline__ float qmc_dot(const qmc_slice<FMT>& b, const h2_t* xo
         const h2_t hd = __builtin_bit_cast(h2_t, b.hdr);
         return __builtin_fmaf((float)hd[0], qcx_code_dot<FMT>(ow, xo, S), (float)hd[1] * S);
     }
+}
+
+// The same slice weight by weight, for a slice with an infinite activation: s sum(q x) + b sum(x) makes NaN of it (0 x inf, inf - inf)
+// where its products with the weights are infinities.  A weight is code s + b in fp32; it is zero only where its f16 rounding is, since
+// scales and biases are multiples of 2^-24.
+template <int FMT>
+__device__ __forceinline__ float qmc_plain_dot(const qmc_slice<FMT>& b, const h8_t* x) {
+    static_assert(QG_FMT_B4 == QW_FMT_B4 && QG_FMT_B8 == QW_FMT_B8 && QG_FMT_B2 == QW_FMT_B2 && QG_FMT_B3 == QW_FMT_B3 && QG_FMT_B6 == QW_FMT_B6, "one numbering");
+    qg_slice<FMT> sl;
+    sl.hdr = b.hdr;
+#pragma unroll
+    for (int j = 0; j < qg_slice_words<FMT>(); ++j) sl.q[j] = b.q[j];
+    const h2_t hd = __builtin_bit_cast(h2_t, b.hdr), one = {(h1_t)1.0f, (h1_t)1.0f}, zero = {(h1_t)0.0f, (h1_t)0.0f};
+    const float s = (float)hd[0], bias = (float)hd[1];
+    float acc = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const h8_t c = qg_dequant_chunk<FMT>(sl, j, one, zero, 0u), xj = x[j];   // the codes
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc = __builtin_fmaf(__builtin_fmaf((float)c[i], s, bias), (float)xj[i], acc);
+    }
+    return acc;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -243,7 +266,7 @@ static __device__ __forceinline__ void run(const qmc_gu_params& p) {
             }
         }
         __syncthreads();
-        e = e_route;
+        e = __builtin_amdgcn_readfirstlane(e_route);
     }
     h1_t* act = p.act + (uint64_t)pair * I;
     if (e < 0) {   // no expert: the pair contributes nothing (uniform over the workgroup)
@@ -275,6 +298,9 @@ static __device__ __forceinline__ void run(const qmc_gu_params& p) {
     h2_t xo[16];
     const float S = qmc_operands_of<FMT>(xs + g * 5, xo);
     const float c1 = 1024.0f * S;
+    // an infinite or NaN activation under this wave: every sum of the pair comes out infinite or NaN, and the plain form says which
+    unsigned long long odd = 0ull;
+    if constexpr (FMT != QW_FMT_M5) odd = __ballot(!qw_finite(S));
 #pragma unroll
     for (int r0 = 0; r0 < R; r0 += D) {
         qmc_slice<FMT> blk[D];
@@ -303,6 +329,23 @@ static __device__ __forceinline__ void run(const qmc_gu_params& p) {
                     v = qw_reduce32_dpp(v);
                     if (lane == 31u) part[(m * 64u + set * R + r0 + j) * cpr + chunk] = v;
                 }
+            }
+        }
+    }
+    if constexpr (FMT != QW_FMT_M5) {
+        if (__builtin_expect(odd != 0ull, 0)) {
+            uint32_t td = tid;   // the lane's places anew: kept from above they would cost the whole kernel registers
+            asm volatile("" : "+v"(td));
+            const uint32_t hs = (td >> 5) / cpr, hc = (td >> 5) - hs * cpr, gc = hc * 32u + (td & 31u), gg = min(gc, nb - 1u);
+            uint32_t ho, po;
+            qmc_offsets<FMT>(gg, p.gshift, p.bb, ho, po);
+#pragma unroll 1
+            for (uint32_t r = 0; r < (uint32_t)R; ++r) {
+                const uint32_t s = hs * R + r;
+                qmc_slice<FMT> b;
+                qmc_load<FMT>(bank, ((s >> 5) * I + min(n0 + (s & 31u), I - 1u)) * row_bytes, ho, po, b);
+                const float v = qw_reduce32_dpp(gc < nb ? qmc_plain_dot<FMT>(b, xs + gg * 5) : 0.0f);
+                if ((td & 31u) == 31u) part[s * cpr + hc] = v;
             }
         }
     }
@@ -394,12 +437,40 @@ static __device__ __forceinline__ void run(const qmc_dn_params& p) {
     h2_t xo[16];
     const float S = qmc_operands_of<FMT>(xr, xo);
     const float c1 = 1024.0f * S;
+    unsigned long long odd = 0ull;   // as in the gate|up kernel
+    if constexpr (FMT != QW_FMT_M5) odd = __ballot(valid && !qw_finite(S));
 #pragma unroll
     for (int j = 0; j < D; ++j) {
         float r = qmc_dot<FMT>(buf[j], xo, S, c1) * wk;
         r = valid ? r : 0.0f;
         r = qw_reduce32_dpp(r);
         if (lane == 31u) part[(set * D + j) * cprv + chunk] = r;
+    }
+    if constexpr (FMT != QW_FMT_M5) {
+        if (__builtin_expect(odd != 0ull, 0)) {
+            uint32_t td = tid;
+            asm volatile("" : "+v"(td));
+            const uint32_t hs = (td >> 5) / cprv, hc = (td >> 5) - hs * cprv, vv = hc * 32u + (td & 31u);
+            const uint32_t kk = min(vv, p.nbv - 1u) / p.nbI, bb = min(vv, p.nbv - 1u) - kk * p.nbI, pr = src * p.top_k + kk;
+            const int32_t ee = p.idx[pr];
+            bool live = vv < p.nbv && ee >= 0;
+            if constexpr (GRP) {
+                live = live && ((uint32_t)ee & 0xFFFFu) < n_experts;
+                live = live && p.labels[live ? ((uint32_t)ee & 0xFFFFu) : 0u] == grp;
+            }
+            const uint8_t* eb = p.bank + (uint64_t)(live ? ((uint32_t)ee & 0xFFFFu) : 0u) * p.expert_bytes;
+            const h8_t* xp = (const h8_t*)(p.act + ((uint64_t)(p.x_div > 1u ? pr / p.x_div : pr) * p.nbI + bb) * 32u);
+            uint32_t ho, po;
+            qmc_offsets<FMT>(bb, p.gshift, p.bb, ho, po);
+#pragma unroll 1
+            for (uint32_t j = 0; j < (uint32_t)D; ++j) {
+                const uint32_t s = hs * D + j;
+                qmc_slice<FMT> sl;
+                qmc_load<FMT>(eb + (uint64_t)min(n0 + s, H - 1u) * row_bytes, 0u, ho, po, sl);
+                const float r = qw_reduce32_dpp(live ? qmc_plain_dot<FMT>(sl, xp) * (p.wts ? p.wts[pr] : 1.0f) : 0.0f);
+                if ((td & 31u) == 31u) part[s * cprv + hc] = r;
+            }
+        }
     }
     __syncthreads();
     if (tid < p.sets * D) {

@@ -393,6 +393,44 @@ def test_moe_decode_column_form_of_every_container(dev, fmt, t, experts, hidden,
     assert qo.normalized_error(out.download(np.float32, (t, hidden)), ref) <= TOL
 
 
+@pytest.mark.parametrize("fmt", ["aq4_g32", "hq4_g128", "hq8_g64", "aq8_g256", "aq2_g64", "aq6_g128", "hq3_g32"])
+@pytest.mark.parametrize("pre", [0, qwhip.X_PREROTATED])
+def test_routed_projections_keep_infinities(dev, fmt, pre):
+    """An infinite activation gives the infinities (or, against a weight of zero or another infinity, the NaN) of its products with the
+    f16 weights: gate|up as the general kernel gives them, down as the plain sum; rows without one are left alone."""
+    rot = H.FORMATS[fmt][4]
+    t, experts, hidden, inter, k = 4, 3, 1280, 256, 2
+    gu_blocks, _, dn_blocks, dn16 = _moe_banks(experts, hidden, inter, seed=61, fmt=fmt)
+    rng = np.random.default_rng(62)
+    x = rng.standard_normal((t, hidden)).astype(np.float16)
+    x[0, 5], x[1, 1100], x[2, 40], x[2, 700] = np.inf, -np.inf, np.inf, -np.inf
+    idx, wts = np.array([[0, 1], [2, 0], [1, 2], [0, 2]], np.int32), (rng.random((t, k)) + 0.2).astype(np.float32)
+    act = rng.standard_normal((t, k, inter)).astype(np.float16)
+    act[0, 1, 3], act[1, 0, 255], act[2, 0, 32], act[2, 1, 64], act[2, 1, 70] = np.inf, -np.inf, np.nan, np.inf, np.inf
+    lib, st = dev.lib, dev.stream.handle
+    gub, dnb, xb, ib, wb, ab = dev.put(gu_blocks), dev.put(dn_blocks), dev.put(x), dev.put(idx), dev.put(wts), dev.put(act)
+    outs = [dev.alloc(t * k * inter * 2) for _ in range(2)] + [dev.alloc(t * hidden * 4)]
+    vgu, vdn = H.view_of(dev, gub, fmt, experts * 2 * inter, hidden), H.view_of(dev, dnb, fmt, experts * hidden, inter)
+    for flags, o in ((pre, outs[0]), (pre | (2 << 8), outs[1])):
+        qwhip.check(lib.qwhip_moe_gateup_decode(st, C.byref(vgu), experts, xb.ptr, qwhip.F16, flags, ib.ptr, t, k, o.ptr))
+    qwhip.check(lib.qwhip_moe_down_decode(st, C.byref(vdn), experts, ab.ptr, ib.ptr, wb.ptr, t, k, None, None, outs[2].ptr, qwhip.F32))
+    dev.stream.sync()
+    col, general = (o.download(np.float16, (t, k, inter)).astype(np.float32) for o in outs[:2])
+    odd = ~np.isfinite(general)
+    assert odd[:3].any() and not odd[3].any()
+    assert np.array_equal(col[odd], general[odd], equal_nan=True)
+    assert np.isfinite(col[~odd]).all() and qo.normalized_error(col[~odd].astype(np.float64), general[~odd].astype(np.float64)) <= TOL
+    with np.errstate(invalid="ignore"):
+        want = np.stack([sum(float(wts[r, j]) * (dn16[idx[r, j]].astype(np.float64) * act[r, j].astype(np.float64)).sum(axis=1)
+                             for j in range(k)) for r in range(t)])
+    got = outs[2].download(np.float32, (t, hidden))
+    assert np.isinf(want[:2]).any() and np.isnan(want[2]).all() and np.isfinite(want[3]).all()
+    assert np.array_equal(got[:3], want[:3].astype(np.float32), equal_nan=True)
+    assert qo.normalized_error(got[3], want[3]) <= TOL
+    for b in (gub, dnb, xb, ib, wb, ab, *outs):
+        b.free()
+
+
 @pytest.mark.parametrize("xdt", ["f16", "bf16"])
 @pytest.mark.parametrize("hidden,inter", [(256, 96), (2048, 160), (3072, 64), (5120, 40)])
 @pytest.mark.parametrize("t,k,experts", [(2, 8, 12), (3, 4, 6), (4, 8, 40), (4, 16, 20), (4, 8, 8)])
