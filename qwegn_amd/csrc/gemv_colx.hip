@@ -165,7 +165,7 @@ static __device__ __forceinline__ void run(const P& pp) {
                 }
             }
         }
-        S[m] = qcx_operands<FMT>(xr, xo[m]);
+        S[m] = qcx_operands<FMT, false>(xr, xo[m]);
         __builtin_amdgcn_sched_barrier(0);   // keeps the conversion of row m + 1 from overlapping row m's registers
     }
 
@@ -199,7 +199,7 @@ static __device__ __forceinline__ void run(const P& pp) {
                     if (lane == 31u && rslot < nrows) qcx_part[(rslot * cpr + chunk) * MR + m] = v;
                     continue;
                 }
-                const float q = qcx_code_dot<FMT>(ow, xo[m], S[m]);
+                const float q = qcx_code_dot<FMT, false>(ow, xo[m], S[m]);
                 float v = __builtin_fmaf(sc, q, bi * S[m]);
                 v = gvalid ? v : 0.0f;
                 v = qw_reduce32_dpp(v);

@@ -82,7 +82,7 @@ __device__ __forceinline__ void qmc_load(const uint8_t* bank, uint32_t row, uint
 template <int FMT>
 __device__ __forceinline__ float qmc_operands_of(const h8_t* v, h2_t* xo) {
     if constexpr (FMT == QW_FMT_M5) return qmc_operands(v, xo);
-    else return qcx_operands<FMT>(v, xo);
+    else return qcx_operands<FMT, true>(v, xo);
 }
 
 template <int FMT>
@@ -93,12 +93,12 @@ __device__ __forceinline__ float qmc_dot(const qmc_slice<FMT>& b, const h2_t* xo
         uint32_t ow[16];
         qcx_mask<FMT>(b, ow);
         const h2_t hd = __builtin_bit_cast(h2_t, b.hdr);
-        return __builtin_fmaf((float)hd[0], qcx_code_dot<FMT>(ow, xo, S), (float)hd[1] * S);
+        return __builtin_fmaf((float)hd[0], qcx_code_dot<FMT, true>(ow, xo, S), (float)hd[1] * S);
     }
 }
 
 // The same slice weight by weight, for a slice with an infinite activation: s sum(q x) + b sum(x) makes NaN of it (0 x inf, inf - inf)
-// where its products with the weights are infinities.  A weight is code s + b in fp32; it is zero only where its f16 rounding is, since
+// where its products with the weights are infinities; and for one that holds an activation past the scale of its operands.  A weight is code s + b in fp32; it is zero only where its f16 rounding is, since
 // scales and biases are multiples of 2^-24.
 template <int FMT>
 __device__ __forceinline__ float qmc_plain_dot(const qmc_slice<FMT>& b, const h8_t* x) {
@@ -298,7 +298,7 @@ static __device__ __forceinline__ void run(const qmc_gu_params& p) {
     h2_t xo[16];
     const float S = qmc_operands_of<FMT>(xs + g * 5, xo);
     const float c1 = 1024.0f * S;
-    // an infinite or NaN activation under this wave: every sum of the pair comes out infinite or NaN, and the plain form says which
+    // an activation under this wave is not finite, or not as an operand: the wave's sums are taken again in the plain form
     unsigned long long odd = 0ull;
     if constexpr (FMT != QW_FMT_M5) odd = __ballot(!qw_finite(S));
 #pragma unroll

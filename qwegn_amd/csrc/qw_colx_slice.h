@@ -27,43 +27,49 @@ struct qcx_slice {
 __device__ constexpr int QCX_B3_LO[16] = {0, 3, 10, 13, 20, 23, 30, 1, 4, 11, 14, 21, 24, 2, 12, 22};
 __device__ constexpr int QCX_B3_HI[16] = {5, 8, 15, 18, 25, 28, 31, 6, 9, 16, 19, 26, 29, 7, 17, 27};
 
-template <int FMT>
+// The fields of a masked 3- or 6-bit word sit at different places in its two halves: the low code of a 3-bit word reads twice the
+// high one, the high code of a 6-bit word four times the low one, and the operands make up for it.  EXACT: they multiply (1x, 2x and
+// 4x, 1x), which keeps every bit of an activation, subnormals too; one past 32,752 or 16,376 becomes infinite, shows in the sum
+// returned, and is the caller's to see.  Not EXACT: they divide (1/2x, 1x and 1x, 1/4x); any activation passes, and those under
+// 2^-13 or 2^-12 lose their last one or two bits (rows of magnitude 1e-5: 6e-3 and 1.3e-2 of the result, 1e-4: 5e-4 and 9e-4).
+template <int FMT, bool EXACT>
+struct qcx_scale {
+    static constexpr float LO = FMT == QW_FMT_B3 ? (EXACT ? 1.0f : 0.5f) : FMT == QW_FMT_B6 ? (EXACT ? 4.0f : 1.0f) : 1.0f;
+    static constexpr float HI = FMT == QW_FMT_B3 ? (EXACT ? 2.0f : 1.0f) : FMT == QW_FMT_B6 ? (EXACT ? 1.0f : 0.25f) : 1.0f;
+    static constexpr float PLAIN = FMT == QW_FMT_B3 ? HI : LO;   // the operand of codes 30 and 31, cut out in step
+    static constexpr float BACK = 16777216.0f / PLAIN;           // 2^24, the codes' place as f16 subnormals, over the scale
+};
+
+// 16 operand pairs of the lane's slice and the sum of its activations.
+template <int FMT, bool EXACT>
 __device__ __forceinline__ float qcx_operands(const h8_t* v, h2_t* xo) {
     const h2_t one = {(h1_t)1.0f, (h1_t)1.0f};
     float s0 = 0.f, s1 = 0.f;
-    if constexpr (FMT == QW_FMT_B6) {
+    if constexpr (FMT == QW_FMT_B6 || FMT == QW_FMT_B3) {
+        using sc = qcx_scale<FMT, EXACT>;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const h2_t nat = {v[j][2 * k], v[j][2 * k + 1]};
-                if (k & 1) s1 = __builtin_amdgcn_fdot2(nat, one, s1, false);
-                else s0 = __builtin_amdgcn_fdot2(nat, one, s0, false);
+        for (int i = 0; i < 16; ++i) {   // 6-bit operand i: elements (e, e + 3), e = 6 (i / 3) + i % 3
+            const bool plain = i == (FMT == QW_FMT_B6 ? 15 : 6);
+            const int lo = FMT == QW_FMT_B3 ? QCX_B3_LO[i] : plain ? 30 : 6 * (i / 3) + i % 3;
+            const int hi = FMT == QW_FMT_B3 ? QCX_B3_HI[i] : plain ? 31 : lo + 3;
+            const float a = plain ? sc::PLAIN : sc::LO, b = plain ? sc::PLAIN : sc::HI;
+            xo[i] = h2_t{v[lo >> 3][lo & 7] * (h1_t)a, v[hi >> 3][hi & 7] * (h1_t)b};
+            if constexpr (EXACT) {
+                const h2_t inv = {(h1_t)(1.0f / a), (h1_t)(1.0f / b)};
+                if (i & 1) s1 = __builtin_amdgcn_fdot2(xo[i], inv, s1, false);
+                else s0 = __builtin_amdgcn_fdot2(xo[i], inv, s0, false);
             }
         }
+        if constexpr (!EXACT) {
 #pragma unroll
-        for (int i = 0; i < 15; ++i) {   // operand i: elements (e, e + 3), e = 6 (i / 3) + i % 3
-            const int lo = 6 * (i / 3) + i % 3, hi = lo + 3;
-            xo[i] = h2_t{v[lo >> 3][lo & 7], v[hi >> 3][hi & 7] * (h1_t)0.25f};
-        }
-        xo[15] = h2_t{v[3][6], v[3][7]};
-        return s0 + s1;
-    }
-    if constexpr (FMT == QW_FMT_B3) {
+            for (int j = 0; j < 4; ++j) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const h2_t nat = {v[j][2 * k], v[j][2 * k + 1]};
-                if (k & 1) s1 = __builtin_amdgcn_fdot2(nat, one, s1, false);
-                else s0 = __builtin_amdgcn_fdot2(nat, one, s0, false);
+                for (int k = 0; k < 4; ++k) {
+                    const h2_t nat = {v[j][2 * k], v[j][2 * k + 1]};
+                    if (k & 1) s1 = __builtin_amdgcn_fdot2(nat, one, s1, false);
+                    else s0 = __builtin_amdgcn_fdot2(nat, one, s0, false);
+                }
             }
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int lo = QCX_B3_LO[i], hi = QCX_B3_HI[i];
-            const h1_t xl = v[lo >> 3][lo & 7], xh = v[hi >> 3][hi & 7];
-            xo[i] = h2_t{i == 6 ? xl : xl * (h1_t)0.5f, xh};   // the windows' low fields read twice their code
         }
         return s0 + s1;
     }
@@ -175,8 +181,8 @@ __device__ __forceinline__ void qcx_mask(const qcx_slice<FMT>& b, uint32_t* ow) 
     }
 }
 
-// sum_i q_i x_i of a slice (HQ4_G32_M5: sum_i (1024 + q_i) x_i).
-template <int FMT>
+// sum_i q_i x_i of a slice, on the operands of the same EXACT (HQ4_G32_M5: sum_i (1024 + q_i) x_i).
+template <int FMT, bool EXACT>
 __device__ __forceinline__ float qcx_code_dot(const uint32_t* ow, const h2_t* xo, float S) {
     float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
     if constexpr (FMT == QW_FMT_B3) {
@@ -201,10 +207,11 @@ __device__ __forceinline__ float qcx_code_dot(const uint32_t* ow, const h2_t* xo
     }
     float q;
     if constexpr (FMT == QW_FMT_B3) {
-        q = __builtin_fmaf(a2, 2097152.0f, (a0 + a1) * 16777216.0f);   // fields at bits 4 / 3 of the halves: 8 q
-        q = __builtin_fmaf(a3, 262144.0f, q);                          // bits 7 / 6: 64 q
+        constexpr float B = qcx_scale<FMT, EXACT>::BACK;
+        q = __builtin_fmaf(a2, B * 0.125f, (a0 + a1) * B);   // fields at bits 4 / 3 of the halves: 8 q
+        q = __builtin_fmaf(a3, B * 0.015625f, q);            // bits 7 / 6: 64 q
     } else if constexpr (FMT == QW_FMT_B8 || FMT == QW_FMT_B6) {
-        q = ((a0 + a1) + (a2 + a3)) * 16777216.0f;
+        q = ((a0 + a1) + (a2 + a3)) * qcx_scale<FMT, EXACT>::BACK;
     } else if constexpr (FMT == QW_FMT_B2) {
         q = __builtin_fmaf(a1, 4194304.0f, a0 * 16777216.0f);     // codes at bits 0..1 and 2..3 of a byte
         q = __builtin_fmaf(a2, 1048576.0f, q);                    // bits 4..5

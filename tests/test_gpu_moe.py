@@ -431,6 +431,62 @@ def test_routed_projections_keep_infinities(dev, fmt, pre):
         b.free()
 
 
+@pytest.mark.parametrize("fmt", ["hq6_g32", "aq6_g128", "hq3_g32", "aq2_g64", "hq8_g64", "aq4_g32"])
+@pytest.mark.parametrize("mag,spike", [(1.0, 0.0), (1e-2, 0.0), (1e-4, 0.0), (1e-5, 0.0), (1e-5, 16376.0), (1e-5, 16384.0), (1e-4, 32752.0),
+                                       (1e-4, 65504.0)])
+def test_routed_down_keeps_every_bit_of_small_activations(dev, fmt, mag, spike):
+    """f16 subnormal activations (gated activations have no norm behind them) and, in one group of a row, a value near the largest f16,
+    against the un-rounded affine weights: exact products, so fp32 sums and the cancellation of s sum(q x) against b sum(x), at most
+    some 30 times the result, are all there is: 2^-24 x 30 x a few."""
+    kind, bits, group, is_m5, _ = H.FORMATS[fmt]
+    t, e, k, h, inter = 2, 3, 2, 80, 768
+    blocks, _ = H.make_bank(fmt, e * h, inter, 51)
+    w = qo.weights_affine_f64(blocks, bits, group, is_m5).reshape(e, h, inter)
+    rng = np.random.default_rng(52)
+    act = (rng.standard_normal((t, k, inter)) * mag).astype(np.float16)
+    if spike:
+        act[1, 0, 37], act[1, 1, 64 + 30] = spike, -spike
+    idx, wts = np.array([[2, 0], [1, 2]], np.int32), (rng.random((t, k)) + 0.2).astype(np.float32)
+    ref = np.zeros((t, h))
+    for r in range(t):
+        for j in range(k):
+            ref[r] += float(wts[r, j]) * (w[idx[r, j]] @ act[r, j].astype(np.float64))
+    bank, ab, ib, wb, out = dev.put(blocks), dev.put(act), dev.put(idx), dev.put(wts), dev.alloc(t * h * 4)
+    v = H.view_of(dev, bank, fmt, e * h, inter)
+    qwhip.check(dev.lib.qwhip_moe_down_decode(dev.stream.handle, C.byref(v), e, ab.ptr, ib.ptr, wb.ptr, t, k, None, None, out.ptr, qwhip.F32))
+    got = out.download(np.float32, (t, h))
+    for r in range(t):   # row by row: the spike's row must not hide the other
+        assert qo.normalized_error(got[r], ref[r]) <= 2e-5, r
+    for b in (bank, ab, ib, wb, out):
+        b.free()
+
+
+@pytest.mark.parametrize("fmt", ["hq6_g32", "aq6_g128", "hq3_g32"])
+@pytest.mark.parametrize("spike", [16376.0, 16392.0, 32752.0, 32768.0, 65504.0])
+def test_routed_gate_up_takes_the_largest_activations(dev, fmt, spike):
+    """An activation at, and past, the largest one the scaled operands hold: the general kernel's result, up to its weights' f16 rounding."""
+    kind, bits, group, is_m5, rot = H.FORMATS[fmt]
+    t, e, k, h, inter = 2, 2, 2, 1280, 96
+    w = H.make_weights(e * 2 * inter, h, 53, std=2e-4)
+    blocks, _ = qo.quant_hq_blocks(w, bits=bits, group=group, is_m5=is_m5, rotate=rot)
+    rng = np.random.default_rng(54)
+    x = rng.standard_normal((t, h)).astype(np.float16)
+    x[0, 7], x[0, 1030], x[1, 31] = spike, -spike, -spike
+    idx = np.array([[0, 1], [1, 0]], np.int32)
+    bank, xb, ib = dev.put(blocks), dev.put(x), dev.put(idx)
+    outs = [dev.alloc(t * k * inter * 2) for _ in range(2)]
+    v = H.view_of(dev, bank, fmt, e * 2 * inter, h)
+    for flags, o in ((0, outs[0]), (2 << 8, outs[1])):
+        qwhip.check(dev.lib.qwhip_moe_gateup_decode(dev.stream.handle, C.byref(v), e, xb.ptr, qwhip.F16, flags | qwhip.X_PREROTATED, ib.ptr, t, k, o.ptr))
+    dev.stream.sync()
+    col, general = (o.download(np.float16, (t, k * inter)).astype(np.float64) for o in outs)
+    assert np.isfinite(general).all() and np.abs(general).max() > 0.1
+    for r in range(t):
+        assert qo.normalized_error(col[r], general[r]) <= TOL
+    for b in (bank, xb, ib, *outs):
+        b.free()
+
+
 @pytest.mark.parametrize("xdt", ["f16", "bf16"])
 @pytest.mark.parametrize("hidden,inter", [(256, 96), (2048, 160), (3072, 64), (5120, 40)])
 @pytest.mark.parametrize("t,k,experts", [(2, 8, 12), (3, 4, 6), (4, 8, 40), (4, 16, 20), (4, 8, 8)])
