@@ -1,5 +1,6 @@
 // Router logits and the dense fp32 GEMV door: out[t, e] = sum_h x[t, h] * w[e, h] on un-quantized weights, fp32 accumulate.
 #include <algorithm>
+#include <type_traits>
 
 #include "qwhip_common.h"
 
@@ -18,14 +19,25 @@ __device__ __forceinline__ float qw_f32_gemv_epilogue(float y, uint32_t epi, flo
 
 typedef __bf16 qw_bf8_t __attribute__((ext_vector_type(8)));
 
-// Eight consecutive elements as they are stored (16 bytes, or 32 for fp32), 16-byte aligned.
+struct __attribute__((packed, aligned(4))) qw_words4 { u4_t v; };   // 16 bytes at any 4-byte boundary
+
+// Eight consecutive elements as they are stored: 16 bytes, 16-byte aligned, or for fp32 32 bytes, 4-byte aligned.
 template <int DT>
 struct qw_raw8 {
     u4_t v[DT == QWHIP_F32 ? 2 : 1];
     __device__ __forceinline__ void load(const void* p, uint64_t i) {
-        const u4_t* q = (const u4_t*)((const uint8_t*)p + i * (DT == QWHIP_F32 ? 4u : 2u));
-        v[0] = q[0];
-        if constexpr (DT == QWHIP_F32) v[1] = q[1];
+        const uint8_t* q = (const uint8_t*)p + i * (DT == QWHIP_F32 ? 4u : 2u);
+        if constexpr (DT == QWHIP_F32) {
+            v[0] = ((const qw_words4*)q)[0].v;
+            v[1] = ((const qw_words4*)q)[1].v;
+        } else {
+            v[0] = *(const u4_t*)q;
+        }
+    }
+    // Keeps a load from sinking into the branch behind which its value is used: all of a batch are in flight together.
+    __device__ __forceinline__ void pin() {
+        asm volatile("" : "+v"(v[0]));
+        if constexpr (DT == QWHIP_F32) asm volatile("" : "+v"(v[1]));
     }
     __device__ __forceinline__ void floats(float* f) const {
         if constexpr (DT == QWHIP_F32) {
@@ -60,39 +72,155 @@ __device__ __forceinline__ qw_bf8_t qw_take_bf16(float* f) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// Two token rows and more: 16 tokens x 16 NT weight rows a workgroup on the matrix cores, the hidden dimension dealt in chunks
-// of 32 to its W waves (chunk c to wave c % W) and the waves' sums added in wave order, so an output does not depend on how
-// many rows or experts the call has.  Operands go from memory to registers as they lie (lane (r, g): row r, columns 8 g .. 8 g + 7
-// of a chunk; nothing is shared between waves, so LDS would only add a copy), four chunks in flight per wave.
+// One summation order for every call on a weight type: a token's logits do not depend on the rows or experts beside it, so a
+// token decodes, verifies and prefills to the same experts.  The hidden dimension goes in chunks of 32 columns; chunk c adds to
+// partial sum c % 16, ascending, and the sixteen end as Q[i] = P[i] + P[i + 8], ((Q0 + Q1) + (Q2 + Q3)) + ((Q4 + Q5) + (Q6 + Q7)).
+// bf16 weights: a chunk is one bf16 matrix product per term of the activations.  Other weights: a partial is four fp32 FMA chains
+// over the columns 8 g .. 8 g + 7 of its chunks, ended as (g0 + g1) + (g2 + g3): with partial p and chain g in lane 4 p + g, a
+// wavefront's own order over pieces of 512 columns (qw_router_dot), and the order of the fp32 product of four 16x1x16 blocks.
+// ------------------------------------------------------------------------------------------------
+
+// Sum over the wavefront, in that order; every lane gets it.
+__device__ __forceinline__ float qw_router_fold(float v) {
+    v += __shfl_xor(v, 1, 64);
+    v += __shfl_xor(v, 2, 64);
+    v += __shfl_xor(v, 32, 64);
+    v += __shfl_xor(v, 4, 64);
+    v += __shfl_xor(v, 8, 64);
+    v += __shfl_xor(v, 16, 64);
+    return v;
+}
+
+// R rows of x (rows past `rows` repeat the last) against one weight row by a wavefront: 16-byte loads, P pieces of 512 columns in flight.
+// `w` is 4-byte aligned, `x` 16-byte.
+template <int XDT, int WDT, int R, int P>
+__device__ __forceinline__ void qw_router_dot(const void* x, uint32_t rows, const void* w, uint64_t wbase, uint32_t H, uint32_t lane, float* out) {
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+    for (uint32_t h0 = lane * 8u; h0 < H; h0 += 512u * P) {
+        qw_raw8<XDT> a[P][R];
+        qw_raw8<WDT> b[P];
+#pragma unroll
+        for (uint32_t u = 0; u < P; ++u) {
+            const uint32_t h = h0 + 512u * u < H ? h0 + 512u * u : h0;
+            b[u].load(w, wbase + h);
+#pragma unroll
+            for (int r = 0; r < R; ++r) a[u][r].load(x, (uint64_t)min((uint32_t)r, rows - 1u) * H + h);
+        }
+#pragma unroll
+        for (uint32_t u = 1; u < P; ++u) {
+            b[u].pin();
+#pragma unroll
+            for (int r = 0; r < R; ++r) a[u][r].pin();
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < P; ++u) {
+            float fb[8];
+            b[u].floats(fb);
+            if (u > 0 && h0 + 512u * u >= H) break;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                float fa[8];
+                a[u][r].floats(fa);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc[r] = fmaf(fb[j], fa[j], acc[r]);
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) out[r] = qw_router_fold(acc[r]);
+}
+
+// The same for bf16 weights, on the matrix cores: a piece of 512 columns is sixteen chunks, lane 16 g + p holds columns
+// 8 g .. 8 g + 7 of chunk p of both rows, and the products' diagonal is what the sixteen partial sums gain.  `w` is 16-byte aligned.
+template <int XDT, int R, int P>
+__device__ __forceinline__ void qw_router_dot_bf16(const void* x, uint32_t rows, const void* w, uint64_t wbase, uint32_t H, uint32_t lane, float* out) {
+    constexpr int TERMS = XDT == QWHIP_BF16 ? 1 : (XDT == QWHIP_F16 ? 2 : 3);
+    f4_t acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = f4_t{0.f, 0.f, 0.f, 0.f};
+    const uint32_t mine = 32u * (lane & 15u) + 8u * (lane >> 4);
+    for (uint32_t base = 0; base < H; base += 512u * P) {          // uniform
+        qw_raw8<XDT> a[P][R];
+        qw_raw8<QWHIP_BF16> b[P];
+#pragma unroll
+        for (uint32_t u = 0; u < P; ++u) {
+            const uint32_t h = base + 512u * u + mine < H ? base + 512u * u + mine : 0u;
+            b[u].load(w, wbase + h);
+#pragma unroll
+            for (int r = 0; r < R; ++r) a[u][r].load(x, (uint64_t)min((uint32_t)r, rows - 1u) * H + h);
+        }
+#pragma unroll
+        for (uint32_t u = 1; u < P; ++u) {
+            b[u].pin();
+#pragma unroll
+            for (int r = 0; r < R; ++r) a[u][r].pin();
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < P; ++u) {
+            if (u > 0 && base + 512u * u >= H) break;   // uniform
+            const bool in = base + 512u * u + mine < H;   // a chunk past the row adds zeros
+            const u4_t zero = {0u, 0u, 0u, 0u};
+            const qw_bf8_t wt = __builtin_bit_cast(qw_bf8_t, in ? b[u].v[0] : zero);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                qw_bf8_t xt[TERMS];
+                if constexpr (XDT == QWHIP_BF16) {
+                    xt[0] = __builtin_bit_cast(qw_bf8_t, in ? a[u][r].v[0] : zero);
+                } else {
+                    float f[8];
+                    a[u][r].floats(f);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) f[j] = in ? f[j] : 0.0f;
+#pragma unroll
+                    for (int p = 0; p < TERMS; ++p) xt[p] = qw_take_bf16(f);
+                }
+#pragma unroll
+                for (int p = TERMS - 1; p >= 0; --p) acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xt[p], wt, acc[r], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        // partial sum p is row p of column p: register p & 3 of lane 16 (p >> 2) + p
+        const uint32_t i = lane & 3u;
+        float v = i == 0u ? acc[r][0] : i == 1u ? acc[r][1] : i == 2u ? acc[r][2] : acc[r][3];
+        v = __shfl(v, (int)(((lane & 12u) << 2) | (lane & 15u)), 64);
+        v += __shfl_xor(v, 8, 64);
+        v += __shfl_xor(v, 1, 64);
+        v += __shfl_xor(v, 2, 64);
+        v += __shfl_xor(v, 4, 64);
+        if constexpr (XDT != QWHIP_BF16) {   // what the tiles sum again (below), the wavefront does here
+            if (v != v) qw_router_dot<XDT, QWHIP_BF16, 1, 4>((const uint8_t*)x + (uint64_t)min((uint32_t)r, rows - 1u) * H * (XDT == QWHIP_F32 ? 4u : 2u), 1u, w, wbase, H, lane, &v);
+        }
+        out[r] = v;
+    }
+}
+
+// 16 tokens x 16 NT weight rows a workgroup on the matrix cores, chunk c to wave c % W.  Operands go from memory to registers as
+// they lie (lane (r, g): row r, columns 8 g .. 8 g + 7 of a chunk; nothing is shared between waves, so LDS would only add a copy),
+// U chunks in flight per wave.
 // bf16 weights meet the activations as one to three bf16 products that hold every bit of them (exact products, fp32 sums: 48
 // matrix-core clocks a chunk for fp32 rows, where fp32 products take 256); other weights take the fp32 matrix product.
 // What bounded the kernel before (one lane per hidden column, every weight x token product one vector instruction and one LDS
-// operand): 2048 x 128 x 2048 with fp32 rows took 93 us, now 17 (two passes over 16 MB of rows); 4 x 256 x 2048 with f16 rows 19 us, now 5.5.
+// operand): 2048 x 128 x 2048 with fp32 rows 94 us, now 13 (two passes over 16 MB of rows); 4 x 256 x 2048 7.2 us, now 5.0;
+// 2048 x 128 x 2048 all fp32 96 us, now 21, all f16 85 us, now 17.
 // The last band (gate_y) is the shared-expert gate: a dot product with an fp32 row per token.
-// ------------------------------------------------------------------------------------------------
 template <int XDT, int WDT, int NT, int W>
 __global__ __launch_bounds__(64 * W) void qw_router_mfma_kernel(const void* __restrict__ x, const void* __restrict__ wr, float* __restrict__ out,
                                                                 uint32_t T, uint32_t E, uint32_t H, const float* __restrict__ sh_w,
                                                                 float* __restrict__ sh_out, uint32_t gate_y, uint32_t epi, float scale) {
+    static_assert(W == 8 || W == 16, "sixteen partial sums");
+    typedef float f16_t __attribute__((ext_vector_type(16)));
     constexpr uint32_t PITCH = NT * 16 + 4;   // rows 4 apart fall 16 banks apart
     __shared__ float part[W][16 * PITCH];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t t0 = blockIdx.x * 16u;
     if (blockIdx.y == gate_y) {
         for (uint32_t t = t0 + wave; t < min(t0 + 16u, T); t += W) {
-            float v = 0.0f;
-            for (uint32_t h = lane * 8u; h < H; h += 512u) {
-                qw_raw8<XDT> a;
-                qw_raw8<QWHIP_F32> b;
-                a.load(x, (uint64_t)t * H + h);
-                b.load(sh_w, h);
-                float fa[8], fb[8];
-                a.floats(fa);
-                b.floats(fb);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) v = fmaf(fb[j], fa[j], v);
-            }
-            v = qw_reduce64(v);
+            float v;
+            qw_router_dot<XDT, QWHIP_F32, 1, 4>((const uint8_t*)x + (uint64_t)t * H * (XDT == QWHIP_F32 ? 4u : 2u), 1u, sh_w, 0u, H, lane, &v);
             if (lane == 0) sh_out[t] = 1.0f / (1.0f + expf(-v));
         }
         return;
@@ -102,63 +230,90 @@ __global__ __launch_bounds__(64 * W) void qw_router_mfma_kernel(const void* __re
     uint64_t wi[NT];
 #pragma unroll
     for (int n = 0; n < NT; ++n) wi[n] = (uint64_t)min(e0 + 16u * n + r, E - 1u) * H + 8u * g;
-    f4_t acc[NT];
-#pragma unroll
-    for (int n = 0; n < NT; ++n) acc[n] = f4_t{0.f, 0.f, 0.f, 0.f};
     const uint32_t chunks = H >> 5;
-    constexpr int U = 4;
-    for (uint32_t c = wave; c < chunks; c += W * U) {
-        qw_raw8<XDT> xa[U];
-        qw_raw8<WDT> wb[U][NT];
+    constexpr int U = 4, A = 16 / W;   // the wave's partial sums: wave and, with eight waves, wave + 8
+    // one product takes a register quad and the partials go side by side; four blocks take sixteen and they go one after the other
+    constexpr bool SIDE = WDT == QWHIP_BF16;
+    constexpr uint32_t STEP = SIDE ? W : 16;
+    using acc_t = std::conditional_t<SIDE, f4_t, f16_t>;
+    f4_t sum[NT];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const uint32_t h = 32u * (c + W * u < chunks ? c + W * u : c);
-            xa[u].load(x, xi + h);
+    for (int a = 0; a < (SIDE ? 1 : A); ++a) {
+        acc_t acc[SIDE ? A : 1][NT];
 #pragma unroll
-            for (int n = 0; n < NT; ++n) wb[u][n].load(wr, wi[n] + h);
+        for (int s = 0; s < (SIDE ? A : 1); ++s)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[s][n] = acc_t{};
+        for (uint32_t c = wave + W * a; c < chunks; c += STEP * U) {
+            qw_raw8<XDT> xa[U];
+            qw_raw8<WDT> wb[U][NT];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint32_t h = 32u * (c + STEP * u < chunks ? c + STEP * u : c);
+                xa[u].load(x, xi + h);
+#pragma unroll
+                for (int n = 0; n < NT; ++n) wb[u][n].load(wr, wi[n] + h);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (u > 0 && c + STEP * u >= chunks) break;   // wave-uniform
+                if constexpr (SIDE) {
+                    constexpr int M = A - 1;
+                    constexpr int P = XDT == QWHIP_BF16 ? 1 : (XDT == QWHIP_F16 ? 2 : 3);
+                    qw_bf8_t xt[P];
+                    if constexpr (XDT == QWHIP_BF16) {
+                        xt[0] = __builtin_bit_cast(qw_bf8_t, xa[u].v[0]);
+                    } else {
+                        float f[8];
+                        xa[u].floats(f);
+#pragma unroll
+                        for (int p = 0; p < P; ++p) xt[p] = qw_take_bf16(f);
+                    }
+                    // the smallest terms first
+#pragma unroll
+                    for (int p = P - 1; p >= 0; --p)
+#pragma unroll
+                        for (int n = 0; n < NT; ++n)
+                            acc[u & M][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xt[p], __builtin_bit_cast(qw_bf8_t, wb[u][n].v[0]), acc[u & M][n], 0, 0, 0);
+                } else {
+                    float fa[8], fb[NT][8];
+                    xa[u].floats(fa);
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) wb[u][n].floats(fb[n]);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+#pragma unroll
+                        for (int n = 0; n < NT; ++n) acc[0][n] = __builtin_amdgcn_mfma_f32_16x16x1f32(fa[j], fb[n][j], acc[0][n], 0, 0, 0);
+                }
+            }
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (u > 0 && c + W * u >= chunks) break;   // wave-uniform
-            if constexpr (WDT == QWHIP_BF16) {
-                constexpr int P = XDT == QWHIP_BF16 ? 1 : (XDT == QWHIP_F16 ? 2 : 3);
-                qw_bf8_t a[P];
-                if constexpr (XDT == QWHIP_BF16) {
-                    a[0] = __builtin_bit_cast(qw_bf8_t, xa[u].v[0]);
-                } else {
-                    float f[8];
-                    xa[u].floats(f);
+        for (int n = 0; n < NT; ++n) {
 #pragma unroll
-                    for (int p = 0; p < P; ++p) a[p] = qw_take_bf16(f);
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (SIDE) {
+                    sum[n][i] = A == 1 ? acc[0][n][i] : acc[0][n][i] + acc[A - 1][n][i];
+                } else {   // block g in registers 4 g .. 4 g + 3
+                    const float q = (acc[0][n][i] + acc[0][n][4 + i]) + (acc[0][n][8 + i] + acc[0][n][12 + i]);
+                    sum[n][i] = a == 0 ? q : sum[n][i] + q;
                 }
-                // the smallest terms first
-#pragma unroll
-                for (int p = P - 1; p >= 0; --p)
-#pragma unroll
-                    for (int n = 0; n < NT; ++n)
-                        acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[p], __builtin_bit_cast(qw_bf8_t, wb[u][n].v[0]), acc[n], 0, 0, 0);
-            } else {
-                float fa[8], fb[NT][8];
-                xa[u].floats(fa);
-#pragma unroll
-                for (int n = 0; n < NT; ++n) wb[u][n].floats(fb[n]);
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-#pragma unroll
-                    for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[j], fb[n][j], acc[n], 0, 0, 0);
             }
         }
     }
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) part[wave][(4u * g + i) * PITCH + 16u * n + r] = acc[n][i];
+        for (int i = 0; i < 4; ++i) part[wave][(4u * g + i) * PITCH + 16u * n + r] = sum[n][i];
     __syncthreads();
     for (uint32_t o = threadIdx.x; o < 16u * 16u * NT; o += 64u * W) {
         const uint32_t row = o / (16u * NT), col = o % (16u * NT);
-        float v = 0.0f;
+        float q[8];
 #pragma unroll
-        for (int w = 0; w < W; ++w) v += part[w][row * PITCH + col];
+        for (int w = 0; w < 8; ++w) {
+            q[w] = part[w][row * PITCH + col];
+            if constexpr (W == 16) q[w] += part[w + 8][row * PITCH + col];
+        }
+        float v = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
         if (t0 + row >= T || e0 + col >= E) continue;
         if constexpr (WDT == QWHIP_BF16 && XDT != QWHIP_BF16) {
             // the bf16 terms of an infinity, and zero terms against an infinite weight, make NaN of what may be an infinity:
@@ -173,44 +328,25 @@ __global__ __launch_bounds__(64 * W) void qw_router_mfma_kernel(const void* __re
     }
 }
 
-// One token row: a wavefront is a workgroup and owns one weight row (the last one the shared-expert gate), 16-byte loads, four of
-// them in flight.  A row of 2048 bf16 weights is four of those loads a lane, all in flight: the launch is its own latency
-// (128 x 2048: 3.2 us, with 2-byte loads and 32 workgroups 6.6).
-template <int XDT, int WDT>
-__global__ __launch_bounds__(64) void qw_router_row_kernel(const void* __restrict__ x, const void* __restrict__ wr, float* __restrict__ out,
-                                                           uint32_t E, uint32_t H, const float* __restrict__ sh_w, float* __restrict__ sh_out,
-                                                           uint32_t epi, float scale) {
+// A few token rows: a wavefront is a workgroup and owns one weight row (the last one the shared-expert gate).  A row of 2048
+// weights is four loads a lane, all in flight: the launch is its own latency, where a tile of sixteen rows takes the fp32 matrix
+// pipe of a compute unit 1.7 us, and repeats a row's loads and terms sixteen times.
+template <int XDT, int WDT, int R>
+__global__ __launch_bounds__(64) void qw_router_rows_kernel(const void* __restrict__ x, const void* __restrict__ wr, float* __restrict__ out,
+                                                            uint32_t T, uint32_t E, uint32_t H, const float* __restrict__ sh_w,
+                                                            float* __restrict__ sh_out, uint32_t epi, float scale) {
+    constexpr int P = R <= 2 ? 4 : 2;
     const uint32_t e = blockIdx.x, lane = threadIdx.x;
-    float acc[2] = {0.0f, 0.0f};
-    auto dot = [&](auto wt, const void* w, uint64_t base) {
-        constexpr int WT = decltype(wt)::value;
-        for (uint32_t h0 = lane * 8u; h0 < H; h0 += 2048u) {
-            qw_raw8<XDT> a[4];
-            qw_raw8<WT> b[4];
+    float v[R];
+    if (e == E) qw_router_dot<XDT, QWHIP_F32, R, P>(x, T, sh_w, 0u, H, lane, v);
+    else if constexpr (WDT == QWHIP_BF16) qw_router_dot_bf16<XDT, R, P>(x, T, wr, (uint64_t)e * H, H, lane, v);
+    else qw_router_dot<XDT, WDT, R, P>(x, T, wr, (uint64_t)e * H, H, lane, v);
+    if (lane != 0) return;
 #pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {
-                const uint32_t h = h0 + 512u * u < H ? h0 + 512u * u : h0;
-                a[u].load(x, h);
-                b[u].load(w, base + h);
-            }
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) {
-                float fa[8], fb[8];
-                a[u].floats(fa);
-                b[u].floats(fb);
-                if (u == 0 || h0 + 512u * u < H) {
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) acc[j & 1] = fmaf(fb[j], fa[j], acc[j & 1]);
-                }
-            }
-        }
-    };
-    if (e == E) dot(std::integral_constant<int, QWHIP_F32>{}, sh_w, 0);
-    else dot(std::integral_constant<int, WDT>{}, wr, (uint64_t)e * H);
-    const float v = qw_reduce64(acc[0] + acc[1]);
-    if (lane == 0) {
-        if (e == E) *sh_out = 1.0f / (1.0f + expf(-v));
-        else out[e] = qw_f32_gemv_epilogue(v, epi, scale);
+    for (uint32_t t = 0; t < R; ++t) {
+        if (t >= T) break;
+        if (e == E) sh_out[t] = 1.0f / (1.0f + expf(-v[t]));
+        else out[(uint64_t)t * E + e] = qw_f32_gemv_epilogue(v[t], epi, scale);
     }
 }
 
@@ -272,17 +408,33 @@ __global__ __launch_bounds__(256) void qw_router_gemm_kernel(const void* __restr
     }
 }
 
-// Launches the matrix-core or the one-row kernel; false for a type the caller reports.
+// Launches the matrix-core or the few-rows kernel; false for a type the caller reports.  The choice does not show in the results.
+// A wavefront per weight row up to four token rows (fp32 weights, 128 x 2048: 2 / 4 rows 2.3 / 3.1 us, tiles of sixteen rows 6.2 / 6.5),
+// on bf16 weights with rows that split into terms up to two (fp32 rows, 1 / 2 / 4: 2.6 / 3.3 / 5.0 us, tiles 4.5 / 4.7 / 4.9).
 // Tile: 64 weight rows a workgroup (the activations' bf16 terms made once for four products) once that alone is a workgroup for
 // every compute unit, else 16 weight rows and twice the waves: a few token rows are bound by the latency of a wave's own chunks.
 template <int XDT, int WDT>
 static void qw_router_launch(hipStream_t st, const void* x, const void* wr, uint32_t t, uint32_t experts, uint32_t hidden, float* out,
                              const float* sh_w, float* sh_out, uint32_t epi, float scale) {
     const uint32_t gate = sh_w ? 1u : 0u;
+    constexpr bool SPLIT = WDT == QWHIP_BF16 && XDT != QWHIP_BF16;
+#define QW_ROWS(R) \
+    hipLaunchKernelGGL((qw_router_rows_kernel<XDT, WDT, R>), dim3(experts + gate), dim3(64), 0, st, x, wr, out, t, experts, hidden, sh_w, sh_out, epi, scale)
     if (t == 1u) {
-        hipLaunchKernelGGL((qw_router_row_kernel<XDT, WDT>), dim3(experts + gate), dim3(64), 0, st, x, wr, out, experts, hidden, sh_w, sh_out, epi, scale);
+        QW_ROWS(1);
         return;
     }
+    if (t == 2u) {
+        QW_ROWS(2);
+        return;
+    }
+    if constexpr (!SPLIT) {
+        if (t <= 4u) {
+            QW_ROWS(4);
+            return;
+        }
+    }
+#undef QW_ROWS
     const uint32_t gx = qwhip_cdiv(t, 16u);
     if ((uint64_t)gx * qwhip_cdiv(experts, 64u) >= 256u) {
         const uint32_t gy = qwhip_cdiv(experts, 64u);
@@ -331,7 +483,7 @@ static qwhip_status qw_router_gemm_impl(qwhip_stream_t s, const void* x, uint32_
     while (tt > 1u && ((size_t)tt * hidden * 4u > 64u * 1024u || tt >= 2u * t)) tt >>= 1;
     const size_t lds = (size_t)tt * hidden * 4u;
     if (lds > 64u * 1024u) return qwhip_fail(QWHIP_E_BAD_SHAPE, "router gemm: hidden %u exceeds the staged row (<= 16384)", hidden);
-    const bool wide = hidden % 32u == 0 && (((uintptr_t)x | (uintptr_t)wr | (uintptr_t)sh_gate_w) & 15u) == 0;
+    const bool wide = hidden % 32u == 0 && (((uintptr_t)x | (uintptr_t)wr) & 15u) == 0;
     if (wide && qw_router_wide(s->stream, x, x_dtype, wr, w_dtype, t, experts, hidden, logits, sh_gate_w, sh_gate_out, epi, scale)) {
         QWHIP_TRY_HIP(hipGetLastError());
         return QWHIP_OK;

@@ -126,6 +126,43 @@ def test_router_gemm_tiles(dev, t, e, h, xdt, wdt):
         b.free()
 
 
+@pytest.mark.parametrize("xdt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("wdt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("h", [96, 100, 1056, 2048])
+def test_router_rows_do_not_depend_on_the_call(dev, h, xdt, wdt):
+    """A token's logits and gate bit for bit: alone, in windows of 2 to 17 rows, in a prefill that takes the wide tile (65 x 5 tiles of 64
+    weight rows), with fewer experts beside it, and wherever the gate's weights begin."""
+    rng = np.random.default_rng(h)
+    t, e = 1025, 257
+    cast = {"f32": (lambda v: (v.astype(np.float32), qwhip.F32, 4)), "f16": (lambda v: (v.astype(np.float16), qwhip.F16, 2)),
+            "bf16": (lambda v: (qo.f32_to_bf16_bits(v.astype(np.float32)), qwhip.BF16, 2))}
+    xh, xcode, xs = cast[xdt](rng.standard_normal((t, h)))
+    wh, wcode, _ = cast[wdt](rng.standard_normal((e, h)) * 0.05)
+    sb = dev.put(np.concatenate([[7.0], rng.standard_normal(h) * 0.03, np.zeros(8)]).astype(np.float32))
+    xb, wb, lb, gb = dev.put(xh), dev.put(wh), dev.alloc(t * e * 4), dev.alloc(t * 4)
+
+    def run(row, n, experts, skew):
+        # the gate's weights from element 1 on, moved to a 16-byte boundary unless `skew`
+        gate = sb.ptr + 4
+        if not skew:
+            qwhip.check(dev.lib.qwhip_memcpy_d2d(dev.stream.handle, ab.ptr, gate, h * 4))
+            gate = ab.ptr
+        qwhip.check(dev.lib.qwhip_router_gemm_shared_gate(dev.stream.handle, xb.ptr + row * h * xs, xcode, wb.ptr, wcode, n, experts, h, lb.ptr, gate, gb.ptr))
+        return lb.download(np.uint32, (n, experts)), gb.download(np.uint32, (n,))
+
+    ab = dev.alloc(h * 4)
+    want, gate = run(0, t, e, False)
+    for row, n, experts, skew in [(0, 1, e, False), (700, 1, e, True), (1, 2, e, False), (9, 3, e, True), (40, 4, e, False), (1019, 5, e, False),
+                                  (16, 17, e, True), (0, t, 20, False), (0, t, e, True), (3, 1, 1, False)]:
+        if xdt != "f32" and h % 8 != 0 and row % 2:
+            continue   # f16 rows of 100 columns begin at other boundaries
+        got, g = run(row, n, experts, skew)
+        assert np.array_equal(got, want[row : row + n, :experts]), (row, n, experts, skew)
+        assert np.array_equal(g, gate[row : row + n]), (row, n, experts, skew)
+    for b in (xb, wb, sb, ab, lb, gb):
+        b.free()
+
+
 @pytest.mark.parametrize("t,e,k", [(33, 128, 8), (5, 40, 4), (9, 512, 16), (7, 100, 3)])
 @pytest.mark.parametrize("mode", ["bias", "split", "bias+split", "softmax+scale"])
 @pytest.mark.parametrize("norm", [0, 1])
