@@ -367,6 +367,39 @@ def test_router_gemm_keeps_infinities(dev, t, e, h, xdt):
         b.free()
 
 
+@pytest.mark.parametrize("xdt", ["f32", "f16"])
+@pytest.mark.parametrize("t,e", [(2, 33), (17, 33), (1025, 257)])
+def test_router_gemm_rows_that_are_not_finite(dev, t, e, xdt):
+    """Rows of 2080 columns with a NaN or an infinity, summed again by the whole wavefront: the class the plain sum gives, the rows beside
+    them untouched, and the bits of a call of their own."""
+    h, rng = 2080, np.random.default_rng(t)
+    x = rng.standard_normal((t, h)).astype(np.float16)
+    w = qo.round_bf16(rng.standard_normal((e, h)).astype(np.float32) * 0.05)
+    clean = x.copy()
+    x[0, 2079], x[t - 1, 511], x[t - 1, 512] = np.inf, -np.inf, np.inf
+    if t > 2:
+        x[1, 1024] = np.nan
+    cast = (lambda v: v.astype(np.float32)) if xdt == "f32" else (lambda v: v)
+    code = qwhip.F32 if xdt == "f32" else qwhip.F16
+    xb, cb, wb, lb = dev.put(cast(x)), dev.put(cast(clean)), dev.put(qo.f32_to_bf16_bits(w)), dev.alloc(t * e * 4)
+    door = lambda b, n: qwhip.check(dev.lib.qwhip_router_gemm(dev.stream.handle, b, code, wb.ptr, qwhip.BF16, n, e, h, lb.ptr))  # noqa: E731
+    door(cb.ptr, t)
+    want = lb.download(np.float32, (t, e))
+    door(xb.ptr, t)
+    got = lb.download(np.float32, (t, e))
+    with np.errstate(invalid="ignore"):
+        for r in range(t):
+            if np.isfinite(x[r]).all():
+                assert np.array_equal(got[r], want[r])
+            else:
+                plain = (w.astype(np.float64) * x[r].astype(np.float64)).sum(axis=1).astype(np.float32)
+                assert np.array_equal(got[r], plain, equal_nan=True), r
+    door(xb.ptr, 1)
+    assert np.array_equal(lb.download(np.float32, (e,)), got[0], equal_nan=True)
+    for b in (xb, cb, wb, lb):
+        b.free()
+
+
 # (format, gate_up kernel override): every container runs the column-stationary kernels, override 2 keeps gate_up on the
 # general kernel.
 @pytest.mark.parametrize("fmt,gu_flags", [("hq4_g32_m5", 0), ("hq4_g32_m5", 2 << 8), ("hq4_g32", 0), ("hq3_g32", 0), ("hq6_g32", 0)])
