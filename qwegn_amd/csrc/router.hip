@@ -415,8 +415,10 @@ __global__ __launch_bounds__(256) void qw_router_gemm_kernel(const void* __restr
 // Launches the matrix-core or the few-rows kernel; false for a type the caller reports.  The choice does not show in the results.
 // A wavefront per weight row up to four token rows (fp32 weights, 128 x 2048: 2 / 4 rows 2.3 / 3.1 us, tiles of sixteen rows 6.2 / 6.5),
 // on bf16 weights with rows that split into terms up to two (fp32 rows, 1 / 2 / 4: 2.6 / 3.3 / 5.0 us, tiles 4.5 / 4.7 / 4.9).
-// Tile: 64 weight rows a workgroup (the activations' bf16 terms made once for four products) once that alone is a workgroup for
-// every compute unit, else 16 weight rows and twice the waves: a few token rows are bound by the latency of a wave's own chunks.
+// Tile: 64 weight rows a workgroup (the activations' bf16 terms made once for four products) from 160 such tiles on, else 16 weight
+// rows and twice the waves: fewer tiles leave compute units idle and are bound by the latency of a wave's own chunks.  Hidden 2048,
+// 64 / 128 / 192 / 256 tiles, narrow against wide: fp32 rows, bf16 weights 7.6 / 12.7 / 18.0 / 23.3 us against 12.6 / 12.6 / 12.8 / 13.2;
+// f16 rows 5.8 / 9.8 / 13.6 / 17.7 against 10.9 / 11.0 / 11.0 / 11.2; all fp32 9.5 / 16.4 / 23.2 / 30.0 against 20.0 / 20.1 / 20.5 / 20.9.
 template <int XDT, int WDT>
 static void qw_router_launch(hipStream_t st, const void* x, const void* wr, uint32_t t, uint32_t experts, uint32_t hidden, float* out,
                              const float* sh_w, float* sh_out, uint32_t epi, float scale) {
@@ -440,7 +442,7 @@ static void qw_router_launch(hipStream_t st, const void* x, const void* wr, uint
     }
 #undef QW_ROWS
     const uint32_t gx = qwhip_cdiv(t, 16u);
-    if ((uint64_t)gx * qwhip_cdiv(experts, 64u) >= 256u) {
+    if ((uint64_t)gx * qwhip_cdiv(experts, 64u) >= 160u) {
         const uint32_t gy = qwhip_cdiv(experts, 64u);
         hipLaunchKernelGGL((qw_router_mfma_kernel<XDT, WDT, 4, 8>), dim3(gx, gy + gate), dim3(512), 0, st, x, wr, out, t, experts, hidden, sh_w, sh_out,
                            gate ? gy : ~0u, epi, scale);
