@@ -100,14 +100,39 @@ extern "C" qwhip_status qwhip_cast_f32_to_f16(qwhip_stream_t s, const float* src
 // SwiGLU runs in fp32 on the values as stored (f16 inputs are the rounded values the fused prefill
 // path also sees, Sources/QWMetal/include/qw_gemm_nax_swiglu.metalh:132-152); rotation in fp32, one
 // f16 rounding on store.
-// Four lanes a 32-group, a row of act per blockIdx.y: with one lane a group and a 64-bit division by the row length, 4 x 17408
+// Four lanes a 32-group, rows of act along blockIdx.y: with one lane a group and a 64-bit division by the row length, 4 x 17408
 // fp32 pairs (2176 lanes of long serial work) took 5.7 us where an empty launch takes 1.7; now 2.4.
+// From 1024 rows on, rows of up to 1024 channels share a workgroup, 256 / (inter / 8) of them: alone they left most of its lanes
+// idle (fp32, 65536 x 32 30.7 us alone, 3.9 shared; 65536 x 96 30.7 / 10.7; 16384 x 128 9.6 / 3.9; 2048 x 1024 4.0 / 4.1).  Fewer
+// rows are their own latency, to which the division adds (64 x 768 2.45 / 2.6).
+
+// What a thread owns: channels c .. c + 7 (none: c >= inter) of the rows first, first + step, ...
+struct qw_row_share {
+    uint32_t c, first, step;
+};
+__device__ __forceinline__ qw_row_share qw_share_rows(uint32_t inter, uint32_t rpw) {
+    qw_row_share s = {(blockIdx.x * 256u + threadIdx.x) * 8u, blockIdx.y, gridDim.y};
+    if (rpw > 1u) {   // inter / 8 is a multiple of four: the lanes of a 32-group are in one row
+        const uint32_t octets = inter / 8u, r = threadIdx.x / octets;
+        s.c = r < rpw ? (threadIdx.x - r * octets) * 8u : inter;
+        s.first = blockIdx.y * rpw + r;
+        s.step = gridDim.y * rpw;
+    }
+    return s;
+}
+static uint32_t qw_rows_per_workgroup(uint32_t rows, uint32_t inter) { return rows >= 1024u && inter <= 1024u ? 256u / (inter / 8u) : 1u; }
+static dim3 qw_row_grid(uint32_t rows, uint32_t inter) {
+    const uint32_t by = (rows - 1u) / qw_rows_per_workgroup(rows, inter) + 1u;
+    return dim3((inter - 1u) / 2048u + 1u, by < 65535u ? by : 65535u);
+}
+
 template <int DT, bool ROT>
 __global__ __launch_bounds__(256) void qw_swiglu_fwht_kernel(const void* __restrict__ gu, h1_t* __restrict__ act,
-                                                              uint32_t rows, uint32_t inter, const qw_act ga) {
-    const uint32_t c = (blockIdx.x * 256u + threadIdx.x) * 8u;
+                                                              uint32_t rows, uint32_t inter, uint32_t rpw, const qw_act ga) {
+    const qw_row_share s = qw_share_rows(inter, rpw);
+    const uint32_t c = s.c;
     if (c >= inter) return;   // whole groups of four lanes leave together
-    for (uint32_t r = blockIdx.y; r < rows; r += gridDim.y) {
+    for (uint32_t r = s.first; r < rows; r += s.step) {
         const uint64_t at = (uint64_t)r * 2 * inter + c;
         float a[8], b[8];
         qw_load8_f32<DT>(gu, at, a);
@@ -148,13 +173,14 @@ extern "C" qwhip_status qwhip_swiglu_fwht(qwhip_stream_t s, const void* gu, uint
         if (gu_dtype == QWHIP_F16) hipLaunchKernelGGL(qw_swiglu_scalar_kernel<QWHIP_F16>, grid, block, 0, s->stream, gu, act, rows, inter, s->dev->act);
         else hipLaunchKernelGGL(qw_swiglu_scalar_kernel<QWHIP_F32>, grid, block, 0, s->stream, gu, act, rows, inter, s->dev->act);
     } else {
-        const dim3 grid(qwhip_cdiv(inter, 2048u), min(rows, 65535u)), block(256);
+        const dim3 grid = qw_row_grid(rows, inter), block(256);
+        const uint32_t rpw = qw_rows_per_workgroup(rows, inter);
         if (gu_dtype == QWHIP_F16) {
-            if (rotate) hipLaunchKernelGGL((qw_swiglu_fwht_kernel<QWHIP_F16, true>), grid, block, 0, s->stream, gu, act, rows, inter, s->dev->act);
-            else hipLaunchKernelGGL((qw_swiglu_fwht_kernel<QWHIP_F16, false>), grid, block, 0, s->stream, gu, act, rows, inter, s->dev->act);
+            if (rotate) hipLaunchKernelGGL((qw_swiglu_fwht_kernel<QWHIP_F16, true>), grid, block, 0, s->stream, gu, act, rows, inter, rpw, s->dev->act);
+            else hipLaunchKernelGGL((qw_swiglu_fwht_kernel<QWHIP_F16, false>), grid, block, 0, s->stream, gu, act, rows, inter, rpw, s->dev->act);
         } else {
-            if (rotate) hipLaunchKernelGGL((qw_swiglu_fwht_kernel<QWHIP_F32, true>), grid, block, 0, s->stream, gu, act, rows, inter, s->dev->act);
-            else hipLaunchKernelGGL((qw_swiglu_fwht_kernel<QWHIP_F32, false>), grid, block, 0, s->stream, gu, act, rows, inter, s->dev->act);
+            if (rotate) hipLaunchKernelGGL((qw_swiglu_fwht_kernel<QWHIP_F32, true>), grid, block, 0, s->stream, gu, act, rows, inter, rpw, s->dev->act);
+            else hipLaunchKernelGGL((qw_swiglu_fwht_kernel<QWHIP_F32, false>), grid, block, 0, s->stream, gu, act, rows, inter, rpw, s->dev->act);
         }
     }
     QWHIP_TRY_HIP(hipGetLastError());
@@ -226,10 +252,11 @@ extern "C" qwhip_status qwhip_dequant_f16(qwhip_stream_t s, const qwhip_weight_v
 // silu(gate) * up in fp32, then the 32-point transform, fp32 out (qwg_silu_mul_f32, Sources/QWMetal/gemm/qwgemm_f32.metal:291-317;
 // door QWGemm.encodeSiluMulF32, Sources/Operators/QWGEMM/QWGemmF32.swift:83-94).  gu fp32 [rows, 2 inter], inter % 32 == 0.
 __global__ __launch_bounds__(256) void qw_silu_mul_f32_kernel(const float* __restrict__ gu, float* __restrict__ act, uint32_t rows,
-                                                               uint32_t inter, const qw_act ga) {
-    const uint32_t c = (blockIdx.x * 256u + threadIdx.x) * 8u;
+                                                               uint32_t inter, uint32_t rpw, const qw_act ga) {
+    const qw_row_share s = qw_share_rows(inter, rpw);
+    const uint32_t c = s.c;
     if (c >= inter) return;
-    for (uint32_t r = blockIdx.y; r < rows; r += gridDim.y) {
+    for (uint32_t r = s.first; r < rows; r += s.step) {
         const uint64_t at = (uint64_t)r * 2u * inter + c;
         float a[8], b[8];
         qw_load8_f32<QWHIP_F32>(gu, at, a);
@@ -248,7 +275,8 @@ extern "C" qwhip_status qwhip_silu_mul_f32(qwhip_stream_t s, const float* gu, fl
     QWHIP_REQUIRE(act);
     if (inter == 0 || inter % 32u != 0) return qwhip_fail(QWHIP_E_BAD_SHAPE, "f32 silu-mul needs intermediate %% 32 == 0, got %u", inter);
     if (((uintptr_t)gu | (uintptr_t)act) & 15u) return qwhip_fail(QWHIP_E_BAD_SHAPE, "f32 silu-mul needs 16-byte aligned buffers");
-    hipLaunchKernelGGL(qw_silu_mul_f32_kernel, dim3(qwhip_cdiv(inter, 2048u), min(rows, 65535u)), dim3(256), 0, s->stream, gu, act, rows, inter, s->dev->act);
+    hipLaunchKernelGGL(qw_silu_mul_f32_kernel, qw_row_grid(rows, inter), dim3(256), 0, s->stream, gu, act, rows, inter,
+                       qw_rows_per_workgroup(rows, inter), s->dev->act);
     QWHIP_TRY_HIP(hipGetLastError());
     return QWHIP_OK;
 }

@@ -704,6 +704,25 @@ def test_swiglu_fwht_more_rows_than_a_grid_dimension(dev):
     assert qo.normalized_error(ab.download(np.float16, (rows, inter)), want) <= 2e-3
 
 
+@pytest.mark.parametrize("inter", [32, 96, 608, 1024, 1056])
+@pytest.mark.parametrize("rows", [7, 1024, 1501])
+def test_gated_activation_of_rows_that_share_a_workgroup(dev, rows, inter):
+    """From 1024 rows on, rows of up to 1024 channels share workgroups (64 of 32, three of 608, two of 1024): full and part filled last
+    workgroups, and a row count and a row length past the lines.  The fp32 door rounds to the f16 door's bits."""
+    gu = (np.random.default_rng(inter + rows).standard_normal((rows, 2 * inter)) * 2).astype(np.float32)
+    gb, ab, fb = dev.put(gu), dev.alloc(rows * inter * 2), dev.alloc(rows * inter * 4)
+    for rotate in (1, 0):
+        qwhip.check(dev.lib.qwhip_swiglu_fwht(dev.stream.handle, gb.ptr, qwhip.F32, ab.ptr, rows, inter, rotate))
+        got = ab.download(np.float16, (rows, inter))
+        want = qo.swiglu_fwht_f16(gu[:, :inter], gu[:, inter:], rotate=bool(rotate)).astype(np.float32)
+        assert np.max(np.abs(got.astype(np.float32) - want)) <= 2e-3 * max(1.0, float(np.max(np.abs(want))))
+        if rotate:
+            qwhip.check(dev.lib.qwhip_silu_mul_f32(dev.stream.handle, gb.ptr, fb.ptr, rows, inter))
+            assert np.array_equal(fb.download(np.float32, (rows, inter)).astype(np.float16), got)
+    for b in (gb, ab, fb):
+        b.free()
+
+
 def test_swiglu_fwht_matches_oracle(dev):
     rng = np.random.default_rng(2)
     rows, inter = 9, 160
