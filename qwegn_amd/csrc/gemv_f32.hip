@@ -11,7 +11,9 @@
 // four vector FMAs it stands for, but a lane holds 32 activations instead of 128 (those spilled into the accumulator file),
 // so three times the waves fit and eight rows share one pass over the bank.  Against a lane per slice with 32 activations
 // of every row: 17408 x 5120, HQ4_G32_M5, 1 / 2 / 3 / 8 rows 18.6 / 21.6 / 29.9 / 57.0 -> 16.1 / 19.3 / 25.9 / 39.1 us;
-// 5120 x 1024, 4-bit, 5.7 / 8.3 / 10.6 / 21.4 -> 4.6 / 5.4 / 6.2 / 10.0 us.
+// 5120 x 1024, 4-bit, 5.7 / 8.3 / 10.6 / 21.4 -> 4.6 / 5.4 / 6.2 / 10.0 us.  One and two rows of several K ranges are bound by the
+// activations, which every workgroup reads (1 x 4096 x 32768, 4-bit 17.2 us in the old form, 18.6 with four lanes asking for the
+// same 32 columns at the start of each range, 17.8 with a quarter each and a range ahead; 2 x 4096 x 16384, 8-bit 16.8, 18.3, 16.9).
 //
 // Arithmetic: all in fp32.  The reference dequantises one weight as fma(float(code [+ 1024]), scale, bias) in fp32 and
 // feeds an fp32 FMA chain (qwg_unpack_hq4_word8_f32 / qwg_dot_hq4_block_f32_reg, qw_dequant_f32.metalh:10-58); here the
@@ -131,16 +133,38 @@ static __device__ __forceinline__ void run(const qf_params& p) {
             i_left = nmax;
         }
     };
-    // activations of a K range, zero for slices past the row's end; rows past M re-read row M - 1
-    f4_t xv[XR][8];
+    // activations of a K range, zero for slices past the row's end; rows past M re-read row M - 1.  In the vector form the four lanes
+    // of a block hold the same 32: each asks for a quarter, a range ahead, and the block exchanges them.
+    f4_t xv[XR][8], xq[MV ? XR : 1][2];
     auto load_x = [&](uint32_t kr) {
         uint32_t ho, po;
         const uint32_t g = slice_of(kr, ho, po);
 #pragma unroll
         for (int mg = 0; mg < XR; ++mg) {
-            const float* xp = p.x + (uint64_t)min(MV ? (uint32_t)mg : 4u * mg + j, p.M - 1u) * p.K + (uint64_t)g * 32u;
+            const float* xp = p.x + (uint64_t)min(MV ? (uint32_t)mg : 4u * mg + j, p.M - 1u) * p.K + (uint64_t)g * 32u + (MV ? 8u * j : 0u);
 #pragma unroll
-            for (int t = 0; t < 8; ++t) xv[mg][t] = *(const f4_t*)(xp + 4 * t);
+            for (int t = 0; t < (MV ? 2 : 8); ++t) {
+                if constexpr (MV != 0) xq[mg][t] = *(const f4_t*)(xp + 4 * t);
+                else xv[mg][t] = *(const f4_t*)(xp + 4 * t);
+            }
+        }
+    };
+    auto spread_x = [&]() {
+        if constexpr (MV != 0) {
+#pragma unroll
+            for (int mg = 0; mg < XR; ++mg) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float e = xq[mg][t][i];   // (the compiler's bit cast of a vector's element takes element 0)
+                        xv[mg][t][i] = QF_DPP_F32(e, 0x00);        // quad_perm [l,l,l,l]: lane l of the block holds 8 l .. 8 l + 7
+                        xv[mg][2 + t][i] = QF_DPP_F32(e, 0x55);
+                        xv[mg][4 + t][i] = QF_DPP_F32(e, 0xAA);
+                        xv[mg][6 + t][i] = QF_DPP_F32(e, 0xFF);
+                    }
+                }
+            }
         }
     };
     load_x(0);
@@ -150,7 +174,12 @@ static __device__ __forceinline__ void run(const qf_params& p) {
     __builtin_amdgcn_sched_barrier(0);
 
     for (uint32_t kr = 0; kr < p.nkr; ++kr) {
-        if (kr > 0u) load_x(kr);
+        if constexpr (MV != 0) {
+            spread_x();
+            if (kr + 1u < p.nkr) load_x(kr + 1u);
+        } else {
+            if (kr > 0u) load_x(kr);
+        }
         const bool gvalid = (kr * wpr + wv) * 16u + b < p.nsl;
         float S[XR];
 #pragma unroll
@@ -359,9 +388,11 @@ void qw_f32_gemv(hipStream_t st, const qwhip_weight_view* w, int fmt, uint32_t g
     // at most 12 waves per row set (768 threads); longer rows take several K ranges
     const uint32_t nkr = (nch + 11u) / 12u;
     const uint32_t wpr = (nch + nkr - 1u) / nkr;
-    const uint32_t sets = max(1u, 12u / wpr);
-    const uint32_t threads = 64u * wpr * sets;
     const uint32_t nquads = (w->n + 3u) / 4u;
+    // a row set fewer for every 256 quads that are missing: a workgroup of one quad beats a third of the compute units with three
+    // (one row, K = 2048: 128 and 1024 rows 4.8 -> 3.1 us, 8-bit 5.6 -> 3.1; 64 x 1024, three rows 6.4 -> 3.2)
+    const uint32_t sets = max(1u, min(12u / wpr, nquads / 256u));
+    const uint32_t threads = 64u * wpr * sets;
     uint32_t wgs = max(1u, min(256u * max(1u, 12u / (wpr * sets)), nquads / sets));
     // the partial sums of a workgroup's rows stay in LDS: more, smaller workgroups when the bank has very many rows
     auto lds_of = [&](uint32_t g) { return (size_t)qwhip_cdiv(nquads, g) * (wpr * 4u) * (4u * mr) * 16u; };

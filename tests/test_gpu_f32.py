@@ -154,6 +154,27 @@ def test_f32_row_quads_and_k_ranges(dev, fmt, n, k, m):
     assert qo.normalized_error(got, want) <= TOL
 
 
+# banks of a few quads to a few hundred (one to six row sets a workgroup), one to six K ranges
+@pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq8_g32", "hq6_g32", "aq2_g64"])
+@pytest.mark.parametrize("n,k", [(3, 2048), (513, 1024), (2100, 1024), (1030, 2048), (70, 6400), (40, 12352), (5, 32768)])
+def test_f32_one_and_two_rows_equal_rows_together(dev, fmt, n, k):
+    """The vector form, its activations asked for a K range ahead, gives the matrix form's bits."""
+    x = H.make_x(5, k, 19)
+    outs = []
+    blocks, _ = H.make_bank(fmt, n, k, 18)
+    bank, xb, yb = dev.put(blocks), dev.put(x), dev.alloc(5 * n * 4)
+    v = H.view_of(dev, bank, fmt, n, k)
+    for row, m in ((0, 5), (0, 1), (1, 2), (4, 1)):
+        qwhip.check(dev.lib.qwhip_gemv_f32(dev.stream.handle, C.byref(v), xb.ptr + row * k * 4, m, 0, 1.0, yb.ptr))
+        outs.append(yb.download(np.float32, (m, n)))
+    kind, bits, group, is_m5, _ = H.FORMATS[fmt]
+    assert qo.normalized_error(outs[0], qo.gemv_f32(blocks, x, bits, group, is_m5)) <= TOL
+    for got, row in zip(outs[1:], (0, 1, 4)):
+        assert np.array_equal(got.view(np.uint32), outs[0][row : row + len(got)].view(np.uint32)), row
+    for b in (bank, xb, yb):
+        b.free()
+
+
 def test_h32_f32_is_the_reference_butterfly(dev):
     """qwhip_h32_f32 against the golden-pinned fp32 FWHT (same butterfly order: equal bits), out of place and in place."""
     x = H.make_x(9, 1280, 5)
