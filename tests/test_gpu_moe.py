@@ -75,8 +75,8 @@ def test_router_gemm(dev, xdt):
 
 @pytest.mark.parametrize("t,e,h,wdt", [(19, 128, 2048, "f32"), (5, 64, 4096, "bf16"), (33, 40, 5120, "f32"), (3, 8, 16384, "f16")])
 def test_router_gemm_shared_gate_and_wide_rows(dev, t, e, h, wdt):
-    """The shared-expert gate column sigmoid(x . w) beside the logits, on hidden sizes that take 8, 4, 2 and 1 token rows
-    per workgroup; the logits are those of the plain door bit for bit."""
+    """The shared-expert gate column sigmoid(x . w) beside the logits, on hidden sizes up to the largest; the logits are those of
+    the plain door bit for bit."""
     rng = np.random.default_rng(4)
     x = rng.standard_normal((t, h)).astype(np.float32)
     wr = (rng.standard_normal((e, h)) * 0.05).astype(np.float32)
@@ -107,9 +107,9 @@ def test_router_gemm_shared_gate_and_wide_rows(dev, t, e, h, wdt):
 @pytest.mark.parametrize("t,e,h", [(1, 1, 32), (1, 65, 2080), (2, 16, 64), (16, 17, 2048), (17, 33, 1056), (300, 130, 544), (1025, 257, 96)])
 def test_router_gemm_tiles(dev, t, e, h, xdt, wdt):
     """One row, the edges of the 16-row tiles, both tile widths and hidden sizes that leave a wave without a chunk, with the gate
-    column.  Every product and sum is fp32 (bf16 products hold all bits of the activations): h sums of relative size 2^-24 stay
-    below h 2^-24 of the sum of magnitudes, which for signs as they fall is sqrt(h) times the result - 2e-5 at h = 2080 at most,
-    2e-6 where the roundings fall either way."""
+    column.  Every product and sum is fp32 (bf16 products hold all bits of the activations).  A chain has at most 40 terms at
+    h = 2080; roundings of 2^-24 that fall either way leave sqrt(40) 2^-24 = 4e-7 of the result, and the bar is five times that
+    (all the same way they would leave 40 2^-24 = 2.4e-6)."""
     rng = np.random.default_rng(t + e + h)
     cast = {"f32": (lambda v: (v, qwhip.F32, v)), "f16": (lambda v: (v.astype(np.float16), qwhip.F16, v.astype(np.float16).astype(np.float32))),
             "bf16": (lambda v: (qo.f32_to_bf16_bits(v), qwhip.BF16, qo.round_bf16(v)))}
@@ -123,6 +123,46 @@ def test_router_gemm_tiles(dev, t, e, h, xdt, wdt):
     assert qo.normalized_error(got, xv.astype(np.float64) @ wv.astype(np.float64).T) <= 2e-6
     np.testing.assert_allclose(gate, qo.router_shared_gate_f64(xv, shw), rtol=0, atol=2e-6)
     for b in (xb, wb, sb, lb, go):
+        b.free()
+
+
+def _router_operands(rng, t, e, h, xdt, wdt):
+    cast = {"f32": (lambda v: (v, qwhip.F32, v)), "f16": (lambda v: (v.astype(np.float16), qwhip.F16, v.astype(np.float16).astype(np.float32))),
+            "bf16": (lambda v: (qo.f32_to_bf16_bits(v), qwhip.BF16, qo.round_bf16(v)))}
+    return cast[xdt](rng.standard_normal((t, h)).astype(np.float32)), cast[wdt]((rng.standard_normal((e, h)) * 0.05).astype(np.float32))
+
+
+@pytest.mark.parametrize("xdt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("wdt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("t,e,h", [(2048, 128, 2048), (1025, 257, 1056), (1024, 161, 2080)])
+def test_router_gemm_trips_of_the_wide_tile(dev, t, e, h, xdt, wdt):
+    """From 160 tiles of 64 weight rows on: whole trips of the unrolled loop, a trip that ends early, a second one; same bar as above."""
+    (xh, xcode, xv), (wh, wcode, wv) = _router_operands(np.random.default_rng(e), t, e, h, xdt, wdt)
+    xb, wb, lb = dev.put(xh), dev.put(wh), dev.alloc(t * e * 4)
+    qwhip.check(dev.lib.qwhip_router_gemm(dev.stream.handle, xb.ptr, xcode, wb.ptr, wcode, t, e, h, lb.ptr))
+    assert qo.normalized_error(lb.download(np.float32, (t, e)), xv.astype(np.float64) @ wv.astype(np.float64).T) <= 2e-6
+    for b in (xb, wb, lb):
+        b.free()
+
+
+@pytest.mark.parametrize("xdt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("wdt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("t", [1, 2, 3, 9])
+@pytest.mark.parametrize("h,skew", [(100, 0), (1000, 0), (1056, 1)])
+def test_router_gemm_of_any_hidden_size_and_alignment(dev, h, skew, t, xdt, wdt):
+    """Hidden sizes that are no multiple of 32 and rows that begin one element past a 16-byte boundary, in tiles of one to eight token
+    rows, with the gate; chains of up to 17 terms a lane, 64 lanes."""
+    e = 37
+    rng = np.random.default_rng(h + t)
+    (xh, xcode, xv), (wh, wcode, wv) = _router_operands(rng, t, e, h, xdt, wdt)
+    shw = (rng.standard_normal(h) * 0.03).astype(np.float32)
+    put = lambda a: dev.put(np.concatenate([np.zeros(skew, a.dtype), a.ravel()]))  # noqa: E731
+    xb, wb, sb, lb, gb = put(xh), put(wh), put(shw), dev.alloc(t * e * 4), dev.alloc(t * 4)
+    qwhip.check(dev.lib.qwhip_router_gemm_shared_gate(dev.stream.handle, xb.ptr + skew * xh.itemsize, xcode, wb.ptr + skew * wh.itemsize, wcode, t, e, h,
+                                                      lb.ptr, sb.ptr + 4 * skew, gb.ptr))
+    assert qo.normalized_error(lb.download(np.float32, (t, e)), xv.astype(np.float64) @ wv.astype(np.float64).T) <= 2e-6
+    np.testing.assert_allclose(gb.download(np.float32, (t,)), qo.router_shared_gate_f64(xv, shw), rtol=0, atol=2e-6)
+    for b in (xb, wb, sb, lb, gb):
         b.free()
 
 
@@ -674,6 +714,12 @@ def test_fused_route_gateup_decode_equals_the_two_launches(dev, fmt, t, experts,
     assert np.array_equal(a1.download(np.uint16, (t, k, inter)), a2.download(np.uint16, (t, k, inter)))
     ref_idx, ref_w = qo.moe_route(logits, k, True, 2.5)
     assert np.array_equal(i1.download(np.int32, (t, k)), ref_idx)
+
+
+@pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq4_g32"])
+@pytest.mark.parametrize("t,experts", [(2, 300), (1, 512)])
+def test_fused_route_gateup_decode_with_eight_experts_a_lane(dev, fmt, t, experts):
+    test_fused_route_gateup_decode_equals_the_two_launches(dev, fmt, t, experts, 256, 64, 3)
 
 
 def test_online_quantizer_writes_the_packers_bytes(dev):
