@@ -223,8 +223,8 @@ qwhip_status qwhip_gemv_silu_pair(qwhip_stream_t s, const qwhip_weight_view* w, 
  * every container width (2, 3, 4, 6, 8 bits and HQ4_G32_M5).  All arithmetic in fp32: weights are code * scale + bias
  * without the f16 rounding of qwhip_dequant_f16, as in the reference's f32 dequant (qw_dequant_f32.metalh:1-24).
  * epi: 0 none, 1 silu(y / scale), 2 sigmoid(y), 3 silu(y / scale) followed by the FWHT-32 over each 32 consecutive outputs
- * (a last partial group is padded with zeros).  Up to 31 rows: four activation rows share one pass over the bank, all
- * arithmetic in fp32.  From 32 rows on (where the reference switches to its batched kernels) and k % 64 == 0: the
+ * (a last partial group is padded with zeros).  Up to 31 rows: eight activation rows share one pass over the bank, all
+ * arithmetic in fp32, a row's bits whatever the row count.  From 32 rows on (where the reference switches to its batched kernels) and k % 64 == 0: the
  * matrix-core form, 64 activation rows per pass over the bank; activations and weights are each split into two f16
  * numbers (22 bits together) and three products are accumulated in fp32 - the same 2e-5 bar.  Every activation row is
  * scaled by a power of two into the f16 range before its split and back at the store (one small launch into the
@@ -333,7 +333,8 @@ qwhip_status qwhip_moe_route_ex(qwhip_stream_t s, const float* logits, uint32_t 
                                 const float* scale_param, int32_t* idx, float* wts);
 
 /* qwg_router_gemm (qwrouter.metal:460-; encodeFnRouterGemm, QWGemmMoERouter.swift:78-113):
- * logits[t, e] = sum_h x[t, h] * Wr[e, h]; x f16/bf16/f32, Wr f32/f16/bf16, fp32 accumulate. */
+ * logits[t, e] = sum_h x[t, h] * Wr[e, h]; x f16/bf16/f32, Wr f32/f16/bf16, fp32 accumulate.  A token's logits are the same bits
+ * whatever rows and experts the call has (for x and Wr at one alignment: hidden a multiple of 32 and 16-byte aligned rows, or not). */
 /* QWGemm.encodeF32Gemv (QWGemmF32.swift:117-141) -> qwg_f32_gemv / qwg_f32_gemv_bm (qwgemm_f32.metal:120-143): dense fp32
  * weights w [n, k], fp32 rows x [rows, k]: y[t, n] = epilogue(w[n] . x[t]); epi 0 none, 1 silu(y / scale), 2 sigmoid(y),
  * 3 2 sigmoid(y / scale).  k up to 16384. */
@@ -417,14 +418,16 @@ qwhip_status qwhip_moe_combine(qwhip_stream_t s, const void* dn, uint32_t dn_dty
  * (QWGemmMoE.swift:120-199) -> Sources/QWMetal/include/qw_moe_f32_common.metalh:187-452.
  * gate_up: act16 [t, top_k, inter] = f16(FWHT32(silu(Wg[e].x) * (Wu[e].x))), SwiGLU on fp32 accumulators.
  * down:    out [t, hidden] = sum_k wts[t,k] * Wd[e_k] . act16[t,k]  (+ shared_gate[t]*shared[t]).
- * gate_up flags: QWHIP_X_PREROTATED, QWHIP_MOE_REUSE_EXPERTS; bits 8..11 = 2 keep an HQ4_G32_M5 bank on the general
- * kernel (tests). */
+ * Weights are the container's code * scale + bias, not rounded to f16, for hidden up to 16384 (gate_up) and top_k * inter up to 32768 (down);
+ * longer rows and bits 8..11 = 2 of gate_up's flags (tests) take the general kernel and its f16 weights.  gate_up flags:
+ * QWHIP_X_PREROTATED, QWHIP_MOE_REUSE_EXPERTS. */
 qwhip_status qwhip_moe_gateup_decode(qwhip_stream_t s, const qwhip_weight_view* w_gate_up, uint32_t experts,
                                      const void* x, uint32_t x_dtype, uint32_t flags, const int32_t* idx, uint32_t t,
                                      uint32_t top_k, void* act16);
-/* qwhip_moe_route + qwhip_moe_gateup_decode as one launch for the decode step (an HQ4_G32_M5 bank routes inside the gate_up
+/* qwhip_moe_route + qwhip_moe_gateup_decode as one launch for the decode step (every container routes inside the gate_up
  * kernel: every workgroup repeats the token's top-k from its router logits with the arithmetic of qwhip_moe_route and
- * leaves idx / wts [t, top_k] for the down projection; other containers run the two launches).  Same results as the two
+ * leaves idx / wts [t, top_k] for the down projection; shapes past that kernel - hidden over 16384, expert banks of 4 GiB - run the
+ * two launches).  Same results as the two
  * calls; one kernel launch less on a path that is bound by launch latency.  The reference runs encodeFnMoeRoute and
  * encodeMoEGateUpF32R1 back to back (QWMoEOperator.swift); arguments as in those two doors. */
 qwhip_status qwhip_moe_route_gateup_decode(qwhip_stream_t s, const qwhip_weight_view* w_gate_up, uint32_t experts,

@@ -490,7 +490,7 @@ public enum QWGemm {
         try qwCheck(qwhip_moe_gateup_decode(enc.stream, &w, UInt32(experts), x.ptr, x.dtype.rawValue, flags,
                                             ids.i32, UInt32(tokens), UInt32(routes), out.ptr))
     }
-    /// encodeMoEGateUpF32R1 with fuseSiluFwht (QWGemmMoE.swift:120-155), routing folded into the launch for an HQ4_G32_M5 bank.
+    /// encodeMoEGateUpF32R1 with fuseSiluFwht (QWGemmMoE.swift:120-155), routing folded into the launch.
     public static func encodeMoERouteGateUp(_ enc: QWHipEncoder, hal: QWHal, x: QWTensorValue, bank: QWWeightView, experts: Int,
                                             logits: QWTensorValue, idx: QWTensorValue, wts: QWTensorValue, out: QWTensorValue,
                                             routes: Int, tokens: Int, normTopK: Bool, routedScale: Float, xIsRotated: Bool = true,
