@@ -285,8 +285,8 @@ def test_rmsnorm_with_rotation_matches_oracle(dev, rows, hidden, residual, rotat
 @pytest.mark.parametrize("hidden", [256, 4352, 5376, 8192, 8448, 16384])
 @pytest.mark.parametrize("residual", [0, 1])
 def test_rmsnorm_rows_do_not_depend_on_the_row_count(dev, hidden, residual):
-    """Many rows run in more sweeps of fewer threads: the same bits as one row alone, at row lengths that fill the last 512 columns
-    of the sum or leave them part empty."""
+    """Many rows run in more sweeps of fewer threads: the same bits as one row alone, at row lengths that fill the last sweep or
+    leave it part empty."""
     rows = 600
     rng = np.random.default_rng(hidden)
     x16 = (rng.standard_normal((rows, hidden)) * 1.5).astype(np.float16)
