@@ -355,6 +355,47 @@ def test_fused_gate_up_swiglu_equals_the_two_step_chain(dev, fmt, t, experts, hi
     assert qo.normalized_error(one.astype(np.float32), want) <= TOL
 
 
+_SPANS_FEW = [1, 16, 17, 0, 32, 33, 63, 64, 65, 2]                  # at most 48 rows an expert: spans of 64
+_SPANS_MANY = [31, 64, 96, 97, 0, 128, 129, 160, 161, 225, 300]     # spans of 128 (96 on the 6- and 8-bit containers)
+
+
+@pytest.mark.parametrize("fmt", sorted(H.FORMATS))
+@pytest.mark.parametrize("counts,k,inter,xdt,compact", [(_SPANS_FEW, 128, 96, "f16", True), (_SPANS_FEW, 384, 32, "bf16", False),
+                                                        (_SPANS_MANY, 384, 96, "f16", False), (_SPANS_MANY, 128, 160, "bf16", True)])
+def test_grouped_gemm_spans(dev, fmt, counts, k, inter, xdt, compact):
+    """Experts of every span shape (fragment edges, the last row of a span, empty experts), one and three pairs of K-steps, partial
+    column tiles: fp32 sums of k exact products against fp64, f16 and bf16 as their roundings, the fused gate|up bit for bit."""
+    if fmt in ("aq8_g256",):
+        k = 256 * (k // 128)                                          # whole groups; takes the 64-row kernel
+    e, n = len(counts), 2 * inter
+    blocks, w16 = H.make_bank(fmt, e * n, k, seed=21)
+    rng = np.random.default_rng(k + inter)
+    ids = rng.permutation(np.repeat(np.arange(e), counts)).astype(np.int32).reshape(-1, 1)
+    pairs = ids.size
+    x, xcode, xval = _hidden_rows(rng, pairs, k, xdt)
+    g = _group(dev, ids, e, 1, compact)
+    lib, st, b = dev.lib, dev.stream.handle, g["bufs"]
+    bank, xb = dev.put(blocks), dev.put(x)
+    view = H.view_of(dev, bank, fmt, e * n, k)
+    plan = (b["stok"].ptr, b["off"].ptr, b["te"].ptr, b["tr"].ptr, b["tc"].ptr, g["max_tiles"], pairs)
+    y32, y16, yb = dev.alloc(pairs * n * 4), dev.alloc(pairs * n * 2), dev.alloc(pairs * n * 2)
+    act1, act2 = dev.alloc(pairs * inter * 2), dev.alloc(pairs * inter * 2)
+    for y, dt in ((y32, qwhip.F32), (y16, qwhip.F16), (yb, qwhip.BF16)):
+        qwhip.check(lib.qwhip_moe_grouped_gemm(st, C.byref(view), e, xb.ptr, xcode, 0, *plan, y.ptr, dt, 0))
+    qwhip.check(lib.qwhip_moe_grouped_gemm_swiglu(st, C.byref(view), e, xb.ptr, xcode, 0, *plan, 1, act1.ptr, 0))
+    qwhip.check(lib.qwhip_swiglu_fwht(st, y16.ptr, qwhip.F16, act2.ptr, pairs, inter, 1))
+    dev.stream.sync()
+    w = w16.reshape(e, n, k).astype(np.float64)
+    xs = xval.astype(np.float16).astype(np.float64)[g["stok"]]
+    want = np.concatenate([xs[g["off"][i]:g["off"][i + 1]] @ w[i].T for i in range(e)])
+    size = np.concatenate([np.abs(xs[g["off"][i]:g["off"][i + 1]]) @ np.abs(w[i]).T for i in range(e)])
+    got = y32.download(np.float32, (pairs, n))
+    assert np.all(np.abs(got - want) <= k * 2.0 ** -24 * size)        # k rounded additions of exact products
+    assert np.array_equal(y16.download(np.float16, (pairs, n)), got.astype(np.float16))
+    assert np.array_equal(yb.download(np.uint16, (pairs, n)), qo.f32_to_bf16_bits(got))
+    assert np.array_equal(act1.download(np.uint16, (pairs, inter)), act2.download(np.uint16, (pairs, inter)))
+
+
 def test_fused_gate_up_swiglu_refusals(dev):
     blocks, _ = H.make_bank("hq4_g32_m5", 4 * 2 * 48, 64, 1)
     bank, xb, act = dev.put(blocks), dev.put(np.zeros((4, 64), np.float16)), dev.alloc(4096)
