@@ -1280,6 +1280,14 @@ qwhip_status gemm_checks(qwhip_stream_t s, const qwhip_weight_view* w, const voi
 }
 
 // runs EXPR with F bound to the container format as a constant
+// the sum of fp32 planes [splits][M][N] into y, in range order
+hipError_t launch_plane_sum(hipStream_t st, const qw_gemm_params& p, uint32_t splits, const float* part, void* y, uint32_t y_dtype, uint32_t ldy) {
+    const dim3 rgrid((unsigned)(((uint64_t)p.M * (p.N / 4u) + 255u) / 256u));
+    if (y_dtype == QWHIP_F16) hipLaunchKernelGGL(qw_splitk_reduce_kernel<QWHIP_F16>, rgrid, dim3(256), 0, st, part, splits, p.M, p.N, y, ldy);
+    else if (y_dtype == QWHIP_BF16) hipLaunchKernelGGL(qw_splitk_reduce_kernel<QWHIP_BF16>, rgrid, dim3(256), 0, st, part, splits, p.M, p.N, y, ldy);
+    else hipLaunchKernelGGL(qw_splitk_reduce_kernel<QWHIP_F32>, rgrid, dim3(256), 0, st, part, splits, p.M, p.N, y, ldy);
+    return hipGetLastError();
+}
 // split-K launch of the half-height ping-pong tile into fp32 planes at `part`, then the sum into y
 template <int FMT>
 hipError_t launch_splitk(hipStream_t st, const qw_gemm_params& p, uint32_t splits, float* part, void* y, uint32_t y_dtype, uint32_t ldy) {
@@ -1293,11 +1301,7 @@ hipError_t launch_splitk(hipStream_t st, const qw_gemm_params& p, uint32_t split
         hipError_t e = p.x_bf16 ? launch_cfg3<1, 5, 4, 2, FMT, QWHIP_F32, false, QWHIP_BF16>(st, q, grid)
                                 : launch_cfg3<1, 5, 4, 2, FMT, QWHIP_F32>(st, q, grid);
         if (e != hipSuccess) return e;
-        const dim3 rgrid((unsigned)(((uint64_t)p.M * (p.N / 4u) + 255u) / 256u));
-        if (y_dtype == QWHIP_F16) hipLaunchKernelGGL(qw_splitk_reduce_kernel<QWHIP_F16>, rgrid, dim3(256), 0, st, part, splits, p.M, p.N, y, ldy);
-        else if (y_dtype == QWHIP_BF16) hipLaunchKernelGGL(qw_splitk_reduce_kernel<QWHIP_BF16>, rgrid, dim3(256), 0, st, part, splits, p.M, p.N, y, ldy);
-        else hipLaunchKernelGGL(qw_splitk_reduce_kernel<QWHIP_F32>, rgrid, dim3(256), 0, st, part, splits, p.M, p.N, y, ldy);
-        return hipGetLastError();
+        return launch_plane_sum(st, p, splits, part, y, y_dtype, ldy);
     }
 }
 
@@ -1317,6 +1321,57 @@ uint32_t choose_splits(uint32_t m, uint32_t n, uint32_t k, uint64_t used, uint64
     return splits < 2u ? 0u : splits;
 }
 
+// The direct-operand kernel (qw_direct.h) for problems of a few rows to about a thousand: spans of 64 or 128 rows by 256 weight
+// rows, K in whole pairs of 64 over 1 .. 12 ranges.  A workgroup's loop costs 0.68 us a pair and 0.24 a fragment of rows
+// (1.34 times that on the 6- and 8-bit containers), a start and an end 7.1 us; ranges add the planes' traffic, at 7.9 TB/s, and
+// the summing launch; the ping-pong kernel is priced the same way (a K-step 1.36 us in a range, 2.35 and 1.66 a round of its
+// tiles, 0.88 on the 128 x 128 tiles).  Fitted to 224 problems, 20 .. 2000 rows on 13 banks of 7 containers, every combination
+// measured (10 % and 9 % of root mean square error); it is taken where it prices below 0.85 of the other, where the fit held: 64 rows on
+// 7168 x 5120 27 -> 20 us, 333 rows on 2560 x 9728 39 -> 36, gate|up of 333 rows on 2 x 9728 x 2560 61 -> 47, 180 rows on
+// 6144 x 16384 80 -> 56; over all of them 1.18 times as fast, 8 of them slower, by 7 % at most.
+struct direct_plan {
+    bool take, few;
+    uint32_t splits;
+};
+direct_plan choose_direct(const qwhip_weight_view* w, uint32_t m, int fmt, uint32_t old_splits, uint64_t plane_room) {
+    direct_plan best = {false, false, 1u};
+    const uint32_t n = w->n, k = w->k;
+    if (k % 128u != 0 || w->group > 128u || 256u * qwhip_view_row_bytes(w) >= (1ull << 32)) return best;
+    const bool wide = fmt == QG_FMT_B8 || fmt == QG_FMT_B6;
+    const double plane = (double)m * n * 4.0;
+    const uint32_t nk = k / 64u, pairs = nk / 2u, frags = qwhip_cdiv(m, 32u), cols = qwhip_cdiv(n, 256u);
+    double limit;
+    if (old_splits >= 2u) {
+        limit = 7.4 + qwhip_cdiv(nk, old_splits) * 1.36 * (wide ? 1.1 : 1.0) + old_splits * plane * 2.0 / 6.3e6;
+    } else {
+        double step = min(1.66 * priced_rounds((double)qwhip_cdiv(m, 128u) * qwhip_cdiv(n, 320u), 256.0),
+                          2.35 * priced_rounds((double)qwhip_cdiv(m, 256u) * qwhip_cdiv(n, 320u), 256.0));
+        if ((uint64_t)qwhip_cdiv(m, 128u) * qwhip_cdiv(n, 128u) <= 256u) step = min(step, 0.88);
+        limit = 5.4 + nk * step * (wide ? 1.1 : 1.0);
+    }
+    limit *= 0.85;
+    const double bank_us = 7.1 + (double)n * (double)qwhip_view_row_bytes(w) / 3.5e6;   // and no faster than the bank streams to this kernel
+    for (uint32_t few = 0; few < 2u; ++few) {
+        const uint32_t span = few ? 2u : wide ? 3u : 4u;
+        if (!few && frags <= 2u) continue;
+        const uint32_t spans = qwhip_cdiv(frags, span);
+        const double per_pair = (0.68 + 0.24 * min(span, qwhip_cdiv(frags, spans))) * (wide ? 1.34 : 1.0);
+        for (uint32_t splits = 1; splits <= min(12u, pairs); ++splits) {
+            const uint32_t per = qwhip_cdiv(pairs, splits);
+            if (splits > 1u && (m > 1024u || n % 4u != 0 || (splits - 1u) * per >= pairs || splits * plane > (double)plane_room)) continue;
+            const double load = (double)spans * cols * splits / 256.0;
+            const double rounds = load <= 1.0 ? 1.0 : load <= 2.0 ? 2.0 : load + 0.4;
+            double t = 7.1 + per * per_pair * rounds;
+            if (t < bank_us) t = bank_us;
+            if (splits > 1u) t += 1.6 + 0.19 * splits + splits * plane * 2.0 / 7.9e6;
+            if (t < limit) {
+                limit = t;
+                best = {true, few != 0u, splits};
+            }
+        }
+    }
+    return best;
+}
 #define QG_FOR_FMT(fmt, e, EXPR)                                                  \
     switch (fmt) {                                                                \
         case QG_FMT_M5: { constexpr int F = QG_FMT_M5; e = (EXPR); } break;       \
@@ -1367,12 +1422,17 @@ extern "C" qwhip_status qwhip_gemm(qwhip_stream_t s, const qwhip_weight_view* w,
     const bool copy_needed = rotate || (x_dtype == QWHIP_BF16 && (flags & (1u << 16)));   // bf16 rows in the basis are read in place
     const uint64_t sk_used = copy_needed ? ((ws_need + 255u) & ~(uint64_t)255u) : 0u;
     uint32_t splits = 0;
-    if (ov == 0u && pp_ok && workspace && ((uintptr_t)workspace & 15u) == 0 && w->n % 4u == 0 && (!copy_needed || ws_ok))
-        splits = choose_splits(m, w->n, w->k, sk_used, workspace_bytes);
+    const bool planes_ok = workspace && ((uintptr_t)workspace & 15u) == 0 && (!copy_needed || ws_ok);
+    if (ov == 0u && pp_ok && planes_ok && w->n % 4u == 0) splits = choose_splits(m, w->n, w->k, sk_used, workspace_bytes);
+    direct_plan direct = {};
+    if (ov == 0u && pp_ok)
+        direct = choose_direct(w, m, fmt, splits, planes_ok && workspace_bytes > sk_used ? workspace_bytes - sk_used : 0u);
     // bf16 activations already in the basis: the ping-pong kernel converts them while it stages the tile (no pass of its own,
     // no workspace); flags bit 16 keeps the separate pass, for tests and comparisons
     const bool direct_bf16 = !rotate && x_dtype == QWHIP_BF16 && ov != 15u && !(flags & (1u << 16)) && (splits != 0u || gemm3_takes(p, cfg, fmt, y_dtype));
-    if (direct_bf16) {
+    if (direct.take && !copy_needed) {
+        // rows in the basis, f16 or bf16, are read in place
+    } else if (direct_bf16) {
         p.x_bf16 = 1u;
         xdt = QWHIP_F16;   // dispatch as the f16 kernels do; the kernel itself reads bf16
     } else if (rotate) {
@@ -1403,6 +1463,18 @@ extern "C" qwhip_status qwhip_gemm(qwhip_stream_t s, const qwhip_weight_view* w,
     p.bb = qwhip_view_block_bytes(w);
     p.row_bytes = qwhip_view_row_bytes(w);
     hipError_t e;
+    if (direct.take) {
+        if (direct.splits == 1u) {
+            QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, p, 1u, xdt, y_dtype, false, direct.few));
+            return QWHIP_OK;
+        }
+        qw_gemm_params q = p;
+        q.y = (uint8_t*)workspace + sk_used;
+        q.ldy = p.N;
+        QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, q, direct.splits, xdt, QWHIP_F32, false, direct.few));
+        QWHIP_TRY_HIP(launch_plane_sum(s->stream, p, direct.splits, (const float*)q.y, y, y_dtype, ldy));
+        return QWHIP_OK;
+    }
     if (splits != 0u && xdt == QWHIP_F16) {
         float* part = (float*)((uint8_t*)workspace + sk_used);
         QG_FOR_FMT(fmt, e, (launch_splitk<F>(s->stream, p, splits, part, y, y_dtype, ldy)))
@@ -1521,14 +1593,29 @@ extern "C" qwhip_status qwhip_gemm_swiglu(qwhip_stream_t s, const qwhip_weight_v
     {
         const uint64_t x_used = xin == workspace ? ((ws_need + 255u) & ~(uint64_t)255u) : 0u;
         const uint64_t gu_bytes = ((uint64_t)m * w->n * 2u + 255u) & ~(uint64_t)255u;
+        const bool tuned = ((flags >> 8) & 0xFu) != 0u;
+        const bool planes_ok = workspace && ((uintptr_t)workspace & 15u) == 0 && ldact == inter && workspace_bytes >= x_used + gu_bytes;
         uint32_t splits = 0;
-        if (((flags >> 8) & 0xFu) == 0u && workspace && ((uintptr_t)workspace & 15u) == 0 && ldact == inter && workspace_bytes >= x_used + gu_bytes)
-            splits = choose_splits(m, w->n, w->k, x_used + gu_bytes, workspace_bytes);
-        if (splits != 0u) {
+        if (!tuned && planes_ok) splits = choose_splits(m, w->n, w->k, x_used + gu_bytes, workspace_bytes);
+        direct_plan direct = {};
+        if (!tuned) direct = choose_direct(w, m, fmt, splits, planes_ok ? workspace_bytes - x_used - gu_bytes : 0u);
+        if (direct.take && direct.splits == 1u) {
+            QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, p, 1u, QWHIP_F16, QWHIP_F16, true, direct.few));
+            return QWHIP_OK;
+        }
+        if (direct.take || splits != 0u) {
             void* gu = (uint8_t*)workspace + x_used;
             float* part = (float*)((uint8_t*)workspace + x_used + gu_bytes);
             hipError_t e;
-            QG_FOR_FMT(fmt, e, (launch_splitk<F>(s->stream, p, splits, part, gu, QWHIP_F16, w->n)))
+            if (direct.take) {
+                qw_gemm_params q = p;
+                q.y = part;
+                q.ldy = w->n;
+                QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, q, direct.splits, QWHIP_F16, QWHIP_F32, false, direct.few));
+                e = launch_plane_sum(s->stream, p, direct.splits, part, gu, QWHIP_F16, w->n);
+            } else {
+                QG_FOR_FMT(fmt, e, (launch_splitk<F>(s->stream, p, splits, part, gu, QWHIP_F16, w->n)))
+            }
             QWHIP_TRY_HIP(e);
             return qwhip_swiglu_fwht(s, gu, QWHIP_F16, act_f16, m, inter, rotate_act);
         }

@@ -330,6 +330,41 @@ def test_gemm_swiglu_split_k_with_a_roomy_workspace(dev, fmt, m, inter, k, xdtyp
     assert qo.normalized_error(split.astype(np.float32), one.astype(np.float32)) <= TOL
 
 
+@pytest.mark.parametrize("fmt", sorted(f for f in H.FORMATS if f != "aq8_g256"))
+@pytest.mark.parametrize("m,n,k,xdtype,ws_mb", [(17, 272, 1920, "f16", 64), (65, 272, 2048, "bf16", 64), (33, 4112, 2048, "f16", 0),
+                                                (97, 4112, 2048, "bf16", 0), (333, 16384, 2048, "f16", 0)])
+def test_gemm_direct_operand_kernel(dev, fmt, m, n, k, xdtype, ws_mb):
+    """The direct-operand kernel where the price rule takes it: K ranges with a short last one, spans of 64 and of 128 rows (96 on the
+    6- and 8-bit containers), ragged rows, a partial column tile.  fp32 sums of k exact products against fp64; the 2-byte outputs
+    are their roundings, and the gate|up door gives the two doors' bits."""
+    blocks, w16 = H.make_bank(fmt, n, k, seed=31)
+    x32 = H.make_x(m, k, 7)
+    x_host, xcode = (qo.f32_to_bf16_bits(x32), qwhip.BF16) if xdtype == "bf16" else (x32.astype(np.float16), qwhip.F16)
+    xs = (qo.round_bf16(x32) if xdtype == "bf16" else x32).astype(np.float16).astype(np.float64)
+    bank, xb, ws = dev.put(blocks), dev.put(x_host), dev.alloc(max(1, ws_mb << 20))
+    view = H.view_of(dev, bank, fmt, n, k)
+    lib, st, flags = dev.lib, dev.stream.handle, qwhip.X_PREROTATED
+    wsp = (ws.ptr, ws_mb << 20) if ws_mb else (None, 0)
+    y32, y16, yb = dev.alloc(m * n * 4), dev.alloc(m * n * 2), dev.alloc(m * n * 2)
+    for y, dt in ((y32, qwhip.F32), (y16, qwhip.F16), (yb, qwhip.BF16)):
+        qwhip.check(lib.qwhip_gemm(st, C.byref(view), xb.ptr, xcode, m, 0, y.ptr, dt, 0, flags, *wsp))
+    dev.stream.sync()
+    got = y32.download(np.float32, (m, n))
+    w = w16.astype(np.float64)
+    assert np.all(np.abs(got - xs @ w.T) <= k * 2.0 ** -24 * (np.abs(xs) @ np.abs(w).T))      # k rounded additions of exact products
+    assert np.array_equal(y16.download(np.float16, (m, n)), got.astype(np.float16))
+    assert np.array_equal(yb.download(np.uint16, (m, n)), qo.f32_to_bf16_bits(got))
+    if xdtype == "f16" and n % 64 == 0:
+        act1, act2 = dev.alloc(m * n), dev.alloc(m * n)
+        qwhip.check(lib.qwhip_gemm_swiglu(st, C.byref(view), xb.ptr, xcode, m, 0, 1, act1.ptr, 0, flags, *wsp))
+        qwhip.check(lib.qwhip_swiglu_fwht(st, y16.ptr, qwhip.F16, act2.ptr, m, n // 2, 1))
+        dev.stream.sync()
+        assert np.array_equal(act1.download(np.uint16, (m, n // 2)), act2.download(np.uint16, (m, n // 2)))
+        act1.free(), act2.free()
+    for b in (bank, xb, ws, y32, y16, yb):
+        b.free()
+
+
 def test_gemm_swiglu_refusals(dev):
     blocks, _ = H.make_bank("hq8_g32", 128, 64, seed=1)
     bank, xb, act = dev.put(blocks), dev.put(np.zeros((64, 64), np.float16)), dev.alloc(64 * 64 * 2)
