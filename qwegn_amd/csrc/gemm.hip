@@ -18,9 +18,9 @@
 //
 // Grouped launches (MoE) take the tile list of the pair sort: tile t = (expert e, row block) over the
 // expert-major slot range [expert_off[e], expert_off[e+1]); slot rows are gathered through `gather`.
-#include <mutex>
-
+#include <algorithm>
 #include <atomic>
+#include <mutex>
 
 #include "qwhip_common.h"
 #include "qw_gemm.h"
@@ -1344,9 +1344,9 @@ direct_plan choose_direct(const qwhip_weight_view* w, uint32_t m, int fmt, uint3
     if (old_splits >= 2u) {
         limit = 7.4 + qwhip_cdiv(nk, old_splits) * 1.36 * (wide ? 1.1 : 1.0) + old_splits * plane * 2.0 / 6.3e6;
     } else {
-        double step = min(1.66 * priced_rounds((double)qwhip_cdiv(m, 128u) * qwhip_cdiv(n, 320u), 256.0),
-                          2.35 * priced_rounds((double)qwhip_cdiv(m, 256u) * qwhip_cdiv(n, 320u), 256.0));
-        if ((uint64_t)qwhip_cdiv(m, 128u) * qwhip_cdiv(n, 128u) <= 256u) step = min(step, 0.88);
+        double step = std::min(1.66 * priced_rounds((double)qwhip_cdiv(m, 128u) * qwhip_cdiv(n, 320u), 256.0),
+                               2.35 * priced_rounds((double)qwhip_cdiv(m, 256u) * qwhip_cdiv(n, 320u), 256.0));
+        if ((uint64_t)qwhip_cdiv(m, 128u) * qwhip_cdiv(n, 128u) <= 256u) step = std::min(step, 0.88);
         limit = 5.4 + nk * step * (wide ? 1.1 : 1.0);
     }
     limit *= 0.85;
