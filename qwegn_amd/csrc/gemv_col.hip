@@ -584,7 +584,7 @@ bool qw_col_gemv(hipStream_t st, const qwhip_weight_view* w, const void* x, uint
     const uint32_t wdepth = kWindow[kind <= 5u ? kind : 0u];       // 0: the compiled window
     // Waves per compute unit, measured on N = 17408, K = 5120.  Compiled window: 10 (11.2-11.3 us; 11.5 with 20, 13.5+ with
     // 5).  Hand-issued window: 20 (10.8-10.9 us on 1024 workgroups; 11.4 on 512 with the same window, 11.1 on 768; deeper
-    // windows 11.1-11.9, a window of two 11.3).  At least four rows per set, at most 128 row slots per workgroup.
+    // windows 11.1-11.9, a window of two 11.3).  At most 128 row slots per workgroup.
     uint32_t wgs = (256u * (wdepth ? 20u : 10u) + waves / 2u) / waves;
     // whole multiples of the 256 compute units: a grid that leaves some of them a workgroup more than the others was up to
     // 19 % slower (5120 x 17408: 569 workgroups 13.6 us, 512 workgroups 11.2 us; K = 6144 .. 18432 5-10 %)
@@ -592,10 +592,19 @@ bool qw_col_gemv(hipStream_t st, const qwhip_weight_view* w, const void* x, uint
     if ((tune >> 3 & 3u) == 1u) wgs /= 2u;
     if ((tune >> 3 & 3u) == 2u) wgs *= 2u;
     if ((tune >> 3 & 3u) == 3u) wgs += wgs / 2u;
-    wgs = min(wgs, max(1u, w->n / (sets * 4u)));
-    wgs = max(wgs, qwhip_cdiv(w->n, 128u));
-    if (!(tune & 0x40u) && wgs > 256u && wgs % 256u != 0u && (wgs + 255u) / 256u * 256u <= max(1u, w->n / (sets * 4u)))
-        wgs = (wgs + 255u) / 256u * 256u;                          // the row-slot limit raised the grid: up to the next whole multiple
+    // Banks under 20 MB are latency: one or two workgroups on every compute unit, down to two rows a set and on the smallest to one,
+    // rather than four rows a set on half of the units (us, before -> now: 3072 x 2048 3.23 -> 2.92, 2048 x 2048 3.22 -> 2.98, 2048 x 6144 5.10 ->
+    // 4.74, 4096 x 2560 4.60 -> 4.07, 2560 x 8192 5.65 -> 5.10, 6144 x 4096 5.31 -> 4.95, 1024 x 3072 3.72 -> 3.02, 5120 x 5120 level).
+    // Larger ones: at least two rows a set, whole multiples of the units (7168 x 5120: 896 workgroups 6.51 us, 1024 6.40)
+    if (wdepth && !(tune & 0x40u) && (tune >> 3 & 3u) == 0u && (uint64_t)w->n * nb * 20u < 20000000u) {
+        wgs = w->n >= sets * 1024u ? 512u : min(256u, max(1u, w->n / sets));
+        wgs = max(wgs, qwhip_cdiv(w->n, 128u));
+    } else {
+        wgs = min(wgs, max(1u, w->n / (sets * (wdepth ? 2u : 4u))));
+        wgs = max(wgs, qwhip_cdiv(w->n, 128u));
+        if (!(tune & 0x40u) && wgs > 256u && wgs % 256u != 0u && (wgs + 255u) / 256u * 256u <= max(1u, w->n / (sets * 4u)))
+            wgs = (wgs + 255u) / 256u * 256u;                      // the row-slot limit raised the grid: up to the next whole multiple
+    }
     const uint32_t rows_per_wg = qwhip_cdiv(w->n, wgs);
     // partial sums: one float per (row slot, chunk); the hand-issued window rounds the trip count up to whole groups and
     // stores every row slot of every group
@@ -646,9 +655,12 @@ bool qw_col_pair_gemv(hipStream_t st, const qwhip_weight_view* w, const void* x,
     const uint32_t sets = cpr <= 3u ? 4u : 2u, h2 = sets / 2u;
     const uint32_t threads = 32u * cpr * sets;
     const uint32_t waves = (threads + 63u) / 64u;
-    uint32_t wgs = (256u * 10u + waves / 2u) / waves;              // ten waves per compute unit, as the compiled window of the GEMV
-    wgs = max(256u, (wgs + 128u) / 256u * 256u);                   // whole multiples of the compute units
-    wgs = min(wgs, max(1u, inter / (h2 * 4u)));                    // at least four channels per set
+    // ten waves per compute unit, as the compiled window of the GEMV, in whole multiples of the units; three workgroups a unit up to six
+    // waves (2 x 8704 x 2560: 512 workgroups 8.06 us, 768 7.68; 2 x 17408 x 5120 level); at least two channels per set
+    // (2 x 2048 x 1024: four, 256 workgroups, 3.42 us; two, 512, 3.24)
+    uint32_t wgs = (256u * 10u + waves / 2u) / waves;
+    wgs = waves <= 6u ? 768u : max(256u, (wgs + 128u) / 256u * 256u);
+    wgs = min(wgs, max(1u, inter / (h2 * 2u)));
     wgs = max(wgs, qwhip_cdiv(inter, 64u));                        // at most 128 row slots per workgroup
     const uint32_t ch_per_wg = qwhip_cdiv(inter, wgs);
     const size_t lds = (size_t)nb * 80u + (size_t)2u * ch_per_wg * cpr * 4u;
