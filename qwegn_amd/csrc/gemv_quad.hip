@@ -14,8 +14,11 @@
 // Arithmetic is the factorised form of the reference's bit-stream GEMVs (qwg_aq_slice_dot,
 // Sources/QWMetal/include/qw_dequant_multi.metalh:205-208): the masked code words are the A operands as they are
 // (f16 subnormals q * 2^-24, 16 q * 2^-24 for the nibbles at bits 4..7 / 20..23), products exact, fp32 accumulation,
-// and  s * sum(q x) + b * sum(x)  per slice and row afterwards (HQ4_G32_M5: s * (sum(q x) + 1024 sum(x)) + b * sum(x),
-// unpack_hq4_word8, qw_dequant.metalh:42-62).  The header of row i reaches the lanes of its block by quad broadcast.
+// and  s * sum(q x) + b * sum(x)  per slice and row afterwards (HQ4_G32_M5: (1024 s + b) for b, unpack_hq4_word8,
+// qw_dequant.metalh:42-62).  The scale of row i reaches the lanes of its block by quad broadcast; b * sum(x) for four bank rows and
+// four activation rows is one more matrix instruction (K = 1, fp32), whose operands are the headers where they were loaded (against
+// four broadcasts and vector FMAs, 34816 x 5120, HQ4_G32_M5: 4 / 8 / 12 rows 22.8 / 33.3 / 54.5 -> 22.5 / 31.8 / 52.8 us; error of 3
+// rows against 64 bits 1.5e-5 -> 4.5e-6).
 //
 // Launch shape: persistent, grid-stride over row quads (quad slot s of workgroup w is quad s * gridDim.x + w, so the
 // grid reads one contiguous band of the bank at a time).  Wave wv of a row set owns slice chunk kr * wpr + wv
@@ -208,17 +211,13 @@ static __device__ __forceinline__ void run(const qq_params& p) {
                         aw[2 * w + 1] = __builtin_bit_cast(h4_t, hi);
                     }
                 }
-                // the four headers of this block's rows
-                float sc[4], bi[4];
-                const uint32_t hq[4] = {(uint32_t)QQ_DPP(blk.hdr, 0x00), (uint32_t)QQ_DPP(blk.hdr, 0x55),
-                                        (uint32_t)QQ_DPP(blk.hdr, 0xAA), (uint32_t)QQ_DPP(blk.hdr, 0xFF)};   // quad_perm [i,i,i,i]
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const h2_t hd = __builtin_bit_cast(h2_t, hq[i]);
-                    sc[i] = (float)hd[0];
-                    bi[i] = (float)hd[1];
-                    if constexpr (FMT == QW_FMT_B8) sc[i] *= 16777216.0f;   // the codes are f16 subnormals code * 2^-24: exact, once per header
-                }
+                // The header of this lane's row: the scale (times 2^24, exactly: the codes are f16 subnormals code * 2^-24) goes to the
+                // block by quad broadcast, the bias stays where it is as the one operand of a K = 1 product with the slices' sums
+                // (HQ4_G32_M5: w = (1024 + q) s + b; 1024 s + b is exact in fp32, so the large terms meet unrounded)
+                const h2_t hd = __builtin_bit_cast(h2_t, blk.hdr);
+                const float s24 = (float)hd[0] * 16777216.0f;
+                const float bias = FMT == QW_FMT_M5 ? __builtin_fmaf(1024.0f, (float)hd[0], (float)hd[1]) : (float)hd[1];
+                const float sc[4] = {QQ_DPP_F32(s24, 0x00), QQ_DPP_F32(s24, 0x55), QQ_DPP_F32(s24, 0xAA), QQ_DPP_F32(s24, 0xFF)};   // quad_perm [i,i,i,i]
 #pragma unroll
                 for (int mg = 0; mg < MG; ++mg) {
                     f4_t a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
@@ -227,17 +226,12 @@ static __device__ __forceinline__ void run(const qq_params& p) {
                         a0 = __builtin_amdgcn_mfma_f32_4x4x4f16(aw[t], xb[mg][t], a0, 0, 0, 0);
                         a1 = __builtin_amdgcn_mfma_f32_4x4x4f16(aw[t + 1], xb[mg][t + 1], a1, 0, 0, 0);
                     }
+                    const f4_t bs = __builtin_amdgcn_mfma_f32_4x4x1f32(bias, S[mg], f4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
                     f4_t v;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        float q;
-                        if constexpr (FMT == QW_FMT_B8) {
-                            q = a0[i] + a1[i];
-                        } else {
-                            q = __builtin_fmaf(a0[i], 16777216.0f, FMT == QW_FMT_M5 ? 1024.0f * S[mg] : 0.0f);
-                            q = __builtin_fmaf(a1[i], 1048576.0f, q);
-                        }
-                        float r = __builtin_fmaf(sc[i], q, bi[i] * S[mg]);
+                        const float q = FMT == QW_FMT_B8 ? a0[i] + a1[i] : __builtin_fmaf(a1[i], 0.0625f, a0[i]);
+                        float r = __builtin_fmaf(sc[i], q, bs[i]);
                         r += QQ_DPP_F32(r, 0x114);   // row_shr:4
                         r += QQ_DPP_F32(r, 0x118);   // row_shr:8: lanes 12..15 of each 16-lane row hold its four blocks
                         v[i] = r;
