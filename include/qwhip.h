@@ -369,8 +369,7 @@ qwhip_status qwhip_moe_group_pairs(qwhip_stream_t s, const int32_t* ids, uint32_
  * (Sources/QWMetal/include/qw_gemm_nax.metalh:436-504).
  * w: ONE view over the expert-major bank, n = experts * rows_per_expert.  Row slot p in
  * [expert_off[e], expert_off[e+1]) uses expert e.  A row of slot p is x[gather[p]] when gather is
- * not NULL (gate_up: gather = sorted_tok) else x[p] (down).  y [pairs, rows_per_expert].  The tile list is
- * qwhip_moe_group_pairs': all entries of an expert that has any (the kernel deals the expert's rows anew among its entries). */
+ * not NULL (gate_up: gather = sorted_tok) else x[p] (down).  y [pairs, rows_per_expert]. */
 qwhip_status qwhip_moe_grouped_gemm(qwhip_stream_t s, const qwhip_weight_view* w, uint32_t experts,
                                     const void* x, uint32_t x_dtype, uint32_t ldx, const int32_t* gather,
                                     const int32_t* expert_off, const int32_t* tile_e, const int32_t* tile_r,

@@ -1279,7 +1279,6 @@ qwhip_status gemm_checks(qwhip_stream_t s, const qwhip_weight_view* w, const voi
     return QWHIP_OK;
 }
 
-// runs EXPR with F bound to the container format as a constant
 // the sum of fp32 planes [splits][M][N] into y, in range order
 hipError_t launch_plane_sum(hipStream_t st, const qw_gemm_params& p, uint32_t splits, const float* part, void* y, uint32_t y_dtype, uint32_t ldy) {
     const dim3 rgrid((unsigned)(((uint64_t)p.M * (p.N / 4u) + 255u) / 256u));
@@ -1288,6 +1287,7 @@ hipError_t launch_plane_sum(hipStream_t st, const qw_gemm_params& p, uint32_t sp
     else hipLaunchKernelGGL(qw_splitk_reduce_kernel<QWHIP_F32>, rgrid, dim3(256), 0, st, part, splits, p.M, p.N, y, ldy);
     return hipGetLastError();
 }
+
 // split-K launch of the half-height ping-pong tile into fp32 planes at `part`, then the sum into y
 template <int FMT>
 hipError_t launch_splitk(hipStream_t st, const qw_gemm_params& p, uint32_t splits, float* part, void* y, uint32_t y_dtype, uint32_t ldy) {
@@ -1372,6 +1372,8 @@ direct_plan choose_direct(const qwhip_weight_view* w, uint32_t m, int fmt, uint3
     }
     return best;
 }
+
+// runs EXPR with F bound to the container format as a constant
 #define QG_FOR_FMT(fmt, e, EXPR)                                                  \
     switch (fmt) {                                                                \
         case QG_FMT_M5: { constexpr int F = QG_FMT_M5; e = (EXPR); } break;       \

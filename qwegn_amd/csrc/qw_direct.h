@@ -44,7 +44,6 @@ typedef u4_t qd_piece __attribute__((aligned(4)));   // 16 bytes at 4-byte align
 template <int N>
 struct qd_int { static constexpr int value = N; };
 
-
 // The workgroup's work: an expert's rows [m0, m0 + rows_valid), nf fragments of 32, and a column tile.
 struct qd_item {
     uint32_t e, m0, rows_valid, nf, col;
@@ -58,11 +57,17 @@ __device__ __forceinline__ void qd_span_rows(uint32_t rows, uint32_t spans, uint
     it.nf = base_f + (i < more ? 1u : 0u);
     it.rows_valid = min(32u * it.nf, rows - row0);
 }
+// rows of tile-list code `packed`'s tile
+__device__ __forceinline__ uint32_t qd_tile_rows(uint32_t packed) {
+    const uint32_t code = packed >> 24;
+    return code == 1u ? 16u : (code == 2u ? 32u : 64u);
+}
 // Grid: one-dimensional and XCD-aware - workgroup L runs on XCD L % 8 (round-robin dispatch), each XCD takes one contiguous
 // eighth of the expert-sorted tile list and walks (tile, column tile) column-fastest, so the spans of an expert and the column
-// tiles of a span run side by side under one L2.  The list's entries are tiles of at most 64 rows; the expert's 32-row
-// fragments are dealt evenly to as few spans of at most MAXF as hold them, entry i (rows 64 i ..) takes span i, and the other
-// entries leave.
+// tiles of a span run side by side under one L2.  The list's entries are tiles of at most 64 rows.  Where all tiles of an expert
+// are listed one after the other, its 32-row fragments are dealt evenly to as few spans of at most MAXF as hold them, entry i (rows
+// 64 i ..) takes span i and the other entries leave; an entry of any other list (a part of one, another order) takes its own rows.
+// The neighbours that this looks at are asked for together with the entry itself.
 template <int MAXF>
 __device__ __forceinline__ bool qd_find_item(const qw_gemm_params& p, qd_item& it) {
     const uint32_t ncol = p.tiles_n;
@@ -72,20 +77,43 @@ __device__ __forceinline__ bool qd_find_item(const qw_gemm_params& p, qd_item& i
     const uint32_t ti = slot / ncol;
     const uint32_t t = xcd * per_xcd + ti;
     if (ti >= per_xcd || t >= tc) return false;
+    const uint32_t lane = threadIdx.x & 63u, near = t + lane - 31u;   // entries t - 31 .. t + 32; below 0 wraps past tc
+    const uint32_t near_e = near < tc ? (uint32_t)p.tile_e[near] : ~0u, near_r = near < tc ? (uint32_t)p.tile_r[near] : 0u;
     const uint32_t e = (uint32_t)p.tile_e[t];
     const uint32_t packed = (uint32_t)p.tile_r[t];
-    const uint32_t code = packed >> 24;
-    const uint32_t bm = code == 1u ? 16u : (code == 2u ? 32u : 64u);
+    const uint32_t bm = qd_tile_rows(packed);
     const uint32_t first = (packed & 0xFFFFFFu) * bm;              // row of the expert
     const uint32_t off_e = (uint32_t)p.expert_off[e];
     const uint32_t rows_e = (uint32_t)p.expert_off[e + 1] - off_e;
-    const uint32_t spans = (rows_e + 32u * MAXF - 1u) / (32u * MAXF);
-    const uint32_t i_span = first >> 6;
-    if (i_span >= spans) return false;
-    uint32_t row0;
-    qd_span_rows<MAXF>(rows_e, spans, i_span, row0, it);
+    if (first >= rows_e) return false;
     it.e = e;
     it.col = slot - ti * ncol;
+
+    const uint32_t tiles = (rows_e + 63u) >> 6, i = first >> 6;
+    // is (le, lr) the tile of rows 64 q .. of this expert?
+    const auto is_tile = [&](uint32_t le, uint32_t lr, uint32_t q) -> bool {
+        const uint32_t n = qd_tile_rows(lr);
+        return le == e && (lr & 0xFFFFFFu) * n == 64u * q && n >= min(64u, rows_e - 64u * q);
+    };
+    bool whole = t >= i && t - i + tiles <= tc;
+    if (whole) {
+        if (i <= 31u && tiles - i <= 33u) {
+            const uint32_t q = lane + i - 31u;
+            whole = __all(q >= tiles || is_tile(near_e, near_r, q));
+        } else {
+            for (uint32_t q = lane; q < tiles; q += 64u) whole = whole && is_tile((uint32_t)p.tile_e[t - i + q], (uint32_t)p.tile_r[t - i + q], q);
+            whole = __all(whole);
+        }
+    }
+    uint32_t row0 = first;
+    if (whole) {
+        const uint32_t spans = (rows_e + 32u * MAXF - 1u) / (32u * MAXF);
+        if (i >= spans) return false;
+        qd_span_rows<MAXF>(rows_e, spans, i, row0, it);
+    } else {
+        it.rows_valid = min(bm, rows_e - first);
+        it.nf = (it.rows_valid + 31u) >> 5;
+    }
     it.m0 = off_e + row0;
     return true;
 }

@@ -396,6 +396,46 @@ def test_grouped_gemm_spans(dev, fmt, counts, k, inter, xdt, compact):
     assert np.array_equal(act1.download(np.uint16, (pairs, inter)), act2.download(np.uint16, (pairs, inter)))
 
 
+@pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq8_g32"])
+@pytest.mark.parametrize("counts", [_SPANS_FEW, _SPANS_MANY, [2300, 40]])
+def test_grouped_gemm_takes_any_tile_list(dev, fmt, counts):
+    """A caller's own list of tiles - another order, a part of the sort's - gives the rows of the tiles that are in it, the same bits
+    as the whole list, and leaves the other rows alone."""
+    e, k, inter = len(counts), 128, 96
+    n = 2 * inter
+    blocks, _ = H.make_bank(fmt, e * n, k, seed=22)
+    ids = np.repeat(np.arange(e), counts).astype(np.int32).reshape(-1, 1)
+    pairs = ids.size
+    g = _group(dev, ids, e, 1)
+    lib, st, b = dev.lib, dev.stream.handle, g["bufs"]
+    bank, xb = dev.put(blocks), dev.put(H.make_x(pairs, k, 5).astype(np.float16))
+    view = H.view_of(dev, bank, fmt, e * n, k)
+    code_rows = np.array([64, 16, 32, 64])
+    bm = code_rows[g["tr"] >> 24]
+    start = g["off"][g["te"]] + (g["tr"] & 0xFFFFFF) * bm
+    stop = np.minimum(start + bm, g["off"][g["te"] + 1])
+
+    def both_doors(te, tr):
+        bufs = [dev.put(te.astype(np.int32)), dev.put(tr.astype(np.int32)), dev.put(np.array([te.size], np.int32))]
+        y, act = dev.put(np.full((pairs, n), 0x5555, np.uint16)), dev.put(np.full((pairs, inter), 0x5555, np.uint16))
+        plan = (b["stok"].ptr, b["off"].ptr, *(t.ptr for t in bufs), g["max_tiles"], pairs)
+        qwhip.check(lib.qwhip_moe_grouped_gemm(st, C.byref(view), e, xb.ptr, qwhip.F16, 0, *plan, y.ptr, qwhip.F16, 0))
+        qwhip.check(lib.qwhip_moe_grouped_gemm_swiglu(st, C.byref(view), e, xb.ptr, qwhip.F16, 0, *plan, 1, act.ptr, 0))
+        dev.stream.sync()
+        out = np.concatenate([y.download(np.uint16, (pairs, n)), act.download(np.uint16, (pairs, inter))], axis=1)
+        for t in (*bufs, y, act):
+            t.free()
+        return out
+
+    whole = both_doors(g["te"], g["tr"])
+    order = np.random.default_rng(3).permutation(g["tc"])
+    for pick in (np.arange(g["tc"])[::-1], order, np.arange(0, g["tc"], 2), np.arange(1, g["tc"]), order[: g["tc"] // 2]):
+        listed = np.zeros(pairs, bool)
+        for t in pick:
+            listed[start[t]:stop[t]] = True
+        assert np.array_equal(both_doors(g["te"][pick], g["tr"][pick]), np.where(listed[:, None], whole, 0x5555))
+
+
 def test_fused_gate_up_swiglu_refusals(dev):
     blocks, _ = H.make_bank("hq4_g32_m5", 4 * 2 * 48, 64, 1)
     bank, xb, act = dev.put(blocks), dev.put(np.zeros((4, 64), np.float16)), dev.alloc(4096)
