@@ -597,7 +597,10 @@ bool qw_col_gemv(hipStream_t st, const qwhip_weight_view* w, const void* x, uint
     // 4.74, 4096 x 2560 4.60 -> 4.07, 2560 x 8192 5.65 -> 5.10, 6144 x 4096 5.31 -> 4.95, 1024 x 3072 3.72 -> 3.02, 5120 x 5120 level).
     // Larger ones: at least two rows a set, whole multiples of the units (7168 x 5120: 896 workgroups 6.51 us, 1024 6.40)
     if (wdepth && !(tune & 0x40u) && (tune >> 3 & 3u) == 0u && (uint64_t)w->n * nb * 20u < 20000000u) {
-        wgs = w->n >= sets * 1024u ? 512u : min(256u, max(1u, w->n / sets));
+        // past six rows a set four of them are the better ones again (16384 x 1024: 512 workgroups 5.15 us, 1024 4.77; 12288 x 2048:
+        // 512 5.08, 768 5.29)
+        if (w->n > sets * 3072u) wgs = min(wgs, w->n / (sets * 4u));
+        else wgs = w->n >= sets * 1024u ? 512u : min(256u, max(1u, w->n / sets));
         wgs = max(wgs, qwhip_cdiv(w->n, 128u));
     } else {
         wgs = min(wgs, max(1u, w->n / (sets * (wdepth ? 2u : 4u))));
@@ -657,10 +660,12 @@ bool qw_col_pair_gemv(hipStream_t st, const qwhip_weight_view* w, const void* x,
     const uint32_t waves = (threads + 63u) / 64u;
     // ten waves per compute unit, as the compiled window of the GEMV, in whole multiples of the units; three workgroups a unit up to six
     // waves (2 x 8704 x 2560: 512 workgroups 8.06 us, 768 7.68; 2 x 17408 x 5120 level); at least two channels per set
-    // (2 x 2048 x 1024: four, 256 workgroups, 3.42 us; two, 512, 3.24)
+    // (2 x 2048 x 1024: four, 256 workgroups, 3.42 us; two, 512, 3.24), past three workgroups a unit four
     uint32_t wgs = (256u * 10u + waves / 2u) / waves;
-    wgs = waves <= 6u ? 768u : max(256u, (wgs + 128u) / 256u * 256u);
-    wgs = min(wgs, max(1u, inter / (h2 * 2u)));
+    wgs = max(256u, (wgs + 128u) / 256u * 256u);
+    const uint32_t most = min(wgs, inter / (h2 * 4u));
+    if (waves <= 6u) wgs = 768u;
+    wgs = max(most, min(wgs, max(1u, inter / (h2 * 2u))));
     wgs = max(wgs, qwhip_cdiv(inter, 64u));                        // at most 128 row slots per workgroup
     const uint32_t ch_per_wg = qwhip_cdiv(inter, wgs);
     const size_t lds = (size_t)nb * 80u + (size_t)2u * ch_per_wg * cpr * 4u;
