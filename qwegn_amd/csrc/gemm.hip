@@ -1288,35 +1288,29 @@ hipError_t launch_plane_sum(hipStream_t st, const qw_gemm_params& p, uint32_t sp
     return hipGetLastError();
 }
 
-// split-K launch of the half-height ping-pong tile into fp32 planes at `part`, then the sum into y
+// split-K launch of the half-height ping-pong tile into the fp32 planes at p.y
 template <int FMT>
-hipError_t launch_splitk(hipStream_t st, const qw_gemm_params& p, uint32_t splits, float* part, void* y, uint32_t y_dtype, uint32_t ldy) {
-    {
-        qw_gemm_params q = p;
-        q.y = part;
-        q.ldy = p.N;
-        q.tiles_m = qwhip_cdiv(p.M, kCfgBM[CFG_128x320]);
-        q.tiles_n = qwhip_cdiv(p.N, kCfgBN[CFG_128x320]);
-        const dim3 grid(((q.tiles_m * q.tiles_n + 7u) / 8u) * 8u, splits);
-        hipError_t e = p.x_bf16 ? launch_cfg3<1, 5, 4, 2, FMT, QWHIP_F32, false, QWHIP_BF16>(st, q, grid)
-                                : launch_cfg3<1, 5, 4, 2, FMT, QWHIP_F32>(st, q, grid);
-        if (e != hipSuccess) return e;
-        return launch_plane_sum(st, p, splits, part, y, y_dtype, ldy);
-    }
+hipError_t launch_splitk(hipStream_t st, const qw_gemm_params& p, uint32_t splits) {
+    qw_gemm_params q = p;
+    q.tiles_m = qwhip_cdiv(p.M, kCfgBM[CFG_128x320]);
+    q.tiles_n = qwhip_cdiv(p.N, kCfgBN[CFG_128x320]);
+    const dim3 grid(((q.tiles_m * q.tiles_n + 7u) / 8u) * 8u, splits);
+    return p.x_bf16 ? launch_cfg3<1, 5, 4, 2, FMT, QWHIP_F32, false, QWHIP_BF16>(st, q, grid)
+                    : launch_cfg3<1, 5, 4, 2, FMT, QWHIP_F32>(st, q, grid);
 }
 
 // K ranges for a problem of few tiles (0 = one launch): 2..8 ranges of at least 8 K-steps over at most 256 workgroups of
-// 128 x 320 tiles, when `workspace_bytes` holds the fp32 planes behind its first `used` bytes and the ranges pay:
+// 128 x 320 tiles, when the fp32 planes fit `plane_room` bytes and the ranges pay:
 // K-steps taken off the tile's loop (0.72 us each) against writing and re-reading the planes (about 5 TB/s together) and
 // the second launch (4 us).  N = K = 2048 with a workspace: M = 1536 over 3 ranges took 46 us against 36 us in one launch,
 // M = 2048 over 2 ranges 36 against 32; N = K = 5120, M = 1024 over 2: 71 against 84.
-uint32_t choose_splits(uint32_t m, uint32_t n, uint32_t k, uint64_t used, uint64_t workspace_bytes) {
+uint32_t choose_splits(uint32_t m, uint32_t n, uint32_t k, uint64_t plane_room) {
     const uint32_t tiles = qwhip_cdiv(m, kCfgBM[CFG_128x320]) * qwhip_cdiv(n, kCfgBN[CFG_128x320]);
     const uint32_t nk = k / 64u;
     const uint64_t plane = (uint64_t)m * n * 4u;
     uint32_t splits = min(min(8u, 256u / tiles), nk / 8u);
     auto pays = [&](uint32_t sp) { return nk * 0.72 * (1.0 - 1.0 / sp) > sp * (double)plane * 2.0 / 5e6 + 4.0; };
-    while (splits >= 2u && ((uint64_t)(splits - 1u) * qwhip_cdiv(nk, splits) >= nk || used + splits * plane > workspace_bytes || !pays(splits)))
+    while (splits >= 2u && ((uint64_t)(splits - 1u) * qwhip_cdiv(nk, splits) >= nk || splits * plane > plane_room || !pays(splits)))
         --splits;
     return splits < 2u ? 0u : splits;
 }
@@ -1329,14 +1323,17 @@ uint32_t choose_splits(uint32_t m, uint32_t n, uint32_t k, uint64_t used, uint64
 // measured (10 % and 9 % of root mean square error); it is taken where it prices below 0.85 of the other, where the fit held: 64 rows on
 // 7168 x 5120 27 -> 20 us, 333 rows on 2560 x 9728 39 -> 36, gate|up of 333 rows on 2 x 9728 x 2560 61 -> 47, 180 rows on
 // 6144 x 16384 80 -> 56; over all of them 1.18 times as fast, 8 of them slower, by 7 % at most.
-struct direct_plan {
-    bool take, few;
-    uint32_t splits;
+struct gemm_route {
+    bool direct, few;    // the direct-operand kernel, its spans of 64 rows
+    uint32_t splits;     // K ranges into fp32 planes (two and more), or one launch
 };
-direct_plan choose_direct(const qwhip_weight_view* w, uint32_t m, int fmt, uint32_t old_splits, uint64_t plane_room) {
-    direct_plan best = {false, false, 1u};
+inline bool direct_takes(const qwhip_weight_view* w) {
+    return w->k % 128u == 0 && w->group <= 128u && 256u * qwhip_view_row_bytes(w) < (1ull << 32);
+}
+gemm_route choose_direct(const qwhip_weight_view* w, uint32_t m, int fmt, uint32_t old_splits, uint64_t plane_room) {
+    gemm_route best = {false, false, old_splits};
     const uint32_t n = w->n, k = w->k;
-    if (k % 128u != 0 || w->group > 128u || 256u * qwhip_view_row_bytes(w) >= (1ull << 32)) return best;
+    if (!direct_takes(w)) return best;
     const bool wide = fmt == QG_FMT_B8 || fmt == QG_FMT_B6;
     const double plane = (double)m * n * 4.0;
     const uint32_t nk = k / 64u, pairs = nk / 2u, frags = qwhip_cdiv(m, 32u), cols = qwhip_cdiv(n, 256u);
@@ -1373,6 +1370,30 @@ direct_plan choose_direct(const qwhip_weight_view* w, uint32_t m, int fmt, uint3
     return best;
 }
 
+// flags bits 8..11 of the dense doors that name a K-split or direct form, for tuning and tests; bits 12..15: its K ranges (0 = one)
+enum { OV_DIRECT_64 = 6, OV_DIRECT_WIDE = 7, OV_SPLIT_PINGPONG = 8 };
+
+// The route of a dense problem: the automatic choice, or the form that the flags name.  Both dense doors call it with the same
+// room for planes, so that the fused gate|up gives the bits of the plain door and the activation pass after it.
+qwhip_status choose_route(const qwhip_weight_view* w, uint32_t m, int fmt, uint32_t flags, bool y_ok, uint64_t plane_room, gemm_route* r) {
+    const uint32_t ov = (flags >> 8) & 0xFu, ranges = (flags >> 12) & 0xFu;
+    *r = {false, false, 0u};
+    if (ov == 0u) {
+        if (y_ok) *r = choose_direct(w, m, fmt, choose_splits(m, w->n, w->k, plane_room), plane_room);
+        return QWHIP_OK;
+    }
+    if (ov != OV_DIRECT_64 && ov != OV_DIRECT_WIDE && ov != OV_SPLIT_PINGPONG) return QWHIP_OK;
+    const bool direct = ov != OV_SPLIT_PINGPONG;
+    const uint32_t steps = w->k / (direct ? 128u : 64u), splits = ranges ? ranges : 1u;
+    const bool split_ok = direct && splits == 1u ? true
+                                                 : splits >= 2u && (uint64_t)(splits - 1u) * qwhip_cdiv(steps, splits) < steps &&
+                                                       (uint64_t)splits * m * w->n * 4u <= plane_room;
+    if (!y_ok || (direct && !direct_takes(w)) || !split_ok)
+        return qwhip_fail(QWHIP_E_BAD_SHAPE, "the GEMM form %u over %u K ranges that flags %#x name does not take this call", ov, splits, flags);
+    *r = {direct, ov == OV_DIRECT_64, splits};
+    return QWHIP_OK;
+}
+
 // runs EXPR with F bound to the container format as a constant
 #define QG_FOR_FMT(fmt, e, EXPR)                                                  \
     switch (fmt) {                                                                \
@@ -1385,10 +1406,23 @@ direct_plan choose_direct(const qwhip_weight_view* w, uint32_t m, int fmt, uint3
         default: e = hipErrorInvalidValue;                                        \
     }
 
+// a problem's partial sums over the route's K ranges, one fp32 plane [M][N] each at `part`
+hipError_t launch_planes(hipStream_t st, int fmt, const qw_gemm_params& p, const gemm_route& route, uint32_t xdt, float* part) {
+    qw_gemm_params q = p;
+    q.y = part;
+    q.ldy = p.N;
+    if (route.direct) return qw_dense_direct(st, fmt, q, route.splits, xdt, QWHIP_F32, false, route.few);
+    hipError_t e;
+    QG_FOR_FMT(fmt, e, (launch_splitk<F>(st, q, route.splits)))
+    return e;
+}
+
 }  // namespace
 
-// flags bits 8..11: tile shape override for tuning and tests (0 = automatic, 1 + CFG_*; 14 = 256 x 320 on the DMA-fed
-// kernel instead of the ping-pong kernel; 15 = the unpipelined kernel).
+// flags bits 8..11: tile shape override for tuning and tests (0 = automatic, 1 + CFG_*; 6 and 7 = the direct-operand kernel on spans of
+// 64 and of 128 rows, 96 on the 6- and 8-bit containers; 8 = the 128 x 320 ping-pong tile over K ranges; 14 = 256 x 320 on the DMA-fed
+// kernel instead of the ping-pong kernel; 15 = the unpipelined kernel).  Bits 12..15: the K ranges of 6, 7 and 8 (0 = one), which refuse
+// a call that they cannot take.
 extern "C" qwhip_status qwhip_gemm(qwhip_stream_t s, const qwhip_weight_view* w, const void* x, uint32_t x_dtype, uint32_t m,
                                    uint32_t ldx, void* y, uint32_t y_dtype, uint32_t ldy, uint32_t flags, void* workspace,
                                    uint64_t workspace_bytes) {
@@ -1423,16 +1457,15 @@ extern "C" qwhip_status qwhip_gemm(qwhip_stream_t s, const qwhip_weight_view* w,
     // over 2..8 workgroups and a second launch sums the planes in range order.
     const bool copy_needed = rotate || (x_dtype == QWHIP_BF16 && (flags & (1u << 16)));   // bf16 rows in the basis are read in place
     const uint64_t sk_used = copy_needed ? ((ws_need + 255u) & ~(uint64_t)255u) : 0u;
-    uint32_t splits = 0;
     const bool planes_ok = workspace && ((uintptr_t)workspace & 15u) == 0 && (!copy_needed || ws_ok);
-    if (ov == 0u && pp_ok && planes_ok && w->n % 4u == 0) splits = choose_splits(m, w->n, w->k, sk_used, workspace_bytes);
-    direct_plan direct = {};
-    if (ov == 0u && pp_ok)
-        direct = choose_direct(w, m, fmt, splits, planes_ok && workspace_bytes > sk_used ? workspace_bytes - sk_used : 0u);
+    gemm_route route;
+    st = choose_route(w, m, fmt, flags, pp_ok, planes_ok && workspace_bytes > sk_used ? workspace_bytes - sk_used : 0u, &route);
+    if (st != QWHIP_OK) return st;
+    const bool planes = route.splits >= 2u;
     // bf16 activations already in the basis: the ping-pong kernel converts them while it stages the tile (no pass of its own,
     // no workspace); flags bit 16 keeps the separate pass, for tests and comparisons
-    const bool direct_bf16 = !rotate && x_dtype == QWHIP_BF16 && ov != 15u && !(flags & (1u << 16)) && (splits != 0u || gemm3_takes(p, cfg, fmt, y_dtype));
-    if (direct.take && !copy_needed) {
+    const bool direct_bf16 = !rotate && x_dtype == QWHIP_BF16 && ov != 15u && !(flags & (1u << 16)) && (planes || gemm3_takes(p, cfg, fmt, y_dtype));
+    if (route.direct && !copy_needed) {
         // rows in the basis, f16 or bf16, are read in place
     } else if (direct_bf16) {
         p.x_bf16 = 1u;
@@ -1465,22 +1498,14 @@ extern "C" qwhip_status qwhip_gemm(qwhip_stream_t s, const qwhip_weight_view* w,
     p.bb = qwhip_view_block_bytes(w);
     p.row_bytes = qwhip_view_row_bytes(w);
     hipError_t e;
-    if (direct.take) {
-        if (direct.splits == 1u) {
-            QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, p, 1u, xdt, y_dtype, false, direct.few));
-            return QWHIP_OK;
-        }
-        qw_gemm_params q = p;
-        q.y = (uint8_t*)workspace + sk_used;
-        q.ldy = p.N;
-        QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, q, direct.splits, xdt, QWHIP_F32, false, direct.few));
-        QWHIP_TRY_HIP(launch_plane_sum(s->stream, p, direct.splits, (const float*)q.y, y, y_dtype, ldy));
+    if (route.direct && !planes) {
+        QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, p, 1u, xdt, y_dtype, false, route.few));
         return QWHIP_OK;
     }
-    if (splits != 0u && xdt == QWHIP_F16) {
+    if (planes) {
         float* part = (float*)((uint8_t*)workspace + sk_used);
-        QG_FOR_FMT(fmt, e, (launch_splitk<F>(s->stream, p, splits, part, y, y_dtype, ldy)))
-        QWHIP_TRY_HIP(e);
+        QWHIP_TRY_HIP(launch_planes(s->stream, fmt, p, route, xdt, part));
+        QWHIP_TRY_HIP(launch_plane_sum(s->stream, p, route.splits, part, y, y_dtype, ldy));
         return QWHIP_OK;
     }
     if (xdt != QWHIP_F16 || ov == 15u) {
@@ -1595,31 +1620,20 @@ extern "C" qwhip_status qwhip_gemm_swiglu(qwhip_stream_t s, const qwhip_weight_v
     {
         const uint64_t x_used = xin == workspace ? ((ws_need + 255u) & ~(uint64_t)255u) : 0u;
         const uint64_t gu_bytes = ((uint64_t)m * w->n * 2u + 255u) & ~(uint64_t)255u;
-        const bool tuned = ((flags >> 8) & 0xFu) != 0u;
         const bool planes_ok = workspace && ((uintptr_t)workspace & 15u) == 0 && ldact == inter && workspace_bytes >= x_used + gu_bytes;
-        uint32_t splits = 0;
-        if (!tuned && planes_ok) splits = choose_splits(m, w->n, w->k, x_used + gu_bytes, workspace_bytes);
-        direct_plan direct = {};
-        if (!tuned) direct = choose_direct(w, m, fmt, splits, planes_ok ? workspace_bytes - x_used - gu_bytes : 0u);
-        if (direct.take && direct.splits == 1u) {
-            QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, p, 1u, QWHIP_F16, QWHIP_F16, true, direct.few));
-            return QWHIP_OK;
-        }
-        if (direct.take || splits != 0u) {
+        gemm_route route;
+        st = choose_route(w, m, fmt, flags, true, planes_ok ? workspace_bytes - x_used - gu_bytes : 0u, &route);
+        if (st != QWHIP_OK) return st;
+        if (route.splits >= 2u) {
             void* gu = (uint8_t*)workspace + x_used;
             float* part = (float*)((uint8_t*)workspace + x_used + gu_bytes);
-            hipError_t e;
-            if (direct.take) {
-                qw_gemm_params q = p;
-                q.y = part;
-                q.ldy = w->n;
-                QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, q, direct.splits, QWHIP_F16, QWHIP_F32, false, direct.few));
-                e = launch_plane_sum(s->stream, p, direct.splits, part, gu, QWHIP_F16, w->n);
-            } else {
-                QG_FOR_FMT(fmt, e, (launch_splitk<F>(s->stream, p, splits, part, gu, QWHIP_F16, w->n)))
-            }
-            QWHIP_TRY_HIP(e);
+            QWHIP_TRY_HIP(launch_planes(s->stream, fmt, p, route, QWHIP_F16, part));
+            QWHIP_TRY_HIP(launch_plane_sum(s->stream, p, route.splits, part, gu, QWHIP_F16, w->n));
             return qwhip_swiglu_fwht(s, gu, QWHIP_F16, act_f16, m, inter, rotate_act);
+        }
+        if (route.direct) {
+            QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, p, 1u, QWHIP_F16, QWHIP_F16, true, route.few));
+            return QWHIP_OK;
         }
     }
     // The half-height tile where it is the cheaper one by the pricing of choose_cfg (0.78 of the big tile's efficiency per

@@ -73,21 +73,25 @@ def test_elementwise_doors(dev, act):
 
 
 @pytest.mark.parametrize("act", ACTS)
-@pytest.mark.parametrize("fmt,m,inter,k", [("hq4_g32_m5", 256, 352, 256), ("hq4_g64", 64, 160, 128), ("hq8_g32", 128, 96, 256)])
-def test_dense_gate_up_gemm(dev, act, fmt, m, inter, k):
-    """qwhip_gemm_swiglu == qwhip_gemm (f16 out) + qwhip_swiglu_fwht bit for bit, and both meet the oracle."""
+@pytest.mark.parametrize("fmt,m,inter,k,cfg", [("hq4_g32_m5", 256, 352, 256, 0), ("hq4_g64", 64, 160, 128, 0), ("hq8_g32", 128, 96, 256, 0),
+                                               ("hq4_g32_m5", 200, 224, 512, 7), ("hq6_g32", 100, 160, 256, 7), ("hq4_g64", 40, 224, 256, 6),
+                                               ("hq3_g32", 70, 96, 640, 6 | 3 << 4), ("hq4_g32_m5", 130, 96, 512, 8 | 3 << 4)])
+def test_dense_gate_up_gemm(dev, act, fmt, m, inter, k, cfg):
+    """qwhip_gemm_swiglu == qwhip_gemm (f16 out) + qwhip_swiglu_fwht bit for bit, and both meet the oracle: the ping-pong tiles, the
+    direct-operand kernel's spans (flags bits 8..11 = 6, 7) in one launch, and K ranges (bits 12..15) of it and of the tiles (8)."""
+    flags = qwhip.X_PREROTATED | cfg << 8
     n = 2 * inter
     blocks, w16 = H.make_bank(fmt, n, k, seed=5)
     x16 = (H.make_x(m, k, 12) * 2).astype(np.float16)
     bank, xb = dev.put(blocks), dev.put(x16)
     gu, act2, act1 = dev.alloc(m * n * 2), dev.put(np.zeros((m, inter), np.float16)), dev.put(np.zeros((m, inter), np.float16))
-    ws = dev.alloc(max(m * k * 2, m * n * 2) + 256)
+    ws = dev.alloc(max(m * k * 2, m * n * 2) + 256 + (3 * m * n * 4 if cfg >> 4 else 0))
     view = H.view_of(dev, bank, fmt, n, k)
     lib, st = dev.lib, dev.stream.handle
     with activation(dev, *act):
-        qwhip.check(lib.qwhip_gemm(st, C.byref(view), xb.ptr, qwhip.F16, m, 0, gu.ptr, qwhip.F16, 0, qwhip.X_PREROTATED, ws.ptr, ws.nbytes))
+        qwhip.check(lib.qwhip_gemm(st, C.byref(view), xb.ptr, qwhip.F16, m, 0, gu.ptr, qwhip.F16, 0, flags, ws.ptr, ws.nbytes))
         qwhip.check(lib.qwhip_swiglu_fwht(st, gu.ptr, qwhip.F16, act2.ptr, m, inter, 1))
-        qwhip.check(lib.qwhip_gemm_swiglu(st, C.byref(view), xb.ptr, qwhip.F16, m, 0, 1, act1.ptr, 0, qwhip.X_PREROTATED, ws.ptr, ws.nbytes))
+        qwhip.check(lib.qwhip_gemm_swiglu(st, C.byref(view), xb.ptr, qwhip.F16, m, 0, 1, act1.ptr, 0, flags, ws.ptr, ws.nbytes))
         dev.stream.sync()
     one, two = act1.download(np.float16, (m, inter)), act2.download(np.float16, (m, inter))
     assert np.array_equal(one.view(np.uint16), two.view(np.uint16))

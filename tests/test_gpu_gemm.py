@@ -11,6 +11,12 @@ from tests import helpers as H
 
 pytestmark = pytest.mark.gpu
 TOL = 2e-3
+# kernel overrides (flags bits 8..11) with their K ranges (bits 12..15): a form that cannot take the call is refused
+DIRECT_64, DIRECT_WIDE, SPLIT_PINGPONG = 6, 7, 8
+
+
+def form(code, ranges=0):
+    return code | ranges << 4
 
 
 @pytest.fixture(scope="module")
@@ -134,30 +140,48 @@ def test_gemm_ragged_rows_at_the_prefill_shape(dev):
 
 
 @pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq4_g64", "aq2_g64", "hq3_g32", "hq6_g32", "hq8_g32"])
-@pytest.mark.parametrize("m,n,k", [(64, 640, 1024), (200, 400, 2048), (37, 336, 1536), (512, 1280, 5120)])
-def test_gemm_split_k_with_a_workspace_for_partial_planes(dev, fmt, m, n, k):
-    """Few tiles and a workspace that holds fp32 partial planes: the K-steps of a tile are dealt over several workgroups and a
-    second launch sums the planes (2 to 8 ranges here, with a short last range at k = 1536: 24 K-steps over 3 ranges of 8,
-    and at k = 2048 behind the rotated copy of un-rotated rows).  Same bar as the one-launch form."""
+@pytest.mark.parametrize("m,n,k,cfg", [(64, 640, 1024, form(SPLIT_PINGPONG, 2)), (200, 400, 2048, form(SPLIT_PINGPONG, 4)),
+                                       (37, 336, 1536, form(SPLIT_PINGPONG, 5)), (512, 1280, 5120, form(SPLIT_PINGPONG, 8)), (64, 640, 1088, 0)])
+def test_gemm_split_k_with_a_workspace_for_partial_planes(dev, fmt, m, n, k, cfg):
+    """The ping-pong tile with the K-steps of a tile dealt over several workgroups and a second launch that sums the planes: even
+    ranges, a short last one (24 K-steps over five ranges of 5), behind the rotated copy of un-rotated rows; k = 1088, an odd
+    number of K-steps, is the automatic choice's.  Same bar as the one-launch form."""
     big = 64 << 20
-    st, out, ref = run_gemm(dev, fmt, m, n, k, xdtype="f16", ydtype="f32", seed=9, workspace_bytes=big)
+    st, out, ref = run_gemm(dev, fmt, m, n, k, xdtype="f16", ydtype="f32", seed=9, workspace_bytes=big, cfg=cfg)
     assert st == qwhip.OK
     assert qo.normalized_error(out, ref) <= 2e-5
-    st, out1, _ = run_gemm(dev, fmt, m, n, k, xdtype="f16", ydtype="f32", seed=9, workspace=False)
+    st, out1, _ = run_gemm(dev, fmt, m, n, k, xdtype="f16", ydtype="f32", seed=9, workspace=False, cfg=5)
     assert qo.normalized_error(out, out1) <= 2e-6          # the ranges only change the order of the fp32 sums
-    st, out, ref = run_gemm(dev, fmt, m, n, k, xdtype="bf16", ydtype="bf16", seed=10, workspace_bytes=big)
+    assert not np.array_equal(out, out1)                   # and they do
+    st, out, ref = run_gemm(dev, fmt, m, n, k, xdtype="bf16", ydtype="bf16", seed=10, workspace_bytes=big, cfg=cfg)
     assert st == qwhip.OK
     assert qo.normalized_error(out, ref) <= TOL
-    st, out, ref = run_gemm(dev, fmt, m, n, k, xdtype="f16", ydtype="f16", prerot=False, seed=11, workspace_bytes=big)
+    st, out, ref = run_gemm(dev, fmt, m, n, k, xdtype="f16", ydtype="f16", prerot=False, seed=11, workspace_bytes=big, cfg=cfg)
     assert st == qwhip.OK
     assert qo.normalized_error(out, ref) <= TOL
+
+
+@pytest.mark.parametrize("k,cfg,ws_mb", [(1088, form(DIRECT_64), 1), (1088, form(DIRECT_WIDE), 1), (1024, form(DIRECT_64, 2), 0),
+                                         (1024, form(SPLIT_PINGPONG, 2), 0), (1024, form(SPLIT_PINGPONG), 1), (1024, form(SPLIT_PINGPONG, 7), 1)])
+def test_gemm_named_forms_refuse_what_they_cannot_take(dev, k, cfg, ws_mb):
+    """K of an odd number of K-steps on the direct-operand kernel, K ranges without room for their planes, ranges of which one would
+    be empty (16 K-steps over 7), one range of the split form: refused, on both dense doors."""
+    m, n = 33, 64
+    bank, xb, y = dev.put(H.make_bank("hq4_g32_m5", n, k, 1)[0]), dev.put(np.zeros((m, k), np.float16)), dev.alloc(m * n * 2)
+    ws = dev.alloc(max(16, ws_mb << 20))
+    view = H.view_of(dev, bank, "hq4_g32_m5", n, k)
+    lib, st, flags, wsp = dev.lib, dev.stream.handle, qwhip.X_PREROTATED | cfg << 8, (ws.ptr, ws_mb << 20) if ws_mb else (None, 0)
+    assert lib.qwhip_gemm(st, C.byref(view), xb.ptr, qwhip.F16, m, 0, y.ptr, qwhip.F16, 0, flags, *wsp) == qwhip.E_BAD_SHAPE
+    assert lib.qwhip_gemm_swiglu(st, C.byref(view), xb.ptr, qwhip.F16, m, 0, 1, y.ptr, 0, flags, *wsp) == qwhip.E_BAD_SHAPE
 
 
 @pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq4_g64", "hq8_g32"])
-@pytest.mark.parametrize("m,ws_mb", [(333, 0), (333, 64), (2100, 0)])
-def test_gemm_strided_rows_on_every_ping_pong_form(dev, fmt, m, ws_mb):
-    """Activation rows ldx > k apart and output rows ldy > n apart (both in elements) through the one-launch forms (256 x 320
-    and 128 x 320 tiles, ragged row counts) and the split-K form: padding columns of the output stay untouched."""
+@pytest.mark.parametrize("m,ws_mb,cfg", [(333, 0, 1), (333, 0, 5), (333, 64, form(SPLIT_PINGPONG, 3)), (2100, 0, 0), (333, 0, form(DIRECT_64)),
+                                         (333, 0, form(DIRECT_WIDE)), (333, 64, form(DIRECT_WIDE, 3))])
+def test_gemm_strided_rows_on_every_form(dev, fmt, m, ws_mb, cfg):
+    """Activation rows ldx > k apart and output rows ldy > n apart (both in elements) through the one-launch forms of the ping-pong
+    kernel (256 x 320 and 128 x 320 tiles, ragged row counts), its split-K form and the direct-operand kernel's: padding columns of
+    the output stay untouched."""
     n, k, ldx, ldy = 656, 1024, 1024 + 64, 656 + 8
     blocks, w16 = H.make_bank(fmt, n, k, seed=13)
     x32 = H.make_x(m, k, 17)
@@ -168,8 +192,8 @@ def test_gemm_strided_rows_on_every_ping_pong_form(dev, fmt, m, ws_mb):
     yb = dev.put(np.full((m, ldy), 0x7FC0, np.uint16))  # bf16 NaN pattern in the padding
     ws = dev.alloc(ws_mb << 20) if ws_mb else None
     view = H.view_of(dev, bank, fmt, n, k)
-    st = dev.lib.qwhip_gemm(dev.stream.handle, C.byref(view), xb.ptr, qwhip.F16, m, ldx, yb.ptr, qwhip.BF16, ldy, qwhip.X_PREROTATED,
-                            ws.ptr if ws else None, ws.nbytes if ws else 0)
+    st = dev.lib.qwhip_gemm(dev.stream.handle, C.byref(view), xb.ptr, qwhip.F16, m, ldx, yb.ptr, qwhip.BF16, ldy,
+                            qwhip.X_PREROTATED | cfg << 8, ws.ptr if ws else None, ws.nbytes if ws else 0)
     assert st == qwhip.OK
     dev.stream.sync()
     raw = yb.download(np.uint16, (m, ldy))
@@ -289,13 +313,15 @@ def test_gemm_swiglu_every_container_and_row_count_in_one_launch(dev, fmt, m, xd
 
 
 @pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq4_g64", "hq8_g32", "hq3_g32"])
-@pytest.mark.parametrize("m,inter,k,xdtype,prerot", [(64, 320, 2048, "f16", True), (100, 480, 1536, "bf16", True), (37, 160, 1024, "f16", False),
-                                                     (128, 800, 5120, "bf16", False)])
-def test_gemm_swiglu_split_k_with_a_roomy_workspace(dev, fmt, m, inter, k, xdtype, prerot):
-    """Few tiles, a long K and a workspace with room for an f16 gate|up image and fp32 planes behind the activation copy: the
-    fused door deals the K-steps over several workgroups, sums the planes and runs the SwiGLU pass - the same bits as qwhip_gemm
-    (which splits the same way when neither workspace binds) followed by qwhip_swiglu_fwht, within the bar of the oracle, and
-    within rounding of its own one-launch form (flags bits 8..11 set keep that)."""
+@pytest.mark.parametrize("m,inter,k,xdtype,prerot,cfg", [
+    (64, 320, 2048, "f16", True, form(SPLIT_PINGPONG, 4)), (100, 480, 1536, "bf16", True, form(SPLIT_PINGPONG, 5)),
+    (37, 160, 1024, "f16", False, form(DIRECT_64, 3)), (128, 800, 5120, "bf16", False, form(DIRECT_WIDE, 7)),
+    (64, 320, 2048, "f16", True, 0), (100, 480, 1536, "bf16", True, 0), (37, 160, 1088, "f16", False, 0)])
+def test_gemm_swiglu_split_k_with_a_roomy_workspace(dev, fmt, m, inter, k, xdtype, prerot, cfg):
+    """Few tiles, a long K and a workspace with room for planes: the fused door deals the K-steps over several workgroups (the
+    ping-pong tile and both spans of the direct-operand kernel, short last ranges among them, and what it takes by itself), sums the
+    planes and runs the SwiGLU pass - the same bits as qwhip_gemm followed by qwhip_swiglu_fwht, within the bar of the oracle, and
+    within rounding of its own one-launch form (flags bits 8..11 = 1 keep that)."""
     n = 2 * inter
     blocks, w16 = H.make_bank(fmt, n, k, seed=6)
     x32 = H.make_x(m, k, 14)
@@ -307,6 +333,7 @@ def test_gemm_swiglu_split_k_with_a_roomy_workspace(dev, fmt, m, inter, k, xdtyp
         x_val = x_host.astype(np.float32)
     flags = qwhip.X_PREROTATED if (prerot or not rotate) else 0
     x_basis = x_val.astype(np.float16) if flags else qo.fwht32_ortho(x_val).astype(np.float16)
+    named = flags | cfg << 8
     bank, xb = dev.put(blocks), dev.put(x_host)
     gu = dev.alloc(m * n * 2)
     acts = [dev.put(np.zeros((m, inter), np.float16)) for _ in range(3)]
@@ -314,9 +341,9 @@ def test_gemm_swiglu_split_k_with_a_roomy_workspace(dev, fmt, m, inter, k, xdtyp
     view = H.view_of(dev, bank, fmt, n, k)
     lib, st = dev.lib, dev.stream.handle
     # bf16 rows go through the separate conversion pass in both doors (flags bit 16 asks qwhip_gemm for it), so both split alike
-    qwhip.check(lib.qwhip_gemm(st, C.byref(view), xb.ptr, xcode, m, 0, gu.ptr, qwhip.F16, 0, flags | (1 << 16), ws.ptr, ws.nbytes))
+    qwhip.check(lib.qwhip_gemm(st, C.byref(view), xb.ptr, xcode, m, 0, gu.ptr, qwhip.F16, 0, named | (1 << 16), ws.ptr, ws.nbytes))
     qwhip.check(lib.qwhip_swiglu_fwht(st, gu.ptr, qwhip.F16, acts[0].ptr, m, inter, 1))
-    qwhip.check(lib.qwhip_gemm_swiglu(st, C.byref(view), xb.ptr, xcode, m, 0, 1, acts[1].ptr, 0, flags, ws.ptr, ws.nbytes))
+    qwhip.check(lib.qwhip_gemm_swiglu(st, C.byref(view), xb.ptr, xcode, m, 0, 1, acts[1].ptr, 0, named, ws.ptr, ws.nbytes))
     qwhip.check(lib.qwhip_gemm_swiglu(st, C.byref(view), xb.ptr, xcode, m, 0, 1, acts[2].ptr, 0, flags | (1 << 8), ws.ptr, ws.nbytes))
     dev.stream.sync()
     two, split, one = (a.download(np.float16, (m, inter)) for a in acts)
@@ -331,19 +358,22 @@ def test_gemm_swiglu_split_k_with_a_roomy_workspace(dev, fmt, m, inter, k, xdtyp
 
 
 @pytest.mark.parametrize("fmt", sorted(f for f in H.FORMATS if f != "aq8_g256"))
-@pytest.mark.parametrize("m,n,k,xdtype,ws_mb", [(17, 272, 1920, "f16", 64), (65, 272, 2048, "bf16", 64), (33, 4112, 2048, "f16", 0),
-                                                (97, 4112, 2048, "bf16", 0), (333, 16384, 2048, "f16", 0)])
-def test_gemm_direct_operand_kernel(dev, fmt, m, n, k, xdtype, ws_mb):
-    """The direct-operand kernel where the price rule takes it: K ranges with a short last one, spans of 64 and of 128 rows (96 on the
-    6- and 8-bit containers), ragged rows, a partial column tile.  fp32 sums of k exact products against fp64; the 2-byte outputs
-    are their roundings, and the gate|up door gives the two doors' bits."""
+@pytest.mark.parametrize("m,n,k,xdtype,cfg", [
+    (17, 272, 1920, "f16", form(DIRECT_64, 4)), (65, 272, 2048, "bf16", form(DIRECT_64, 6)), (33, 4112, 2048, "f16", form(DIRECT_64)),
+    (40, 1088, 1024, "f16", form(DIRECT_64)), (97, 4112, 2048, "bf16", form(DIRECT_WIDE)), (150, 272, 1920, "bf16", form(DIRECT_WIDE, 4)),
+    (333, 1040, 2048, "f16", form(DIRECT_WIDE, 3)), (129, 1088, 1024, "f16", form(DIRECT_WIDE)), (1, 64, 128, "f16", form(DIRECT_WIDE))])
+def test_gemm_direct_operand_kernel(dev, fmt, m, n, k, xdtype, cfg):
+    """The direct-operand kernel: spans of 64 and of 128 rows (96 on the 6- and 8-bit containers), in one launch and over K ranges with
+    a short last one, f16 and bf16 rows, ragged rows, partial column tiles, one pair of K-steps.  fp32 sums of k exact products against
+    fp64; the 2-byte outputs are their roundings, and the gate|up door (partial tiles of 128 outputs) gives the two doors' bits."""
+    ws_mb = 64 if cfg >> 4 else 0
     blocks, w16 = H.make_bank(fmt, n, k, seed=31)
     x32 = H.make_x(m, k, 7)
     x_host, xcode = (qo.f32_to_bf16_bits(x32), qwhip.BF16) if xdtype == "bf16" else (x32.astype(np.float16), qwhip.F16)
     xs = (qo.round_bf16(x32) if xdtype == "bf16" else x32).astype(np.float16).astype(np.float64)
     bank, xb, ws = dev.put(blocks), dev.put(x_host), dev.alloc(max(1, ws_mb << 20))
     view = H.view_of(dev, bank, fmt, n, k)
-    lib, st, flags = dev.lib, dev.stream.handle, qwhip.X_PREROTATED
+    lib, st, flags = dev.lib, dev.stream.handle, qwhip.X_PREROTATED | cfg << 8
     wsp = (ws.ptr, ws_mb << 20) if ws_mb else (None, 0)
     y32, y16, yb = dev.alloc(m * n * 4), dev.alloc(m * n * 2), dev.alloc(m * n * 2)
     for y, dt in ((y32, qwhip.F32), (y16, qwhip.F16), (yb, qwhip.BF16)):
@@ -355,7 +385,7 @@ def test_gemm_direct_operand_kernel(dev, fmt, m, n, k, xdtype, ws_mb):
     assert np.array_equal(y16.download(np.float16, (m, n)), got.astype(np.float16))
     assert np.array_equal(yb.download(np.uint16, (m, n)), qo.f32_to_bf16_bits(got))
     if xdtype == "f16" and n % 64 == 0:
-        act1, act2 = dev.alloc(m * n), dev.alloc(m * n)
+        act1, act2 = dev.alloc(m * n), dev.alloc(m * n)   # [m, n / 2] f16
         qwhip.check(lib.qwhip_gemm_swiglu(st, C.byref(view), xb.ptr, xcode, m, 0, 1, act1.ptr, 0, flags, *wsp))
         qwhip.check(lib.qwhip_swiglu_fwht(st, y16.ptr, qwhip.F16, act2.ptr, m, n // 2, 1))
         dev.stream.sync()
