@@ -295,10 +295,12 @@ qwhip_status qwhip_embed_bf16_f32(qwhip_stream_t s, const void* table_bf16, uint
  * Requires k % 64 == 0 and n % 16 == 0 else QWHIP_E_BAD_GEOMETRY (the reference's tensor path
  * requires N, K multiples of 64).  Activations must be in the container's basis
  * (QWHIP_X_PREROTATED) unless `workspace` holds m*k f16 elements for the rotated copy.
- * A problem of few tiles (about m * n <= 128 * 128 * 320) whose workspace also holds fp32 planes of m * n
- * elements (after the activation copy, rounded up to 256 bytes, when there is one) runs its K-steps in 2..8
- * ranges and sums the planes in range order in a second launch, when the K-steps saved outweigh the traffic
- * of the planes; the result depends on the workspace size only through that choice, never on its contents. */
+ * Where the workspace also holds fp32 planes of m * n elements (after the activation copy, rounded up to 256 bytes,
+ * when there is one) and that is priced as the faster form, the K-steps run in ranges, one plane each, and a second
+ * launch sums the planes in range order: 2..12 ranges up to 1024 rows, 2..8 on few tiles (about m * n <= 128 * 128 * 320)
+ * at any m.  The result depends on the workspace size only through that choice, never on its contents.
+ * A row's bits may depend on m, with and without planes: the kernels for up to 1024 rows and those for more add the
+ * same exact products in another order (fp32). */
 qwhip_status qwhip_gemm(qwhip_stream_t s, const qwhip_weight_view* w, const void* x, uint32_t x_dtype,
                         uint32_t m, uint32_t ldx, void* y, uint32_t y_dtype, uint32_t ldy, uint32_t flags,
                         void* workspace, uint64_t workspace_bytes);
@@ -380,13 +382,11 @@ qwhip_status qwhip_moe_grouped_gemm(qwhip_stream_t s, const qwhip_weight_view* w
  * (qmm_t_nax_swiglu_impl, Sources/QWMetal/include/qw_gemm_nax_swiglu.metalh:86-167; door
  * Sources/Runtime/QWEngine/Driver/EncodeKernels.swift:156-190).  w: [2 * inter, k], rows [gate | up]; act f16 [m, inter]
  * = f16(FWHT32(silu(g) * u)) with g, u rounded to f16 first - bit-identical to qwhip_gemm (f16 out) followed by
- * qwhip_swiglu_fwht, without the [m, 2 inter] matrix.  One launch for every container and any m; inter % 32 == 0, act
- * 16-byte aligned with ldact % 8 == 0 (0 = inter); x, flags and workspace as qwhip_gemm (bf16 or un-rotated activations
- * need the workspace: m * k * 2 bytes).  A problem of few tiles and a long K whose workspace also holds, behind the
- * activation copy, an f16 image of the gate|up matrix (m * 2 inter * 2 bytes, rounded up to 256) and fp32 planes of
- * m * 2 inter elements runs as qwhip_gemm does with K ranges and then qwhip_swiglu_fwht from the image, when that is
- * the faster form (packed act rows only; flags bits 8..11 != 0 keep the one launch); as there, the result depends on
- * the workspace size only through that choice. */
+ * qwhip_swiglu_fwht with the same rows, flags and workspace, without the [m, 2 inter] matrix.  Every container and any m;
+ * inter % 32 == 0, act 16-byte aligned with ldact % 8 == 0 (0 = inter); x, flags and workspace as qwhip_gemm (bf16 or
+ * un-rotated activations need the workspace: m * k * 2 bytes).  One launch, or K ranges and the sum of their planes, which
+ * applies the activation, where qwhip_gemm would take them; as there, the result depends on the workspace size only
+ * through that choice. */
 qwhip_status qwhip_gemm_swiglu(qwhip_stream_t s, const qwhip_weight_view* w, const void* x, uint32_t x_dtype, uint32_t m,
                                uint32_t ldx, uint32_t rotate_act, void* act_f16, uint32_t ldact, uint32_t flags,
                                void* workspace, size_t workspace_bytes);

@@ -1143,6 +1143,34 @@ __global__ __launch_bounds__(256) void qw_splitk_reduce_kernel(const float* __re
     for (int e = 0; e < 4; ++e) qg_store<YDT>(y, (uint64_t)row * ldy + c + e, acc[e]);
 }
 
+// The same sums of a gate|up matrix with the gated activation (+ FWHT-32) behind them, act f16 [M, ldact]: the arithmetic of
+// qw_splitk_reduce_kernel into f16 and qwhip_swiglu_fwht after it, without the f16 matrix between them, so the fused door needs the
+// planes' room alone, as qwhip_gemm does.  Eight channels a lane, four lanes a rotation group (N % 64 == 0).  Bound by the planes' read.
+template <bool ROT>
+__global__ __launch_bounds__(256) void qw_splitk_gated_kernel(const float* __restrict__ part, uint32_t splits, uint32_t M, uint32_t N,
+                                                              h1_t* __restrict__ act, uint32_t ldact, const qw_act ga) {
+    const uint32_t inter = N / 2u, n8 = inter / 8u;
+    const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+    if (i >= (uint64_t)M * n8) return;   // whole groups of four lanes leave together
+    const uint32_t row = (uint32_t)(i / n8), c = (uint32_t)(i - (uint64_t)row * n8) * 8u;
+    const uint64_t plane = (uint64_t)M * N;
+    typedef float fl4_t __attribute__((ext_vector_type(4)));
+    const float* g = part + (uint64_t)row * N + c;
+    fl4_t acc[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[q] = *(const fl4_t*)(g + (q >> 1) * (uint64_t)inter + (q & 1) * 4);
+    for (uint32_t sidx = 1; sidx < splits; ++sidx) {
+        g += plane;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] += *(const fl4_t*)(g + (q >> 1) * (uint64_t)inter + (q & 1) * 4);
+    }
+    float f[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = qw_gated((float)(h1_t)acc[e >> 2][e & 3], (float)(h1_t)acc[2 + (e >> 2)][e & 3], ga);
+    if (ROT) qw_fwht32_quad(f, threadIdx.x);
+    qw_store8_f16(act + (uint64_t)row * ldact + c, f);
+}
+
 template <int FMT, int YDT, bool SWIGLU, bool GACT = false, int XDT = QWHIP_F16>
 hipError_t launch_cfg4(hipStream_t st, const qw_gemm_params& p, dim3 grid) {
     // two activation stages, or the four epilogue slabs (32 rows x (128 + 16) bytes each) when they are larger
@@ -1288,6 +1316,13 @@ hipError_t launch_plane_sum(hipStream_t st, const qw_gemm_params& p, uint32_t sp
     return hipGetLastError();
 }
 
+hipError_t launch_plane_gated(hipStream_t st, const qw_gemm_params& p, uint32_t splits, const float* part) {
+    const dim3 grid((unsigned)(((uint64_t)p.M * (p.inter / 8u) + 255u) / 256u));
+    if (p.rotate_act) hipLaunchKernelGGL(qw_splitk_gated_kernel<true>, grid, dim3(256), 0, st, part, splits, p.M, p.N, (h1_t*)p.y, p.ldy, p.act);
+    else hipLaunchKernelGGL(qw_splitk_gated_kernel<false>, grid, dim3(256), 0, st, part, splits, p.M, p.N, (h1_t*)p.y, p.ldy, p.act);
+    return hipGetLastError();
+}
+
 // split-K launch of the half-height ping-pong tile into the fp32 planes at p.y
 template <int FMT>
 hipError_t launch_splitk(hipStream_t st, const qw_gemm_params& p, uint32_t splits) {
@@ -1373,8 +1408,9 @@ gemm_route choose_direct(const qwhip_weight_view* w, uint32_t m, int fmt, uint32
 // flags bits 8..11 of the dense doors that name a K-split or direct form, for tuning and tests; bits 12..15: its K ranges (0 = one)
 enum { OV_DIRECT_64 = 6, OV_DIRECT_WIDE = 7, OV_SPLIT_PINGPONG = 8 };
 
-// The route of a dense problem: the automatic choice, or the form that the flags name.  Both dense doors call it with the same
-// room for planes, so that the fused gate|up gives the bits of the plain door and the activation pass after it.
+// The route of a dense problem: the automatic choice, or the form that the flags name.  Both dense doors call it with the room for
+// planes behind a copy of the rows that both make or neither, so that the fused gate|up gives the bits of the plain door and the
+// activation pass after it whatever the workspace holds (2-byte rows of y that are not 16-byte aligned, y_ok = false, excepted).
 qwhip_status choose_route(const qwhip_weight_view* w, uint32_t m, int fmt, uint32_t flags, bool y_ok, uint64_t plane_room, gemm_route* r) {
     const uint32_t ov = (flags >> 8) & 0xFu, ranges = (flags >> 12) & 0xFu;
     *r = {false, false, 0u};
@@ -1585,19 +1621,27 @@ extern "C" qwhip_status qwhip_gemm_swiglu(qwhip_stream_t s, const qwhip_weight_v
     const bool rotate = qwhip_view_rotated(w) && !(flags & QWHIP_X_PREROTATED);
     const uint64_t ws_need = (uint64_t)m * w->k * 2u;
     const bool ws_ok = workspace && workspace_bytes >= ws_need && ldx == w->k && ((uintptr_t)workspace & 15u) == 0;
+    if (rotate && !ws_ok)
+        return qwhip_fail(QWHIP_E_BASIS, "activations are not in the rotated basis: a 16-byte aligned workspace of %llu bytes and packed rows are needed",
+                          (unsigned long long)ws_need);
+    if (x_dtype == QWHIP_BF16 && !ws_ok)
+        return qwhip_fail(QWHIP_E_BAD_GEOMETRY, "bf16 activations need the f16 workspace (%llu bytes, packed rows)", (unsigned long long)ws_need);
+    // The route, from the room for planes that qwhip_gemm finds in the same workspace: bf16 rows in the basis are read in place over K
+    // ranges, as there, and copied for the one launch only.
+    const bool copy_needed = rotate || (x_dtype == QWHIP_BF16 && (flags & (1u << 16)));
+    const uint64_t x_used = copy_needed ? ((ws_need + 255u) & ~(uint64_t)255u) : 0u;
+    const bool planes_ok = workspace && ((uintptr_t)workspace & 15u) == 0;
+    gemm_route route;
+    st = choose_route(w, m, fmt, flags, true, planes_ok && workspace_bytes > x_used ? workspace_bytes - x_used : 0u, &route);
+    if (st != QWHIP_OK) return st;
+    const bool planes = route.splits >= 2u;
     const void* xin = x;
-    if (rotate) {
-        if (!ws_ok)
-            return qwhip_fail(QWHIP_E_BASIS, "activations are not in the rotated basis: a 16-byte aligned workspace of %llu bytes and packed rows are needed",
-                              (unsigned long long)ws_need);
-        st = qwhip_fwht32(s, x, x_dtype, workspace, (uint64_t)m * w->k);
+    uint32_t xdt = x_dtype;
+    if (copy_needed || (x_dtype == QWHIP_BF16 && !planes)) {
+        st = rotate ? qwhip_fwht32(s, x, x_dtype, workspace, (uint64_t)m * w->k) : qw_convert_to_f16(s, x, x_dtype, workspace, (uint64_t)m * w->k);
         if (st != QWHIP_OK) return st;
         xin = workspace;
-    } else if (x_dtype == QWHIP_BF16) {
-        if (!ws_ok) return qwhip_fail(QWHIP_E_BAD_GEOMETRY, "bf16 activations need the f16 workspace (%llu bytes, packed rows)", (unsigned long long)ws_need);
-        st = qw_convert_to_f16(s, x, x_dtype, workspace, (uint64_t)m * w->k);
-        if (st != QWHIP_OK) return st;
-        xin = workspace;
+        xdt = QWHIP_F16;
     }
     qw_gemm_params p = {};
     p.bank = (const uint8_t*)w->blocks;
@@ -1614,27 +1658,17 @@ extern "C" qwhip_status qwhip_gemm_swiglu(qwhip_stream_t s, const qwhip_weight_v
     p.inter = inter;
     p.rotate_act = rotate_act ? 1u : 0u;
     p.act = s->dev->act;
-    // Few tiles and a workspace with room behind the activation copy for an f16 gate|up image and fp32 planes: the K-steps
-    // of a tile are dealt over 2..8 workgroups as in qwhip_gemm, the planes are summed into the image and the SwiGLU pass
-    // reads that - the two doors called one after the other, from one call.  flags bits 8..11 != 0 keep the one launch.
-    {
-        const uint64_t x_used = xin == workspace ? ((ws_need + 255u) & ~(uint64_t)255u) : 0u;
-        const uint64_t gu_bytes = ((uint64_t)m * w->n * 2u + 255u) & ~(uint64_t)255u;
-        const bool planes_ok = workspace && ((uintptr_t)workspace & 15u) == 0 && ldact == inter && workspace_bytes >= x_used + gu_bytes;
-        gemm_route route;
-        st = choose_route(w, m, fmt, flags, true, planes_ok ? workspace_bytes - x_used - gu_bytes : 0u, &route);
-        if (st != QWHIP_OK) return st;
-        if (route.splits >= 2u) {
-            void* gu = (uint8_t*)workspace + x_used;
-            float* part = (float*)((uint8_t*)workspace + x_used + gu_bytes);
-            QWHIP_TRY_HIP(launch_planes(s->stream, fmt, p, route, QWHIP_F16, part));
-            QWHIP_TRY_HIP(launch_plane_sum(s->stream, p, route.splits, part, gu, QWHIP_F16, w->n));
-            return qwhip_swiglu_fwht(s, gu, QWHIP_F16, act_f16, m, inter, rotate_act);
-        }
-        if (route.direct) {
-            QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, p, 1u, QWHIP_F16, QWHIP_F16, true, route.few));
-            return QWHIP_OK;
-        }
+    // K ranges as in qwhip_gemm: the sum of the planes ends in the activation instead of y
+    if (planes) {
+        float* part = (float*)((uint8_t*)workspace + x_used);
+        p.x_bf16 = xdt == QWHIP_BF16 ? 1u : 0u;
+        QWHIP_TRY_HIP(launch_planes(s->stream, fmt, p, route, xdt, part));
+        QWHIP_TRY_HIP(launch_plane_gated(s->stream, p, route.splits, part));
+        return QWHIP_OK;
+    }
+    if (route.direct) {
+        QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, p, 1u, QWHIP_F16, QWHIP_F16, true, route.few));
+        return QWHIP_OK;
     }
     // The half-height tile where it is the cheaper one by the pricing of choose_cfg (0.78 of the big tile's efficiency per
     // area): up to 128 rows, where the big tile is half idle, and where it fills the chip and

@@ -357,6 +357,38 @@ def test_gemm_swiglu_split_k_with_a_roomy_workspace(dev, fmt, m, inter, k, xdtyp
     assert qo.normalized_error(split.astype(np.float32), one.astype(np.float32)) <= TOL
 
 
+@pytest.mark.parametrize("fmt,m,inter,k,xdtype,prerot,ldpad", [
+    ("hq4_g32_m5", 64, 320, 2048, "f16", True, 0), ("hq4_g32_m5", 64, 320, 2048, "bf16", True, 8), ("hq4_g64", 200, 2048, 2048, "f16", True, 0),
+    ("hq6_g32", 33, 352, 1920, "bf16", True, 0), ("aq4_g32", 100, 480, 1088, "f16", True, 16), ("hq3_g32", 37, 160, 2048, "bf16", False, 8)])
+@pytest.mark.parametrize("planes", [0, 1, 2, 3, 4, 9])
+def test_gemm_swiglu_takes_the_k_ranges_of_the_plain_door(dev, fmt, m, inter, k, xdtype, prerot, ldpad, planes):
+    """A workspace that holds exactly `planes` fp32 planes behind the copy of the rows (made by both doors or by neither; where neither
+    makes one, the first plane lies where a bf16 copy would): the fused door gives the bits of the two doors on that workspace, with act
+    rows ldpad elements apart from their neighbours too, whose padding stays as it was."""
+    n = 2 * inter
+    blocks, _ = H.make_bank(fmt, n, k, seed=8)
+    x32 = H.make_x(m, k, 15) * 2
+    x_host, xcode = (qo.f32_to_bf16_bits(x32), qwhip.BF16) if xdtype == "bf16" else (x32.astype(np.float16), qwhip.F16)
+    flags = qwhip.X_PREROTATED if prerot else 0
+    copy = 0 if prerot else (m * k * 2 + 255) // 256 * 256
+    size = max(m * k * 2, copy + planes * m * n * 4)           # the fused door wants room for a copy of bf16 rows in any case
+    bank, xb, ws = dev.put(blocks), dev.put(x_host), dev.alloc(size)
+    gu, act2 = dev.alloc(m * n * 2), dev.alloc(m * inter * 2)
+    ld = inter + ldpad
+    act1 = dev.put(np.full((m, ld), 0x7E01, np.uint16))
+    view = H.view_of(dev, bank, fmt, n, k)
+    lib, st = dev.lib, dev.stream.handle
+    qwhip.check(lib.qwhip_gemm(st, C.byref(view), xb.ptr, xcode, m, 0, gu.ptr, qwhip.F16, 0, flags, ws.ptr, size))
+    qwhip.check(lib.qwhip_swiglu_fwht(st, gu.ptr, qwhip.F16, act2.ptr, m, inter, 1))
+    qwhip.check(lib.qwhip_gemm_swiglu(st, C.byref(view), xb.ptr, xcode, m, 0, 1, act1.ptr, ld, flags, ws.ptr, size))
+    dev.stream.sync()
+    one, two = act1.download(np.uint16, (m, ld)), act2.download(np.uint16, (m, inter))
+    for b in (bank, xb, ws, gu, act1, act2):
+        b.free()
+    assert np.array_equal(one[:, :inter], two)
+    assert np.all(one[:, inter:] == 0x7E01)
+
+
 @pytest.mark.parametrize("fmt", sorted(f for f in H.FORMATS if f != "aq8_g256"))
 @pytest.mark.parametrize("m,n,k,xdtype,cfg", [
     (17, 272, 1920, "f16", form(DIRECT_64, 4)), (65, 272, 2048, "bf16", form(DIRECT_64, 6)), (33, 4112, 2048, "f16", form(DIRECT_64)),
