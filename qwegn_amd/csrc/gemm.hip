@@ -1350,14 +1350,35 @@ uint32_t choose_splits(uint32_t m, uint32_t n, uint32_t k, uint64_t plane_room) 
     return splits < 2u ? 0u : splits;
 }
 
-// The direct-operand kernel (qw_direct.h) for problems of a few rows to about a thousand: spans of 64 or 128 rows by 256 weight
-// rows, K in whole pairs of 64 over 1 .. 12 ranges.  A workgroup's loop costs 0.68 us a pair and 0.24 a fragment of rows
-// (1.34 times that on the 6- and 8-bit containers), a start and an end 7.1 us; ranges add the planes' traffic, at 7.9 TB/s, and
-// the summing launch; the ping-pong kernel is priced the same way (a K-step 1.36 us in a range, 2.35 and 1.66 a round of its
-// tiles, 0.88 on the 128 x 128 tiles).  Fitted to 224 problems, 20 .. 2000 rows on 13 banks of 7 containers, every combination
-// measured (10 % and 9 % of root mean square error); it is taken where it prices below 0.85 of the other, where the fit held: 64 rows on
-// 7168 x 5120 27 -> 20 us, 333 rows on 2560 x 9728 39 -> 36, gate|up of 333 rows on 2 x 9728 x 2560 61 -> 47, 180 rows on
-// 6144 x 16384 80 -> 56; over all of them 1.18 times as fast, 8 of them slower, by 7 % at most.
+// The price, us, of the ping-pong and DMA-fed kernels' route to a dense problem: over K ranges, or choose_cfg's tile in one launch.
+// An XCD takes a contiguous eighth of the tiles, so its 32 units' load is that eighth's, rounded up: 50 tiles over five ranges are 35
+// workgroups on an XCD, and one unit runs two of them.  Fitted to 937 problems, 17 .. 4096 rows on 79 banks of 12 containers: 6 % of root
+// mean square error over ranges, 2 % on 256 x 320 tiles, 7 % on the others (128 x 128 tiles in qwhip_gemm_swiglu's place for a tile of
+// its own: the doors choose alike).
+double price_tiles(uint32_t m, uint32_t n, uint32_t k, int fmt, uint32_t splits) {
+    const bool wide = fmt == QG_FMT_B8 || fmt == QG_FMT_B6;
+    const double nk = k / 64u;
+    if (splits >= 2u) {
+        const double load = qwhip_cdiv(qwhip_cdiv(m, 128u) * qwhip_cdiv(n, 320u), 8u) * splits / 32.0;
+        return 8.5 + 0.225 * splits + qwhip_cdiv(k / 64u, splits) * (1.01 + 0.295 * load) * (wide ? 1.14 : 1.0) +
+               splits * (double)m * n * 4.0 * 2.0 / 6.46e6;
+    }
+    const int cfg = choose_cfg(m, n, fmt == QG_FMT_B8, true, false);
+    const double tiles = (double)qwhip_cdiv(m, kCfgBM[cfg]) * qwhip_cdiv(n, kCfgBN[cfg]);
+    if (cfg == CFG_128x128) return 6.6 + nk * (0.52 + 0.42 * tiles / 256.0) * (wide ? 1.18 : 1.0);
+    if (cfg == CFG_128x320) return 7.8 + priced_rounds(tiles, 256.0) * nk * 1.48 * (wide ? 1.1 : 1.0);
+    return 3.6 + priced_rounds(tiles, 256.0) * (nk * 2.13 * (wide ? 1.064 : 1.0) + 7.5);
+}
+
+// The direct-operand kernel (qw_direct.h): spans of 64 or 128 rows (96 on the 6- and 8-bit containers) by 256 weight rows, K in whole
+// pairs of 64, in one launch at any m and up to 1024 rows over up to twelve ranges.  A workgroup's loop costs 0.86 us a pair and 0.18 a
+// fragment of rows (1.39 times that on the 6- and 8-bit containers), times a slope in the XCDs' load, steeper for the tallest spans; a
+// start and an end 5.3 us; ranges add the planes' traffic, at 7.0 TB/s, and the summing launch.  Fitted to 9756 measured forms of the same
+// problems, 7 % of root mean square error.  It is taken below 0.9 of the other kernels' price.
+// Over 654 other problems, drawn alike: 0.81 of their time (0.67 up to 64 rows, 0.76 to 256, 0.89 to 1024, 0.93 past), three slower by
+// more than 3 % (9 % at most); qwhip_gemm_swiglu over 434 others 0.79, one slower by more than 3 % (10 %).  With the load taken over the
+// whole chip 17 of 766 were slower, by up to 23 % (640 rows on 2560 x 9728 over five ranges 61 us against 53, 333 rows on 7168 x 5120
+// over three 54 against 48).
 struct gemm_route {
     bool direct, few;    // the direct-operand kernel, its spans of 64 rows
     uint32_t splits;     // K ranges into fp32 planes (two and more), or one launch
@@ -1371,31 +1392,22 @@ gemm_route choose_direct(const qwhip_weight_view* w, uint32_t m, int fmt, uint32
     if (!direct_takes(w)) return best;
     const bool wide = fmt == QG_FMT_B8 || fmt == QG_FMT_B6;
     const double plane = (double)m * n * 4.0;
-    const uint32_t nk = k / 64u, pairs = nk / 2u, frags = qwhip_cdiv(m, 32u), cols = qwhip_cdiv(n, 256u);
-    double limit;
-    if (old_splits >= 2u) {
-        limit = 7.4 + qwhip_cdiv(nk, old_splits) * 1.36 * (wide ? 1.1 : 1.0) + old_splits * plane * 2.0 / 6.3e6;
-    } else {
-        double step = std::min(1.66 * priced_rounds((double)qwhip_cdiv(m, 128u) * qwhip_cdiv(n, 320u), 256.0),
-                               2.35 * priced_rounds((double)qwhip_cdiv(m, 256u) * qwhip_cdiv(n, 320u), 256.0));
-        if ((uint64_t)qwhip_cdiv(m, 128u) * qwhip_cdiv(n, 128u) <= 256u) step = std::min(step, 0.88);
-        limit = 5.4 + nk * step * (wide ? 1.1 : 1.0);
-    }
-    limit *= 0.85;
-    const double bank_us = 7.1 + (double)n * (double)qwhip_view_row_bytes(w) / 3.5e6;   // and no faster than the bank streams to this kernel
+    const uint32_t pairs = k / 128u, frags = qwhip_cdiv(m, 32u), cols = qwhip_cdiv(n, 256u);
+    double limit = 0.9 * price_tiles(m, n, k, fmt, old_splits);
+    const double bank_us = 5.3 + (double)n * (double)qwhip_view_row_bytes(w) / 3.5e6;   // no faster than the bank streams to this kernel
     for (uint32_t few = 0; few < 2u; ++few) {
         const uint32_t span = few ? 2u : wide ? 3u : 4u;
         if (!few && frags <= 2u) continue;
         const uint32_t spans = qwhip_cdiv(frags, span);
-        const double per_pair = (0.68 + 0.24 * min(span, qwhip_cdiv(frags, spans))) * (wide ? 1.34 : 1.0);
+        const double per_pair = (0.86 + 0.18 * min(span, qwhip_cdiv(frags, spans))) * (wide ? 1.39 : 1.0);
         for (uint32_t splits = 1; splits <= min(12u, pairs); ++splits) {
             const uint32_t per = qwhip_cdiv(pairs, splits);
             if (splits > 1u && (m > 1024u || n % 4u != 0 || (splits - 1u) * per >= pairs || splits * plane > (double)plane_room)) continue;
-            const double load = (double)spans * cols * splits / 256.0;
-            const double rounds = load <= 1.0 ? 1.0 : load <= 2.0 ? 2.0 : load + 0.4;
-            double t = 7.1 + per * per_pair * rounds;
-            if (t < bank_us) t = bank_us;
-            if (splits > 1u) t += 1.6 + 0.19 * splits + splits * plane * 2.0 / 7.9e6;
+            const double load = qwhip_cdiv(spans * cols, 8u) * splits / 32.0;
+            const double rounds = span == 4u ? (load <= 1.0 ? 1.0 + 0.29 * load : load <= 2.0 ? 1.30 + 0.47 * load : 0.20 + 1.24 * load)
+                                             : (load <= 1.0 ? 1.0 + 0.10 * load : load <= 2.0 ? 1.41 + 0.19 * load : 0.36 + 0.885 * load);
+            double t = std::max(5.3 + per * per_pair * rounds, bank_us);
+            if (splits > 1u) t += 2.0 + 0.24 * splits + splits * plane * 2.0 / 7.0e6;
             if (t < limit) {
                 limit = t;
                 best = {true, few != 0u, splits};

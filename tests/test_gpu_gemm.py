@@ -427,6 +427,19 @@ def test_gemm_direct_operand_kernel(dev, fmt, m, n, k, xdtype, cfg):
         b.free()
 
 
+def test_gemm_ranges_fit_an_xcd(dev):
+    """An eighth of the tiles, rounded up, over the ranges is what an XCD's 32 units hold: 50 tiles over five ranges are 35 workgroups on
+    an XCD although they are 250 on the chip.  The automatic choice is another form (other fp32 sums)."""
+    fmt, m, n, k = "hq4_g64", 640, 2560, 9728
+    st, out, ref = run_gemm(dev, fmt, m, n, k, xdtype="f16", ydtype="f32", seed=9, workspace_bytes=96 << 20)
+    assert st == qwhip.OK
+    assert qo.normalized_error(out, ref) <= 2e-5
+    st, other, _ = run_gemm(dev, fmt, m, n, k, xdtype="f16", ydtype="f32", seed=9, workspace_bytes=96 << 20, cfg=form(DIRECT_WIDE, 5))
+    assert st == qwhip.OK
+    assert qo.normalized_error(out, other) <= 4e-5         # each within 2e-5 of the exact sums
+    assert not np.array_equal(out, other)
+
+
 def test_gemm_swiglu_refusals(dev):
     blocks, _ = H.make_bank("hq8_g32", 128, 64, seed=1)
     bank, xb, act = dev.put(blocks), dev.put(np.zeros((64, 64), np.float16)), dev.alloc(64 * 64 * 2)
