@@ -1728,7 +1728,7 @@ hipError_t launch_grouped_direct(hipStream_t st, const qw_gemm_params& p, dim3 g
 }
 template <int FMT>
 hipError_t launch_grouped_xy(hipStream_t st, const qw_gemm_params& p, dim3 grid, uint32_t xdt, uint32_t ydt) {
-    if (!p.force_gemm2 && (ydt == QWHIP_F32 || (p.ldy % 8u == 0 && ((uintptr_t)p.y & 15u) == 0))) {
+    if (ydt == QWHIP_F32 || (p.ldy % 8u == 0 && ((uintptr_t)p.y & 15u) == 0)) {
         if (xdt == QWHIP_F16) return launch_grouped_direct<FMT, QWHIP_F16>(st, p, grid, ydt);
         return launch_grouped_direct<FMT, QWHIP_BF16>(st, p, grid, ydt);
     }
@@ -1793,8 +1793,8 @@ extern "C" qwhip_status qwhip_moe_grouped_gemm(qwhip_stream_t s, const qwhip_wei
     p.rows_per_expert = rows_per_expert;
     const dim3 grid(qwhip_cdiv(rows_per_expert, 256u), max_tiles);
     hipError_t e;
-    if (!p.force_gemm2 && qw_grouped_direct_takes(p) && (y_dtype == QWHIP_F32 || (ldy % 8u == 0 && ((uintptr_t)y & 15u) == 0))) {
-        p.tiles_n = grid.x;
+    p.tiles_n = grid.x;
+    if (qw_grouped_direct_takes(fmt, p, experts) && (y_dtype == QWHIP_F32 || (ldy % 8u == 0 && ((uintptr_t)y & 15u) == 0))) {
         QWHIP_TRY_HIP(qw_grouped_direct(s->stream, fmt, p, max_tiles, experts, x_dtype, y_dtype, false));
         return QWHIP_OK;
     }
@@ -1853,7 +1853,7 @@ extern "C" qwhip_status qwhip_moe_grouped_gemm_swiglu(qwhip_stream_t s, const qw
     p.rotate_act = rotate_act ? 1u : 0u;
     p.act = s->dev->act;
     p.tiles_n = qwhip_cdiv(inter, 128u);
-    if (qw_grouped_direct_takes(p)) {
+    if (qw_grouped_direct_takes(fmt, p, experts)) {
         QWHIP_TRY_HIP(qw_grouped_direct(s->stream, fmt, p, max_tiles, experts, x_dtype, QWHIP_F16, true));
         return QWHIP_OK;
     }

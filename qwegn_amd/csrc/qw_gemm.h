@@ -34,7 +34,7 @@ __device__ __forceinline__ void qg_store(void* y, uint64_t idx, float v) {
 
 // gemm_direct.hip: grouped GEMM on direct weight operands (K in whole pairs of 64, groups of at most 128); max_tiles as the door's,
 // p.tiles_n column tiles of 256 weight rows (swiglu: of 128 outputs)
-bool qw_grouped_direct_takes(const qw_gemm_params& p);
+bool qw_grouped_direct_takes(int fmt, const qw_gemm_params& p, uint32_t experts);
 hipError_t qw_grouped_direct(hipStream_t st, int fmt, const qw_gemm_params& p, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt,
                              bool swiglu);
 // gemm_mid.hip: the dense form.  splits > 1: fp32 planes [splits][M][ldy] at p.y (ydt f32), no range of K pairs empty; swiglu: f16

@@ -356,20 +356,28 @@ def test_fused_gate_up_swiglu_equals_the_two_step_chain(dev, fmt, t, experts, hi
 
 
 _SPANS_FEW = [1, 16, 17, 0, 32, 33, 63, 64, 65, 2]                  # at most 48 rows an expert: spans of 64
-_SPANS_MANY = [31, 64, 96, 97, 0, 128, 129, 160, 161, 225, 300]     # spans of 128 (96 on the 6- and 8-bit containers)
+_SPANS_MANY = [31, 64, 96, 97, 0, 128, 129, 160, 161, 225, 300]     # spans of 128 (96 on the 6- and 8-bit containers) on wide enough banks
 
 
-@pytest.mark.parametrize("fmt", sorted(H.FORMATS))
-@pytest.mark.parametrize("counts,k,inter,xdt,compact", [(_SPANS_FEW, 128, 96, "f16", True), (_SPANS_FEW, 384, 32, "bf16", False),
-                                                        (_SPANS_MANY, 384, 96, "f16", False), (_SPANS_MANY, 128, 160, "bf16", True)])
+_SPANS_M5 = [3000, 2725]                                            # HQ4_G32_M5 takes them on K past 2048 only
+
+
+@pytest.mark.parametrize("fmt,counts,k,inter,xdt,compact", [
+    (fmt, *case) for fmt in sorted(H.FORMATS)
+    for case in [(_SPANS_FEW, 128, 96, "f16", True), (_SPANS_FEW, 768, 32, "bf16", False), (_SPANS_MANY, 384, 96, "f16", False)]
+    + ([(_SPANS_M5, 2176, 2144, "f16", True)] if fmt == "hq4_g32_m5" else [(_SPANS_MANY, 128, 6688, "bf16", True)])]
+    + [(fmt, _SPANS_MANY, 384, 6688, "f16", False) for fmt in ("hq4_g64", "hq3_g32", "hq6_g32")])
 def test_grouped_gemm_spans(dev, fmt, counts, k, inter, xdt, compact):
-    """Experts of every span shape (fragment edges, the last row of a span, empty experts), one and three pairs of K-steps, partial
-    column tiles: fp32 sums of k exact products against fp64, f16 and bf16 as their roundings, the fused gate|up bit for bit."""
+    """Experts of every span shape (fragment edges, the last row of a span, empty experts), one, three and six pairs of K-steps (up to
+    five of them 8-bit banks this small take the 64-row kernel), partial column tiles: fp32 sums of k exact products against fp64, f16 and bf16 as their roundings, the fused gate|up bit for bit."""
     if fmt in ("aq8_g256",):
         k = 256 * (k // 128)                                          # whole groups; takes the 64-row kernel
     e, n = len(counts), 2 * inter
-    blocks, w16 = H.make_bank(fmt, e * n, k, seed=21)
     rng = np.random.default_rng(k + inter)
+    blocks, w16 = H.make_bank(fmt, min(e * n, 3001), k, seed=21)
+    if e * n > 3001:
+        pick = rng.integers(0, 3001, e * n)                           # a large bank's rows are drawn from fewer
+        blocks, w16 = blocks[pick], w16[pick]
     ids = rng.permutation(np.repeat(np.arange(e), counts)).astype(np.int32).reshape(-1, 1)
     pairs = ids.size
     x, xcode, xval = _hidden_rows(rng, pairs, k, xdt)
@@ -396,14 +404,15 @@ def test_grouped_gemm_spans(dev, fmt, counts, k, inter, xdt, compact):
     assert np.array_equal(act1.download(np.uint16, (pairs, inter)), act2.download(np.uint16, (pairs, inter)))
 
 
-@pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq8_g32"])
-@pytest.mark.parametrize("counts", [_SPANS_FEW, _SPANS_MANY, [2300, 40]])
-def test_grouped_gemm_takes_any_tile_list(dev, fmt, counts):
+@pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq8_g32", "hq4_g64"])
+@pytest.mark.parametrize("counts,inter", [(_SPANS_FEW, 96), (_SPANS_MANY, 96), ([2300, 40], 96), (_SPANS_MANY, 6656), ([2300, 40], 4992)])
+def test_grouped_gemm_takes_any_tile_list(dev, fmt, counts, inter):
     """A caller's own list of tiles - another order, a part of the sort's - gives the rows of the tiles that are in it, the same bits
-    as the whole list, and leaves the other rows alone."""
-    e, k, inter = len(counts), 128, 96
+    as the whole list, and leaves the other rows alone: spans of 64 rows, and on the wide banks of 128 (96), but for HQ4_G32_M5."""
+    e, k = len(counts), 768 if inter == 96 else 128
     n = 2 * inter
-    blocks, _ = H.make_bank(fmt, e * n, k, seed=22)
+    blocks, _ = H.make_bank(fmt, min(e * n, 3001), k, seed=22)
+    blocks = blocks[np.random.default_rng(e).integers(0, len(blocks), e * n)]
     ids = np.repeat(np.arange(e), counts).astype(np.int32).reshape(-1, 1)
     pairs = ids.size
     g = _group(dev, ids, e, 1)
