@@ -658,11 +658,13 @@ bool qw_col_pair_gemv(hipStream_t st, const qwhip_weight_view* w, const void* x,
     const uint32_t sets = cpr <= 3u ? 4u : 2u, h2 = sets / 2u;
     const uint32_t threads = 32u * cpr * sets;
     const uint32_t waves = (threads + 63u) / 64u;
-    // ten waves per compute unit, as the compiled window of the GEMV, in whole multiples of the units, and three workgroups a unit up to
-    // six waves (2 x 8704 x 2560: 512 workgroups 8.06 us, 768 7.68; 2 x 17408 x 5120 level); at least four channels per set, on few
-    // channels two for up to two workgroups a unit (2 x 2048 x 2048: 256 workgroups 4.18 us, 512 3.76; 2 x 4096 x 2048: 512 4.82, 768 5.03)
+    // ten waves per compute unit, as the compiled window of the GEMV, in whole multiples of the units, three workgroups a unit up to six
+    // waves where the channels give them all (2 x 8704 x 2560: 512 workgroups 8.06 us, 768 7.68; 2 x 17408 x 5120 20.1, 19.6; but 2 x 4224 x
+    // 2304: 512 5.5, 528 5.8, 2 x 2560 x 5120: 512 5.6, 640 5.8); at least four channels per set, on few channels two for up to two
+    // workgroups a unit (2 x 2048 x 2048: 256 workgroups 4.18 us, 512 3.76; 2 x 4096 x 2048: 512 4.82, 768 5.03)
     uint32_t wgs = (256u * 10u + waves / 2u) / waves;
-    wgs = max(waves <= 6u ? 768u : 256u, (wgs + 128u) / 256u * 256u);
+    wgs = max(256u, (wgs + 128u) / 256u * 256u);
+    if (waves <= 6u && inter / (h2 * 4u) >= 768u) wgs = max(wgs, 768u);
     wgs = max(min(wgs, inter / (h2 * 4u)), min(min(wgs, 512u), max(1u, inter / (h2 * 2u))));
     wgs = max(wgs, qwhip_cdiv(inter, 64u));                        // at most 128 row slots per workgroup
     const uint32_t ch_per_wg = qwhip_cdiv(inter, wgs);
