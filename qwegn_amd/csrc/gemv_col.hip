@@ -558,6 +558,37 @@ hipError_t qc_launch(hipStream_t st, const qc_params& p, uint32_t wgs, uint32_t 
     return hipGetLastError();
 }
 
+// Workgroups of a launch over n rows of nb blocks: `window` = the hand-issued one; `tune` as qw_col_gemv's.
+uint32_t qc_grid(uint32_t n, uint32_t nb, uint32_t sets, uint32_t waves, bool window, uint32_t tune) {
+    // Waves per compute unit, measured on N = 17408, K = 5120.  Compiled window: 10 (11.2-11.3 us; 11.5 with 20, 13.5+ with
+    // 5).  Hand-issued window: 20 (10.8-10.9 us on 1024 workgroups; 11.4 on 512 with the same window, 11.1 on 768; deeper
+    // windows 11.1-11.9, a window of two 11.3).  At most 128 row slots per workgroup.
+    uint32_t wgs = (256u * (window ? 20u : 10u) + waves / 2u) / waves;
+    // whole multiples of the 256 compute units: a grid that leaves some of them a workgroup more than the others was up to
+    // 19 % slower (5120 x 17408: 569 workgroups 13.6 us, 512 workgroups 11.2 us; K = 6144 .. 18432 5-10 %)
+    if (!(tune & 0x40u)) wgs = max(256u, (wgs + 128u) / 256u * 256u);   // tune bit 6 (tests): the unrounded grid
+    if ((tune >> 3 & 3u) == 1u) wgs /= 2u;
+    if ((tune >> 3 & 3u) == 2u) wgs *= 2u;
+    if ((tune >> 3 & 3u) == 3u) wgs += wgs / 2u;
+    // Banks under 20 MB are latency: one or two workgroups on every compute unit, down to two rows a set and on the smallest to one,
+    // rather than four rows a set on half of the units (us, before -> now: 3072 x 2048 3.23 -> 2.92, 2048 x 2048 3.22 -> 2.98, 2048 x 6144 5.10 ->
+    // 4.74, 4096 x 2560 4.60 -> 4.07, 2560 x 8192 5.65 -> 5.10, 6144 x 4096 5.31 -> 4.95, 1024 x 3072 3.72 -> 3.02, 5120 x 5120 level).
+    // Larger ones: at least two rows a set, whole multiples of the units (7168 x 5120: 896 workgroups 6.51 us, 1024 6.40)
+    if (window && !(tune & 0x40u) && (tune >> 3 & 3u) == 0u && (uint64_t)n * nb * 20u < 20000000u) {
+        // past six rows a set four of them are the better ones again (16384 x 1024: 512 workgroups 5.15 us, 1024 4.77; 12288 x 2048:
+        // 512 5.08, 768 5.29)
+        if (n > sets * 3072u) wgs = min(wgs, n / (sets * 4u));
+        else wgs = n >= sets * 1024u ? 512u : min(256u, max(1u, n / sets));
+        wgs = max(wgs, qwhip_cdiv(n, 128u));
+    } else {
+        wgs = min(wgs, max(1u, n / (sets * (window ? 2u : 4u))));
+        wgs = max(wgs, qwhip_cdiv(n, 128u));
+        if (!(tune & 0x40u) && wgs > 256u && wgs % 256u != 0u && (wgs + 255u) / 256u * 256u <= max(1u, n / (sets * 4u)))
+            wgs = (wgs + 255u) / 256u * 256u;                      // the row-slot limit raised the grid: up to the next whole multiple
+    }
+    return wgs;
+}
+
 }  // namespace
 
 // Tries the column-stationary kernel for a validated m = 1 HQ4_G32_M5 call; false when the shape is outside its envelope.
@@ -582,32 +613,7 @@ bool qw_col_gemv(hipStream_t st, const qwhip_weight_view* w, const void* x, uint
     const uint32_t kind = keys ? 1u : (tune & 7u);
     static const uint32_t kWindow[6] = {3u, 0u, 2u, 3u, 4u, 6u};
     const uint32_t wdepth = kWindow[kind <= 5u ? kind : 0u];       // 0: the compiled window
-    // Waves per compute unit, measured on N = 17408, K = 5120.  Compiled window: 10 (11.2-11.3 us; 11.5 with 20, 13.5+ with
-    // 5).  Hand-issued window: 20 (10.8-10.9 us on 1024 workgroups; 11.4 on 512 with the same window, 11.1 on 768; deeper
-    // windows 11.1-11.9, a window of two 11.3).  At most 128 row slots per workgroup.
-    uint32_t wgs = (256u * (wdepth ? 20u : 10u) + waves / 2u) / waves;
-    // whole multiples of the 256 compute units: a grid that leaves some of them a workgroup more than the others was up to
-    // 19 % slower (5120 x 17408: 569 workgroups 13.6 us, 512 workgroups 11.2 us; K = 6144 .. 18432 5-10 %)
-    if (!(tune & 0x40u)) wgs = max(256u, (wgs + 128u) / 256u * 256u);   // tune bit 6 (tests): the unrounded grid
-    if ((tune >> 3 & 3u) == 1u) wgs /= 2u;
-    if ((tune >> 3 & 3u) == 2u) wgs *= 2u;
-    if ((tune >> 3 & 3u) == 3u) wgs += wgs / 2u;
-    // Banks under 20 MB are latency: one or two workgroups on every compute unit, down to two rows a set and on the smallest to one,
-    // rather than four rows a set on half of the units (us, before -> now: 3072 x 2048 3.23 -> 2.92, 2048 x 2048 3.22 -> 2.98, 2048 x 6144 5.10 ->
-    // 4.74, 4096 x 2560 4.60 -> 4.07, 2560 x 8192 5.65 -> 5.10, 6144 x 4096 5.31 -> 4.95, 1024 x 3072 3.72 -> 3.02, 5120 x 5120 level).
-    // Larger ones: at least two rows a set, whole multiples of the units (7168 x 5120: 896 workgroups 6.51 us, 1024 6.40)
-    if (wdepth && !(tune & 0x40u) && (tune >> 3 & 3u) == 0u && (uint64_t)w->n * nb * 20u < 20000000u) {
-        // past six rows a set four of them are the better ones again (16384 x 1024: 512 workgroups 5.15 us, 1024 4.77; 12288 x 2048:
-        // 512 5.08, 768 5.29)
-        if (w->n > sets * 3072u) wgs = min(wgs, w->n / (sets * 4u));
-        else wgs = w->n >= sets * 1024u ? 512u : min(256u, max(1u, w->n / sets));
-        wgs = max(wgs, qwhip_cdiv(w->n, 128u));
-    } else {
-        wgs = min(wgs, max(1u, w->n / (sets * (wdepth ? 2u : 4u))));
-        wgs = max(wgs, qwhip_cdiv(w->n, 128u));
-        if (!(tune & 0x40u) && wgs > 256u && wgs % 256u != 0u && (wgs + 255u) / 256u * 256u <= max(1u, w->n / (sets * 4u)))
-            wgs = (wgs + 255u) / 256u * 256u;                      // the row-slot limit raised the grid: up to the next whole multiple
-    }
+    const uint32_t wgs = qc_grid(w->n, nb, sets, waves, wdepth != 0u, tune);
     const uint32_t rows_per_wg = qwhip_cdiv(w->n, wgs);
     // partial sums: one float per (row slot, chunk); the hand-issued window rounds the trip count up to whole groups and
     // stores every row slot of every group
@@ -703,9 +709,7 @@ extern "C" qwhip_status qwhip_plane_checksum_rows(qwhip_stream_t s, const void* 
         return qwhip_fail(QWHIP_E_BAD_SHAPE, "row checksum takes rows of whole 20-byte pieces, at most 1024 of them, under 4 GiB in all; got %u rows of %u bytes", rows, row_bytes);
     const uint32_t sets = cpr <= 3u ? 4u : (cpr <= 12u ? 2u : 1u);
     const uint32_t threads = 32u * cpr * sets, waves = (threads + 63u) / 64u;
-    uint32_t wgs = (256u * 20u + waves / 2u) / waves;      // the decode GEMV's grid
-    wgs = min(wgs, max(1u, rows / (sets * 4u)));
-    wgs = max(wgs, qwhip_cdiv(rows, 128u));
+    const uint32_t wgs = qc_grid(rows, nb, sets, waves, true, 0u);
     qcs_params p;
     p.bank = (const uint8_t*)plane;
     p.sum = (unsigned long long*)sum;
