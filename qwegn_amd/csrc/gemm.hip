@@ -344,12 +344,8 @@ __global__ __launch_bounds__(WVM* WVN * 64) void qw_gemm2_kernel(const qw_gemm_p
     // compiler wait on the load right where it is issued).
     for (uint32_t kt = 0; kt + 1 < nk; ++kt) {
         const uint32_t cur = kt & 1u, nxt = cur ^ 1u;
-#ifndef QW_PROBE_SKIP_ADMA
         dma_a(kt + 1, nxt);
-#endif
-#ifndef QW_PROBE_SKIP_BLOAD
         load_b(kt + 1);
-#endif
         __builtin_amdgcn_sched_barrier(0);             // keep the loads at the top: their latency hides behind the MFMAs
         mfma_step(lds2 + cur * STAGE);
         store_b(nxt);
@@ -1500,9 +1496,9 @@ extern "C" qwhip_status qwhip_gemm(qwhip_stream_t s, const qwhip_weight_view* w,
     p.ldy = ldy;
     p.y = y;
     p.force_gemm2 = ov == 14u ? 1u : 0u;
-    // Split-K: a problem of few tiles is one tile's K loop long (80 K-steps of ~1.1 us on K = 5120, whatever M).  When the
-    // workspace also holds fp32 partial planes (after the activation copy, if there is one), the K-steps of a tile are dealt
-    // over 2..8 workgroups and a second launch sums the planes in range order.
+    // K ranges: a problem of few tiles is one tile's K loop long (80 K-steps of ~1.1 us on K = 5120, whatever M).  When the workspace
+    // also holds fp32 partial planes (after the activation copy, if there is one), the K-steps of a tile are dealt over several
+    // workgroups (choose_splits, choose_direct) and a second launch sums the planes in range order.
     const bool copy_needed = rotate || (x_dtype == QWHIP_BF16 && (flags & (1u << 16)));   // bf16 rows in the basis are read in place
     const uint64_t sk_used = copy_needed ? ((ws_need + 255u) & ~(uint64_t)255u) : 0u;
     const bool planes_ok = workspace && ((uintptr_t)workspace & 15u) == 0 && (!copy_needed || ws_ok);

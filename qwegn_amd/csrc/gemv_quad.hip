@@ -213,7 +213,8 @@ static __device__ __forceinline__ void run(const qq_params& p) {
                 }
                 // The header of this lane's row: the scale (times 2^24, exactly: the codes are f16 subnormals code * 2^-24) goes to the
                 // block by quad broadcast, the bias stays where it is as the one operand of a K = 1 product with the slices' sums
-                // (HQ4_G32_M5: w = (1024 + q) s + b; 1024 s + b is exact in fp32, so the large terms meet unrounded)
+                // (HQ4_G32_M5: w = (1024 + q) s + b; 1024 s + b is exact in fp32 while the two lie within 12 binades, as
+                // the quantizer's do, whose b is about -1032 s, and one rounding otherwise: the large terms meet before they are multiplied)
                 const h2_t hd = __builtin_bit_cast(h2_t, blk.hdr);
                 const float s24 = (float)hd[0] * 16777216.0f;
                 const float bias = FMT == QW_FMT_M5 ? __builtin_fmaf(1024.0f, (float)hd[0], (float)hd[1]) : (float)hd[1];
