@@ -1,39 +1,10 @@
 // Host side of the grouped (MoE) GEMM on direct weight operands (qw_direct.h).
 #include <algorithm>
 
-#include "qw_direct.h"
+#include "qw_direct_launch.h"
 
 namespace {
 
-template <int FMT, int YDT, bool SWIGLU, bool GACT, int XDT, int MAXF>
-hipError_t launch6(hipStream_t st, const qw_gemm_params& p, uint32_t max_tiles) {
-    constexpr size_t lds = 2u * MAXF * 4096u + 256u * qd_pitch<FMT>();
-    auto kern = qw_gemm6_kernel<FMT, YDT, SWIGLU, GACT, XDT, MAXF>;
-    static std::atomic<bool> attr_done{false};
-    if (!attr_done.load(std::memory_order_acquire)) {
-        const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
-        if (e != hipSuccess) return e;
-        attr_done.store(true, std::memory_order_release);
-    }
-    const dim3 grid(8u * qwhip_cdiv(max_tiles, 8u) * p.tiles_n);   // XCD-aware one-dimensional grid over (tile, column tile)
-    hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, p);
-    return hipGetLastError();
-}
-template <int FMT, int YDT, bool SWIGLU, bool GACT, int XDT>
-hipError_t launch_rows(hipStream_t st, const qw_gemm_params& p, uint32_t max_tiles, bool few) {
-    if (few) return launch6<FMT, YDT, SWIGLU, GACT, XDT, 2>(st, p, max_tiles);
-    return launch6<FMT, YDT, SWIGLU, GACT, XDT, qd_span<FMT>()>(st, p, max_tiles);
-}
-template <int FMT, int XDT>
-hipError_t launch_out(hipStream_t st, const qw_gemm_params& p, uint32_t max_tiles, uint32_t ydt, bool swiglu, bool few) {
-    if (swiglu) {
-        if (p.act.kind) return launch_rows<FMT, QWHIP_F16, true, true, XDT>(st, p, max_tiles, few);
-        return launch_rows<FMT, QWHIP_F16, true, false, XDT>(st, p, max_tiles, few);
-    }
-    if (ydt == QWHIP_F16) return launch_rows<FMT, QWHIP_F16, false, false, XDT>(st, p, max_tiles, few);
-    if (ydt == QWHIP_BF16) return launch_rows<FMT, QWHIP_BF16, false, false, XDT>(st, p, max_tiles, few);
-    return launch_rows<FMT, QWHIP_F32, false, false, XDT>(st, p, max_tiles, few);
-}
 // workgroups of tall spans a unit, from the mean of rows an expert (half a span of remainder where they are more than one's)
 double tall_load(int fmt, const qw_gemm_params& p, uint32_t experts) {
     const double used = std::min(experts, p.M), span = fmt == QG_FMT_B8 || fmt == QG_FMT_B6 ? 96.0 : 128.0;
@@ -54,10 +25,8 @@ bool few_rows(const qw_gemm_params& p, uint32_t experts) {
     return load < 3.0 || p.K <= (FMT == QG_FMT_M5 ? 2048u : 512u);
 }
 template <int FMT>
-hipError_t launch_x(hipStream_t st, const qw_gemm_params& p, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt, bool swiglu) {
-    const bool few = few_rows<FMT>(p, experts);
-    if (xdt == QWHIP_F16) return launch_out<FMT, QWHIP_F16>(st, p, max_tiles, ydt, swiglu, few);
-    return launch_out<FMT, QWHIP_BF16>(st, p, max_tiles, ydt, swiglu, few);
+hipError_t launch(hipStream_t st, const qw_gemm_params& p, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt, bool swiglu) {
+    return qd_launch_x<FMT, false>(st, p, max_tiles, xdt, ydt, swiglu, few_rows<FMT>(p, experts));
 }
 
 }  // namespace
@@ -72,11 +41,11 @@ bool qw_grouped_direct_takes(int fmt, const qw_gemm_params& p, uint32_t experts)
 hipError_t qw_grouped_direct(hipStream_t st, int fmt, const qw_gemm_params& p, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt,
                              bool swiglu) {
     switch (fmt) {
-        case QG_FMT_M5: return launch_x<QG_FMT_M5>(st, p, max_tiles, experts, xdt, ydt, swiglu);
-        case QG_FMT_B4: return launch_x<QG_FMT_B4>(st, p, max_tiles, experts, xdt, ydt, swiglu);
-        case QG_FMT_B8: return launch_x<QG_FMT_B8>(st, p, max_tiles, experts, xdt, ydt, swiglu);
-        case QG_FMT_B2: return launch_x<QG_FMT_B2>(st, p, max_tiles, experts, xdt, ydt, swiglu);
-        case QG_FMT_B3: return launch_x<QG_FMT_B3>(st, p, max_tiles, experts, xdt, ydt, swiglu);
-        default: return launch_x<QG_FMT_B6>(st, p, max_tiles, experts, xdt, ydt, swiglu);
+        case QG_FMT_M5: return launch<QG_FMT_M5>(st, p, max_tiles, experts, xdt, ydt, swiglu);
+        case QG_FMT_B4: return launch<QG_FMT_B4>(st, p, max_tiles, experts, xdt, ydt, swiglu);
+        case QG_FMT_B8: return launch<QG_FMT_B8>(st, p, max_tiles, experts, xdt, ydt, swiglu);
+        case QG_FMT_B2: return launch<QG_FMT_B2>(st, p, max_tiles, experts, xdt, ydt, swiglu);
+        case QG_FMT_B3: return launch<QG_FMT_B3>(st, p, max_tiles, experts, xdt, ydt, swiglu);
+        default: return launch<QG_FMT_B6>(st, p, max_tiles, experts, xdt, ydt, swiglu);
     }
 }
