@@ -15,14 +15,14 @@ double tall_load(int fmt, const qw_gemm_params& p, uint32_t experts) {
 // taller, fewer ones leave units idle (16 experts, 128 rows each: down of 1536 x 1536 20.4 us / 33.8, gate|up of 3072 x 1536 67 / 94); past
 // that 4-bit and narrower containers 0.96 .. 0.99 up to three and 1.03 .. 1.08 past, 6- and 8-bit ones 1.03 .. 1.13; on short K, whose starts
 // and ends weigh more, 0.85 .. 1.0 (64 experts, 128 rows each, 2048 x 512: 37.7 / 41.6).  HQ4_G32_M5's short unpack has nothing to
-// amortise on K up to 2048 (0.78 .. 1.01).  Up to 48 rows an expert both are the same spans and the three waves win (0.92 .. 1.0), but for
+// amortise on K up to 1536 (0.83 .. 1.0; past three workgroups a unit 0.99 .. 1.04 up to K = 2048, 1.05 past).  Up to 48 rows an expert both are the same spans and the three waves win (0.92 .. 1.0), but for
 // three to four workgroups a unit, two rounds of either (1.04 .. 1.08).
 template <int FMT>
 bool few_rows(const qw_gemm_params& p, uint32_t experts) {
     const double rows = p.M / (double)std::min(experts, p.M), load = tall_load(FMT, p, experts);
     if (FMT == QG_FMT_B8 || FMT == QG_FMT_B6) return rows <= 48.0 || load < (p.K <= 512u ? 3.0 : 1.5);
     if (rows <= 48.0) return !(load > 3.0 && load <= 4.0);
-    return load < 3.0 || p.K <= (FMT == QG_FMT_M5 ? 2048u : 512u);
+    return load < 3.0 || p.K <= (FMT == QG_FMT_M5 ? 1536u : 512u);
 }
 template <int FMT>
 hipError_t launch(hipStream_t st, const qw_gemm_params& p, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt, bool swiglu) {

@@ -359,7 +359,7 @@ _SPANS_FEW = [1, 16, 17, 0, 32, 33, 63, 64, 65, 2]                  # at most 48
 _SPANS_MANY = [31, 64, 96, 97, 0, 128, 129, 160, 161, 225, 300]     # spans of 128 (96 on the 6- and 8-bit containers) on wide enough banks
 
 
-_SPANS_M5 = [3000, 2725]                                            # HQ4_G32_M5 takes them on K past 2048 only
+_SPANS_M5 = [3000, 2725]                                            # HQ4_G32_M5 takes them on K past 1536 only
 
 
 @pytest.mark.parametrize("fmt,counts,k,inter,xdt,compact", [
