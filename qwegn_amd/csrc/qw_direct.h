@@ -1,5 +1,5 @@
 // GEMM with the weights dequantized straight into the matrix cores' operand registers (K in whole pairs of 64, groups of at most
-// 128): grouped (MoE; gemm.hip has the form for the rest), and dense for a few rows to about a thousand.
+// 128): grouped (MoE; gemm.hip has the form for the rest), and dense where choose_direct in gemm.hip prices it below the tiles.
 //
 // A workgroup of four waves owns 256 weight rows of one expert and up to 32 * MAXF of its sorted rows; wave w owns tile columns
 // [64 w, 64 w + 64) for all of them: NF x 2 fragments of v_mfma_f32_32x32x16_f16, NF = 1 .. MAXF (a switch in front of the K loop:
@@ -14,10 +14,11 @@
 //  - Activations: a 64-column stage per K-step through registers into LDS, XOR-swizzled, one barrier per K-step.
 //  - Everything a sub-step needs is asked for one sub-step ahead: fragment a of the next one as soon as the two products that
 //    read it are issued, the next weight chunk between this one's products.
-// Bound, 2048 rows x top-8 of 128 experts of 2048 x 768: gate|up 157 us (HQ4_G32_M5; 7.7 vector instructions a matrix product, whose
-// issue takes 13 + 4 * 7.7 of 32 cycles: the products wait for the unpack); at 32 rows an expert and fewer the bank's
-// stream, 252 MB in 72 us.  Layers against the 64-row form: HQ4_G32_M5 2048 / 256 / 16 rows 316 -> 304, 157 -> 144, 120 -> 106 us;
-// 1500 rows, top-6 of 64 experts: 4-bit affine g64 230 -> 186, 8-bit 330 -> 236, 6-bit 302 -> 226 us.
+// Bound, 2048 rows x top-8 of 128 experts of 2048 x 768: gate|up 153 .. 162 us by the card (HQ4_G32_M5; 6.1 vector instructions beside a
+// matrix product on spans of 128, 8.8 on 64; the matrix pipe is busy 38 % of the cycles on either: at two and three waves a SIMD the
+// products wait for the unpack and its operands); at 32 rows an expert and fewer the bank's stream, 252 MB in 72 us.  Layers against the
+// 64-row kernel before, one box: HQ4_G32_M5 2048 / 256 / 16 rows 286 -> 274, 134 -> 125, 100 -> 87 us; 1500 rows, top-6 of 64 experts:
+// 4-bit affine g64 230 -> 186, 8-bit 330 -> 236, 6-bit 302 -> 226 us.
 #pragma once
 #include <atomic>
 
