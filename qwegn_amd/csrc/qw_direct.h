@@ -17,7 +17,7 @@
 // Bound, 2048 rows x top-8 of 128 experts of 2048 x 768: gate|up 153 .. 162 us by the card (HQ4_G32_M5; 6.1 vector instructions beside a
 // matrix product on spans of 128, 8.8 on 64; the matrix pipe is busy 38 % of the cycles on either: at two and three waves a SIMD the
 // products wait for the unpack and its operands); at 32 rows an expert and fewer the bank's stream, 252 MB in 72 us.  Layers against the
-// 64-row kernel before, one box: HQ4_G32_M5 2048 / 256 / 16 rows 286 -> 274, 134 -> 125, 100 -> 87 us; 1500 rows, top-6 of 64 experts:
+// 64-row kernel before, in turn: HQ4_G32_M5 2048 / 256 / 16 rows 286 -> 274, 134 -> 125, 100 -> 87 us; 1500 rows, top-6 of 64 experts:
 // 4-bit affine g64 230 -> 186, 8-bit 330 -> 236, 6-bit 302 -> 226 us.
 #pragma once
 #include <atomic>
