@@ -1017,11 +1017,41 @@ bool qw_col_gemv(hipStream_t st, const qwhip_weight_view* w, const void* x, uint
 bool qw_sk_gemv(qwhip_stream_t s, const qwhip_weight_view* w, int fmt, uint32_t gshift, uint32_t bb, uint64_t row_bytes,
                 const void* x, uint32_t x_dtype, uint32_t m, void* y16, float* y32, uint32_t tune, hipError_t* err);
 
+// gemv_rows.hip
+bool qw_rows_gemv(qwhip_stream_t s, const qwhip_weight_view* w, int fmt, uint32_t gshift, uint32_t bb, uint64_t row_bytes, const void* x,
+                  uint32_t x_dtype, uint32_t m, bool f16w, void* y16, float* y32, uint32_t inter, bool rotate_out, uint32_t tune, hipError_t* err);
+
+// Does the row-tile kernel pay?  From 86 banks of each of six containers (K = 1024 .. 17408, N = 1024 .. 32768) at 2 .. 16 rows, its time
+// over that of the kernel that a call took before.  13 rows on 0.62 .. 0.72 in the mean (1.10 at most), 9 to 12 rows 0.63 .. 0.79 (1.13), 8 rows
+// 0.81 .. 0.85.  Below that the 4x4x4-block kernel, whose cost is a third of this one's at four rows, keeps the banks whose launch is
+// neither so short that its one trip through LDS counts nor so long that the memory system sets the time: 5 .. 7 rows on 4096 .. 12288
+// columns of up to 5120 rows (1.0 .. 1.2; 8-bit streams of any height, up to eight rows, 1.0 .. 1.15), 2 .. 4 rows past 2048 columns (1.0 .. 1.5).
+// 2-, 3- and 6-bit streams: the dot2 kernel's work grows with m, from three rows on 0.78 .. 0.86 (0.55 .. 0.63 at six), two rows 1.2, and
+// three and four rows on 1024 bank rows 1.0 .. 1.28.
+static bool qw_rows_pays(int fmt, uint32_t m, uint32_t n, uint32_t k) {
+    if (m < 2u || m > 16u) return false;
+    if (fmt >= QW_FMT_B2) return m >= 5u || (m >= 3u && n >= 2048u);
+    if (m >= 9u) return true;
+    if (fmt == QW_FMT_B8 && m >= 5u) return k <= 3072u || k > 12288u;
+    if (m == 8u) return true;
+    if (m >= 5u) return k <= 3072u || k > 12288u || n > 5120u;
+    if (n > 12288u) return false;
+    return m == 4u ? k <= 2048u : fmt != QW_FMT_B4 && (m == 3u ? k <= 2048u : k <= 1024u);
+}
+// Which weights the kernels before it contracted: the exact f16 ones on the transposing (13 rows on) and the split-K kernel.
+static bool qw_rows_f16_weights(qwhip_stream_t s, const qwhip_weight_view* w, int fmt, uint32_t gshift, uint32_t bb, uint64_t row_bytes, const void* x,
+                                uint32_t x_dtype, uint32_t m) {
+    if (fmt >= QW_FMT_B2) return false;
+    if (m >= 13u) return true;
+    return m >= 6u && w->k >= 8192u && fmt != QW_FMT_B8 &&
+           qw_sk_gemv(s, w, fmt, gshift, bb, row_bytes, x, x_dtype, m, nullptr, nullptr, m > 8u ? 26u : 0u, nullptr);
+}
+
 // flags bits 8..11: kernel override for tuning and tests (0 = automatic, 1 = dot2, 2 = direct-load mfma, 3 = DMA streamer,
 // 4 = column-stationary persistent kernel, 5 = column-stationary MFMA kernel, 6 = column-stationary small-M kernel,
-// 7 = 4x4x4-block MFMA kernel, 8 = transposing MFMA kernel, 9 = split-K MFMA kernel);
+// 7 = 4x4x4-block MFMA kernel, 8 = transposing MFMA kernel, 9 = split-K MFMA kernel, 10 = row-tile kernel);
 // bits 12..15: row tiles per wave for the direct-load mfma kernel / K-split of the streamer / tuning code of the
-// column-stationary kernel (0 = automatic); bits 12..18: tuning code of the split-K kernel.
+// column-stationary kernel (0 = automatic); bits 12..18: tuning code of the split-K and the row-tile kernel.
 // `token` (head door only): where the column-stationary kernel's fused fold leaves the argmax; *folded tells whether it ran
 static qwhip_status qw_gemv_impl(qwhip_stream_t s, const qwhip_weight_view* w, const void* x, uint32_t x_dtype, uint32_t m,
                                  uint32_t flags, void* y16, float* y32, int32_t* token, bool* folded) {
@@ -1103,6 +1133,21 @@ static qwhip_status qw_gemv_impl(qwhip_stream_t s, const qwhip_weight_view* w, c
         if (st != QWHIP_OK) return st;
         return qw_gemv_impl(s, w, xr, QWHIP_F16, m, flags | QWHIP_X_PREROTATED, y16, y32, token, folded);
     }
+    // Row-tile kernel: two to sixteen rows already in the basis, every container.  It contracts the exact f16 weights where the kernels
+    // before it did (13 rows on; six on long rows that the split-K kernel takes), and the codes themselves, scaled in fp32, elsewhere.
+    if (variant == 10 || (variant == 0 && !rotate && qw_rows_pays(fmt, m, w->n, w->k))) {
+        hipError_t e = hipSuccess;
+        const bool f16w = qw_rows_f16_weights(s, w, fmt, a.gshift, a.bb, a.row_bytes, x, x_dtype, m);
+        // (rows too long for the dot2 kernel of the 2-, 3- and 6-bit streams stay refused)
+        const bool known = variant == 10 || fmt < QW_FMT_B2 ||
+                           qw_colx_gemv(s->stream, w, fmt, a.gshift, a.bb, a.row_bytes, x, x_dtype, min(m, 8u), false, y16, y32, rt, nullptr);
+        if (!rotate && m >= 2 && known &&
+            qw_rows_gemv(s, w, fmt, a.gshift, a.bb, a.row_bytes, x, x_dtype, m, f16w, y16, y32, 0, false, (flags >> 12) & 0x7Fu, &e)) {
+            QWHIP_TRY_HIP(e);
+            return QWHIP_OK;
+        }
+        if (variant == 10) return qwhip_fail(QWHIP_E_BAD_GEOMETRY, "the row-tile kernel takes 2..16 rows already in the basis, K ranges within the stream's scratch");
+    }
     // 2-, 3- and 6-bit streams: the column-stationary dot2 kernel is their one decode kernel (eight rows per launch)
     if (fmt >= QW_FMT_B2) {
         if (rotate && m > 1)
@@ -1173,13 +1218,9 @@ static qwhip_status qw_gemv_impl(qwhip_stream_t s, const qwhip_weight_view* w, c
         return QWHIP_OK;
     }
 
-    // split-K matrix-core kernel: activations already in the basis, 2..16 rows.  Its cost is flat in m (two launches, one
-    // dequantization per weight whatever m is), so it takes over where rows are long and few and m is large: N = 5120,
-    // K = 17408, HQ4_G64 measured 18.7 / 18.7 / 20.7 us at m = 6 / 8 / 16 against 21.2 / 23.2 / 34.9 for the kernels below
-    // (16.7 against 18.6 at m = 4); on K = 5120 banks (N = 7168 HQ8, N = 17408 or 5120 HQ4) the kernels below stay ahead.
-    // 13..16 rows on an 8-bit stream of short rows take it too, four waves a workgroup, four groups in flight, the image in
-    // 128 KiB (tuning code 60): two K ranges and the second launch, 15.7 us on N = 7168, K = 5120 against 16.9 for the
-    // transposing kernel and 17.7 for the 4x4x4-block kernel.
+    // split-K matrix-core kernel: what the row-tile kernel leaves (banks of 4 GiB and more, partial sums past the stream's scratch) on
+    // long rows, N = 5120, K = 17408, HQ4_G64: 18.7 / 18.7 / 20.7 us at m = 6 / 8 / 16 against 21.2 / 23.2 / 34.9 for the kernels below, and
+    // 13..16 rows on an 8-bit stream of short rows, four waves a workgroup, four groups in flight, the image in 128 KiB (tuning code 60).
     const bool sk_long = !rotate && m >= 6 && w->k >= 8192 && fmt != QW_FMT_B8;
     const bool sk_wide8 = !rotate && m >= 13 && w->k < 8192 && fmt == QW_FMT_B8;
     if (variant == 9 || (variant == 0 && (sk_long || sk_wide8))) {
@@ -1194,9 +1235,7 @@ static qwhip_status qw_gemv_impl(qwhip_stream_t s, const qwhip_weight_view* w, c
         if (variant == 9)
             return qwhip_fail(QWHIP_E_BAD_GEOMETRY, "the split-K kernel takes 2..16 rows already in the basis, k %% 128 == 0, partial sums within the stream's scratch");
     }
-    // transposing MFMA kernel: activations already in the basis.  Its cost barely grows with m: measured best from 13 rows
-    // on (N = 7168, K = 5120, HQ8: 16.0 / 16.9 us at m = 13 / 16 against 16.6 / 17.9 for the 4x4x4-block kernel and 18.6 for
-    // the column-stationary MFMA kernel; N = 5120, K = 17408, HQ4_G64: level with the 4x4x4-block kernel, 31.5 / 34.6 us).
+    // transposing MFMA kernel: activations already in the basis, from 13 rows on (the row-tile kernel takes these calls first)
     if (variant == 8 || (variant == 0 && !rotate && m >= 13)) {
         hipError_t e = hipSuccess;
         bool done = false;
@@ -1209,9 +1248,8 @@ static qwhip_status qw_gemv_impl(qwhip_stream_t s, const qwhip_weight_view* w, c
         }
         if (variant == 8) return qwhip_fail(QWHIP_E_BAD_GEOMETRY, "the transposing MFMA kernel needs activations in the basis");
     }
-    // 4x4x4-block MFMA kernel: activations already in the basis.  Measured best for 2..12 rows (N = 7168, K = 5120, HQ8:
-    // 11.0 / 11.9 / 13.2 us at m = 2 / 4 / 8, 14.4 / 15.7 at m = 9 / 12 against 15.2 / 16.0 for the transposing kernel;
-    // N = 5120, K = 17408, HQ4_G64: 23.4 us at m = 8, 25.9 / 27.9 at m = 9 / 12 against 28.1 / 31.1).
+    // 4x4x4-block MFMA kernel: activations already in the basis, 2 to 12 rows where the row-tile kernel does not pay (N = 7168, K = 5120,
+    // HQ8: 11.0 / 11.9 us at m = 2 / 4)
     if (variant == 7 || (variant == 0 && !rotate && m >= 2 && m <= 12)) {
         hipError_t e = hipSuccess;
         if (!rotate && qw_quad_gemv(s->stream, w, fmt, a.gshift, a.bb, a.row_bytes, x, x_dtype, m, y16, y32, rt, &e)) {
@@ -1286,6 +1324,17 @@ extern "C" qwhip_status qwhip_gemv_silu_pair(qwhip_stream_t s, const qwhip_weigh
     // partial-sum area, then the gated activation (+ rotation) pass over it - every weight is read once whatever m is (the MoE
     // decode kernel reads the bank once per row: 40 / 70 / 125 us at m = 2 / 4 / 8 on 2 x 17408 x 5120).
     if (m >= 2u && m <= 16u && ((flags >> 8) & 0xFu) == 0u && s->scratch && (!rot_out || ((uintptr_t)act16 & 15u) == 0)) {
+        // f16 rows in the basis: the row-tile kernel on the gate and up rows of a channel block, the gated activation where it sums them
+        if (!rotate && !(flags & QWHIP_GEMV_ROW_INVARIANT) && x_dtype == QWHIP_F16) {
+            hipError_t e = hipSuccess;
+            const uint32_t gshift = log2_u32(w->group / 32), bb = qwhip_view_block_bytes(w);
+            const uint64_t row_bytes = qwhip_view_row_bytes(w);
+            const bool f16w = qw_rows_f16_weights(s, w, fmt, gshift, bb, row_bytes, x, x_dtype, m);
+            if (qw_rows_gemv(s, w, fmt, gshift, bb, row_bytes, x, x_dtype, m, f16w, act16, nullptr, inter, rot_out, 0, &e)) {
+                QWHIP_TRY_HIP(e);
+                return QWHIP_OK;
+            }
+        }
         const size_t need = (((size_t)m * w->n * 4u) + 255u) & ~(size_t)255u;
         const size_t area = s->scratch_bytes - QWHIP_STREAM_COUNTER_BYTES - QWHIP_STREAM_XROT_BYTES;
         if (need <= area / 2u) {

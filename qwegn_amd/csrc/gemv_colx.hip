@@ -346,6 +346,7 @@ bool qw_colx_gemv(hipStream_t st, const qwhip_weight_view* w, int fmt, uint32_t 
     if (rotate && (threads >> 6) * 5u * 16u < nsl) return false;   // rotation tiles: five per full wave
     const size_t lds = (size_t)rows_per_wg * cpr * mr * 4u + (rotate ? (size_t)nsl * 80u : 0u);
     if (lds > 60u * 1024u) return false;
+    if (!err) return true;   // the caller only asks
     qcx_params p;
     p.bank = (const uint8_t*)w->blocks;
     p.x = x;

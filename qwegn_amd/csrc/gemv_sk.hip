@@ -278,6 +278,11 @@ hipError_t qsk_launch(hipStream_t st, const qsk_params& p, uint32_t wgs, uint32_
 
 }  // namespace
 
+hipError_t qw_sk_sum(hipStream_t st, const float* part, void* y16, float* y32, uint32_t n, uint32_t m, uint32_t n16, uint32_t nkr) {
+    hipLaunchKernelGGL(qw_gemv_sk_reduce_kernel, dim3(qwhip_cdiv(m * (n16 / 4u), 256u)), dim3(256), 0, st, part, (h1_t*)y16, y32, n, m, n16, nkr);
+    return hipGetLastError();
+}
+
 // Tries the split-K matrix-core kernel for a validated call with m = 2..16 rows already in the container's basis; false when
 // the shape is outside its envelope (rows that are not whole groups of four slices, partial sums that do not fit the stream's
 // scratch).  fmt: QW_FMT_M5 / QW_FMT_B4 / QW_FMT_B8 (the same codes as the GEMM's).
@@ -317,6 +322,7 @@ bool qw_sk_gemv(qwhip_stream_t s, const qwhip_weight_view* w, int fmt, uint32_t 
     const uint64_t part_bytes = nkr > 1u ? (uint64_t)nkr * m * ntiles * 16u * 4u : 0u;
     if (nkr > 1u && (!s->scratch || part_bytes + s->scratch_reserved > s->scratch_bytes - QWHIP_STREAM_COUNTER_BYTES - QWHIP_STREAM_XROT_BYTES))
         return false;
+    if (!err) return true;   // the caller only asks
     qsk_params p;
     p.bank = (const uint8_t*)w->blocks;
     p.x = x;
@@ -345,12 +351,7 @@ bool qw_sk_gemv(qwhip_stream_t s, const qwhip_weight_view* w, int fmt, uint32_t 
     else if (fmt == QW_FMT_B4) { QSK_FMT(QG_FMT_B4) }
     else { QSK_FMT(QG_FMT_B8) }
 #undef QSK_FMT
-    if (e == hipSuccess && nkr > 1u) {
-        const uint32_t quads = m * ntiles * 4u;
-        hipLaunchKernelGGL(qw_gemv_sk_reduce_kernel, dim3(qwhip_cdiv(quads, 256u)), dim3(256), 0, s->stream, p.part, p.y16, p.y32, p.N, m,
-                           ntiles * 16u, nkr);
-        e = hipGetLastError();
-    }
+    if (e == hipSuccess && nkr > 1u) e = qw_sk_sum(s->stream, p.part, p.y16, p.y32, p.N, m, ntiles * 16u, nkr);
     *err = e;
     return true;
 }

@@ -265,6 +265,89 @@ def test_gemv_split_k_mfma_kernel_refusals_and_stream_order(dev):
         g16, g32, ref = _run_gemv(dev, "hq4_g32_m5", n, k, m, prerot=True, seed=n, variant=0)     # automatic: k >= 8192, m >= 6
         assert qo.normalized_error(g32, ref) <= 2e-5
 
+_ROWS_FORMATS = ["hq4_g32_m5", "aq4_g32", "hq4_g128", "hq8_g32", "aq8_g256", "aq2_g64", "hq3_g32", "aq6_g128"]
+
+
+@pytest.mark.parametrize("fmt", _ROWS_FORMATS)
+@pytest.mark.parametrize("n,k,m,xdtype", [
+    (270, 1536, 2, "f16"),       # one step a wave, a partial row tile
+    (5, 256, 7, "bf16"),         # a bank smaller than a tile, two waves
+    (37, 1792, 16, "f16"),       # every activation row there
+    (1000, 2304, 12, "bf16"),    # two steps a wave, the last wave half empty
+    (16 * 300 + 3, 512, 13, "f16"),   # several tiles a workgroup, the last sum short
+    (300, 4352, 5, "f16"),       # four steps a wave
+    (96, 6400, 9, "f16"),        # two K ranges, partial sums through the stream's scratch
+    (50, 17408, 3, "bf16"),      # three K ranges
+])
+def test_gemv_row_tile_kernel(dev, fmt, n, k, m, xdtype):
+    """Row-tile kernel (override 10): tight against what it computes - the codes' own weights up to 12 rows, the exact f16 weights on
+    13 and more (4- and 8-bit banks) and on six and more long 4-bit rows.  fp32 sums: K products of two exact f16, one rounding a
+    slice and product of 32; 2e-6 is about three times the largest error measured against 64 bits (7.5e-7)."""
+    g16, g32, ref = _run_gemv(dev, fmt, n, k, m, prerot=True, xdtype=xdtype, seed=5, variant=10)
+    four = fmt in ("hq4_g32_m5", "aq4_g32", "hq4_g128")
+    exact_f16 = (four or "8_" in fmt) and (m >= 13 or (four and m >= 6 and k >= 8192))
+    assert qo.normalized_error(g32, ref if exact_f16 else _affine_ref(fmt, n, k, m, 5, xdtype)) <= 2e-6
+    assert qo.normalized_error(g32, ref) <= TOL
+    assert qo.normalized_error(g16, ref) <= TOL
+
+
+@pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq8_g64", "hq3_g32", "aq6_g128"])
+@pytest.mark.parametrize("m", [5, 16])
+def test_gemv_row_tile_kernel_keeps_an_infinity_in_its_row(dev, fmt, m):
+    """The m activation rows share the instructions: a row that is not finite leaves the others' bits alone."""
+    n, k = 48, 1536
+    blocks, _ = H.make_bank(fmt, n, k, 3)
+    x16 = H.make_x(m, k, 4).astype(np.float16)
+    bad = x16.copy()
+    bad[2, 700] = np.inf
+    bank, outs = dev.put(blocks), []
+    view = H.view_of(dev, bank, fmt, n, k)
+    for x in (x16, bad):
+        xb, y = dev.put(x), dev.alloc(m * n * 4)
+        qwhip.check(dev.lib.qwhip_gemv(dev.stream.handle, C.byref(view), xb.ptr, qwhip.F16, m, qwhip.X_PREROTATED | (10 << 8), None, y.ptr))
+        dev.stream.sync()
+        outs.append(y.download(np.float32, (m, n)))
+        xb.free()
+        y.free()
+    bank.free()
+    rest = [i for i in range(m) if i != 2]
+    assert np.array_equal(outs[0][rest].view(np.uint32), outs[1][rest].view(np.uint32))
+    assert not np.isfinite(outs[1][2]).any()
+
+
+def test_gemv_row_tile_kernel_refuses_what_was_refused(dev):
+    """Rows in the basis only, two to sixteen; 2-, 3- and 6-bit rows too long for the dot2 kernel are refused by the automatic choice."""
+    lib, st = dev.lib, dev.stream.handle
+    blocks, _ = H.make_bank("hq6_g32", 32, 17408, 0)
+    bank, xb, y = dev.put(blocks), dev.put(np.zeros((7, 17408), np.float16)), dev.alloc(7 * 32 * 4)
+    v = H.view_of(dev, bank, "hq6_g32", 32, 17408)
+    assert lib.qwhip_gemv(st, C.byref(v), xb.ptr, qwhip.F16, 7, qwhip.X_PREROTATED, None, y.ptr) == qwhip.E_BAD_GEOMETRY
+    assert lib.qwhip_gemv(st, C.byref(v), xb.ptr, qwhip.F16, 7, 10 << 8, None, y.ptr) == qwhip.E_BAD_GEOMETRY
+    assert lib.qwhip_gemv(st, C.byref(v), xb.ptr, qwhip.F16, 1, qwhip.X_PREROTATED | (10 << 8), None, y.ptr) == qwhip.E_BAD_GEOMETRY
+    for b in (bank, xb, y):
+        b.free()
+
+
+@pytest.mark.parametrize("fmt", _ROWS_FORMATS)
+@pytest.mark.parametrize("inter,k,m,rot_out", [(32, 512, 2, 1), (160, 1536, 6, 1), (176, 2560, 13, 0), (48, 5120, 16, 0), (4128, 1024, 3, 1)])
+def test_gemv_silu_pair_row_tiles(dev, fmt, inter, k, m, rot_out):
+    """The gated form (16 or, rotated, 32 channels a unit; 4128 channels leave workgroups a second one): bit for bit the plain row-tile
+    GEMV, the gated activation and the rotation one after the other, whose sums and roundings are the same."""
+    blocks, _ = H.make_bank(fmt, 2 * inter, k, seed=inter)
+    x16 = H.make_x(m, k, 9).astype(np.float16)
+    xb, bank = dev.put(x16), dev.put(blocks)
+    a1, a2, gu = dev.alloc(m * inter * 2), dev.alloc(m * inter * 2), dev.alloc(m * 2 * inter * 4)
+    view = H.view_of(dev, bank, fmt, 2 * inter, k)
+    st, fl = dev.stream.handle, qwhip.X_PREROTATED
+    qwhip.check(dev.lib.qwhip_gemv_silu_pair(st, C.byref(view), xb.ptr, qwhip.F16, m, fl, rot_out, a1.ptr))
+    qwhip.check(dev.lib.qwhip_gemv(st, C.byref(view), xb.ptr, qwhip.F16, m, fl | (10 << 8), None, gu.ptr))
+    qwhip.check(dev.lib.qwhip_swiglu_fwht(st, gu.ptr, qwhip.F32, a2.ptr, m, inter, rot_out))
+    dev.stream.sync()
+    one, two = a1.download(np.uint16, (m, inter)), a2.download(np.uint16, (m, inter))
+    for b in (bank, xb, a1, a2, gu):
+        b.free()
+    assert np.array_equal(one, two)
+
 
 @pytest.mark.parametrize("fmt", ["aq2_g64", "hq3_g32", "hq6_g32", "aq6_g128"])
 @pytest.mark.parametrize("m", [1, 3, 8, 12])
