@@ -12,8 +12,8 @@
 // masks of qw_colx_slice.h).
 // Bound by the latency of one chain (route, expert id, first weight rows), not by bandwidth; all rows of a lane are asked for
 // at once.  Against the general kernels these containers took before (matrix tiles of 16 rows, a route launch in front):
-// 4 rows x top-8 of 256 experts, 4-bit affine, 2048 x 512: route 4.5 + gate|up 17 + down 9.4 us -> 13.8 (routing inside) + 5.5 us,
-// the layer 52 -> 40 us.
+// 4 rows x top-8 of 256 experts, 4-bit affine, 2048 x 512: route 4.5 + gate|up 17 + down 9.4 us -> 11.8 (routing inside; 5.7 at 1 row x 128 experts
+// with the route given, 7.7 with the routing) + 5.5 us.
 #include <type_traits>
 
 #include "qw_colx_slice.h"
@@ -125,15 +125,16 @@ __device__ __forceinline__ float qmc_plain_dot(const qmc_slice<FMT>& b, const h8
 // Epilogue: act[pair, n] = f16(FWHT32(silu(g) * u)) over the 32 outputs of the workgroup (rotation optional).
 // blockDim.x = 32 * cpr * SETS; dynamic LDS = nb * 80 + 64 * cpr * 4 bytes.
 // ------------------------------------------------------------------------------------------------
-// logits, idx_out, wts_out, experts, norm, routed_scale (JN > 0): the routing is done here.  The first wave of every workgroup
+// route: the pairs' experts (JN == 0; NULL: one dense bank) or, JN > 0, the router's logits, which with `experts` come in registers: the
+// chain starts with them.  idx_out, wts_out, norm, routed_scale (JN > 0): the routing is done here.  The first wave of every workgroup
 // routes the pair's token from its router logits (the arithmetic of qw_moe_route_kernel, so the same experts and weights) and
 // the workgroup takes rank pair % top_k; the workgroups of the first row block leave the pair's expert and weight in idx_out /
 // wts_out for the down projection.  x_rows: activation row of every pair (NULL: the pair's token).  ga: the device's gated
 // activation (all zero: SwiGLU).
 #define QMC_GU_FIELDS(X)                                                                                                     \
-    X(const uint8_t*, bank) X(const void*, x) X(h1_t*, act) X(const int32_t*, idx) X(const float*, logits) X(uint32_t, top_k)    \
-    X(uint32_t, nb) X(uint32_t, cpr) X(uint32_t, I) X(uint32_t, rotate) X(uint32_t, rot_out) X(uint64_t, expert_bytes)           \
-    X(const int32_t*, x_rows) X(uint32_t, experts) X(int32_t*, idx_out) X(float*, wts_out) X(uint32_t, norm)                     \
+    X(const uint8_t*, bank) X(const void*, x) X(h1_t*, act) X(const void*, route) X(uint32_t, top_k) X(uint32_t, nb) X(uint32_t, cpr)  \
+    X(uint32_t, I) X(uint32_t, experts) X(uint32_t, rotate) X(uint32_t, rot_out) X(uint64_t, expert_bytes)                       \
+    X(const int32_t*, x_rows) X(int32_t*, idx_out) X(float*, wts_out) X(uint32_t, norm)                                          \
     X(float, routed_scale) X(qw_act, ga) X(uint32_t, gshift) X(uint32_t, bb) X(uint32_t, row_bytes)
 QW_ARG_BLOCK(qmc_gu_params, QMC_GU_FIELDS)
 
@@ -171,7 +172,9 @@ static __device__ __forceinline__ void run(const qmc_gu_params& p) {
 
     // memory order: the route's expert id, the token's activations, the first weight rows; the rotation runs under them
     int32_t e = 0;                               // no route list: one dense gate|up bank
-    if constexpr (JN == 0 && MT == 1) e = p.idx ? p.idx[pair] : 0;
+    const int32_t* const idx = (const int32_t*)p.route;
+    const float* const logits = (const float*)p.route;
+    if constexpr (JN == 0 && MT == 1) e = idx ? idx[pair] : 0;
     const uint32_t token = pair / p.top_k;
     uint32_t xrow = token;
     if constexpr (MT == 1) xrow = (JN == 0 && p.x_rows) ? (uint32_t)max(p.x_rows[pair], 0) : token;
@@ -199,7 +202,7 @@ static __device__ __forceinline__ void run(const qmc_gu_params& p) {
             if (wave < ntok) {   // one wave per token routes it
                 int32_t isel;
                 float wsel;
-                qw_route_wave<JN>(p.logits + (uint64_t)wave * p.experts, p.experts, K, p.norm, p.routed_scale, l64, isel, wsel);
+                qw_route_wave<JN>(logits + (uint64_t)wave * p.experts, p.experts, K, p.norm, p.routed_scale, l64, isel, wsel);
                 if (l64 < K) {
                     tab_e[wave * K + l64] = isel;
                     tab_w[wave * K + l64] = wsel;
@@ -212,7 +215,7 @@ static __device__ __forceinline__ void run(const qmc_gu_params& p) {
                 p.wts_out[pair] = tab_w[pair];
             }
         } else {
-            if (l64 < pairs) my_e = p.idx[l64];
+            if (l64 < pairs) my_e = idx[l64];
         }
         uint32_t my_row = l64 / K;
         if constexpr (JN == 0) {
@@ -250,26 +253,33 @@ static __device__ __forceinline__ void run(const qmc_gu_params& p) {
             }
         }
     }
+    float route_p = 0.0f;
     if constexpr (JN > 0 && MT == 1) {
         __shared__ int32_t e_route;
         if (wave == 0) {   // one wave routes (the others would only compete for the same SIMDs), the workgroup reads its result
             int32_t isel;
-            float wsel;
-            qw_route_wave<JN>(p.logits + (uint64_t)token * p.experts, p.experts, p.top_k, p.norm, p.routed_scale, l64, isel, wsel);
             const uint32_t rank = pair - token * p.top_k;
-            if (l64 == rank) {
-                e_route = isel;
-                if (blockIdx.x == 0) {
-                    p.idx_out[pair] = isel;
-                    p.wts_out[pair] = wsel;
-                }
-            }
+            // the row block that stores the route needs every rank for the weights' sum, the others theirs
+            qw_route_select<JN>(logits + (uint64_t)token * p.experts, p.experts, blockIdx.x == 0 ? p.top_k : rank + 1u, l64, isel, route_p);
+            if (l64 == rank) e_route = isel;
         }
         __syncthreads();
         e = __builtin_amdgcn_readfirstlane(e_route);
     }
+    auto store_route = [&]() __attribute__((always_inline)) {   // nothing in this launch waits for it: behind the first weight rows' loads
+        if constexpr (JN > 0 && MT == 1) {
+            if (blockIdx.x == 0 && wave == 0) {
+                const float w = qw_route_weight(route_p, p.top_k, p.norm, p.routed_scale);
+                if (l64 == pair - token * p.top_k) {
+                    p.idx_out[pair] = e;
+                    p.wts_out[pair] = w;
+                }
+            }
+        }
+    };
     h1_t* act = p.act + (uint64_t)pair * I;
     if (e < 0) {   // no expert: the pair contributes nothing (uniform over the workgroup)
+        store_route();
         if (tid < 32u && n0 + tid < I) act[n0 + tid] = (h1_t)0.0f;
         return;
     }
@@ -283,6 +293,7 @@ static __device__ __forceinline__ void run(const qmc_gu_params& p) {
 #pragma unroll
     for (int j = 0; j < D; ++j) qmc_load<FMT>(bank, row_off(j), hdr_off, pay_off, buf[j]);
     __builtin_amdgcn_sched_barrier(0);
+    store_route();
     {
         h8_t h_lo, h_hi;
         qw_hadamard_pair(l64 & 15u, l64 >> 4, h_lo, h_hi);
@@ -514,7 +525,7 @@ bool qw_moe_gateup_col(hipStream_t st, const qwhip_weight_view* w, int fmt, uint
     p.bank = (const uint8_t*)w->blocks;
     p.x = x;
     p.act = (h1_t*)act16;
-    p.idx = idx;
+    p.route = logits ? (const void*)logits : (const void*)idx;
     p.x_rows = x_rows;
     p.ga = act;
     p.I = inter;
@@ -527,7 +538,6 @@ bool qw_moe_gateup_col(hipStream_t st, const qwhip_weight_view* w, int fmt, uint
     p.gshift = (uint32_t)__builtin_ctz(w->group / 32u);
     p.bb = (uint32_t)qwhip_view_block_bytes(w);
     p.row_bytes = (uint32_t)row_bytes;
-    p.logits = logits;
     p.idx_out = idx_out;
     p.wts_out = wts_out;
     p.experts = experts;

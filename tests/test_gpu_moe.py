@@ -53,6 +53,40 @@ def test_moe_route_ties_and_non_finite(dev):
     np.testing.assert_allclose(wts[0], 0.25, rtol=1e-6)
 
 
+# one to eight experts a lane, the last lanes without one; a single expert; a full last lane
+@pytest.mark.parametrize("e", [1, 63, 64, 65, 128, 129, 256, 257, 511])
+def test_route_edges_of_the_expert_count(dev, e):
+    """Rows of ties, of one candidate, of none, of the lowest finite logits and of infinities: ids and weights as the oracle's; the fused
+    projection, whose later row blocks stop at their own rank, leaves the same ids, weights and activations."""
+    k, hidden, inter = min(e, 8), 256, 96
+    rng = np.random.default_rng(e)
+    logits = rng.standard_normal((8, e)).astype(np.float32)
+    logits[1] = 0.25
+    logits[2, : e - 1] = np.nan
+    logits[3] = -np.inf
+    logits[4] = -np.finfo(np.float32).max
+    logits[4, e // 2] = -3.0e38
+    logits[5, ::2] = np.inf
+    logits[6, e - 1] = np.finfo(np.float32).max
+    logits[7] = np.round(logits[7] * 2)              # ties between some
+    idx, wts = _route(dev, logits, k, scale=1.5)
+    with np.errstate(over="ignore"):
+        ridx, rwts = qo.moe_route(logits, k, True, 1.5)
+    assert np.array_equal(idx, ridx)
+    np.testing.assert_allclose(wts, rwts, rtol=2e-6, atol=1e-9)
+    lib, st = dev.lib, dev.stream.handle
+    blocks, _, _, _ = _moe_banks(e, hidden, inter, seed=3, fmt="hq4_g32")
+    bank, xb, lb = dev.put(blocks), dev.put(rng.standard_normal((8, hidden)).astype(np.float16)), dev.put(logits)
+    view = H.view_of(dev, bank, "hq4_g32", e * 2 * inter, hidden)
+    ib, wb, ab, a2 = dev.alloc(8 * k * 4 + 256), dev.alloc(8 * k * 4 + 256), dev.alloc(8 * k * inter * 2), dev.alloc(8 * k * inter * 2)
+    qwhip.check(lib.qwhip_moe_route_gateup_decode(st, C.byref(view), e, xb.ptr, qwhip.F16, 0, lb.ptr, 8, k, 1, 1.5, ib.ptr, wb.ptr, ab.ptr))
+    qwhip.check(lib.qwhip_moe_gateup_decode(st, C.byref(view), e, xb.ptr, qwhip.F16, 0, ib.ptr, 8, k, a2.ptr))
+    dev.stream.sync()
+    assert np.array_equal(ib.download(np.int32, (8, k)), idx)
+    assert np.array_equal(wb.download(np.uint32, (8, k)), wts.view(np.uint32))
+    assert np.array_equal(ab.download(np.uint16, (8, k, inter)), a2.download(np.uint16, (8, k, inter)))
+
+
 @pytest.mark.parametrize("xdt", ["f32", "bf16", "f16"])
 def test_router_gemm(dev, xdt):
     t, e, h = 19, 128, 2048
