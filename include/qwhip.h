@@ -302,7 +302,7 @@ qwhip_status qwhip_embed_bf16_f32(qwhip_stream_t s, const void* table_bf16, uint
  * A row's bits may depend on m, with and without planes: the kernels among which a call's m, n, k and container decide
  * add the same exact products in different orders (fp32).
  * flags bits 8..15 name a kernel form and its K ranges, for tuning and tests (0 = automatic; bits 8..11 = 1 .. 5 keep one
- * launch of the tiles, 6 .. 8 are refused with QWHIP_E_BAD_SHAPE where the form cannot take the call). */
+ * launch of the tiles, and so does 9 where its form does not take the call; 6 .. 8 are refused with QWHIP_E_BAD_SHAPE there). */
 qwhip_status qwhip_gemm(qwhip_stream_t s, const qwhip_weight_view* w, const void* x, uint32_t x_dtype,
                         uint32_t m, uint32_t ldx, void* y, uint32_t y_dtype, uint32_t ldy, uint32_t flags,
                         void* workspace, uint64_t workspace_bytes);

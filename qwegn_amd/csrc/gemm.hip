@@ -1378,20 +1378,20 @@ double price_tiles(uint32_t m, uint32_t n, uint32_t k, int fmt, uint32_t splits)
 struct gemm_route {
     bool direct, few;    // the direct-operand kernel, its spans of 64 rows
     uint32_t splits;     // K ranges into fp32 planes (two and more), or one launch
+    uint32_t rows;       // steps a wave of the row-tile kernel, which reads the rows as the direct-operand kernel does (0: another kernel)
 };
 inline bool direct_takes(const qwhip_weight_view* w) {
     return w->k % 128u == 0 && w->group <= 128u && 256u * qwhip_view_row_bytes(w) < (1ull << 32);
 }
 gemm_route choose_direct(const qwhip_weight_view* w, uint32_t m, int fmt, uint32_t old_splits, uint64_t plane_room) {
-    gemm_route best = {false, false, old_splits};
+    gemm_route best = {false, false, old_splits, 0u};
     const uint32_t n = w->n, k = w->k;
-    if (!direct_takes(w)) return best;
+    double limit = 0.9 * price_tiles(m, n, k, fmt, old_splits);
     const bool wide = fmt == QG_FMT_B8 || fmt == QG_FMT_B6;
     const double plane = (double)m * n * 4.0;
     const uint32_t pairs = k / 128u, frags = qwhip_cdiv(m, 32u), cols = qwhip_cdiv(n, 256u);
-    double limit = 0.9 * price_tiles(m, n, k, fmt, old_splits);
     const double bank_us = 5.3 + (double)n * (double)qwhip_view_row_bytes(w) / 3.5e6;   // no faster than the bank streams to this kernel
-    for (uint32_t few = 0; few < 2u; ++few) {
+    for (uint32_t few = 0; few < 2u && direct_takes(w); ++few) {
         const uint32_t span = few ? 2u : wide ? 3u : 4u;
         if (!few && frags <= 2u) continue;
         const uint32_t spans = qwhip_cdiv(frags, span);
@@ -1406,25 +1406,35 @@ gemm_route choose_direct(const qwhip_weight_view* w, uint32_t m, int fmt, uint32
             if (splits > 1u) t += 2.0 + 0.24 * splits + splits * plane * 2.0 / 7.0e6;
             if (t < limit) {
                 limit = t;
-                best = {true, few != 0u, splits};
+                best = {true, few != 0u, splits, 0u};
             }
         }
     }
+    // the row-tile kernel (gemm_rows.hip), below 0.92 of the price so far
+    uint32_t steps, ranges;
+    if (qw_gemm_rows_choose(fmt, m, n, k, qwhip_view_row_bytes(w), plane_room, 0u, 0.92 * (best.direct ? limit : limit / 0.9), &steps, &ranges))
+        best = {true, true, ranges, steps};
     return best;
 }
 
 // flags bits 8..11 of the dense doors that name a K-split or direct form, for tuning and tests; bits 12..15: its K ranges (0 = one)
-enum { OV_DIRECT_64 = 6, OV_DIRECT_WIDE = 7, OV_SPLIT_PINGPONG = 8 };
+enum { OV_DIRECT_64 = 6, OV_DIRECT_WIDE = 7, OV_SPLIT_PINGPONG = 8, OV_ROWS = 9 };
 
 // The route of a dense problem: the automatic choice, or the form that the flags name.  Both dense doors call it with the room for
 // planes behind a copy of the rows that both make or neither, so that the fused gate|up gives the bits of the plain door and the
 // activation pass after it whatever the workspace holds (2-byte rows of y that are not 16-byte aligned, y_ok = false, excepted).
 qwhip_status choose_route(const qwhip_weight_view* w, uint32_t m, int fmt, uint32_t flags, bool y_ok, uint64_t plane_room, gemm_route* r) {
     const uint32_t ov = (flags >> 8) & 0xFu, ranges = (flags >> 12) & 0xFu;
-    *r = {false, false, 0u};
+    *r = {false, false, 0u, 0u};
     if (ov == 0u) {
         if (y_ok) *r = choose_direct(w, m, fmt, choose_splits(m, w->n, w->k, plane_room), plane_room);
         return QWHIP_OK;
+    }
+    if (ov == OV_ROWS && y_ok) {
+        uint32_t steps, n_ranges;
+        if (qw_gemm_rows_choose(fmt, m, w->n, w->k, qwhip_view_row_bytes(w), plane_room, ranges ? ranges : 1u, 1e30, &steps, &n_ranges))
+            *r = {true, true, n_ranges, steps};
+        return QWHIP_OK;   // else the tiles in one launch
     }
     if (ov != OV_DIRECT_64 && ov != OV_DIRECT_WIDE && ov != OV_SPLIT_PINGPONG) return QWHIP_OK;
     const bool direct = ov != OV_SPLIT_PINGPONG;
@@ -1434,7 +1444,7 @@ qwhip_status choose_route(const qwhip_weight_view* w, uint32_t m, int fmt, uint3
                                                        (uint64_t)splits * m * w->n * 4u <= plane_room;
     if (!y_ok || (direct && !direct_takes(w)) || !split_ok)
         return qwhip_fail(QWHIP_E_BAD_SHAPE, "the GEMM form %u over %u K ranges that flags %#x name does not take this call", ov, splits, flags);
-    *r = {direct, ov == OV_DIRECT_64, splits};
+    *r = {direct, ov == OV_DIRECT_64, splits, 0u};
     return QWHIP_OK;
 }
 
@@ -1455,6 +1465,7 @@ hipError_t launch_planes(hipStream_t st, int fmt, const qw_gemm_params& p, const
     qw_gemm_params q = p;
     q.y = part;
     q.ldy = p.N;
+    if (route.rows) return qw_gemm_rows(st, fmt, q, route.rows, route.splits, xdt, QWHIP_F32, false);
     if (route.direct) return qw_dense_direct(st, fmt, q, route.splits, xdt, QWHIP_F32, false, route.few);
     hipError_t e;
     QG_FOR_FMT(fmt, e, (launch_splitk<F>(st, q, route.splits)))
@@ -1464,9 +1475,9 @@ hipError_t launch_planes(hipStream_t st, int fmt, const qw_gemm_params& p, const
 }  // namespace
 
 // flags bits 8..11: tile shape override for tuning and tests (0 = automatic, 1 + CFG_*; 6 and 7 = the direct-operand kernel on spans of
-// 64 and of 128 rows, 96 on the 6- and 8-bit containers; 8 = the 128 x 320 ping-pong tile over K ranges; 14 = 256 x 320 on the DMA-fed
-// kernel instead of the ping-pong kernel; 15 = the unpipelined kernel).  Bits 12..15: the K ranges of 6, 7 and 8 (0 = one), which refuse
-// a call that they cannot take.
+// 64 and of 128 rows, 96 on the 6- and 8-bit containers; 8 = the 128 x 320 ping-pong tile over K ranges; 9 = the row-tile kernel where it
+// takes the call, else one launch of the tiles; 14 = 256 x 320 on the DMA-fed kernel instead of the ping-pong kernel; 15 = the unpipelined
+// kernel).  Bits 12..15: the K ranges of 6 to 9 (0 = one); 6, 7 and 8 refuse a call that they cannot take.
 extern "C" qwhip_status qwhip_gemm(qwhip_stream_t s, const qwhip_weight_view* w, const void* x, uint32_t x_dtype, uint32_t m,
                                    uint32_t ldx, void* y, uint32_t y_dtype, uint32_t ldy, uint32_t flags, void* workspace,
                                    uint64_t workspace_bytes) {
@@ -1543,7 +1554,8 @@ extern "C" qwhip_status qwhip_gemm(qwhip_stream_t s, const qwhip_weight_view* w,
     p.row_bytes = qwhip_view_row_bytes(w);
     hipError_t e;
     if (route.direct && !planes) {
-        QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, p, 1u, xdt, y_dtype, false, route.few));
+        QWHIP_TRY_HIP(route.rows ? qw_gemm_rows(s->stream, fmt, p, route.rows, 1u, xdt, y_dtype, false)
+                                 : qw_dense_direct(s->stream, fmt, p, 1u, xdt, y_dtype, false, route.few));
         return QWHIP_OK;
     }
     if (planes) {
@@ -1640,12 +1652,13 @@ extern "C" qwhip_status qwhip_gemm_swiglu(qwhip_stream_t s, const qwhip_weight_v
     const uint64_t x_used = copy_needed ? ((ws_need + 255u) & ~(uint64_t)255u) : 0u;
     const bool planes_ok = workspace && ((uintptr_t)workspace & 15u) == 0;
     gemm_route route;
-    st = choose_route(w, m, fmt, flags, true, planes_ok && workspace_bytes > x_used ? workspace_bytes - x_used : 0u, &route);
+    const uint64_t plane_room = planes_ok && workspace_bytes > x_used ? workspace_bytes - x_used : 0u;
+    st = choose_route(w, m, fmt, flags, true, plane_room, &route);
     if (st != QWHIP_OK) return st;
-    const bool planes = route.splits >= 2u;
+    const bool planes = route.splits >= 2u || (route.rows && (uint64_t)m * w->n * 4u <= plane_room && !qw_gemm_rows_fuses(fmt, m, w->n, w->k, route.rows));
     const void* xin = x;
     uint32_t xdt = x_dtype;
-    if (copy_needed || (x_dtype == QWHIP_BF16 && !planes)) {
+    if (copy_needed || (x_dtype == QWHIP_BF16 && !planes && !route.rows)) {
         st = rotate ? qwhip_fwht32(s, x, x_dtype, workspace, (uint64_t)m * w->k) : qw_convert_to_f16(s, x, x_dtype, workspace, (uint64_t)m * w->k);
         if (st != QWHIP_OK) return st;
         xin = workspace;
@@ -1675,7 +1688,8 @@ extern "C" qwhip_status qwhip_gemm_swiglu(qwhip_stream_t s, const qwhip_weight_v
         return QWHIP_OK;
     }
     if (route.direct) {
-        QWHIP_TRY_HIP(qw_dense_direct(s->stream, fmt, p, 1u, QWHIP_F16, QWHIP_F16, true, route.few));
+        QWHIP_TRY_HIP(route.rows ? qw_gemm_rows(s->stream, fmt, p, route.rows, 1u, xdt, QWHIP_F16, true)
+                                 : qw_dense_direct(s->stream, fmt, p, 1u, QWHIP_F16, QWHIP_F16, true, route.few));
         return QWHIP_OK;
     }
     // The half-height tile where it is the cheaper one by the pricing of choose_cfg (0.78 of the big tile's efficiency per

@@ -40,3 +40,8 @@ hipError_t qw_grouped_direct(hipStream_t st, int fmt, const qw_gemm_params& p, u
 // gemm_mid.hip: the dense form.  splits > 1: fp32 planes [splits][M][ldy] at p.y (ydt f32), no range of K pairs empty; swiglu: f16
 // rows; few: spans of 64 rows.
 hipError_t qw_dense_direct(hipStream_t st, int fmt, const qw_gemm_params& p, uint32_t splits, uint32_t xdt, uint32_t ydt, bool swiglu, bool few);
+// gemm_rows.hip: dense, at most 64 rows, `steps` 128-column steps a wave over K ranges; the planes and swiglu as qw_dense_direct's.
+hipError_t qw_gemm_rows(hipStream_t st, int fmt, const qw_gemm_params& p, uint32_t steps, uint32_t ranges, uint32_t xdt, uint32_t ydt, bool swiglu);
+bool qw_gemm_rows_choose(int fmt, uint32_t m, uint32_t n, uint32_t k, uint64_t row_bytes, uint64_t plane_room, uint32_t ranges, double limit,
+                         uint32_t* steps, uint32_t* chosen);
+bool qw_gemm_rows_fuses(int fmt, uint32_t m, uint32_t n, uint32_t k, uint32_t steps);

@@ -427,6 +427,51 @@ def test_gemm_direct_operand_kernel(dev, fmt, m, n, k, xdtype, cfg):
         b.free()
 
 
+@pytest.mark.parametrize("fmt", sorted(H.FORMATS))
+@pytest.mark.parametrize("m,n,k,xdtype,ranges", [
+    (17, 272, 1920, "f16", 1), (32, 64, 64, "bf16", 1), (1, 1040, 192, "f16", 1), (33, 4160, 1088, "bf16", 2), (48, 320, 2048, "f16", 1),
+    (64, 8384, 1280, "f16", 1), (49, 4112, 2112, "bf16", 3), (64, 128, 4096, "f16", 4), (31, 16448, 4096, "f16", 1)])
+def test_gemm_row_tile_kernel(dev, fmt, m, n, k, xdtype, ranges):
+    """The row-tile kernel: two, three and four fragments of rows, half a step to the most steps a wave, one workgroup to several tiles
+    each, one launch and K ranges, strided rows.  fp32 sums of k exact products against fp64; the 2-byte outputs are their roundings; the
+    gate|up door gives the two doors' bits in one launch (no workspace) and over one plane."""
+    group = max(64, H.FORMATS[fmt][2])
+    k = -(-k // group) * group
+    cfg, ldx, ldy = form(9, ranges), k + 24, n + 8
+    blocks, w16 = H.make_bank(fmt, n, k, seed=33)
+    x32 = H.make_x(m, k, 8)
+    x_host, xcode = (qo.f32_to_bf16_bits(x32), qwhip.BF16) if xdtype == "bf16" else (x32.astype(np.float16), qwhip.F16)
+    xs = (qo.round_bf16(x32) if xdtype == "bf16" else x32).astype(np.float16).astype(np.float64)
+    strided = np.zeros((m, ldx), x_host.dtype)
+    strided[:, :k] = x_host
+    strided[:, k:] = 0x7E00 if xdtype == "bf16" else np.nan    # not read
+    bank, xb, xp, ws = dev.put(blocks), dev.put(strided), dev.put(x_host), dev.alloc(64 << 20)
+    view = H.view_of(dev, bank, fmt, n, k)
+    lib, st, flags = dev.lib, dev.stream.handle, qwhip.X_PREROTATED | cfg << 8
+    y32, y16, yb = dev.alloc(m * ldy * 4), dev.alloc(m * ldy * 2), dev.alloc(m * ldy * 2)
+    for y, dt in ((y32, qwhip.F32), (y16, qwhip.F16), (yb, qwhip.BF16)):
+        qwhip.check(lib.qwhip_gemm(st, C.byref(view), xb.ptr, xcode, m, ldx, y.ptr, dt, ldy, flags, ws.ptr, 64 << 20))
+    dev.stream.sync()
+    got = y32.download(np.float32, (m, ldy))[:, :n]
+    w = w16.astype(np.float64)
+    assert np.all(np.abs(got - xs @ w.T) <= k * 2.0 ** -24 * (np.abs(xs) @ np.abs(w).T))      # k rounded additions of exact products
+    assert np.array_equal(y16.download(np.float16, (m, ldy))[:, :n], got.astype(np.float16))
+    assert np.array_equal(yb.download(np.uint16, (m, ldy))[:, :n], qo.f32_to_bf16_bits(got))
+    if n % 64 == 0:
+        act1, act2 = dev.alloc(m * n), dev.alloc(m * n)   # [m, n / 2] f16
+        flat = dev.put(got.astype(np.float16))
+        rooms = [64 << 20, m * k * 2] if xdtype == "bf16" or ranges > 1 else [64 << 20, 0]
+        for rot in (0, 1):
+            qwhip.check(lib.qwhip_swiglu_fwht(st, flat.ptr, qwhip.F16, act2.ptr, m, n // 2, rot))
+            for room in rooms if ranges == 1 else rooms[:1]:
+                qwhip.check(lib.qwhip_gemm_swiglu(st, C.byref(view), xp.ptr, xcode, m, 0, rot, act1.ptr, 0, flags, ws.ptr if room else None, room))
+                dev.stream.sync()
+                assert np.array_equal(act1.download(np.uint16, (m, n // 2)), act2.download(np.uint16, (m, n // 2))), (rot, room)
+        act1.free(), act2.free(), flat.free()
+    for b in (bank, xb, xp, ws, y32, y16, yb):
+        b.free()
+
+
 def test_gemm_ranges_fit_an_xcd(dev):
     """An eighth of the tiles, rounded up, over the ranges is what an XCD's 32 units hold: 50 tiles over five ranges are 35 workgroups on
     an XCD although they are 250 on the chip.  The automatic choice is another form (other fp32 sums)."""
