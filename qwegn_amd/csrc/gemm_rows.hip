@@ -25,48 +25,6 @@ QW_ARG_BLOCK(qwr_params, QWR_FIELDS)
 // Waves of a workgroup, by the registers of MF fragments over S steps: 128, 168 or 256 a lane.
 constexpr uint32_t qwr_waves(uint32_t mf, uint32_t s) { return mf * s <= 4u ? 16u : mf * s <= 6u ? 12u : 8u; }
 
-// Step g of a 16-row tile out of the wave's image against MF fragments, the exact f16 weights: lane (n, c) has slice 4 g + c of row n.
-template <int FMT, int S, int MF>
-__device__ __forceinline__ void qwr_step(const uint32_t* img, uint32_t g, uint32_t n, uint32_t c, const h8_t (&xo)[MF][4], uint32_t magic, f4_t (&acc)[MF]) {
-    using im = qr_image<FMT, S>;
-    qg_slice<FMT> blk;
-    blk.hdr = img[16u * im::RS + n * im::HS + 4u * g + c];
-    const uint32_t* src = img + n * im::RS + (4u * g + c) * im::PW;
-    if constexpr (im::PW % 4u == 0u) {
-#pragma unroll
-        for (uint32_t k = 0; k < im::PW; k += 4) {
-            const u4_t v = *(const u4_t*)(src + k);
-            blk.q[k] = v[0], blk.q[k + 1] = v[1], blk.q[k + 2] = v[2], blk.q[k + 3] = v[3];
-        }
-    } else if constexpr (im::PW % 2u == 0u) {
-#pragma unroll
-        for (uint32_t k = 0; k < im::PW; k += 2) {
-            const u2_t v = *(const u2_t*)(src + k);
-            blk.q[k] = v[0], blk.q[k + 1] = v[1];
-        }
-    } else {
-#pragma unroll
-        for (uint32_t k = 0; k < im::PW; ++k) blk.q[k] = src[k];
-    }
-    const h2_t s2 = qw_splat_lo(blk.hdr), b2 = qw_splat_hi(blk.hdr);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const h8_t w = qg_dequant_chunk<FMT>(blk, j, s2, b2, magic);
-#pragma unroll
-        for (int f = 0; f < MF; ++f) acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xo[f][j], w, acc[f], 0, 0, 0);
-    }
-}
-
-// Four activation rows 4 q .. of bank row rr of the tile at `part`, over the waves in order.
-template <int MF>
-__device__ __forceinline__ f4_t qwr_sum(const f4_t* part, uint32_t W, uint32_t q, uint32_t rr) {
-    const f4_t* src = part + (q >> 2) * 64u + (q & 3u) * 16u + rr;
-    f4_t v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-    for (uint32_t w = 0; w < W; ++w) v += src[w * MF * 64u];
-    return v;
-}
-
 // blockDim.x = 64 * ceil(steps / (S nkr)); dynamic LDS = the waves' images, 2 * flush * waves * MF KiB of partial tiles and, GATED, the
 // unit's sums, 4 tiles of 16 MF activation rows by 16 + 1.
 template <int FMT, int MF, int S, bool GATED>
@@ -141,7 +99,7 @@ static __device__ __forceinline__ void run(const qwr_params& p) {
         for (int f = 0; f < MF; ++f) acc[f] = f4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int u = 0; u < S; ++u) {
-            qwr_step<FMT, S, MF>(img, u, n, c, xo[u], magic, acc);
+            qr_weight_step<FMT, S, MF>(img, u, n, c, xo[u], magic, acc);
             __builtin_amdgcn_sched_barrier(0);
         }
         f4_t* mine = parts + ((size_t)(side * p.flush + in_flush) * W + wave) * (MF * 64u) + lane;
@@ -155,7 +113,7 @@ static __device__ __forceinline__ void run(const qwr_params& p) {
             const uint32_t quads = 4u * ((p.M + 15u) >> 4);
             for (uint32_t e = tid; e < in_flush * 16u * quads; e += blockDim.x) {
                 const uint32_t rr = e & 15u, sq = e >> 4, s = sq / quads, q = sq - s * quads;
-                const f4_t v = qwr_sum<MF>(part + (size_t)s * W * MF * 64u, W, q, rr);
+                const f4_t v = qr_wave_sum<MF>(part + (size_t)s * W * MF * 64u, W, q, rr);
                 if constexpr (GATED) {   // one tile a sum
                     float* to = sums + ((slot & 3u) * ROWS + 4u * q) * 17u + rr;
 #pragma unroll

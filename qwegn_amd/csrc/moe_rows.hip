@@ -1,0 +1,318 @@
+// Grouped (MoE) GEMM of few rows an expert on the row-tile form of gemv_rows.hip: one or two fragments of an expert's sorted rows
+// share a tile of 16 of its bank rows.
+//
+// A workgroup takes up to 32 rows of a tile-list entry and a band of the expert's row tiles; its waves split the columns and keep the
+// rows' columns in registers for all the band.  The launch reads every routed expert's bank once and is bound by that stream: the
+// direct-operand kernel's four waves wait for a K-step's loads and their way through LDS at a barrier each, with 1 to 32 rows to
+// multiply.
+#include <algorithm>
+#include <atomic>
+#include <cmath>
+
+#include "qw_gemm.h"
+#include "qw_rows.h"
+
+namespace {
+
+#define QMR_FIELDS(X)                                                                                                       \
+    X(const uint8_t*, bank) X(const int32_t*, tile_count) X(const int32_t*, tile_e) X(const int32_t*, tile_r)                    \
+    X(const int32_t*, expert_off) X(uint32_t, bands) X(uint32_t, nsl) X(uint32_t, gshift) X(uint32_t, bb) X(const int32_t*, gather)  \
+    X(const void*, x) X(uint64_t, expert_bytes) X(uint32_t, row_bytes) X(uint32_t, N) X(uint32_t, units) X(uint32_t, K) X(uint32_t, ldx)   \
+    X(uint32_t, x_bf16) X(uint32_t, flush) X(uint32_t, inter) X(uint32_t, rotate) X(void*, y) X(uint32_t, ldy) X(uint32_t, y_dtype)        \
+    X(qw_act, act)
+QW_ARG_BLOCK(qmr_params, QMR_FIELDS)
+
+// Waves of a workgroup, by the registers of MF fragments over S steps.
+constexpr uint32_t qmr_waves(uint32_t mf, uint32_t s) { return mf * s <= 2u ? 16u : 12u; }
+
+// blockDim.x = 64 * ceil(steps / S); dynamic LDS = the waves' images, 2 * flush * waves * MF KiB of partial tiles and, GATED, the unit's
+// sums, 4 tiles of 16 MF rows by 16 + 1.  Grid: as the direct-operand kernel's, an XCD takes a contiguous eighth of the tile list and walks
+// (entry, band) band-fastest.
+template <int FMT, int S, int MF, bool GATED>
+struct qw_moe_rows_kernel {
+static constexpr int kLaunchBound = 64 * qmr_waves(MF, S);
+
+static __device__ __forceinline__ void rows(const qmr_params& p, const uint8_t* bank, uint32_t m0, uint32_t M, uint32_t band, uint32_t* lds) {
+    using im = qr_image<FMT, S>;
+    constexpr uint32_t SPU = GATED ? 4u : 1u, RPL = 16u / S, ROWS = 16u * MF;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, W = blockDim.x >> 6, G = p.bands;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t n = lane & 15u, c = lane >> 4;             // contraction role
+    const uint32_t lb = lane / RPL, lj = lane & (RPL - 1u);   // load role: slice lb of the wave's, row RPL q + lj of the tile
+    uint32_t* const img = lds + wave * im::DWORDS;
+    f4_t* const parts = (f4_t*)(lds + W * im::DWORDS);
+    float* const sums = (float*)(parts + (size_t)2u * p.flush * W * MF * 64u);
+    const uint32_t slots = (p.units - band + G - 1u) / G * SPU;
+    const uint32_t magic = qw_vgpr_const(0x64006400u);
+
+    // the rows' places first: the activations wait for them, the bank's first tile for nothing
+    const uint32_t xrow = min(lane, M - 1u);
+    const uint32_t src_row = p.gather ? (uint32_t)p.gather[m0 + xrow] : m0 + xrow;
+    struct place { const uint8_t* bank; uint32_t nsl, gshift, bb; } at = {bank, p.nsl, p.gshift, p.bb};
+    uint32_t hdr, codes;
+    qr_slice_at<FMT>(at, 4u * S * wave + lb, hdr, codes);
+    qg_slice<FMT> buf[S];
+    auto request = [&](uint32_t slot) __attribute__((always_inline)) {
+        uint32_t row;
+        if constexpr (!GATED) {
+            row = 16u * (slot * G + band);
+        } else {
+            const uint32_t k = slot >> 2, q = slot & 3u;
+            row = 32u * (k * G + band) + 16u * (q & 1u) + (q >= 2u ? p.inter : 0u);
+        }
+        qr_for<S>([&](auto q) {
+            const uint32_t ro = min(row + RPL * q + lj, p.N - 1u) * p.row_bytes;
+            qr_load<FMT>(at, ro + hdr, ro + codes, buf[q]);
+        });
+    };
+    request(0);
+    __builtin_amdgcn_sched_barrier(0);
+    u4_t raw[4 * S * MF];   // step, fragment, four rows a load: runs of 256 bytes; zero past M and past the row's end
+    qr_for<4 * MF>([&](auto f) {
+        const uint32_t row = 4u * f + c, from = (uint32_t)__shfl((int)src_row, (int)min(row, 63u), 64);
+        qr_for<S>([&](auto u) {
+            const uint32_t col = 128u * (wave * S + u) + 8u * n;
+            u4_t v = {0u, 0u, 0u, 0u};
+            if (row < M && col < p.K) v = *(const u4_t*)((const uint8_t*)p.x + (2u * from * p.ldx + 2u * col));
+            raw[4 * MF * u + f] = v;
+        });
+    });
+    __builtin_amdgcn_sched_barrier(0);
+    h8_t xo[S][MF][4];
+    qr_for<S>([&](auto u) {
+        qr_for<MF>([&](auto f) {
+            qr_for<4>([&](auto q) {
+                const u4_t v = raw[4 * MF * u + 4 * f + q];
+                *(h8_t*)(img + (4u * q + c) * QR_XS + 4u * n) = p.x_bf16 ? qg_to_f16x8<QWHIP_BF16>(v) : qg_to_f16x8<QWHIP_F16>(v);
+            });
+            asm volatile("" ::: "memory");   // a wave's own LDS operations complete in order
+            qr_for<4>([&](auto t) { xo[u][f][t] = *(const h8_t*)(img + n * QR_XS + 4u * (4u * c + t)); });
+            asm volatile("" ::: "memory");
+        });
+    });
+
+    uint32_t in_flush = 0, side = 0, first = 0;   // row tiles since the last sum, the half of the partial tiles, its first slot
+#pragma unroll 1
+    for (uint32_t slot = 0; slot < slots; ++slot) {
+        qr_for<S>([&](auto q) { qr_park<FMT, S>(img, RPL * q + lj, lb, buf[q]); });
+        asm volatile("" ::: "memory");
+        if (slot + 1u < slots) request(slot + 1u);
+        __builtin_amdgcn_sched_barrier(0);
+        f4_t acc[MF];
+#pragma unroll
+        for (int f = 0; f < MF; ++f) acc[f] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < S; ++u) {
+            qr_weight_step<FMT, S, MF>(img, u, n, c, xo[u], magic, acc);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        f4_t* mine = parts + ((size_t)(side * p.flush + in_flush) * W + wave) * (MF * 64u) + lane;
+#pragma unroll
+        for (int f = 0; f < MF; ++f) mine[f * 64] = acc[f];
+        asm volatile("" ::: "memory");
+        ++in_flush;
+        if (in_flush == p.flush || slot + 1u == slots) {
+            __syncthreads();   // the other half of the partial tiles is free again: its sums lie before this barrier
+            const f4_t* part = parts + (size_t)side * p.flush * W * MF * 64u;
+            const uint32_t quads = (M + 3u) >> 2;
+            for (uint32_t e = tid; e < in_flush * 16u * quads; e += blockDim.x) {
+                const uint32_t rr = e & 15u, sq = e >> 4, s = sq / quads, q = sq - s * quads;
+                const f4_t v = qr_wave_sum<MF>(part + (size_t)s * W * MF * 64u, W, q, rr);
+                if constexpr (GATED) {   // one tile a sum
+                    float* to = sums + ((slot & 3u) * ROWS + 4u * q) * 17u + rr;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) to[r * 17] = (float)(h1_t)v[r];   // what the plain door stores
+                } else {
+                    const uint32_t row = 16u * ((first + s) * G + band) + rr;
+#pragma unroll
+                    for (uint32_t r = 0; r < 4; ++r) {
+                        const uint32_t m = 4u * q + r;
+                        if (m >= M || row >= p.N) continue;
+                        const uint64_t to = (uint64_t)(m0 + m) * p.ldy + row;
+                        if (p.y_dtype == QWHIP_F32) qg_store<QWHIP_F32>(p.y, to, v[r]);
+                        else if (p.y_dtype == QWHIP_F16) qg_store<QWHIP_F16>(p.y, to, v[r]);
+                        else qg_store<QWHIP_BF16>(p.y, to, v[r]);
+                    }
+                }
+            }
+            in_flush = 0;
+            side ^= 1u;
+            first = slot + 1u;
+            if constexpr (GATED) {
+                if ((slot & 3u) == 3u) {
+                    __syncthreads();
+                    const uint32_t j = tid & 31u, c0 = 32u * ((slot >> 2) * G + band);
+                    const qw_fwht32_signs sg = qw_fwht32_lane_signs(j);
+                    for (uint32_t e = tid; e < ((32u * M + 63u) & ~63u); e += blockDim.x) {   // whole waves: the rotation exchanges lanes
+                        const uint32_t m = min(e >> 5, M - 1u);
+                        const float* g = sums + ((j >> 4) * ROWS + m) * 17u + (j & 15u);
+                        float v = qw_gated(g[0], g[2u * ROWS * 17u], p.act);
+                        if (p.rotate) {
+                            v = qw_fwht32_lanes(v, sg) * QW_INV_SQRT32;
+                            asm volatile("" : "+v"(v));   // rounded to fp32 and then to f16, as the rotation pass does (not by one mixed instruction)
+                        }
+                        if (e < 32u * M) ((h1_t*)p.y)[(uint64_t)(m0 + m) * p.ldy + c0 + j] = (h1_t)v;
+                    }
+                    // the next unit's sums lie behind the next tile's barrier
+                }
+            }
+        }
+    }
+}
+
+static __device__ __forceinline__ void run(const qmr_params& p) {
+    extern __shared__ __attribute__((aligned(16))) uint32_t qmr_lds[];
+    const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
+    const uint32_t tc = (uint32_t)max(p.tile_count[0], 0), per_xcd = (tc + 7u) >> 3;
+    const uint32_t ti = slot / p.bands, t = xcd * per_xcd + ti;
+    if (ti >= per_xcd || t >= tc) return;
+    const uint32_t e = (uint32_t)p.tile_e[t], packed = (uint32_t)p.tile_r[t];
+    const uint32_t code = packed >> 24, bm = code == 1u ? 16u : code == 2u ? 32u : 64u;   // rows of the entry's tile
+    const uint32_t first = (packed & 0xFFFFFFu) * bm;                                     // row of the expert
+    const uint32_t off = (uint32_t)p.expert_off[e], rows_e = (uint32_t)p.expert_off[e + 1] - off;
+    if (first >= rows_e) return;
+    const uint32_t M = min(bm, rows_e - first);
+    const uint8_t* bank = p.bank + (uint64_t)e * p.expert_bytes;
+#pragma unroll 1
+    for (uint32_t r = 0; r < M; r += 16u * MF) {
+        if (r > 0) __syncthreads();
+        rows(p, bank, off + first + r, min(16u * MF, M - r), slot - ti * p.bands, qmr_lds);
+    }
+}
+};
+
+template <int FMT, int S, int MF, bool GATED>
+hipError_t qmr_go(hipStream_t st, const qmr_params& p, uint32_t wgs, uint32_t waves, size_t lds) {
+    using K = qw_moe_rows_kernel<FMT, S, MF, GATED>;
+    static std::atomic<bool> attr_done{false};   // per instantiation
+    if (!attr_done.load(std::memory_order_acquire)) {
+        const hipError_t e = hipFuncSetAttribute(qw_scalar_kernel_ptr<K>((const qmr_params*)nullptr), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) return e;
+        attr_done.store(true, std::memory_order_release);
+    }
+    qw_launch_scalar<K>(dim3(wgs), dim3(64u * waves), lds, st, p);
+    return hipGetLastError();
+}
+template <int FMT>
+constexpr uint32_t qmr_image_bytes(uint32_t s) { return 4u * (s == 1u ? qr_image<FMT, 1>::DWORDS : qr_image<FMT, 2>::DWORDS); }
+uint32_t qmr_image_bytes(int fmt, uint32_t s) {
+    switch (fmt) {
+        case QG_FMT_M5: return qmr_image_bytes<QG_FMT_M5>(s);
+        case QG_FMT_B4: return qmr_image_bytes<QG_FMT_B4>(s);
+        case QG_FMT_B8: return qmr_image_bytes<QG_FMT_B8>(s);
+        case QG_FMT_B2: return qmr_image_bytes<QG_FMT_B2>(s);
+        case QG_FMT_B3: return qmr_image_bytes<QG_FMT_B3>(s);
+        default: return qmr_image_bytes<QG_FMT_B6>(s);
+    }
+}
+
+// Steps a wave: by the bank's container and columns alone, so that both doors add in one order.  Two, the waves of several workgroups to a
+// unit; one where that would leave two waves, and on 8-bit banks up to 1536 columns (32 experts, 6 rows each, 1536 x 1536: 18.6 us, 19.5).
+uint32_t qmr_steps(int fmt, uint32_t k) {
+    const uint32_t steps = k / 128u;
+    return steps <= 5u || (fmt == QG_FMT_B8 && steps <= 12u) ? 1u : 2u;
+}
+
+struct qmr_config {
+    uint32_t waves, mf, units, bands, flush, lds;   // waves = 0: none fits
+    double us;
+};
+// The launch with the lowest price, us: fragments of rows and bands of an expert's row tiles.  A launch 4.2; then rounds of workgroups,
+// one's start 1.5, its activations and row tiles for every 16 mf rows of its expert (rows an expert: Poisson), a tile costing 0.54, its
+// waves' sums and every step's unpacking and products on a SIMD; no faster than 5.7 TB/s of the experts that have rows.  Fitted to the
+// choice among 16 forms each of 122 problems (8 .. 256 experts, up to 8 rows each, 12 containers): 0.71 of the direct-operand kernel's
+// time where the best of the forms took 0.69.
+qmr_config qmr_choose(int fmt, const qw_gemm_params& p, uint32_t experts, bool gated) {
+    const uint32_t s = qmr_steps(fmt, p.K), waves = qwhip_cdiv(p.K / 128u, s), most = 160u * 1024u, units = gated ? p.inter / 32u : qwhip_cdiv(p.N, 16u);
+    const double unpack = fmt == QG_FMT_B8 ? 1.38 : fmt == QG_FMT_B6 ? 0.9 : fmt == QG_FMT_B3 ? 2.2 : 1.0;
+    const double mean = p.M / (double)experts, none = std::exp(-mean), used = experts * (1.0 - none);
+    const double stream = 4.2 + used * (double)p.N * (double)p.row_bytes / 5.7e6;
+    qmr_config best = {};
+    best.us = 1e30;
+    for (uint32_t mf = 1; mf <= 2u; ++mf) {
+        const uint32_t image = waves * qmr_image_bytes(fmt, s), part = 2u * waves * mf * 1024u, sums = 4u * 16u * mf * 17u * 4u;
+        if (waves > qmr_waves(mf, s) || image + part + sums > most) continue;
+        double passes = 0.0, chance = none;   // of an expert with rows
+        for (uint32_t k = 1; k < 64u; ++k) chance *= mean / k, passes += chance * qwhip_cdiv(k, 16u * mf);
+        passes /= 1.0 - none;
+        const uint32_t per_cu = max(1u, min(qmr_waves(mf, s) / waves, most / (image + part + sums)));
+        for (uint32_t bands : {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u, 24u, 32u, 48u}) {
+            if (bands > units) break;
+            const double wgs = used * bands / 256.0, side = std::min((double)per_cu, std::max(1.0, std::ceil(wgs)));
+            const uint32_t tiles = qwhip_cdiv(units, bands) * (gated ? 4u : 1u);
+            const double tile = 0.54 + 0.029 * waves * s + waves * side / 4.0 * s * (0.116 * unpack + 0.034 * mf);
+            const double rounds = std::max(1.0, std::ceil(wgs / side - 0.01));
+            const double us = std::max(stream, 4.2 + rounds * (1.5 + passes * (0.32 * s * mf + tiles * tile)));
+            if (us >= best.us) continue;
+            best.waves = waves, best.mf = mf, best.units = units, best.bands = bands, best.us = us;
+            best.flush = gated ? 1u : max(1u, min(min(4u, tiles), (most / per_cu - image) / part));
+            best.lds = image + best.flush * part + (gated ? sums : 0u);
+        }
+    }
+    return best;
+}
+
+template <int FMT>
+hipError_t qmr_launch(hipStream_t st, const qmr_params& p, const qmr_config& c, uint32_t s, uint32_t max_tiles, bool gated) {
+    const uint32_t wgs = 8u * qwhip_cdiv(max_tiles, 8u) * c.bands;
+#define QMR_GO(S, M) (gated ? qmr_go<FMT, S, M, true>(st, p, wgs, c.waves, c.lds) : qmr_go<FMT, S, M, false>(st, p, wgs, c.waves, c.lds))
+    if (s == 1u) return c.mf == 1u ? QMR_GO(1, 1) : QMR_GO(1, 2);
+    return c.mf == 1u ? QMR_GO(2, 1) : QMR_GO(2, 2);
+#undef QMR_GO
+}
+
+}  // namespace
+
+// A mean of up to eight rows an expert, at which the direct-operand kernel multiplies 32 and waits; by price against its own, the dense
+// form's (choose_direct) without ranges, which is a tenth below the grouped kernel's measured times.  Past eight rows the second fragment
+// and the experts of several passes take the lead away (16 rows and more each 1.1 to 1.5 times its time).
+bool qw_grouped_rows_takes(int fmt, const qw_gemm_params& p, uint32_t experts) {
+    if (p.M > 8u * experts) return false;
+    const qmr_config c = qmr_choose(fmt, p, experts, false);
+    if (c.waves == 0u) return false;
+    const double used = experts * (1.0 - std::exp(-(p.M / (double)experts))), load = used * qwhip_cdiv(p.N, 256u) / 256.0;
+    const double rounds = load <= 1.0 ? 1.0 + 0.10 * load : load <= 2.0 ? 1.41 + 0.19 * load : 0.36 + 0.885 * load;
+    const bool wide = fmt == QG_FMT_B8 || fmt == QG_FMT_B6;
+    const double direct = 5.3 + std::max(p.K / 128u * 1.04 * (wide ? 1.39 : 1.0) * rounds, used * (double)p.N * (double)p.row_bytes / 3.5e6);
+    return c.us < 1.1 * direct;
+}
+hipError_t qw_grouped_rows(hipStream_t st, int fmt, const qw_gemm_params& g, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt,
+                           bool swiglu) {
+    const qmr_config c = qmr_choose(fmt, g, experts, swiglu);
+    if (c.waves == 0u || (uint64_t)max_tiles * c.bands >= (1u << 30)) return hipErrorInvalidValue;
+    const uint32_t s = qmr_steps(fmt, g.K);
+    qmr_params p;
+    p.bank = g.bank;
+    p.tile_count = g.tile_count;
+    p.tile_e = g.tile_e;
+    p.tile_r = g.tile_r;
+    p.expert_off = g.expert_off;
+    p.bands = c.bands;
+    p.nsl = g.K / 32u;
+    p.gshift = g.gshift;
+    p.bb = g.bb;
+    p.gather = g.gather;
+    p.x = g.x;
+    p.expert_bytes = (uint64_t)g.rows_per_expert * g.row_bytes;
+    p.row_bytes = (uint32_t)g.row_bytes;
+    p.N = g.N;
+    p.units = c.units;
+    p.K = g.K;
+    p.ldx = g.ldx;
+    p.x_bf16 = xdt == QWHIP_BF16 ? 1u : 0u;
+    p.flush = c.flush;
+    p.inter = g.inter;
+    p.rotate = g.rotate_act;
+    p.y = g.y;
+    p.ldy = g.ldy;
+    p.y_dtype = ydt;
+    p.act = g.act;
+    switch (fmt) {
+        case QG_FMT_M5: return qmr_launch<QG_FMT_M5>(st, p, c, s, max_tiles, swiglu);
+        case QG_FMT_B4: return qmr_launch<QG_FMT_B4>(st, p, c, s, max_tiles, swiglu);
+        case QG_FMT_B8: return qmr_launch<QG_FMT_B8>(st, p, c, s, max_tiles, swiglu);
+        case QG_FMT_B2: return qmr_launch<QG_FMT_B2>(st, p, c, s, max_tiles, swiglu);
+        case QG_FMT_B3: return qmr_launch<QG_FMT_B3>(st, p, c, s, max_tiles, swiglu);
+        default: return qmr_launch<QG_FMT_B6>(st, p, c, s, max_tiles, swiglu);
+    }
+}

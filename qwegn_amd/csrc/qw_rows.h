@@ -1,5 +1,5 @@
 // A tile of 16 bank rows against fragments of 16 f16 activation rows, as the row-tile kernels take it (gemv_rows.hip has the whole,
-// gemm_rows.hip two and four fragments): a wave's LDS image of the slices, the codes as f16 operands, one step of 128 columns.
+// gemm_rows.hip and moe_rows.hip several fragments): a wave's LDS image of the slices, the codes as f16 operands, one step of 128 columns.
 #pragma once
 #include <type_traits>
 
@@ -201,6 +201,48 @@ __device__ __forceinline__ void qr_for(F&& f) {   // arrays of slices stay in re
         f(std::integral_constant<int, I>{});
         qr_for<N, I + 1>(f);
     }
+}
+
+// Step g of a 16-row tile out of the wave's image against MF fragments, the exact f16 weights: lane (n, c) has slice 4 g + c of row n.
+template <int FMT, int S, int MF>
+__device__ __forceinline__ void qr_weight_step(const uint32_t* img, uint32_t g, uint32_t n, uint32_t c, const h8_t (&xo)[MF][4], uint32_t magic, f4_t (&acc)[MF]) {
+    using im = qr_image<FMT, S>;
+    qg_slice<FMT> blk;
+    blk.hdr = img[16u * im::RS + n * im::HS + 4u * g + c];
+    const uint32_t* src = img + n * im::RS + (4u * g + c) * im::PW;
+    if constexpr (im::PW % 4u == 0u) {
+#pragma unroll
+        for (uint32_t k = 0; k < im::PW; k += 4) {
+            const u4_t v = *(const u4_t*)(src + k);
+            blk.q[k] = v[0], blk.q[k + 1] = v[1], blk.q[k + 2] = v[2], blk.q[k + 3] = v[3];
+        }
+    } else if constexpr (im::PW % 2u == 0u) {
+#pragma unroll
+        for (uint32_t k = 0; k < im::PW; k += 2) {
+            const u2_t v = *(const u2_t*)(src + k);
+            blk.q[k] = v[0], blk.q[k + 1] = v[1];
+        }
+    } else {
+#pragma unroll
+        for (uint32_t k = 0; k < im::PW; ++k) blk.q[k] = src[k];
+    }
+    const h2_t s2 = qw_splat_lo(blk.hdr), b2 = qw_splat_hi(blk.hdr);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const h8_t w = qg_dequant_chunk<FMT>(blk, j, s2, b2, magic);
+#pragma unroll
+        for (int f = 0; f < MF; ++f) acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xo[f][j], w, acc[f], 0, 0, 0);
+    }
+}
+
+// Four activation rows 4 q .. of bank row rr of the tile at `part`, over the waves in order.
+template <int MF>
+__device__ __forceinline__ f4_t qr_wave_sum(const f4_t* part, uint32_t W, uint32_t q, uint32_t rr) {
+    const f4_t* src = part + (q >> 2) * 64u + (q & 3u) * 16u + rr;
+    f4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (uint32_t w = 0; w < W; ++w) v += src[w * MF * 64u];
+    return v;
 }
 
 }  // namespace

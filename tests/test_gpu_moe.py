@@ -438,6 +438,18 @@ def test_grouped_gemm_spans(dev, fmt, counts, k, inter, xdt, compact):
     assert np.array_equal(act1.download(np.uint16, (pairs, inter)), act2.download(np.uint16, (pairs, inter)))
 
 
+_FEW_EACH = [1, 16, 17, 0, 32, 33, 64, 65, 3, 2, 5] + [0] * 29     # six rows an expert: the row-tile kernel, one to four passes of 16
+
+
+@pytest.mark.parametrize("fmt", sorted(f for f in H.FORMATS if f != "aq8_g256"))
+@pytest.mark.parametrize("counts,k,inter,xdt,compact", [
+    (_FEW_EACH, 640, 96, "f16", True), (_FEW_EACH, 1024, 32, "bf16", False), (_FEW_EACH, 2176, 160, "f16", True),
+    (_FEW_EACH, 3968, 32, "f16", False), ([15, 1, 9, 0, 3], 1536, 1024, "bf16", True)])
+def test_grouped_gemm_of_few_rows_an_expert(dev, fmt, counts, k, inter, xdt, compact):
+    """The row-tile kernel's edges: fragments and passes, one step a wave and two, a last half step, one to several bands of row tiles."""
+    test_grouped_gemm_spans(dev, fmt, counts, k, inter, xdt, compact)
+
+
 @pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq8_g32", "hq4_g64"])
 @pytest.mark.parametrize("counts,inter", [(_SPANS_FEW, 96), (_SPANS_MANY, 96), ([2300, 40], 96), (_SPANS_MANY, 6656), ([2300, 40], 4992)])
 def test_grouped_gemm_takes_any_tile_list(dev, fmt, counts, inter):
