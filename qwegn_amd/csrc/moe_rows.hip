@@ -264,17 +264,20 @@ hipError_t qmr_launch(hipStream_t st, const qmr_params& p, const qmr_config& c, 
 }  // namespace
 
 // A mean of up to eight rows an expert, at which the direct-operand kernel multiplies 32 and waits; by price against its own, the dense
-// form's (choose_direct) without ranges, which is a tenth below the grouped kernel's measured times.  Past eight rows the second fragment
-// and the experts of several passes take the lead away (16 rows and more each 1.1 to 1.5 times its time).
+// form's (choose_direct) without ranges, which is a tenth below the grouped kernel's measured times.  Over 200 other problems 0.77 of its
+// time, 3 % slower at most.  Past that where the direct-operand kernel's workgroups leave units idle and the price says so clearly (ratio
+// 0.8): up to ten rows under 0.8 of a workgroup a unit, up to 24 under 0.6 (280 problems of 8 to 60 experts, 8 to 24 rows each: 0.84 of
+// the time over all, one slower by 10 %; on more experts the second fragment and the experts of several passes made up to 1.3 of it, at 24
+// to 48 rows four of 26 were slower by 14 to 20 %).
 bool qw_grouped_rows_takes(int fmt, const qw_gemm_params& p, uint32_t experts) {
-    if (p.M > 8u * experts) return false;
+    if (p.M > 24u * experts) return false;
     const qmr_config c = qmr_choose(fmt, p, experts, false);
     if (c.waves == 0u) return false;
     const double used = experts * (1.0 - std::exp(-(p.M / (double)experts))), load = used * qwhip_cdiv(p.N, 256u) / 256.0;
     const double rounds = load <= 1.0 ? 1.0 + 0.10 * load : load <= 2.0 ? 1.41 + 0.19 * load : 0.36 + 0.885 * load;
     const bool wide = fmt == QG_FMT_B8 || fmt == QG_FMT_B6;
     const double direct = 5.3 + std::max(p.K / 128u * 1.04 * (wide ? 1.39 : 1.0) * rounds, used * (double)p.N * (double)p.row_bytes / 3.5e6);
-    return c.us < 1.1 * direct;
+    return p.M <= 8u * experts ? c.us < 1.1 * direct : load <= (p.M <= 10u * experts ? 0.8 : 0.6) && c.us < 0.8 * direct;
 }
 hipError_t qw_grouped_rows(hipStream_t st, int fmt, const qw_gemm_params& g, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt,
                            bool swiglu) {

@@ -444,7 +444,7 @@ _FEW_EACH = [1, 16, 17, 0, 32, 33, 64, 65, 3, 2, 5] + [0] * 29     # six rows an
 @pytest.mark.parametrize("fmt", sorted(f for f in H.FORMATS if f != "aq8_g256"))
 @pytest.mark.parametrize("counts,k,inter,xdt,compact", [
     (_FEW_EACH, 640, 96, "f16", True), (_FEW_EACH, 1024, 32, "bf16", False), (_FEW_EACH, 2176, 160, "f16", True),
-    (_FEW_EACH, 3968, 32, "f16", False), ([15, 1, 9, 0, 3], 1536, 1024, "bf16", True)])
+    (_FEW_EACH, 3968, 32, "f16", False), ([15, 1, 9, 0, 3], 1536, 1024, "bf16", True), ([40, 20, 0, 33, 15], 1536, 96, "f16", True)])
 def test_grouped_gemm_of_few_rows_an_expert(dev, fmt, counts, k, inter, xdt, compact):
     """The row-tile kernel's edges: fragments and passes, one step a wave and two, a last half step, one to several bands of row tiles."""
     test_grouped_gemm_spans(dev, fmt, counts, k, inter, xdt, compact)
