@@ -32,6 +32,8 @@ struct qgf_params {
     uint64_t row_bytes;
     float scale;
     const float* row_down;   // [M] powers of two: row r is contracted as x[r] * row_down[r]
+    float* part;             // K ranges of `per` steps (gridDim.z > 1): planes [range][M][N] of the scaled rows' sums
+    uint32_t per;
 };
 
 // row_down[r] = 2^-e with 2^e <= max |x[r]| * 2^-13 < 2^(e + 1); 1 for a row of zeros.  e is kept inside the exponents
@@ -164,10 +166,10 @@ __global__ __launch_bounds__(256) void qw_gemm_f32x_kernel(const qgf_params p) {
     };
 
     f16_t acc = {}, acc_lo = {};
-    const uint32_t nk = p.K / 64u;
+    const uint32_t k0 = blockIdx.z * p.per, nk = min(p.K / 64u, k0 + p.per);
     const uint32_t frow = lane & 31u, k_half = lane >> 5;
-    issue(0);
-    for (uint32_t kt = 0; kt < nk; ++kt) {
+    issue(k0);
+    for (uint32_t kt = k0; kt < nk; ++kt) {
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -205,20 +207,36 @@ __global__ __launch_bounds__(256) void qw_gemm_f32x_kernel(const qgf_params p) {
         for (int r = 0; r < 16; ++r) {
             const uint32_t row = m0 + wm * 32u + 8u * (r >> 2) + 4u * k_half + (r & 3);
             if (row < p.M) {
-                const float up = 1.0f / p.row_down[row];     // a power of two: exact
-                p.y[(uint64_t)row * p.N + n] = qgf_epilogue(__builtin_fmaf(acc_lo[r], 1.0f / 2048.0f, acc[r]) * up, p.epi, p.scale);
+                const float v = __builtin_fmaf(acc_lo[r], 1.0f / 2048.0f, acc[r]);
+                if (gridDim.z > 1u) {
+                    p.part[((uint64_t)blockIdx.z * p.M + row) * p.N + n] = v;
+                } else {
+                    const float up = 1.0f / p.row_down[row];     // a power of two: exact
+                    p.y[(uint64_t)row * p.N + n] = qgf_epilogue(v * up, p.epi, p.scale);
+                }
             }
         }
     }
 }
 
+// The planes' sum in range order, the rows' scale and the epilogue.
+__global__ __launch_bounds__(256) void qw_f32_plane_sum_kernel(const float* __restrict__ part, uint32_t ranges, uint32_t M, uint32_t N,
+                                                               const float* __restrict__ row_down, uint32_t epi, float scale, float* __restrict__ y) {
+    const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x, plane = (uint64_t)M * N;
+    if (i >= plane) return;
+    float v = part[i];
+    for (uint32_t r = 1; r < ranges; ++r) v += part[r * plane + i];
+    y[i] = qgf_epilogue(v * (1.0f / row_down[i / N]), epi, scale);
+}
+
 }  // namespace
 
 // Runs the batched form for a validated call; false when the shape is outside it (K not a multiple of 64).
-// `row_down`: device scratch for m floats (the rows' scaling factors, written by the first of the two launches).
+// `row_down`: `scratch_bytes` of device scratch: m floats (the rows' scaling factors, written by the first launch), then the planes of
+// the K ranges, which a last launch sums.
 // Epilogue 3's rotation over the outputs is the caller's second launch, as for the GEMV form.
 bool qw_f32_gemm(hipStream_t st, const qwhip_weight_view* w, int fmt, uint32_t gshift, uint32_t bb, uint64_t row_bytes,
-                 const float* x, uint32_t m, uint32_t epi, float scale, float* y, float* row_down) {
+                 const float* x, uint32_t m, uint32_t epi, float scale, float* y, float* row_down, uint64_t scratch_bytes) {
     if (w->k % 64u != 0 || ((uintptr_t)x & 15u) != 0 || !row_down) return false;
     hipLaunchKernelGGL(qw_row_scale_kernel, dim3(qwhip_cdiv(m, 4u)), dim3(256), 0, st, x, m, w->k, row_down);
     qgf_params p;
@@ -234,12 +252,26 @@ bool qw_f32_gemm(hipStream_t st, const qwhip_weight_view* w, int fmt, uint32_t g
     p.epi = epi;
     p.row_bytes = row_bytes;
     p.scale = scale;
-    const dim3 grid(qwhip_cdiv(w->n, 64u), qwhip_cdiv(m, 64u));
+    const uint32_t tiles = max(1u, qwhip_cdiv(w->n, 64u) * qwhip_cdiv(m, 64u)), steps = w->k / 64u;
+    const uint64_t head = ((uint64_t)m + 63u) / 64u * 256u, plane = (uint64_t)m * w->n * 4u;   // bytes
+    // K ranges to two workgroups a unit, of two steps at least, where the scratch holds their planes.  A step of a lone workgroup is 1.2 us,
+    // loads, splits and two barriers one after the other, and 64 x 64 tiles leave most units without one: 208 x 1088 x 3840 75.9 -> 29 us,
+    // 40 x 1024 x 8192 144 -> 23.7, 130 x 2048 x 2048 43.2 -> 23, 33 x 1024 x 1024 24.1 -> 11.3 (on 256 tiles, 100 x 8192 x 1024, 27.9 -> 26.1).
+    // The error against 64 bits falls with the ranges: 3.9e-7 -> 1.6e-7, 5.9e-7 -> 1.8e-7, 2.9e-7 -> 1.5e-7.
+    uint32_t ranges = min(min(512u / tiles, steps / 2u), 16u);
+    while (ranges > 1u && head + ranges * plane > scratch_bytes) --ranges;
+    ranges = max(ranges, 1u);
+    p.per = qwhip_cdiv(steps, ranges);
+    ranges = qwhip_cdiv(steps, p.per);
+    p.part = (float*)((uint8_t*)row_down + head);
+    const dim3 grid(qwhip_cdiv(w->n, 64u), qwhip_cdiv(m, 64u), ranges);
     switch (fmt) {
 #define QGF_GO(F) case F: hipLaunchKernelGGL(qw_gemm_f32x_kernel<F>, grid, dim3(256), 0, st, p); break;
         QGF_GO(QW_FMT_M5) QGF_GO(QW_FMT_B4) QGF_GO(QW_FMT_B8) QGF_GO(QW_FMT_B2) QGF_GO(QW_FMT_B3) QGF_GO(QW_FMT_B6)
 #undef QGF_GO
         default: return false;
     }
+    if (ranges > 1u)
+        hipLaunchKernelGGL(qw_f32_plane_sum_kernel, dim3((unsigned)((plane / 4u + 255u) / 256u)), dim3(256), 0, st, p.part, ranges, m, w->n, row_down, epi, scale, y);
     return true;
 }

@@ -1591,7 +1591,7 @@ void qw_f32_gemv(hipStream_t st, const qwhip_weight_view* w, int fmt, uint32_t g
 void qw_h32_f32_launch(hipStream_t st, const float* x, float* out, uint32_t rows, uint32_t hidden);
 // gemm_f32.hip
 bool qw_f32_gemm(hipStream_t st, const qwhip_weight_view* w, int fmt, uint32_t gshift, uint32_t bb, uint64_t row_bytes,
-                 const float* x, uint32_t m, uint32_t epi, float scale, float* y, float* row_down);
+                 const float* x, uint32_t m, uint32_t epi, float scale, float* y, float* row_down, uint64_t scratch_bytes);
 
 // fp32 activations in the container's basis -> fp32 outputs with the scalar epilogues of the reference's f32 family
 // (QWGemm.encodeHQ4F32V4 / encodeHQ4F32BM, Sources/Operators/QWGEMM/QWGemmF32.swift:178-199,311-350): the rows go through
@@ -1616,10 +1616,11 @@ extern "C" qwhip_status qwhip_gemv_f32(qwhip_stream_t s, const qwhip_weight_view
     const uint32_t per = qw_f32_gemv_rows(w, row_bytes);
     if (per == 0) return qwhip_fail(QWHIP_E_BAD_GEOMETRY, "no f32 gemv kernel for n=%u k=%u (rows up to 32768 columns, banks under 1 GiB)", w->n, w->k);
     const uint32_t gshift = log2_u32(w->group / 32), bb = qwhip_view_block_bytes(w);
-    // the batched form keeps one scaling factor per activation row (at most 65535 floats) at the head of the stream's
+    // the batched form keeps one scaling factor per activation row (at most 65535 floats) and the planes of its K ranges in the stream's
     // partial-sum scratch: launches on a stream are ordered, and nothing else of this call uses the scratch
     float* row_down = s->scratch ? (float*)(s->scratch + QWHIP_STREAM_COUNTER_BYTES) : nullptr;
-    const bool batched = m >= 32u && qw_f32_gemm(s->stream, w, fmt, gshift, bb, row_bytes, x, m, epi, scale, y, row_down);
+    const uint64_t room = s->scratch ? s->scratch_bytes - QWHIP_STREAM_COUNTER_BYTES - QWHIP_STREAM_XROT_BYTES - s->scratch_reserved : 0u;
+    const bool batched = m >= 32u && qw_f32_gemm(s->stream, w, fmt, gshift, bb, row_bytes, x, m, epi, scale, y, row_down, room);
     if (batched) QWHIP_TRY_HIP(hipGetLastError());
     for (uint32_t m0 = 0; !batched && m0 < m; m0 += per) {
         const uint32_t mm = min(per, m - m0);
