@@ -194,10 +194,10 @@ qwhip_status qwhip_dequant_f16(qwhip_stream_t s, const qwhip_weight_view* w, voi
  * Sources/QWMetal/include/qw_dequant_multi.metalh:205-208); the others contract the f16 weights of qwhip_dequant_f16.
  * flags: QWHIP_X_PREROTATED; bits 8..11 pick one kernel for tuning and tests (0 = automatic, 1 = half-wave dot2,
  * 2 = MFMA streamer, 3 = DMA streamer, 4 = column-stationary HQ4 kernel, 5 = column-stationary MFMA kernel,
- * 6 = column-stationary dot2 kernel, 7 = 4x4x4-block MFMA kernel, 8 = transposing MFMA kernel, 9 = split-K MFMA kernel; a
- * kernel that does not take the shape returns QWHIP_E_BAD_GEOMETRY); bits 12..15 its tuning code (bits 12..17 for the
+ * 6 = column-stationary dot2 kernel, 7 = 4x4x4-block MFMA kernel, 8 = transposing MFMA kernel, 9 = split-K MFMA kernel,
+ * 10 = row-tile MFMA kernel; a kernel that does not take the shape returns QWHIP_E_BAD_GEOMETRY); bits 12..15 its tuning code (bits 12..17 for the
  * column-stationary HQ4 kernel: window form, grid scale, row sets; bits 12..18 for the
- * split-K kernel).  The split-K kernel (automatic for 4-bit banks with k >= 8192 and m >= 6) keeps its partial sums in
+ * split-K kernel).  The split-K kernel and the row-tile kernel on rows past 6144 columns keep their partial sums in
  * the stream's scratch: calls on one stream are ordered; calls on different streams do not share it. */
 qwhip_status qwhip_gemv(qwhip_stream_t s, const qwhip_weight_view* w, const void* x, uint32_t x_dtype,
                         uint32_t m, uint32_t flags, void* y16, float* y32);
@@ -210,8 +210,8 @@ qwhip_status qwhip_gemv(qwhip_stream_t s, const qwhip_weight_view* w, const void
  * rotation is a second, small launch over fp32 gated values in the stream's scratch.  Without it the call is 2-3 us shorter
  * (20.7 against 23.5 us on 2 x 17408 x 5120, HQ4_G32_M5): a dense MLP decode step is fastest as this call with rotate_out = 0
  * followed by qwhip_gemv on the down bank without QWHIP_X_PREROTATED, whose fused rotation costs nothing at one row.
- * Two to sixteen rows run qwhip_gemv over the whole bank into an fp32 image in the stream's scratch and qwhip_swiglu_fwht
- * over that (calls on one stream are ordered; calls on different streams do not share the scratch).
+ * Two to sixteen f16 rows in the basis run one launch of the row-tile kernel where its whole units divide well, the others qwhip_gemv
+ * over the whole bank into an fp32 image in the stream's scratch and qwhip_swiglu_fwht over that, the same bits (calls on one stream are ordered; calls on different streams do not share the scratch).
  * flags bits 8..11 (tests): 2 = the general kernel, 3 = HQ4_G32_M5 on the MoE decode kernel. */
 qwhip_status qwhip_gemv_silu_pair(qwhip_stream_t s, const qwhip_weight_view* w, const void* x, uint32_t x_dtype,
                                   uint32_t m, uint32_t flags, uint32_t rotate_out, void* act16);
@@ -225,7 +225,8 @@ qwhip_status qwhip_gemv_silu_pair(qwhip_stream_t s, const qwhip_weight_view* w, 
  * epi: 0 none, 1 silu(y / scale), 2 sigmoid(y), 3 silu(y / scale) followed by the FWHT-32 over each 32 consecutive outputs
  * (a last partial group is padded with zeros).  Up to 31 rows: eight activation rows share one pass over the bank, all
  * arithmetic in fp32, a row's bits whatever the row count.  From 32 rows on (where the reference switches to its batched kernels) and k % 64 == 0: the
- * matrix-core form, 64 activation rows per pass over the bank; activations and weights are each split into two f16
+ * matrix-core form, 64 activation rows per pass over the bank (over K ranges, with fp32 planes in the stream's scratch, where the tiles are
+ * few); activations and weights are each split into two f16
  * numbers (22 bits together) and three products are accumulated in fp32 - the same 2e-5 bar.  Every activation row is
  * scaled by a power of two into the f16 range before its split and back at the store (one small launch into the
  * stream's scratch), so any finite fp32 row is taken at every row count. */
