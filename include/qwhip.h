@@ -195,8 +195,8 @@ qwhip_status qwhip_dequant_f16(qwhip_stream_t s, const qwhip_weight_view* w, voi
  * flags: QWHIP_X_PREROTATED; bits 8..11 pick one kernel for tuning and tests (0 = automatic, 1 = half-wave dot2,
  * 2 = MFMA streamer, 3 = DMA streamer, 4 = column-stationary HQ4 kernel, 5 = column-stationary MFMA kernel,
  * 6 = column-stationary dot2 kernel, 7 = 4x4x4-block MFMA kernel, 8 = transposing MFMA kernel, 9 = split-K MFMA kernel,
- * 10 = row-tile MFMA kernel; a kernel that does not take the shape returns QWHIP_E_BAD_GEOMETRY); bits 12..15 its tuning code (bits 12..17 for the
- * column-stationary HQ4 kernel: window form, grid scale, row sets; bits 12..18 for the
+ * 10 = row-tile MFMA kernel; a kernel that does not take the shape returns QWHIP_E_BAD_GEOMETRY); bits 12..15 its tuning code
+ * (bits 12..17 for the column-stationary HQ4 kernel: window form, grid scale, row sets; bits 12..18 for the
  * split-K kernel).  The split-K kernel and the row-tile kernel on rows past 6144 columns keep their partial sums in
  * the stream's scratch: calls on one stream are ordered; calls on different streams do not share it. */
 qwhip_status qwhip_gemv(qwhip_stream_t s, const qwhip_weight_view* w, const void* x, uint32_t x_dtype,
@@ -210,8 +210,9 @@ qwhip_status qwhip_gemv(qwhip_stream_t s, const qwhip_weight_view* w, const void
  * rotation is a second, small launch over fp32 gated values in the stream's scratch.  Without it the call is 2-3 us shorter
  * (20.7 against 23.5 us on 2 x 17408 x 5120, HQ4_G32_M5): a dense MLP decode step is fastest as this call with rotate_out = 0
  * followed by qwhip_gemv on the down bank without QWHIP_X_PREROTATED, whose fused rotation costs nothing at one row.
- * Two to sixteen f16 rows in the basis run one launch of the row-tile kernel where its whole units divide well, the others qwhip_gemv
- * over the whole bank into an fp32 image in the stream's scratch and qwhip_swiglu_fwht over that, the same bits (calls on one stream are ordered; calls on different streams do not share the scratch).
+ * Two to sixteen f16 rows in the basis run one launch of the row-tile kernel where its whole units divide well; the others run
+ * qwhip_gemv over the whole bank into an fp32 image in the stream's scratch and qwhip_swiglu_fwht
+ * over that (calls on one stream are ordered; calls on different streams do not share the scratch).
  * flags bits 8..11 (tests): 2 = the general kernel, 3 = HQ4_G32_M5 on the MoE decode kernel. */
 qwhip_status qwhip_gemv_silu_pair(qwhip_stream_t s, const qwhip_weight_view* w, const void* x, uint32_t x_dtype,
                                   uint32_t m, uint32_t flags, uint32_t rotate_out, void* act16);
