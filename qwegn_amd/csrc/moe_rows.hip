@@ -16,7 +16,7 @@ namespace {
 
 #define QMR_FIELDS(X)                                                                                                       \
     X(const uint8_t*, bank) X(const int32_t*, tile_count) X(const int32_t*, tile_e) X(const int32_t*, tile_r)                    \
-    X(const int32_t*, expert_off) X(uint32_t, bands) X(uint32_t, nsl) X(uint32_t, gshift) X(uint32_t, bb) X(const int32_t*, gather)  \
+    X(const int32_t*, expert_off) X(uint32_t, bands) X(uint32_t, stride) X(uint32_t, nsl) X(uint32_t, gshift) X(uint32_t, bb) X(const int32_t*, gather)  \
     X(const void*, x) X(uint64_t, expert_bytes) X(uint32_t, row_bytes) X(uint32_t, N) X(uint32_t, units) X(uint32_t, K) X(uint32_t, ldx)   \
     X(uint32_t, x_bf16) X(uint32_t, flush) X(uint32_t, inter) X(uint32_t, rotate) X(void*, y) X(uint32_t, ldy) X(uint32_t, y_dtype)        \
     X(qw_act, act)
@@ -27,7 +27,9 @@ constexpr uint32_t qmr_waves(uint32_t mf, uint32_t s) { return mf * s <= 2u ? 16
 
 // blockDim.x = 64 * ceil(steps / S); dynamic LDS = the waves' images, 2 * flush * waves * MF KiB of partial tiles and, GATED, the unit's
 // sums, 4 tiles of 16 MF rows by 16 + 1.  Grid: as the direct-operand kernel's, an XCD takes a contiguous eighth of the tile list and walks
-// (entry, band) band-fastest.
+// (rows 16 MF chunk .. of an entry, entry, band) band-fastest: the chunks past the first, which most experts do not have, leave last.  One
+// workgroup for all of an entry's chunks made a busy expert the launch's time: 64 rows x top-8 of 128 experts, 2048 x 768, all tokens on the
+// same eight 98 us, now 35 (the direct-operand kernel 25), routes falling as 1 / rank 114, 80 (65), even ones 51, 50 (71).
 template <int FMT, int S, int MF, bool GATED>
 struct qw_moe_rows_kernel {
 static constexpr int kLaunchBound = 64 * qmr_waves(MF, S);
@@ -162,22 +164,18 @@ static __device__ __forceinline__ void rows(const qmr_params& p, const uint8_t* 
 
 static __device__ __forceinline__ void run(const qmr_params& p) {
     extern __shared__ __attribute__((aligned(16))) uint32_t qmr_lds[];
-    const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
+    const uint32_t xcd = blockIdx.x & 7u, chunk = (blockIdx.x >> 3) / p.stride, slot = (blockIdx.x >> 3) - chunk * p.stride;
     const uint32_t tc = (uint32_t)max(p.tile_count[0], 0), per_xcd = (tc + 7u) >> 3;
     const uint32_t ti = slot / p.bands, t = xcd * per_xcd + ti;
     if (ti >= per_xcd || t >= tc) return;
     const uint32_t e = (uint32_t)p.tile_e[t], packed = (uint32_t)p.tile_r[t];
     const uint32_t code = packed >> 24, bm = code == 1u ? 16u : code == 2u ? 32u : 64u;   // rows of the entry's tile
-    const uint32_t first = (packed & 0xFFFFFFu) * bm;                                     // row of the expert
+    if (16u * MF * chunk >= bm) return;
+    const uint32_t first = (packed & 0xFFFFFFu) * bm + 16u * MF * chunk;                  // row of the expert
     const uint32_t off = (uint32_t)p.expert_off[e], rows_e = (uint32_t)p.expert_off[e + 1] - off;
     if (first >= rows_e) return;
-    const uint32_t M = min(bm, rows_e - first);
-    const uint8_t* bank = p.bank + (uint64_t)e * p.expert_bytes;
-#pragma unroll 1
-    for (uint32_t r = 0; r < M; r += 16u * MF) {
-        if (r > 0) __syncthreads();
-        rows(p, bank, off + first + r, min(16u * MF, M - r), slot - ti * p.bands, qmr_lds);
-    }
+    const uint32_t M = min(min(16u * MF, bm - 16u * MF * chunk), rows_e - first);
+    rows(p, p.bank + (uint64_t)e * p.expert_bytes, off + first, M, slot - ti * p.bands, qmr_lds);
 }
 };
 
@@ -254,7 +252,7 @@ qmr_config qmr_choose(int fmt, const qw_gemm_params& p, uint32_t experts, bool g
 
 template <int FMT>
 hipError_t qmr_launch(hipStream_t st, const qmr_params& p, const qmr_config& c, uint32_t s, uint32_t max_tiles, bool gated) {
-    const uint32_t wgs = 8u * qwhip_cdiv(max_tiles, 8u) * c.bands;
+    const uint32_t wgs = 8u * p.stride * (4u / c.mf);
 #define QMR_GO(S, M) (gated ? qmr_go<FMT, S, M, true>(st, p, wgs, c.waves, c.lds) : qmr_go<FMT, S, M, false>(st, p, wgs, c.waves, c.lds))
     if (s == 1u) return c.mf == 1u ? QMR_GO(1, 1) : QMR_GO(1, 2);
     return c.mf == 1u ? QMR_GO(2, 1) : QMR_GO(2, 2);
@@ -282,7 +280,7 @@ bool qw_grouped_rows_takes(int fmt, const qw_gemm_params& p, uint32_t experts) {
 hipError_t qw_grouped_rows(hipStream_t st, int fmt, const qw_gemm_params& g, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt,
                            bool swiglu) {
     const qmr_config c = qmr_choose(fmt, g, experts, swiglu);
-    if (c.waves == 0u || (uint64_t)max_tiles * c.bands >= (1u << 30)) return hipErrorInvalidValue;
+    if (c.waves == 0u || (uint64_t)max_tiles * c.bands >= (1u << 28)) return hipErrorInvalidValue;
     const uint32_t s = qmr_steps(fmt, g.K);
     qmr_params p;
     p.bank = g.bank;
@@ -291,6 +289,7 @@ hipError_t qw_grouped_rows(hipStream_t st, int fmt, const qw_gemm_params& g, uin
     p.tile_r = g.tile_r;
     p.expert_off = g.expert_off;
     p.bands = c.bands;
+    p.stride = qwhip_cdiv(max_tiles, 8u) * c.bands;
     p.nsl = g.K / 32u;
     p.gshift = g.gshift;
     p.bb = g.bb;
