@@ -190,7 +190,7 @@ hipError_t qr_launch(hipStream_t st, qr_params& p, size_t part_bytes, uint32_t o
     // as few steps a wave as 16 waves (one or two steps, 128 registers) or 12 (168) hold; longer rows in K ranges
     const uint32_t steps = qwhip_cdiv(p.nsl, 4u);
     uint32_t s = steps <= 16u ? 1u : steps <= 32u ? 2u : 4u;
-    if (tune & 7u) s = max(tune & 7u, s);
+    if (tune & 7u) s = max((tune & 7u) == 3u ? 4u : min(tune & 7u, 4u), s);   // the forms there are: 1, 2 and 4
     const uint32_t spu = out ? 2u * out : 1u;
     p.units = out ? p.inter / (16u * out) : qwhip_cdiv(p.N, 16u);
     p.nkr = qwhip_cdiv(steps, s * (s <= 2u ? 16u : 12u));
@@ -239,7 +239,7 @@ hipError_t qr_launch(hipStream_t st, qr_params& p, size_t part_bytes, uint32_t o
 // Tries the row-tile kernel for a validated call with m = 1..16 rows already in the container's basis; false when the shape is outside
 // its envelope.  fmt: QW_FMT_* (the codes of qw_slice.h).  f16w: contract the exact f16 weights (HQ4_G32_M5, 4- and 8-bit streams).
 // inter > 0: the bank is gate|up, y16 the gated activations [m][inter], with `rotate_out` in the rotated basis.
-// `tune` (0 = automatic): bits 0..2 steps a wave at least / row tiles a workgroup on long rows, bits 3.. workgroups a unit / waves / 4.
+// `tune` (0 = automatic): bits 0..2 steps a wave at least (3 and more: 4), bits 3..4 workgroups a unit.
 bool qw_rows_gemv(qwhip_stream_t s, const qwhip_weight_view* w, int fmt, uint32_t gshift, uint32_t bb, uint64_t row_bytes, const void* x,
                   uint32_t x_dtype, uint32_t m, bool f16w, void* y16, float* y32, uint32_t inter, bool rotate_out, uint32_t tune, hipError_t* err) {
     if (m == 0u || m > 16u || ((uintptr_t)x & 15u) != 0) return false;

@@ -291,6 +291,14 @@ def test_gemv_row_tile_kernel(dev, fmt, n, k, m, xdtype):
     assert qo.normalized_error(g16, ref) <= TOL
 
 
+@pytest.mark.parametrize("tune", range(1, 8))
+@pytest.mark.parametrize("k", [640, 2560, 5120])
+def test_gemv_row_tile_kernel_steps_codes(dev, k, tune):
+    """Any code for the steps a wave contracts every column (5 steps, 20 and 40 of 128 columns)."""
+    _, g32, _ = _run_gemv(dev, "hq4_g32_m5", 100, k, 8, prerot=True, seed=5, variant=10, rt=tune)
+    assert qo.normalized_error(g32, _affine_ref("hq4_g32_m5", 100, k, 8, 5, "f16")) <= 2e-6
+
+
 @pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq8_g64", "hq3_g32", "aq6_g128"])
 @pytest.mark.parametrize("m", [5, 16])
 def test_gemv_row_tile_kernel_keeps_an_infinity_in_its_row(dev, fmt, m):
