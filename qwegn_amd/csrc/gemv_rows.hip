@@ -218,7 +218,7 @@ hipError_t qr_launch(hipStream_t st, qr_params& p, size_t part_bytes, uint32_t o
         if ((longer + plain * tiles) * p.K > 5500.0f) return hipErrorNotSupported;
     }
     uint32_t per_cu = cus / 256u;
-    if ((tune >> 3) & 3u) per_cu = (tune >> 3) & 3u;
+    if ((tune >> 3) & 3u) per_cu = min((tune >> 3) & 3u, most / (image + part));   // as many as LDS holds
     const uint32_t bands = min(p.units, 256u * per_cu / p.nkr), wgs = bands * p.nkr;
     p.flush = out ? 1u : max(1u, min(min(4u, qwhip_cdiv(p.units, bands)), (most / per_cu - image) / part));
     const size_t lds = (size_t)image + p.flush * part;

@@ -299,6 +299,22 @@ def test_gemv_row_tile_kernel_steps_codes(dev, k, tune):
     assert qo.normalized_error(g32, _affine_ref("hq4_g32_m5", 100, k, 8, 5, "f16")) <= 2e-6
 
 
+@pytest.mark.parametrize("tune", [0x08, 0x10, 0x18])
+def test_gemv_row_tile_kernel_workgroups_code(dev, tune):
+    """The code for the workgroups a unit: the grid alone changes, also where LDS holds fewer (twelve waves, several tiles each)."""
+    n, k, m = 64 * 577, 6144, 5
+    bank = dev.put(np.tile(H.make_bank("hq4_g32_m5", 64, k, 3)[0].reshape(-1), 577))
+    xb, y = dev.put(H.make_x(m, k, 4).astype(np.float16)), dev.alloc(m * n * 4)
+    view, outs = H.view_of(dev, bank, "hq4_g32_m5", n, k), []
+    for code in (0, tune):
+        qwhip.check(dev.lib.qwhip_gemv(dev.stream.handle, C.byref(view), xb.ptr, qwhip.F16, m, qwhip.X_PREROTATED | (10 << 8) | (code << 12), None, y.ptr))
+        dev.stream.sync()
+        outs.append(y.download(np.uint32, (m, n)))
+    for b in (bank, xb, y):
+        b.free()
+    assert np.array_equal(*outs) and np.array_equal(outs[0][:, :64], outs[0][:, -64:])
+
+
 @pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq8_g64", "hq3_g32", "aq6_g128"])
 @pytest.mark.parametrize("m", [5, 16])
 def test_gemv_row_tile_kernel_keeps_an_infinity_in_its_row(dev, fmt, m):
