@@ -197,7 +197,8 @@ qwhip_status qwhip_dequant_f16(qwhip_stream_t s, const qwhip_weight_view* w, voi
  * 6 = column-stationary dot2 kernel, 7 = 4x4x4-block MFMA kernel, 8 = transposing MFMA kernel, 9 = split-K MFMA kernel,
  * 10 = row-tile MFMA kernel; a kernel that does not take the shape returns QWHIP_E_BAD_GEOMETRY); bits 12..15 its tuning code
  * (bits 12..17 for the column-stationary HQ4 kernel: window form, grid scale, row sets; bits 12..18 for the
- * split-K kernel).  The split-K kernel and the row-tile kernel on rows past 6144 columns keep their partial sums in
+ * split-K kernel; bits 12..16 for the row-tile kernel, which reads them only where it is named).
+ * The split-K kernel and the row-tile kernel on rows past 6144 columns keep their partial sums in
  * the stream's scratch: calls on one stream are ordered; calls on different streams do not share it. */
 qwhip_status qwhip_gemv(qwhip_stream_t s, const qwhip_weight_view* w, const void* x, uint32_t x_dtype,
                         uint32_t m, uint32_t flags, void* y16, float* y32);

@@ -1051,7 +1051,7 @@ static bool qw_rows_f16_weights(qwhip_stream_t s, const qwhip_weight_view* w, in
 // 4 = column-stationary persistent kernel, 5 = column-stationary MFMA kernel, 6 = column-stationary small-M kernel,
 // 7 = 4x4x4-block MFMA kernel, 8 = transposing MFMA kernel, 9 = split-K MFMA kernel, 10 = row-tile kernel);
 // bits 12..15: row tiles per wave for the direct-load mfma kernel / K-split of the streamer / tuning code of the
-// column-stationary kernel (0 = automatic); bits 12..18: tuning code of the split-K and the row-tile kernel.
+// column-stationary kernel (0 = automatic); bits 12..18: tuning code of the split-K kernel, 12..16 of the row-tile kernel where it is named.
 // `token` (head door only): where the column-stationary kernel's fused fold leaves the argmax; *folded tells whether it ran
 static qwhip_status qw_gemv_impl(qwhip_stream_t s, const qwhip_weight_view* w, const void* x, uint32_t x_dtype, uint32_t m,
                                  uint32_t flags, void* y16, float* y32, int32_t* token, bool* folded) {
@@ -1142,7 +1142,7 @@ static qwhip_status qw_gemv_impl(qwhip_stream_t s, const qwhip_weight_view* w, c
         const bool known = variant == 10 || fmt < QW_FMT_B2 ||
                            qw_colx_gemv(s->stream, w, fmt, a.gshift, a.bb, a.row_bytes, x, x_dtype, min(m, 8u), false, y16, y32, rt, nullptr);
         if (!rotate && m >= 2 && known &&
-            qw_rows_gemv(s, w, fmt, a.gshift, a.bb, a.row_bytes, x, x_dtype, m, f16w, y16, y32, 0, false, (flags >> 12) & 0x7Fu, &e)) {
+            qw_rows_gemv(s, w, fmt, a.gshift, a.bb, a.row_bytes, x, x_dtype, m, f16w, y16, y32, 0, false, variant == 10 ? (flags >> 12) & 0x1Fu : 0u, &e)) {
             QWHIP_TRY_HIP(e);
             return QWHIP_OK;
         }

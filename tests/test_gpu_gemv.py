@@ -315,6 +315,13 @@ def test_gemv_row_tile_kernel_workgroups_code(dev, tune):
     assert np.array_equal(*outs) and np.array_equal(outs[0][:, :64], outs[0][:, -64:])
 
 
+def test_gemv_row_tile_kernel_reads_its_code_where_it_is_named(dev):
+    """Tuning bits without an override leave the automatic choice's sums alone; with the override another split of the columns over the
+    waves adds in another order."""
+    runs = [_run_gemv(dev, "hq4_g32_m5", 64, 1024, 8, prerot=True, seed=5, variant=v, rt=rt)[1] for v, rt in ((0, 0), (0, 2), (0, 4), (10, 0), (10, 4))]
+    assert all(np.array_equal(runs[0], r) for r in runs[1:4]) and not np.array_equal(runs[0], runs[4])
+
+
 @pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq8_g64", "hq3_g32", "aq6_g128"])
 @pytest.mark.parametrize("m", [5, 16])
 def test_gemv_row_tile_kernel_keeps_an_infinity_in_its_row(dev, fmt, m):
