@@ -194,6 +194,7 @@ hipError_t qr_launch(hipStream_t st, qr_params& p, size_t part_bytes, uint32_t o
     const uint32_t spu = out ? 2u * out : 1u;
     p.units = out ? p.inter / (16u * out) : qwhip_cdiv(p.N, 16u);
     p.nkr = qwhip_cdiv(steps, s * (s <= 2u ? 16u : 12u));
+    if (p.nkr > (out ? 1u : 254u)) return hipErrorNotSupported;   // at most 256 ranges (1560576 columns): a workgroup each at least
     if (p.nkr > 1u) {   // of the least number of ranges and the two after it, the one whose workgroups walk the fewest wave steps
         uint32_t best = ~0u, least = p.nkr;
         for (uint32_t k = least; k < least + 3u; ++k) {
@@ -203,7 +204,7 @@ hipError_t qr_launch(hipStream_t st, qr_params& p, size_t part_bytes, uint32_t o
     }
     const uint32_t waves = qwhip_cdiv(steps, s * p.nkr);
     p.nkr = qwhip_cdiv(steps, s * waves);
-    if (p.nkr > 1u && (out || (uint64_t)p.nkr * p.M * p.units * 64u > part_bytes)) return hipErrorNotSupported;
+    if (p.nkr > 1u && (uint64_t)p.nkr * p.M * p.units * 64u > part_bytes) return hipErrorNotSupported;
     const uint32_t image = waves * 4u * (s == 1u ? qr_image<FMT, 1>::DWORDS : s == 2u ? qr_image<FMT, 2>::DWORDS : qr_image<FMT, 4>::DWORDS);
     const uint32_t part = 2u * spu * waves * 1024u, most = 160u * 1024u;   // bytes of the images, of the partial tiles of a unit
     if (image + part > most) return hipErrorNotSupported;

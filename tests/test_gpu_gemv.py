@@ -346,6 +346,21 @@ def test_gemv_row_tile_kernel_keeps_an_infinity_in_its_row(dev, fmt, m):
     assert not np.isfinite(outs[1][2]).any()
 
 
+def test_gemv_row_tile_kernel_longest_rows(dev):
+    """254 ranges of 6144 columns and their 1.56 million columns; one step more is refused on the host, whose range count would divide a
+    unit count of zero."""
+    k = 254 * 6144
+    g32, ref = _run_gemv(dev, "hq4_g32_m5", 16, k, 2, prerot=True, seed=5, variant=10)[1:]
+    assert qo.normalized_error(g32, ref) <= TOL      # the codes against their f16 weights
+    bank, xb, y = dev.alloc(16 * (k + 128) // 32 * 20), dev.alloc(2 * (k + 128) * 2), dev.alloc(2 * 16 * 4)
+    v = dev.view(bank, 16, k + 128, qwhip.KIND_HQ4_G32_M5)
+    assert dev.lib.qwhip_gemv(dev.stream.handle, C.byref(v), xb.ptr, qwhip.F16, 2, qwhip.X_PREROTATED | (10 << 8), None, y.ptr) == qwhip.E_BAD_GEOMETRY
+    v = dev.view(bank, 1, 16 * (k + 128), qwhip.KIND_HQ4_G32_M5)
+    assert dev.lib.qwhip_gemv(dev.stream.handle, C.byref(v), xb.ptr, qwhip.F16, 2, qwhip.X_PREROTATED | (10 << 8), None, y.ptr) == qwhip.E_BAD_GEOMETRY
+    for b in (bank, xb, y):
+        b.free()
+
+
 def test_gemv_row_tile_kernel_refuses_what_was_refused(dev):
     """Rows in the basis only, two to sixteen; 2-, 3- and 6-bit rows too long for the dot2 kernel are refused by the automatic choice."""
     lib, st = dev.lib, dev.stream.handle
