@@ -1038,13 +1038,15 @@ static bool qw_rows_pays(int fmt, uint32_t m, uint32_t n, uint32_t k) {
     if (n > 12288u) return false;
     return m == 4u ? k <= 2048u : fmt != QW_FMT_B4 && (m == 3u ? k <= 2048u : k <= 1024u);
 }
-// Which weights the kernels before it contracted: the exact f16 ones on the transposing (13 rows on) and the split-K kernel.
-static bool qw_rows_f16_weights(qwhip_stream_t s, const qwhip_weight_view* w, int fmt, uint32_t gshift, uint32_t bb, uint64_t row_bytes, const void* x,
-                                uint32_t x_dtype, uint32_t m) {
+// Which weights the row-tile kernel contracts, by shape alone (the plain and the gate|up door agree, whatever is in the scratch): the exact f16
+// ones at 13 rows and more, and at six and more on 4-bit rows of 8192 columns and more, as the transposing and the split-K kernel, which had
+// these calls and whose results they are; the codes elsewhere.  The split-K kernel had them where its planes, of ranges of 3072 columns,
+// fitted the partial-sum area, here beside an image of the rows: longer and taller banks were and are contracted by their codes.
+static bool qw_rows_f16_weights(int fmt, uint32_t m, uint32_t n, uint32_t k) {
     if (fmt >= QW_FMT_B2) return false;
     if (m >= 13u) return true;
-    return m >= 6u && w->k >= 8192u && fmt != QW_FMT_B8 &&
-           qw_sk_gemv(s, w, fmt, gshift, bb, row_bytes, x, x_dtype, m, nullptr, nullptr, m > 8u ? 26u : 0u, nullptr);
+    const uint64_t area = QWHIP_STREAM_SCRATCH_BYTES - QWHIP_STREAM_COUNTER_BYTES - QWHIP_STREAM_XROT_BYTES;
+    return m >= 6u && k >= 8192u && k % 128u == 0 && fmt != QW_FMT_B8 && (1u + (uint64_t)qwhip_cdiv(k, 3072u)) * m * qwhip_cdiv(n, 16u) * 64u <= area;
 }
 
 // flags bits 8..11: kernel override for tuning and tests (0 = automatic, 1 = dot2, 2 = direct-load mfma, 3 = DMA streamer,
@@ -1137,7 +1139,7 @@ static qwhip_status qw_gemv_impl(qwhip_stream_t s, const qwhip_weight_view* w, c
     // before it did (13 rows on; six on long rows that the split-K kernel takes), and the codes themselves, scaled in fp32, elsewhere.
     if (variant == 10 || (variant == 0 && !rotate && qw_rows_pays(fmt, m, w->n, w->k))) {
         hipError_t e = hipSuccess;
-        const bool f16w = qw_rows_f16_weights(s, w, fmt, a.gshift, a.bb, a.row_bytes, x, x_dtype, m);
+        const bool f16w = qw_rows_f16_weights(fmt, m, w->n, w->k);
         // (rows too long for the dot2 kernel of the 2-, 3- and 6-bit streams stay refused)
         const bool known = variant == 10 || fmt < QW_FMT_B2 ||
                            qw_colx_gemv(s->stream, w, fmt, a.gshift, a.bb, a.row_bytes, x, x_dtype, min(m, 8u), false, y16, y32, rt, nullptr);
@@ -1221,7 +1223,7 @@ static qwhip_status qw_gemv_impl(qwhip_stream_t s, const qwhip_weight_view* w, c
     // split-K matrix-core kernel: what the row-tile kernel leaves (banks of 4 GiB and more, partial sums past the stream's scratch) on
     // long rows, N = 5120, K = 17408, HQ4_G64: 18.7 / 18.7 / 20.7 us at m = 6 / 8 / 16 against 21.2 / 23.2 / 34.9 for the kernels below, and
     // 13..16 rows on an 8-bit stream of short rows, four waves a workgroup, four groups in flight, the image in 128 KiB (tuning code 60).
-    const bool sk_long = !rotate && m >= 6 && w->k >= 8192 && fmt != QW_FMT_B8;
+    const bool sk_long = !rotate && w->k >= 8192 && fmt != QW_FMT_B8 && qw_rows_f16_weights(fmt, m, w->n, w->k);
     const bool sk_wide8 = !rotate && m >= 13 && w->k < 8192 && fmt == QW_FMT_B8;
     if (variant == 9 || (variant == 0 && (sk_long || sk_wide8))) {
         hipError_t e = hipSuccess;
@@ -1329,7 +1331,7 @@ extern "C" qwhip_status qwhip_gemv_silu_pair(qwhip_stream_t s, const qwhip_weigh
             hipError_t e = hipSuccess;
             const uint32_t gshift = log2_u32(w->group / 32), bb = qwhip_view_block_bytes(w);
             const uint64_t row_bytes = qwhip_view_row_bytes(w);
-            const bool f16w = qw_rows_f16_weights(s, w, fmt, gshift, bb, row_bytes, x, x_dtype, m);
+            const bool f16w = qw_rows_f16_weights(fmt, m, w->n, w->k);
             if (qw_rows_gemv(s, w, fmt, gshift, bb, row_bytes, x, x_dtype, m, f16w, act16, nullptr, inter, rot_out, 0, &e)) {
                 QWHIP_TRY_HIP(e);
                 return QWHIP_OK;

@@ -198,6 +198,7 @@ hipError_t qr_launch(hipStream_t st, qr_params& p, size_t part_bytes, uint32_t o
     if (p.nkr > 1u) {   // of the least number of ranges and the two after it, the one whose workgroups walk the fewest wave steps
         uint32_t best = ~0u, least = p.nkr;
         for (uint32_t k = least; k < least + 3u; ++k) {
+            if (k > least && (uint64_t)k * p.M * p.units * 64u > part_bytes) break;
             const uint32_t cost = qwhip_cdiv(p.units, 256u / k) * qwhip_cdiv(steps, s * k);
             if (cost < best) best = cost, p.nkr = k;
         }

@@ -346,6 +346,25 @@ def test_gemv_row_tile_kernel_keeps_an_infinity_in_its_row(dev, fmt, m):
     assert not np.isfinite(outs[1][2]).any()
 
 
+@pytest.mark.parametrize("m", [8, 12])
+def test_gemv_row_tile_kernel_weights_follow_the_shape(dev, m):
+    """The plain door, whose planes have all of the partial-sum area, and the gate|up door, whose image takes a part of it, contract the
+    same weights: the bits of one are those of the other and the activation pass."""
+    reps, k = 8 * 1094 // m, 8192
+    n = 64 * reps
+    bank = dev.put(np.tile(H.make_bank("hq4_g32_m5", 64, k, 3)[0].reshape(-1), reps))
+    xb, gu, a1, a2 = dev.put(H.make_x(m, k, 4).astype(np.float16)), dev.alloc(m * n * 4), dev.alloc(m * n), dev.alloc(m * n)
+    view, lib, st, fl = H.view_of(dev, bank, "hq4_g32_m5", n, k), dev.lib, dev.stream.handle, qwhip.X_PREROTATED
+    qwhip.check(lib.qwhip_gemv(st, C.byref(view), xb.ptr, qwhip.F16, m, fl, None, gu.ptr))
+    qwhip.check(lib.qwhip_swiglu_fwht(st, gu.ptr, qwhip.F32, a2.ptr, m, n // 2, 0))
+    qwhip.check(lib.qwhip_gemv_silu_pair(st, C.byref(view), xb.ptr, qwhip.F16, m, fl, 0, a1.ptr))
+    dev.stream.sync()
+    one, two = a1.download(np.uint16, (m, n // 2)), a2.download(np.uint16, (m, n // 2))
+    for b in (bank, xb, gu, a1, a2):
+        b.free()
+    assert np.array_equal(one, two)
+
+
 def test_gemv_row_tile_kernel_longest_rows(dev):
     """254 ranges of 6144 columns and their 1.56 million columns; one step more is refused on the host, whose range count would divide a
     unit count of zero."""
