@@ -1805,8 +1805,9 @@ extern "C" qwhip_status qwhip_moe_grouped_gemm(qwhip_stream_t s, const qwhip_wei
     hipError_t e;
     p.tiles_n = grid.x;
     if (qw_grouped_direct_takes(fmt, p, experts) && (y_dtype == QWHIP_F32 || (ldy % 8u == 0 && ((uintptr_t)y & 15u) == 0))) {
-        QWHIP_TRY_HIP(qw_grouped_rows_takes(fmt, p, experts) ? qw_grouped_rows(s->stream, fmt, p, max_tiles, experts, x_dtype, y_dtype, false)
-                                                             : qw_grouped_direct(s->stream, fmt, p, max_tiles, experts, x_dtype, y_dtype, false));
+        if (!qw_grouped_rows(s->stream, fmt, p, max_tiles, experts, x_dtype, y_dtype, false, &e))
+            e = qw_grouped_direct(s->stream, fmt, p, max_tiles, experts, x_dtype, y_dtype, false);
+        QWHIP_TRY_HIP(e);
         return QWHIP_OK;
     }
     QG_FOR_FMT(fmt, e, (launch_grouped_xy<F>(s->stream, p, grid, x_dtype, y_dtype)))
@@ -1865,8 +1866,10 @@ extern "C" qwhip_status qwhip_moe_grouped_gemm_swiglu(qwhip_stream_t s, const qw
     p.act = s->dev->act;
     p.tiles_n = qwhip_cdiv(inter, 128u);
     if (qw_grouped_direct_takes(fmt, p, experts)) {
-        QWHIP_TRY_HIP(qw_grouped_rows_takes(fmt, p, experts) ? qw_grouped_rows(s->stream, fmt, p, max_tiles, experts, x_dtype, QWHIP_F16, true)
-                                                             : qw_grouped_direct(s->stream, fmt, p, max_tiles, experts, x_dtype, QWHIP_F16, true));
+        hipError_t e;
+        if (!qw_grouped_rows(s->stream, fmt, p, max_tiles, experts, x_dtype, QWHIP_F16, true, &e))
+            e = qw_grouped_direct(s->stream, fmt, p, max_tiles, experts, x_dtype, QWHIP_F16, true);
+        QWHIP_TRY_HIP(e);
         return QWHIP_OK;
     }
     const dim3 grid(8u * qwhip_cdiv(max_tiles, 8u) * p.tiles_n);   // XCD-aware one-dimensional grid over (tile, column tile)

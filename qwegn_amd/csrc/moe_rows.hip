@@ -16,28 +16,35 @@ namespace {
 
 #define QMR_FIELDS(X)                                                                                                       \
     X(const uint8_t*, bank) X(const int32_t*, tile_count) X(const int32_t*, tile_e) X(const int32_t*, tile_r)                    \
-    X(const int32_t*, expert_off) X(uint32_t, bands) X(uint32_t, stride) X(uint32_t, nsl) X(uint32_t, gshift) X(uint32_t, bb) X(const int32_t*, gather)  \
-    X(const void*, x) X(uint64_t, expert_bytes) X(uint32_t, row_bytes) X(uint32_t, N) X(uint32_t, units) X(uint32_t, K) X(uint32_t, ldx)   \
+    X(const int32_t*, expert_off) X(uint32_t, max_tiles) X(uint32_t, wgs) X(uint32_t, units) X(uint32_t, nsl) X(uint32_t, gshift) X(uint32_t, bb) X(const int32_t*, gather)  \
+    X(const void*, x) X(uint64_t, expert_bytes) X(uint32_t, row_bytes) X(uint32_t, N) X(uint32_t, K) X(uint32_t, ldx)   \
     X(uint32_t, x_bf16) X(uint32_t, flush) X(uint32_t, inter) X(uint32_t, rotate) X(void*, y) X(uint32_t, ldy) X(uint32_t, y_dtype)        \
     X(qw_act, act)
 QW_ARG_BLOCK(qmr_params, QMR_FIELDS)
+
+constexpr uint32_t QMR_LISTS = 12;                  // 64 entries of the tile list each
+constexpr uint32_t QMR_LDS = 160u * 1024u - 512u;   // dynamic LDS of a unit, beside the items found
 
 // Waves of a workgroup, by the registers of MF fragments over S steps.
 constexpr uint32_t qmr_waves(uint32_t mf, uint32_t s) { return mf * s <= 2u ? 16u : 12u; }
 
 // blockDim.x = 64 * ceil(steps / S); dynamic LDS = the waves' images, 2 * flush * waves * MF KiB of partial tiles and, GATED, the unit's
-// sums, 4 tiles of 16 MF rows by 16 + 1.  Grid: as the direct-operand kernel's, an XCD takes a contiguous eighth of the tile list and walks
-// (rows 16 MF chunk .. of an entry, entry, band) band-fastest: the chunks past the first, which most experts do not have, leave last.  One
-// workgroup for all of an entry's chunks made a busy expert the launch's time: 64 rows x top-8 of 128 experts, 2048 x 768, all tokens on the
-// same eight 98 us, now 35 (the direct-operand kernel 25), routes falling as 1 / rank 114, 80 (65), even ones 51, 50 (71).
+// sums, 4 tiles of 16 MF rows by 16 + 1.
+// Grid: every 16 MF rows of an entry are a chunk, and the chunks that there are, counted here, share the launch's workgroups, each in as many
+// bands as come out even; an XCD takes a contiguous eighth of (entry, band, chunk), so that the chunks of a busy expert run side by side under
+// one L2 and no XCD has more than another however the routes fall.  (With the host's bands, a grid for four chunks of every entry and eighths
+// of the list, the late chunks were a round of their own behind the empty workgroups, and the XCD of the busy experts had most of them.)
+// 64 rows x top-8 of 128 experts, 2048 x 768, gate|up and down, us: even routes 51 and 29 (the direct-operand kernel 70 and 42), routes
+// falling as 1 / rank 50 and 28 (before 77 and 44, direct-operand 65 and 38), all tokens on the same eight 15 and 10 (35 and 19; 25 and 12).
+// Finding its chunk costs a workgroup 0.4 us: 22 rows x top-2 of 8 experts, 1024 x 384, 5.2 -> 5.6.
 template <int FMT, int S, int MF, bool GATED>
 struct qw_moe_rows_kernel {
 static constexpr int kLaunchBound = 64 * qmr_waves(MF, S);
 
-static __device__ __forceinline__ void rows(const qmr_params& p, const uint8_t* bank, uint32_t m0, uint32_t M, uint32_t band, uint32_t* lds) {
+static __device__ __forceinline__ void rows(const qmr_params& p, const uint8_t* bank, uint32_t m0, uint32_t M, uint32_t band, uint32_t G, uint32_t* lds) {
     using im = qr_image<FMT, S>;
     constexpr uint32_t SPU = GATED ? 4u : 1u, RPL = 16u / S, ROWS = 16u * MF;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, W = blockDim.x >> 6, G = p.bands;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, W = blockDim.x >> 6;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t n = lane & 15u, c = lane >> 4;             // contraction role
     const uint32_t lb = lane / RPL, lj = lane & (RPL - 1u);   // load role: slice lb of the wave's, row RPL q + lj of the tile
@@ -162,20 +169,68 @@ static __device__ __forceinline__ void rows(const qmr_params& p, const uint8_t* 
     }
 }
 
+// The workgroup's entry, chunk of rows and band, and the bands of this launch.  Every wave finds them: no barrier in front of the bank's loads.
+struct item { uint32_t e, packed, chunk, band, bands, valid; };
+static __device__ __forceinline__ item find(const qmr_params& p, uint32_t lane) {
+    const uint32_t tc = min((uint32_t)max(p.tile_count[0], 0), p.max_tiles);   // the lists end there
+    uint32_t te[QMR_LISTS], tr[QMR_LISTS];
+#pragma unroll
+    for (uint32_t j = 0; j < QMR_LISTS; ++j) {
+        if (64u * j >= tc) break;
+        const uint32_t t = min(64u * j + lane, tc - 1u);
+        te[j] = (uint32_t)p.tile_e[t];
+        tr[j] = (uint32_t)p.tile_r[t];
+    }
+    // chunks of an entry of 16, 32 or 64 rows: 1, 2 or 4 (MF = 1), 1, 1 or 2
+    auto count = [&](uint32_t j) { return 64u * j + lane >= tc ? 0u : tr[j] >> 24 == 1u ? 1u : tr[j] >> 24 == 2u ? 2u / MF : 4u / MF; };
+    uint32_t total = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < QMR_LISTS; ++j) {
+        if (64u * j >= tc) break;
+        const uint32_t n = count(j);
+        total += __popcll(__ballot(n > 0u)) + __popcll(__ballot(n > 1u)) + 2u * __popcll(__ballot(n > 2u));
+    }
+    item it = {};
+    if (total == 0u) return it;
+    const uint32_t bands = min(max(p.wgs / total, 1u), p.units);
+    const uint32_t items = total * bands, per_xcd = (items + 7u) >> 3, at = blockIdx.x >> 3, i = (blockIdx.x & 7u) * per_xcd + at, q = i / bands;
+    if (at >= per_xcd || i >= items) return it;
+    uint32_t before = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < QMR_LISTS; ++j) {
+        if (64u * j >= tc) break;
+        const uint32_t n = count(j);
+        const unsigned long long b0 = __ballot(n > 0u), b1 = __ballot(n > 1u), b2 = __ballot(n > 2u);
+        auto lower = [](unsigned long long b) { return __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u)); };
+        const uint32_t mine = before + lower(b0) + lower(b1) + 2u * lower(b2);
+        const unsigned long long hit = __ballot(q >= mine && q < mine + n);
+        if (hit != 0ull) {
+            const uint32_t l = (uint32_t)__builtin_ctzll(hit);
+            const uint32_t local = i - __builtin_amdgcn_readlane(mine, l) * bands, chunks = __builtin_amdgcn_readlane(n, l);
+            it.band = local >> (chunks >> 1);   // 1, 2 or 4
+            it.chunk = local & (chunks - 1u);
+            it.e = __builtin_amdgcn_readlane(te[j], l);
+            it.packed = __builtin_amdgcn_readlane(tr[j], l);
+            it.bands = bands;
+            it.valid = 1u;
+            return it;
+        }
+        before += __popcll(b0) + __popcll(b1) + 2u * __popcll(b2);
+    }
+    return it;
+}
+
 static __device__ __forceinline__ void run(const qmr_params& p) {
     extern __shared__ __attribute__((aligned(16))) uint32_t qmr_lds[];
-    const uint32_t xcd = blockIdx.x & 7u, chunk = (blockIdx.x >> 3) / p.stride, slot = (blockIdx.x >> 3) - chunk * p.stride;
-    const uint32_t tc = (uint32_t)max(p.tile_count[0], 0), per_xcd = (tc + 7u) >> 3;
-    const uint32_t ti = slot / p.bands, t = xcd * per_xcd + ti;
-    if (ti >= per_xcd || t >= tc) return;
-    const uint32_t e = (uint32_t)p.tile_e[t], packed = (uint32_t)p.tile_r[t];
+    const item it = find(p, threadIdx.x & 63u);
+    if (it.valid == 0u) return;
+    const uint32_t e = it.e, packed = it.packed, chunk = it.chunk;
     const uint32_t code = packed >> 24, bm = code == 1u ? 16u : code == 2u ? 32u : 64u;   // rows of the entry's tile
-    if (16u * MF * chunk >= bm) return;
     const uint32_t first = (packed & 0xFFFFFFu) * bm + 16u * MF * chunk;                  // row of the expert
     const uint32_t off = (uint32_t)p.expert_off[e], rows_e = (uint32_t)p.expert_off[e + 1] - off;
     if (first >= rows_e) return;
     const uint32_t M = min(min(16u * MF, bm - 16u * MF * chunk), rows_e - first);
-    rows(p, p.bank + (uint64_t)e * p.expert_bytes, off + first, M, slot - ti * p.bands, qmr_lds);
+    rows(p, p.bank + (uint64_t)e * p.expert_bytes, off + first, M, it.band, it.bands, qmr_lds);
 }
 };
 
@@ -184,7 +239,7 @@ hipError_t qmr_go(hipStream_t st, const qmr_params& p, uint32_t wgs, uint32_t wa
     using K = qw_moe_rows_kernel<FMT, S, MF, GATED>;
     static std::atomic<bool> attr_done{false};   // per instantiation
     if (!attr_done.load(std::memory_order_acquire)) {
-        const hipError_t e = hipFuncSetAttribute(qw_scalar_kernel_ptr<K>((const qmr_params*)nullptr), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        const hipError_t e = hipFuncSetAttribute(qw_scalar_kernel_ptr<K>((const qmr_params*)nullptr), hipFuncAttributeMaxDynamicSharedMemorySize, (int)QMR_LDS);
         if (e != hipSuccess) return e;
         attr_done.store(true, std::memory_order_release);
     }
@@ -212,38 +267,46 @@ uint32_t qmr_steps(int fmt, uint32_t k) {
 }
 
 struct qmr_config {
-    uint32_t waves, mf, units, bands, flush, lds;   // waves = 0: none fits
+    uint32_t waves, mf, units, wgs, flush, lds;   // waves = 0: none fits
     double us;
 };
-// The launch with the lowest price, us: fragments of rows and bands of an expert's row tiles.  A launch 4.2; then rounds of workgroups,
-// one's start 1.5, its activations and row tiles for every 16 mf rows of its expert (rows an expert: Poisson), a tile costing 0.54, its
-// waves' sums and every step's unpacking and products on a SIMD; no faster than 5.7 TB/s of the experts that have rows.  Fitted to the
-// choice among 16 forms each of 122 problems (8 .. 256 experts, up to 8 rows each, 12 containers): 0.71 of the direct-operand kernel's
-// time where the best of the forms took 0.69.
+// The launch with the lowest price, us: fragments of rows, and workgroups for the bands of row tiles of all chunks together (find).  A launch
+// 4.2; then rounds of workgroups, one's start 1.5, its activations and row tiles, a tile costing 0.54, its waves' sums and every step's
+// unpacking and products on a SIMD; no faster than 5.7 TB/s of the experts that have rows.  The chunks are those of even routes (rows an
+// expert: Poisson) and a tenth more, in the mean of both prices: skewed routes leave experts without rows and give others several chunks,
+// 0.9 .. 1.13 of the even ones' number on routes falling as 1 / rank.  Over 140 layers (8 .. 256 experts, up to 24 rows each, 12 containers,
+// both kinds of routes) the form taken is 4 % slower than the best of up to ten measured ones.
 qmr_config qmr_choose(int fmt, const qw_gemm_params& p, uint32_t experts, bool gated) {
-    const uint32_t s = qmr_steps(fmt, p.K), waves = qwhip_cdiv(p.K / 128u, s), most = 160u * 1024u, units = gated ? p.inter / 32u : qwhip_cdiv(p.N, 16u);
+    const uint32_t s = qmr_steps(fmt, p.K), waves = qwhip_cdiv(p.K / 128u, s), units = gated ? p.inter / 32u : qwhip_cdiv(p.N, 16u);
     const double unpack = fmt == QG_FMT_B8 ? 1.38 : fmt == QG_FMT_B6 ? 0.9 : fmt == QG_FMT_B3 ? 2.2 : 1.0;
     const double mean = p.M / (double)experts, none = std::exp(-mean), used = experts * (1.0 - none);
     const double stream = 4.2 + used * (double)p.N * (double)p.row_bytes / 5.7e6;
+    double chunks[2] = {0.0, 0.0}, chance = none;   // of 16 and of 32 rows
+    for (uint32_t k = 1; k < 64u && (k < mean + 2.0 || chance > 1e-5); ++k) {
+        chance *= mean / k;
+        chunks[0] += chance * ((k + 15u) >> 4);
+        chunks[1] += chance * ((k + 31u) >> 5);
+    }
     qmr_config best = {};
     best.us = 1e30;
     for (uint32_t mf = 1; mf <= 2u; ++mf) {
         const uint32_t image = waves * qmr_image_bytes(fmt, s), part = 2u * waves * mf * 1024u, sums = 4u * 16u * mf * 17u * 4u;
-        if (waves > qmr_waves(mf, s) || image + part + sums > most) continue;
-        double passes = 0.0, chance = none;   // of an expert with rows
-        for (uint32_t k = 1; k < 64u; ++k) chance *= mean / k, passes += chance * qwhip_cdiv(k, 16u * mf);
-        passes /= 1.0 - none;
-        const uint32_t per_cu = max(1u, min(qmr_waves(mf, s) / waves, most / (image + part + sums)));
-        for (uint32_t bands : {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u, 24u, 32u, 48u}) {
-            if (bands > units) break;
-            const double wgs = used * bands / 256.0, side = std::min((double)per_cu, std::max(1.0, std::ceil(wgs)));
-            const uint32_t tiles = qwhip_cdiv(units, bands) * (gated ? 4u : 1u);
-            const double tile = 0.54 + 0.029 * waves * s + waves * side / 4.0 * s * (0.116 * unpack + 0.034 * mf);
-            const double rounds = std::max(1.0, std::ceil(wgs / side - 0.01));
-            const double us = std::max(stream, 4.2 + rounds * (1.5 + passes * (0.32 * s * mf + tiles * tile)));
+        if (waves > qmr_waves(mf, s) || image + part + sums > QMR_LDS) continue;
+        const uint32_t per_cu = max(1u, min(qmr_waves(mf, s) / waves, QMR_LDS / (image + part + sums)));
+        for (uint32_t i : {1u, 2u, 3u, 4u, 6u, 8u}) {   // workgroups a unit in all
+            if (i > 2u * per_cu) break;
+            double us = 0.0;
+            uint32_t tiles = 1;
+            for (double c : {experts * chunks[mf - 1u], 1.1 * experts * chunks[mf - 1u]}) {
+                const uint32_t bands = min(max(1u, (uint32_t)(256u * i / c)), units), longest = qwhip_cdiv(units, bands);
+                const double load = c * qwhip_cdiv(units, longest) / 256.0, side = std::min((double)min(per_cu, i), std::max(1.0, std::ceil(load)));
+                tiles = longest * (gated ? 4u : 1u);
+                const double tile = 0.54 + 0.029 * waves * s + waves * side / 4.0 * s * (0.116 * unpack + 0.034 * mf);
+                us += 0.5 * std::max(stream, 4.2 + std::max(1.0, std::ceil(load / side - 0.01)) * (1.5 + 0.32 * s * mf + tiles * tile));
+            }
             if (us >= best.us) continue;
-            best.waves = waves, best.mf = mf, best.units = units, best.bands = bands, best.us = us;
-            best.flush = gated ? 1u : max(1u, min(min(4u, tiles), (most / per_cu - image) / part));
+            best.waves = waves, best.mf = mf, best.units = units, best.wgs = 256u * i, best.us = us;
+            best.flush = gated ? 1u : max(1u, min(min(4u, tiles), (QMR_LDS / min(per_cu, i) - image) / part));
             best.lds = image + best.flush * part + (gated ? sums : 0u);
         }
     }
@@ -251,8 +314,8 @@ qmr_config qmr_choose(int fmt, const qw_gemm_params& p, uint32_t experts, bool g
 }
 
 template <int FMT>
-hipError_t qmr_launch(hipStream_t st, const qmr_params& p, const qmr_config& c, uint32_t s, uint32_t max_tiles, bool gated) {
-    const uint32_t wgs = 8u * p.stride * (4u / c.mf);
+hipError_t qmr_launch(hipStream_t st, const qmr_params& p, const qmr_config& c, uint32_t s, bool gated) {
+    const uint32_t wgs = max(c.wgs, 8u * qwhip_cdiv(p.max_tiles * (4u / c.mf), 8u));   // a workgroup for every chunk there can be
 #define QMR_GO(S, M) (gated ? qmr_go<FMT, S, M, true>(st, p, wgs, c.waves, c.lds) : qmr_go<FMT, S, M, false>(st, p, wgs, c.waves, c.lds))
     if (s == 1u) return c.mf == 1u ? QMR_GO(1, 1) : QMR_GO(1, 2);
     return c.mf == 1u ? QMR_GO(2, 1) : QMR_GO(2, 2);
@@ -262,25 +325,24 @@ hipError_t qmr_launch(hipStream_t st, const qmr_params& p, const qmr_config& c, 
 }  // namespace
 
 // A mean of up to eight rows an expert, at which the direct-operand kernel multiplies 32 and waits; by price against its own, the dense
-// form's (choose_direct) without ranges, which is a tenth below the grouped kernel's measured times.  Over 200 other problems 0.77 of its
-// time, 3 % slower at most.  Past that where the direct-operand kernel's workgroups leave units idle and the price says so clearly (ratio
-// 0.8): up to ten rows under 0.8 of a workgroup a unit, up to 24 under 0.6 (280 problems of 8 to 60 experts, 8 to 24 rows each: 0.84 of
-// the time over all, one slower by 10 %; on more experts the second fragment and the experts of several passes made up to 1.3 of it, at 24
-// to 48 rows four of 26 were slower by 14 to 20 %).
-bool qw_grouped_rows_takes(int fmt, const qw_gemm_params& p, uint32_t experts) {
-    if (p.M > 24u * experts) return false;
-    const qmr_config c = qmr_choose(fmt, p, experts, false);
+// form's (choose_direct) without ranges, which is a fourteenth below the grouped kernel's measured times where the price here is a fifth above
+// its own: level at 1.3.  Past that where the direct-operand kernel's workgroups leave units idle and the price says so clearly (ratio
+// 0.9): up to ten rows under 0.8 of a workgroup a unit, up to 24 under 0.6.
+// Over 140 calls of 70 layers (8 .. 256 experts, up to 24 rows each, 12 containers): 0.76 of the direct-operand kernel's time on even routes,
+// 0.77 on routes of log-normal popularity and on routes falling as 1 / rank, 3 % slower at most; all tokens on the same experts 0.65, three
+// of 140 slower, by up to 1.4 (100 rows on eight of 256: entries of 64 rows, each unpacked four times).
+// Both doors take the kernel by the plain door's price: one arithmetic.
+bool qw_grouped_rows(hipStream_t st, int fmt, const qw_gemm_params& g, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt, bool swiglu,
+                     hipError_t* err) {
+    if (g.M > 24u * experts || max_tiles > 64u * QMR_LISTS) return false;
+    qmr_config c = qmr_choose(fmt, g, experts, false);
     if (c.waves == 0u) return false;
-    const double used = experts * (1.0 - std::exp(-(p.M / (double)experts))), load = used * qwhip_cdiv(p.N, 256u) / 256.0;
+    const double used = experts * (1.0 - std::exp(-(g.M / (double)experts))), load = used * qwhip_cdiv(g.N, 256u) / 256.0;
     const double rounds = load <= 1.0 ? 1.0 + 0.10 * load : load <= 2.0 ? 1.41 + 0.19 * load : 0.36 + 0.885 * load;
     const bool wide = fmt == QG_FMT_B8 || fmt == QG_FMT_B6;
-    const double direct = 5.3 + std::max(p.K / 128u * 1.04 * (wide ? 1.39 : 1.0) * rounds, used * (double)p.N * (double)p.row_bytes / 3.5e6);
-    return p.M <= 8u * experts ? c.us < 1.1 * direct : load <= (p.M <= 10u * experts ? 0.8 : 0.6) && c.us < 0.8 * direct;
-}
-hipError_t qw_grouped_rows(hipStream_t st, int fmt, const qw_gemm_params& g, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt,
-                           bool swiglu) {
-    const qmr_config c = qmr_choose(fmt, g, experts, swiglu);
-    if (c.waves == 0u || (uint64_t)max_tiles * c.bands >= (1u << 28)) return hipErrorInvalidValue;
+    const double direct = 5.3 + std::max(g.K / 128u * 1.04 * (wide ? 1.39 : 1.0) * rounds, used * (double)g.N * (double)g.row_bytes / 3.5e6);
+    if (!(g.M <= 8u * experts ? c.us < 1.3 * direct : load <= (g.M <= 10u * experts ? 0.8 : 0.6) && c.us < 0.9 * direct)) return false;
+    if (swiglu) c = qmr_choose(fmt, g, experts, true);   // fits where the plain form does
     const uint32_t s = qmr_steps(fmt, g.K);
     qmr_params p;
     p.bank = g.bank;
@@ -288,8 +350,8 @@ hipError_t qw_grouped_rows(hipStream_t st, int fmt, const qw_gemm_params& g, uin
     p.tile_e = g.tile_e;
     p.tile_r = g.tile_r;
     p.expert_off = g.expert_off;
-    p.bands = c.bands;
-    p.stride = qwhip_cdiv(max_tiles, 8u) * c.bands;
+    p.max_tiles = max_tiles;
+    p.wgs = c.wgs;
     p.nsl = g.K / 32u;
     p.gshift = g.gshift;
     p.bb = g.bb;
@@ -310,11 +372,12 @@ hipError_t qw_grouped_rows(hipStream_t st, int fmt, const qw_gemm_params& g, uin
     p.y_dtype = ydt;
     p.act = g.act;
     switch (fmt) {
-        case QG_FMT_M5: return qmr_launch<QG_FMT_M5>(st, p, c, s, max_tiles, swiglu);
-        case QG_FMT_B4: return qmr_launch<QG_FMT_B4>(st, p, c, s, max_tiles, swiglu);
-        case QG_FMT_B8: return qmr_launch<QG_FMT_B8>(st, p, c, s, max_tiles, swiglu);
-        case QG_FMT_B2: return qmr_launch<QG_FMT_B2>(st, p, c, s, max_tiles, swiglu);
-        case QG_FMT_B3: return qmr_launch<QG_FMT_B3>(st, p, c, s, max_tiles, swiglu);
-        default: return qmr_launch<QG_FMT_B6>(st, p, c, s, max_tiles, swiglu);
+        case QG_FMT_M5: *err = qmr_launch<QG_FMT_M5>(st, p, c, s, swiglu); break;
+        case QG_FMT_B4: *err = qmr_launch<QG_FMT_B4>(st, p, c, s, swiglu); break;
+        case QG_FMT_B8: *err = qmr_launch<QG_FMT_B8>(st, p, c, s, swiglu); break;
+        case QG_FMT_B2: *err = qmr_launch<QG_FMT_B2>(st, p, c, s, swiglu); break;
+        case QG_FMT_B3: *err = qmr_launch<QG_FMT_B3>(st, p, c, s, swiglu); break;
+        default: *err = qmr_launch<QG_FMT_B6>(st, p, c, s, swiglu); break;
     }
+    return true;
 }

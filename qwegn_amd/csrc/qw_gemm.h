@@ -37,10 +37,9 @@ __device__ __forceinline__ void qg_store(void* y, uint64_t idx, float v) {
 bool qw_grouped_direct_takes(int fmt, const qw_gemm_params& p, uint32_t experts);
 hipError_t qw_grouped_direct(hipStream_t st, int fmt, const qw_gemm_params& p, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt,
                              bool swiglu);
-// moe_rows.hip: grouped, few rows an expert
-bool qw_grouped_rows_takes(int fmt, const qw_gemm_params& p, uint32_t experts);
-hipError_t qw_grouped_rows(hipStream_t st, int fmt, const qw_gemm_params& p, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt,
-                           bool swiglu);
+// moe_rows.hip: grouped, few rows an expert; false where it does not take the call.
+bool qw_grouped_rows(hipStream_t st, int fmt, const qw_gemm_params& p, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt, bool swiglu,
+                     hipError_t* err);
 // gemm_mid.hip: the dense form.  splits > 1: fp32 planes [splits][M][ldy] at p.y (ydt f32), no range of K pairs empty; swiglu: f16
 // rows; few: spans of 64 rows.
 hipError_t qw_dense_direct(hipStream_t st, int fmt, const qw_gemm_params& p, uint32_t splits, uint32_t xdt, uint32_t ydt, bool swiglu, bool few);
