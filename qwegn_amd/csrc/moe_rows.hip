@@ -36,7 +36,7 @@ constexpr uint32_t qmr_waves(uint32_t mf, uint32_t s) { return mf * s <= 2u ? 16
 // of the list, the late chunks were a round of their own behind the empty workgroups, and the XCD of the busy experts had most of them.)
 // 64 rows x top-8 of 128 experts, 2048 x 768, gate|up and down, us: even routes 51 and 29 (the direct-operand kernel 70 and 42), routes
 // falling as 1 / rank 50 and 28 (before 77 and 44, direct-operand 65 and 38), all tokens on the same eight 15 and 10 (35 and 19; 25 and 12).
-// Finding its chunk costs a workgroup 0.4 us: 22 rows x top-2 of 8 experts, 1024 x 384, 5.2 -> 5.6.
+// Finding its chunk costs a workgroup 0.4 us: 25 rows x top-2 of 16 experts, down of 2304 x 384, HQ4_G32, 6.0 -> 6.5.
 template <int FMT, int S, int MF, bool GATED>
 struct qw_moe_rows_kernel {
 static constexpr int kLaunchBound = 64 * qmr_waves(MF, S);

@@ -85,9 +85,10 @@ def test_batched_f32_form_shapes(dev, fmt, n, k, m):
     assert qo.normalized_error(got, want) <= TOL
 
 
-# a last range of one step and of two, sixteen ranges, one (too few steps; more tiles than units), planes past the scratch
+# ranges of two and of three steps, sixteen of eight, one (too few steps; tiles enough), a last range of one step, four that the scratch makes three
 @pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq8_g32", "hq3_g32"])
-@pytest.mark.parametrize("n,k,m,epi", [(77, 1088, 33, 0), (200, 2240, 40, 1), (64, 8192, 64, 3), (4100, 192, 32, 2), (33000, 128, 65, 0), (8000, 512, 256, 0)])
+@pytest.mark.parametrize("n,k,m,epi", [(77, 1088, 33, 0), (200, 2240, 40, 1), (64, 8192, 64, 3), (4100, 192, 32, 2), (33000, 128, 65, 0), (8000, 512, 256, 0),
+                                       (77, 448, 33, 0), (8192, 512, 64, 1)])
 def test_batched_f32_form_over_k_ranges(dev, fmt, n, k, m, epi):
     got, want, _ = _run(dev, fmt, n, k, m, epi, 1.5, seed=23)
     assert qo.normalized_error(got, want) <= TOL

@@ -454,6 +454,11 @@ def test_gemm_row_tile_kernel(dev, fmt, m, n, k, xdtype, ranges):
     dev.stream.sync()
     got = y32.download(np.float32, (m, ldy))[:, :n]
     w = w16.astype(np.float64)
+    y32b = dev.alloc(m * ldy * 4)
+    qwhip.check(lib.qwhip_gemm(st, C.byref(view), xb.ptr, xcode, m, ldx, y32b.ptr, qwhip.F32, ldy, qwhip.X_PREROTATED | 5 << 8, None, 0))
+    dev.stream.sync()
+    assert not np.array_equal(got, y32b.download(np.float32, (m, ldy))[:, :n])               # not the tiles, which add in another order
+    y32b.free()
     assert np.all(np.abs(got - xs @ w.T) <= k * 2.0 ** -24 * (np.abs(xs) @ np.abs(w).T))      # k rounded additions of exact products
     assert np.array_equal(y16.download(np.float16, (m, ldy))[:, :n], got.astype(np.float16))
     assert np.array_equal(yb.download(np.uint16, (m, ldy))[:, :n], qo.f32_to_bf16_bits(got))

@@ -261,9 +261,10 @@ def test_gemv_split_k_mfma_kernel_refusals_and_stream_order(dev):
     assert lib.qwhip_gemv(st, C.byref(v128), xb.ptr, qwhip.F16, 2, 9 << 8, y.ptr, None) == qwhip.E_BAD_GEOMETRY  # not in the basis
     for b in (bank, xb, y):
         b.free()
-    for n, k, m in ((640, 17408, 16), (96, 8192, 6)):
-        g16, g32, ref = _run_gemv(dev, "hq4_g32_m5", n, k, m, prerot=True, seed=n, variant=0)     # automatic: k >= 8192, m >= 6
-        assert qo.normalized_error(g32, ref) <= 2e-5
+    for variant in (0, 9, 10):      # the automatic choice is the row-tile kernel's ranges
+        for n, k, m in ((640, 17408, 16), (96, 8192, 6)):
+            g16, g32, ref = _run_gemv(dev, "hq4_g32_m5", n, k, m, prerot=True, seed=n, variant=variant)
+            assert qo.normalized_error(g32, ref) <= 2e-5
 
 _ROWS_FORMATS = ["hq4_g32_m5", "aq4_g32", "hq4_g128", "hq8_g32", "aq8_g256", "aq2_g64", "hq3_g32", "aq6_g128"]
 
