@@ -454,7 +454,7 @@ def test_grouped_gemm_of_few_rows_an_expert(dev, fmt, counts, k, inter, xdt, com
 _LISTS = [[5], [1] * 64, [2] * 65, [int(c) for c in np.random.default_rng(1).integers(0, 4, 448)] + [70, 33], [0] * 20 + [96] + [0] * 19]
 
 
-@pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq8_g32"])
+@pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq6_g32"])
 @pytest.mark.parametrize("counts", _LISTS, ids=["one", "64", "65", "450", "same"])
 def test_grouped_row_tiles_find_every_chunk(dev, fmt, counts):
     """The row-tile kernel deals (entry, chunk of rows, band) over its workgroups: each is somebody's, once."""
@@ -466,23 +466,27 @@ def test_grouped_row_tiles_take_any_tile_list(dev, fmt):
     test_grouped_gemm_takes_any_tile_list(dev, fmt, _FEW_EACH, 96)
 
 
-@pytest.mark.parametrize("capacity", [768, 769, 4000])
-def test_grouped_row_tiles_capacity_of_the_tile_list(dev, capacity):
-    """Lists of more places than entries: the entries alone are read, up to what the row-tile kernel looks through and past it."""
+def test_grouped_row_tiles_capacity_of_the_tile_list(dev):
+    """Lists of more places than entries: the entries alone are read.  Up to 768 places the row-tile kernel looks through them, past that the
+    direct-operand kernel has the call, whose fp32 sums add in another order."""
     fmt, e, k, inter = "hq4_g32_m5", len(_FEW_EACH), 768, 96
     n = 2 * inter
     blocks, w16 = H.make_bank(fmt, e * n, k, seed=22)
     ids = np.repeat(np.arange(e), _FEW_EACH).astype(np.int32).reshape(-1, 1)
     pairs, g, x = ids.size, _group(dev, ids, e, 1), H.make_x(ids.size, k, 5).astype(np.float16)
     b, bank, xb, y = g["bufs"], dev.put(blocks), dev.put(x), dev.alloc(pairs * n * 4)
-    view = H.view_of(dev, bank, fmt, e * n, k)
-    qwhip.check(dev.lib.qwhip_moe_grouped_gemm(dev.stream.handle, C.byref(view), e, xb.ptr, qwhip.F16, 0, b["stok"].ptr, b["off"].ptr, b["te"].ptr,
-                                               b["tr"].ptr, b["tc"].ptr, capacity, pairs, y.ptr, qwhip.F32, 0))
-    dev.stream.sync()
+    view, got = H.view_of(dev, bank, fmt, e * n, k), []
+    for capacity in (g["max_tiles"], 768, 769, 4000):
+        qwhip.check(dev.lib.qwhip_moe_grouped_gemm(dev.stream.handle, C.byref(view), e, xb.ptr, qwhip.F16, 0, b["stok"].ptr, b["off"].ptr, b["te"].ptr,
+                                                   b["tr"].ptr, b["tc"].ptr, capacity, pairs, y.ptr, qwhip.F32, 0))
+        dev.stream.sync()
+        got.append(y.download(np.float32, (pairs, n)))
     xs, w = x.astype(np.float64)[g["stok"]], w16.reshape(e, n, k).astype(np.float64)
     rows = [(xs[g["off"][i]:g["off"][i + 1]], w[i].T) for i in range(e)]
     want, size = np.concatenate([a @ c for a, c in rows]), np.concatenate([np.abs(a) @ np.abs(c) for a, c in rows])
-    assert np.all(np.abs(y.download(np.float32, (pairs, n)) - want) <= k * 2.0 ** -24 * size)      # k rounded additions of exact products
+    for out in got:
+        assert np.all(np.abs(out - want) <= k * 2.0 ** -24 * size)      # k rounded additions of exact products
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[2], got[3]) and not np.array_equal(got[0], got[2])
 
 
 @pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq8_g32", "hq4_g64"])
