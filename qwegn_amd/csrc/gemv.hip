@@ -1021,13 +1021,13 @@ bool qw_sk_gemv(qwhip_stream_t s, const qwhip_weight_view* w, int fmt, uint32_t 
 bool qw_rows_gemv(qwhip_stream_t s, const qwhip_weight_view* w, int fmt, uint32_t gshift, uint32_t bb, uint64_t row_bytes, const void* x,
                   uint32_t x_dtype, uint32_t m, bool f16w, void* y16, float* y32, uint32_t inter, bool rotate_out, uint32_t tune, hipError_t* err);
 
-// Does the row-tile kernel pay?  From 86 banks of each of six containers (K = 1024 .. 17408, N = 1024 .. 32768) at 2 .. 16 rows, its time
-// over that of the kernel that a call took before.  13 rows on 0.62 .. 0.72 in the mean (1.10 at most), 9 to 12 rows 0.63 .. 0.79 (1.13), 8 rows
-// 0.81 .. 0.85.  Below that the 4x4x4-block kernel, whose cost is a third of this one's at four rows, keeps the banks whose launch is
+// Does the row-tile kernel pay?  Its time over that of the kernel that a call took before, where the rule takes it, over 240 banks of 12
+// containers (K = 1024 .. 17408, N = 1024 .. 36000): 13 rows on 0.71 in the mean (1.02 at most), 9 to 12 rows 0.70 (1.04), 8 rows 0.80
+// (1.04), 5 to 7 rows 0.83 (1.06), 2- to 4-row calls 0.76 (1.05); 2-, 3- and 6-bit streams, whose dot2 kernel's work grows with m, 0.29, 0.38, 0.51,
+// 0.54 and 0.73.  Elsewhere the 4x4x4-block kernel, whose cost is a third of this one's at four rows, keeps the banks whose launch is
 // neither so short that its one trip through LDS counts nor so long that the memory system sets the time: 5 .. 7 rows on 4096 .. 12288
-// columns of up to 5120 rows (1.0 .. 1.2; 8-bit streams of any height, up to eight rows, 1.0 .. 1.15), 2 .. 4 rows past 2048 columns (1.0 .. 1.5).
-// 2-, 3- and 6-bit streams: the dot2 kernel's work grows with m, from three rows on 0.78 .. 0.86 (0.55 .. 0.63 at six), two rows 1.2, and
-// three and four rows on 1024 bank rows 1.0 .. 1.28.
+// columns of up to 5120 rows (1.0 .. 1.2; 8-bit streams of any height, up to eight rows, 1.0 .. 1.15), 2 .. 4 rows past 2048 columns (1.0 .. 1.5),
+// and the dot2 kernel two rows (1.2), three and four rows on 1024 bank rows (1.0 .. 1.28).
 static bool qw_rows_pays(int fmt, uint32_t m, uint32_t n, uint32_t k) {
     if (m < 2u || m > 16u) return false;
     if (fmt >= QW_FMT_B2) return m >= 5u || (m >= 3u && n >= 2048u);
@@ -1326,7 +1326,7 @@ extern "C" qwhip_status qwhip_gemv_silu_pair(qwhip_stream_t s, const qwhip_weigh
     // partial-sum area, then the gated activation (+ rotation) pass over it - every weight is read once whatever m is (the MoE
     // decode kernel reads the bank once per row: 40 / 70 / 125 us at m = 2 / 4 / 8 on 2 x 17408 x 5120).
     if (m >= 2u && m <= 16u && ((flags >> 8) & 0xFu) == 0u && s->scratch && (!rot_out || ((uintptr_t)act16 & 15u) == 0)) {
-        // f16 rows in the basis: the row-tile kernel on the gate and up rows of a channel block, the gated activation where it sums them
+        // f16 rows in the basis: the row-tile kernel on the gate and up rows of a channel block, the gated activation where it sums them.
         if (!rotate && !(flags & QWHIP_GEMV_ROW_INVARIANT) && x_dtype == QWHIP_F16) {
             hipError_t e = hipSuccess;
             const uint32_t gshift = log2_u32(w->group / 32), bb = qwhip_view_block_bytes(w);

@@ -21,8 +21,8 @@
 // loads, LDS, products, sums.  Against the kernels before, launches on cold banks back to back (us): 34816 x 5120 HQ4_G32_M5 at
 // 8 / 12 / 16 rows 31.8 / 53.1 / 29.5 -> 25.3 / 26.9 / 27.4 (5.2 TB/s at 8), 3072 x 2048 6.9 / 8.7 / 10.9 -> 4.5 / 4.6 / 4.7; 24576 x 4096 in
 // 36-byte blocks 17.9 / 23.6 / 17.7 -> 15.2 / 16.0 / 17.0; 22784 x 4608 at 6 bits 45 / 70 / 90 -> 24.4 / 25.4 / 25.4; 16384 x 2304 at 3 bits
-// 22.4 / 37.8 / 44.9 -> 9.2 / 9.7 / 9.9; 4096 x 12288 4-bit 19.3 / 19.7 / 19.8 -> 13.1 / 13.9 / 14.4; 6144 x 24576 33.5 / 34.5 / 34.7 -> 23.0 / 24.3 /
-// 25.1; 5120 x 17408 HQ8_G32 29.6 / 34.0 / 51.1 -> 25.1 / 26.2 / 26.6.  Error against 64 bits of the codes' own weights (FACT), 8 rows of
+// 22.4 / 37.8 / 44.9 -> 9.2 / 9.7 / 9.9; 4096 x 12288 4-bit 20.3 / 20.5 / 20.5 -> 12.7 / 13.2 / 13.8; 6144 x 24576 34.5 / 35.6 / 35.8 -> 24.3 / 24.6 /
+// 25.5; 5120 x 17408 HQ8_G32 31.1 / 35.6 / 51.6 -> 26.8 / 26.9 / 26.9.  Error against 64 bits of the codes' own weights (FACT), 8 rows of
 // 1536 columns: HQ4_G32_M5 6.5e-6 -> 5.2e-7, HQ8_G32 4.0e-7 -> 1.7e-7, 2 bits 1.0e-5 -> 3.9e-7.
 #include <atomic>
 
@@ -185,31 +185,50 @@ hipError_t qr_go(hipStream_t st, const qr_params& p, uint32_t wgs, uint32_t wave
     return hipGetLastError();
 }
 
+template <int FMT>
+constexpr uint32_t qr_image_bytes(uint32_t s) { return 4u * (s == 1u ? qr_image<FMT, 1>::DWORDS : s == 2u ? qr_image<FMT, 2>::DWORDS : qr_image<FMT, 4>::DWORDS); }
+constexpr uint32_t qr_most_waves(uint32_t s) { return s <= 2u ? 16u : 12u; }   // of 128 and of 168 registers
+constexpr uint32_t QR_LDS = 160u * 1024u;
+
+// Steps a wave (at least `least`) and K ranges of rows past 6144 columns, by the lowest price, us: the launches 5.1 and the activations; row
+// tiles one after the other on a compute unit, each 0.27 for the barrier, 0.021 for every wave's part of the sums, and every step on a SIMD;
+// the planes at 1.4 TB/s; and the bank's stream (8.5 TB/s, in quadrature).  Weighed by the choice it makes among 11000 measured forms of 170
+// banks (n 1024 .. 20000, k 6400 .. 28672, 12 containers) at 4 to 16 rows: the form taken is 2 % slower than the best.  (Four steps a wave and
+// as few ranges as hold the row, the rule before, was 13 % slower than the best: 2368 x 7936 HQ8_G32 at nine rows 15.4 us, the 4x4x4-block
+// kernel 12.1, this choice 10.5.)  False where nothing fits.
+template <int FMT>
+bool qr_ranges(const qr_params& p, uint32_t steps, uint32_t least, size_t part_bytes, uint32_t* s_out, uint32_t* nkr_out) {
+    const float unpack = FMT == QG_FMT_B8 ? 2.0f : FMT == QG_FMT_B6 ? 1.8f : FMT == QG_FMT_B3 ? 1.6f : 1.0f;
+    const float bank = (float)p.N * (float)p.row_bytes / 8.5e6f;
+    float best = 3e38f;
+    for (uint32_t s = 1; s <= 4u; s *= 2u) {
+        const uint32_t lo = max(2u, qwhip_cdiv(steps, s * qr_most_waves(s)));
+        for (uint32_t k = lo; s >= least && k < lo + 7u && k <= 256u && (uint64_t)k * p.M * p.units * 64u <= part_bytes; ++k) {
+            const uint32_t waves = qwhip_cdiv(steps, s * k), need = waves * (qr_image_bytes<FMT>(s) + 2048u);
+            if (waves < 2u || need > QR_LDS || (k - 1u) * s * waves >= steps) continue;
+            const uint32_t per_cu = max(1u, min(qr_most_waves(s) / waves, QR_LDS / need)), bands = min(p.units, 256u * per_cu / k);
+            const float simd = waves * qwhip_cdiv(bands * k, 256u) * s / 4.0f;   // steps on a SIMD, side by side
+            const float tile = 0.27f + 0.021f * waves + 0.076f * unpack * (s == 1u ? 0.55f : s == 2u ? 1.0f : 2.5f) * simd;
+            const float t = 5.1f + 0.43f * simd + qwhip_cdiv(p.units, bands) * tile + (float)k * p.M * p.N * 8.0f / 1.43e6f, us = t * t + bank * bank;
+            if (us < best) best = us, *s_out = s, *nkr_out = k;
+        }
+    }
+    return best < 3e38f;
+}
+
 template <int FMT, int XDT, bool F16W>
 hipError_t qr_launch(hipStream_t st, qr_params& p, size_t part_bytes, uint32_t out, uint32_t tune) {
     // as few steps a wave as 16 waves (one or two steps, 128 registers) or 12 (168) hold; longer rows in K ranges
-    const uint32_t steps = qwhip_cdiv(p.nsl, 4u);
-    uint32_t s = steps <= 16u ? 1u : steps <= 32u ? 2u : 4u;
-    if (tune & 7u) s = max((tune & 7u) == 3u ? 4u : min(tune & 7u, 4u), s);   // the forms there are: 1, 2 and 4
+    const uint32_t steps = qwhip_cdiv(p.nsl, 4u), code = (tune & 7u) == 3u ? 4u : min(tune & 7u, 4u);   // the forms there are: 1, 2 and 4
+    uint32_t s = max(code, steps <= 16u ? 1u : steps <= 32u ? 2u : 4u);
     const uint32_t spu = out ? 2u * out : 1u;
     p.units = out ? p.inter / (16u * out) : qwhip_cdiv(p.N, 16u);
-    p.nkr = qwhip_cdiv(steps, s * (s <= 2u ? 16u : 12u));
-    if (p.nkr > (out ? 1u : 254u)) return hipErrorNotSupported;   // at most 256 ranges (1560576 columns): a workgroup each at least
-    if (p.nkr > 1u) {   // of the least number of ranges and the two after it, the one whose workgroups walk the fewest wave steps
-        uint32_t best = ~0u, least = p.nkr;
-        for (uint32_t k = least; k < least + 3u; ++k) {
-            if (k > least && (uint64_t)k * p.M * p.units * 64u > part_bytes) break;
-            const uint32_t cost = qwhip_cdiv(p.units, 256u / k) * qwhip_cdiv(steps, s * k);
-            if (cost < best) best = cost, p.nkr = k;
-        }
-    }
+    p.nkr = 1;
+    if (steps > s * qr_most_waves(s) && (out || !qr_ranges<FMT>(p, steps, code, part_bytes, &s, &p.nkr))) return hipErrorNotSupported;
     const uint32_t waves = qwhip_cdiv(steps, s * p.nkr);
-    p.nkr = qwhip_cdiv(steps, s * waves);
-    if (p.nkr > 1u && (uint64_t)p.nkr * p.M * p.units * 64u > part_bytes) return hipErrorNotSupported;
-    const uint32_t image = waves * 4u * (s == 1u ? qr_image<FMT, 1>::DWORDS : s == 2u ? qr_image<FMT, 2>::DWORDS : qr_image<FMT, 4>::DWORDS);
-    const uint32_t part = 2u * spu * waves * 1024u, most = 160u * 1024u;   // bytes of the images, of the partial tiles of a unit
+    const uint32_t image = waves * qr_image_bytes<FMT>(s), part = 2u * spu * waves * 1024u, most = QR_LDS;   // bytes of the images, of the partial tiles of a unit
     if (image + part > most) return hipErrorNotSupported;
-    const uint32_t cus = 256u * max(1u, min((s <= 2u ? 16u : 12u) / waves, most / (image + part)));
+    const uint32_t cus = 256u * max(1u, min(qr_most_waves(s) / waves, most / (image + part)));
     if (out) {
         // The launch that is saved is worth 2 to 2.5 us (2 x 8192 x 3072: 9.3 us, in two launches 11.5; 2 x 7552 x 2560 8.7 / 11.1; 2 x 3840 x 1536
         // 5.8 / 7.2).  Whole units leave workgroups with a unit more than others, a row tile being 0.4 to 0.5 us per 1024 columns (2 x 8448 x

@@ -367,9 +367,9 @@ def test_gemv_row_tile_kernel_weights_follow_the_shape(dev, m):
 
 
 def test_gemv_row_tile_kernel_longest_rows(dev):
-    """254 ranges of 6144 columns and their 1.56 million columns; one step more is refused on the host, whose range count would divide a
-    unit count of zero."""
-    k = 254 * 6144
+    """256 ranges of 6144 columns; one step more, and rows of 25 million columns, are refused on the host: more ranges than compute units
+    would divide by zero."""
+    k = 256 * 6144
     g32, ref = _run_gemv(dev, "hq4_g32_m5", 16, k, 2, prerot=True, seed=5, variant=10)[1:]
     assert qo.normalized_error(g32, ref) <= TOL      # the codes against their f16 weights
     bank, xb, y = dev.alloc(16 * (k + 128) // 32 * 20), dev.alloc(2 * (k + 128) * 2), dev.alloc(2 * 16 * 4)
