@@ -1326,8 +1326,12 @@ extern "C" qwhip_status qwhip_gemv_silu_pair(qwhip_stream_t s, const qwhip_weigh
     // partial-sum area, then the gated activation (+ rotation) pass over it - every weight is read once whatever m is (the MoE
     // decode kernel reads the bank once per row: 40 / 70 / 125 us at m = 2 / 4 / 8 on 2 x 17408 x 5120).
     if (m >= 2u && m <= 16u && ((flags >> 8) & 0xFu) == 0u && s->scratch && (!rot_out || ((uintptr_t)act16 & 15u) == 0)) {
-        // f16 rows in the basis: the row-tile kernel on the gate and up rows of a channel block, the gated activation where it sums them.
-        if (!rotate && !(flags & QWHIP_GEMV_ROW_INVARIANT) && x_dtype == QWHIP_F16) {
+        // f16 rows in the basis: the row-tile kernel on the gate and up rows of a channel block, the gated activation where it sums them.  At four
+        // steps a wave (rows past 4096 columns) where it has the plain call too, and 4-bit banks from five rows on: elsewhere there the launch
+        // that is saved does not pay for the kernel (8-bit 9024 x 5376, five rows, 20.8 us / 16.7; 27 calls 1.05; HQ4_G32_M5 4928 x 4608, six
+        // rows, 8.8 / 10.4)
+        const bool gated_pays = w->k <= 4096u || qw_rows_pays(fmt, m, w->n, w->k) || (m >= 5u && (fmt == QW_FMT_M5 || fmt == QW_FMT_B4));
+        if (!rotate && !(flags & QWHIP_GEMV_ROW_INVARIANT) && x_dtype == QWHIP_F16 && gated_pays) {
             hipError_t e = hipSuccess;
             const uint32_t gshift = log2_u32(w->group / 32), bb = qwhip_view_block_bytes(w);
             const uint64_t row_bytes = qwhip_view_row_bytes(w);
