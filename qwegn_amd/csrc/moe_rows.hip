@@ -266,51 +266,84 @@ uint32_t qmr_steps(int fmt, uint32_t k) {
     return steps <= 5u || (fmt == QG_FMT_B8 && steps <= 12u) ? 1u : 2u;
 }
 
+// What the routes make of a call: the experts that have rows and their tiles of 16, 32 and 64 rows.
+struct qmr_load {
+    double used, tiles[3], stream;   // stream: us of a launch that reads those experts' banks
+};
+// The host does not see the routes.  Prices are taken for three: even ones (rows an expert: Poisson), rows falling as 1 / rank (experts of
+// neighbouring ranks together) and all rows on four experts.
+void qmr_loads(const qw_gemm_params& p, uint32_t experts, qmr_load (&out)[3]) {
+    const uint32_t rows = p.M;
+    auto add = [](qmr_load& l, double n, double mean) {   // n experts; the tiles of Poisson rows to 5 % (up to 19 % at 0.75 of a tile)
+        const double some = 1.0 - std::exp(-mean);
+        l.used += n * some;
+        for (int i = 0; i < 3; ++i) {
+            const double b = 16 << i;
+            l.tiles[i] += n * (mean < 2.2 * b ? some + std::max(0.0, mean / b - 0.55) : mean / b + 0.5);
+        }
+    };
+    for (qmr_load& l : out) l = {};
+    add(out[0], experts, rows / (double)experts);
+    const double all = std::log((double)experts) + 0.577;
+    for (uint32_t lo = 1, hi; lo <= experts; lo = hi + 1u) {
+        hi = min(experts, max(lo, lo * 3u / 2u));
+        const double n = hi - lo + 1u;
+        add(out[1], n, rows * std::log((hi + 0.5) / (lo - 0.5)) / (all * n));
+    }
+    const uint32_t few = min(experts, 4u);
+    add(out[2], few, rows / (double)few);
+    for (qmr_load& l : out) l.stream = 3.9 + l.used * (double)p.N * (double)p.row_bytes / 4.75e6;
+}
+
 struct qmr_config {
     uint32_t waves, mf, units, wgs, flush, lds;   // waves = 0: none fits
-    double us;
+    double us[3];                                 // by kind of route
 };
-// The launch with the lowest price, us: fragments of rows, and workgroups for the bands of row tiles of all chunks together (find).  A launch
-// 4.2; then rounds of workgroups, one's start 1.5, its activations and row tiles, a tile costing 0.54, its waves' sums and every step's
-// unpacking and products on a SIMD; no faster than 5.7 TB/s of the experts that have rows.  The chunks are those of even routes (rows an
-// expert: Poisson) and a tenth more, in the mean of both prices: skewed routes leave experts without rows and give others several chunks,
-// 0.9 .. 1.13 of the even ones' number on routes falling as 1 / rank.  Over 140 layers (8 .. 256 experts, up to 24 rows each, 12 containers,
-// both kinds of routes) the form taken is 4 % slower than the best of up to ten measured ones.
-qmr_config qmr_choose(int fmt, const qw_gemm_params& p, uint32_t experts, bool gated) {
+// The launch with the lowest price, us, over the three kinds of routes (the product): fragments of rows, and workgroups for the bands of row
+// tiles of all chunks together (find).  A launch 3.9; then rounds of workgroups, one's activations and row tiles, a tile costing 0.36 (gate|up
+// 0.42) and every step's unpacking and products on a SIMD; no faster than 4.75 TB/s of the experts that have rows.  The chunks as they are and a
+// tenth more, in the mean of both: one more than the workgroups hold is another round of them.  Fitted to 19000 measured launches: up to 12
+// forms of 800 calls (16 .. 256 experts, 0.1 .. 24 rows each, 12 containers) on each kind of routes, 11 % of root mean square error.
+qmr_config qmr_choose(int fmt, const qw_gemm_params& p, const qmr_load (&loads)[3], bool gated) {
     const uint32_t s = qmr_steps(fmt, p.K), waves = qwhip_cdiv(p.K / 128u, s), units = gated ? p.inter / 32u : qwhip_cdiv(p.N, 16u);
-    const double unpack = fmt == QG_FMT_B8 ? 1.38 : fmt == QG_FMT_B6 ? 0.9 : fmt == QG_FMT_B3 ? 2.2 : 1.0;
-    const double mean = p.M / (double)experts, none = std::exp(-mean), used = experts * (1.0 - none);
-    const double stream = 4.2 + used * (double)p.N * (double)p.row_bytes / 5.7e6;
-    double chunks[2] = {0.0, 0.0}, chance = none;   // of 16 and of 32 rows
-    for (uint32_t k = 1; k < 64u && (k < mean + 2.0 || chance > 1e-5); ++k) {
-        chance *= mean / k;
-        chunks[0] += chance * ((k + 15u) >> 4);
-        chunks[1] += chance * ((k + 31u) >> 5);
-    }
+    const double unpack = fmt == QG_FMT_B8 ? 1.87 : fmt == QG_FMT_B6 ? 2.04 : fmt == QG_FMT_B3 ? 1.66 : fmt == QG_FMT_B2 ? 1.42 : fmt == QG_FMT_B4 ? 1.33 : 1.0;
     qmr_config best = {};
-    best.us = 1e30;
+    double lowest = 1e300;
     for (uint32_t mf = 1; mf <= 2u; ++mf) {
         const uint32_t image = waves * qmr_image_bytes(fmt, s), part = 2u * waves * mf * 1024u, sums = 4u * 16u * mf * 17u * 4u;
         if (waves > qmr_waves(mf, s) || image + part + sums > QMR_LDS) continue;
         const uint32_t per_cu = max(1u, min(qmr_waves(mf, s) / waves, QMR_LDS / (image + part + sums)));
         for (uint32_t i : {1u, 2u, 3u, 4u, 6u, 8u}) {   // workgroups a unit in all
             if (i > 2u * per_cu) break;
-            double us = 0.0;
-            uint32_t tiles = 1;
-            for (double c : {experts * chunks[mf - 1u], 1.1 * experts * chunks[mf - 1u]}) {
-                const uint32_t bands = min(max(1u, (uint32_t)(256u * i / c)), units), longest = qwhip_cdiv(units, bands);
-                const double load = c * qwhip_cdiv(units, longest) / 256.0, side = std::min((double)min(per_cu, i), std::max(1.0, std::ceil(load)));
-                tiles = longest * (gated ? 4u : 1u);
-                const double tile = 0.54 + 0.029 * waves * s + waves * side / 4.0 * s * (0.116 * unpack + 0.034 * mf);
-                us += 0.5 * std::max(stream, 4.2 + std::max(1.0, std::ceil(load / side - 0.01)) * (1.5 + 0.32 * s * mf + tiles * tile));
+            double us[3];
+            uint32_t run = 1;   // row tiles of a workgroup on even routes
+            for (int r = 2; r >= 0; --r) {
+                us[r] = 0.0;
+                for (double c : {1.1 * loads[r].tiles[mf - 1u], loads[r].tiles[mf - 1u]}) {
+                    const uint32_t bands = min(max(1u, (uint32_t)(256u * i / c)), units), longest = qwhip_cdiv(units, bands);
+                    const double load = c * qwhip_cdiv(units, longest) / 256.0, side = std::min((double)min(per_cu, i), std::max(1.0, std::ceil(load)));
+                    run = longest * (gated ? 4u : 1u);
+                    const double tile = (gated ? 0.416 : 0.355) + waves * side / 4.0 * s * (0.118 * unpack + 0.054 * mf);
+                    us[r] += 0.5 * std::max(loads[r].stream, 3.9 + std::max(1.0, std::ceil(load / side - 0.01)) * (0.25 * s * mf + run * tile));
+                }
             }
-            if (us >= best.us) continue;
-            best.waves = waves, best.mf = mf, best.units = units, best.wgs = 256u * i, best.us = us;
-            best.flush = gated ? 1u : max(1u, min(min(4u, tiles), (QMR_LDS / min(per_cu, i) - image) / part));
+            if (us[0] * us[1] * us[2] >= lowest) continue;
+            lowest = us[0] * us[1] * us[2];
+            best.waves = waves, best.mf = mf, best.units = units, best.wgs = 256u * i;
+            for (int r = 0; r < 3; ++r) best.us[r] = us[r];
+            best.flush = gated ? 1u : max(1u, min(min(4u, run), (QMR_LDS / min(per_cu, i) - image) / part));
             best.lds = image + best.flush * part + (gated ? sums : 0u);
         }
     }
     return best;
+}
+// The direct-operand kernel's price, on spans of 64 rows, which it takes for this few rows an expert: 9 % of root mean square error on the
+// same 2400 calls.
+double qmr_direct_us(int fmt, const qw_gemm_params& p, const qmr_load& l) {
+    const double load = l.tiles[2] * qwhip_cdiv(p.N, 256u) / 256.0, deep = 1.0 + 0.07 * (std::max(1.0, l.tiles[1] / l.tiles[2]) - 1.0);
+    const double rounds = load <= 1.0 ? 1.0 + 0.48 * load : load <= 2.0 ? 1.41 + 0.59 * load : 0.34 + 1.32 * load;
+    const double step = fmt == QG_FMT_B8 ? 1.67 : fmt == QG_FMT_B6 ? 1.54 : fmt == QG_FMT_B2 ? 1.09 : fmt == QG_FMT_B4 ? 1.17 : 1.15;
+    return 4.8 + std::max(p.K / 128u * step * rounds * deep, l.used * (double)p.N * (double)p.row_bytes / 3.8e6);
 }
 
 template <int FMT>
@@ -324,25 +357,23 @@ hipError_t qmr_launch(hipStream_t st, const qmr_params& p, const qmr_config& c, 
 
 }  // namespace
 
-// A mean of up to eight rows an expert, at which the direct-operand kernel multiplies 32 and waits; by price against its own, the dense
-// form's (choose_direct) without ranges, which is a fourteenth below the grouped kernel's measured times where the price here is a fifth above
-// its own: level at 1.3.  Past that where the direct-operand kernel's workgroups leave units idle and the price says so clearly (ratio
-// 0.9): up to ten rows under 0.8 of a workgroup a unit, up to 24 under 0.6.
-// Over 140 calls of 70 layers (8 .. 256 experts, up to 24 rows each, 12 containers): 0.76 of the direct-operand kernel's time on even routes,
-// 0.77 on routes of log-normal popularity and on routes falling as 1 / rank, 3 % slower at most; all tokens on the same experts 0.65, three
-// of 140 slower, by up to 1.4 (100 rows on eight of 256: entries of 64 rows, each unpacked four times).
+// Up to 24 rows an expert, where the price is under the direct-operand kernel's, 0.95 of it, on each kind of routes.  Over 1400 calls (16 .. 256
+// experts, 0.1 .. 24 rows each, 12 containers, cold banks), of that kernel's time where this one takes them: even routes 0.67, 1 / rank 0.66, all
+// tokens on the same experts 0.52; down projections 3 % slower at most, of 545 gate|up calls 15 by more than 3 %, up to 1.33.  (The price of even
+// routes alone, which decided before, let through calls up to 2.1 times as slow on the same experts and 1.9 times on 1 / rank, each chunk of 16
+// rows unpacking the expert again: 966 rows x top-2 of 256 experts, 1792 x 512, 20.6 us, now 11.0.  Refused with them are some even calls that
+// it served better: 43 rows x top-8 of 64 experts, 3328 x 896, 30 -> 42 us.)
 // Both doors take the kernel by the plain door's price: one arithmetic.
 bool qw_grouped_rows(hipStream_t st, int fmt, const qw_gemm_params& g, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt, bool swiglu,
                      hipError_t* err) {
     if (g.M > 24u * experts || max_tiles > 64u * QMR_LISTS) return false;
-    qmr_config c = qmr_choose(fmt, g, experts, false);
+    qmr_load loads[3];
+    qmr_loads(g, experts, loads);
+    qmr_config c = qmr_choose(fmt, g, loads, false);
     if (c.waves == 0u) return false;
-    const double used = experts * (1.0 - std::exp(-(g.M / (double)experts))), load = used * qwhip_cdiv(g.N, 256u) / 256.0;
-    const double rounds = load <= 1.0 ? 1.0 + 0.10 * load : load <= 2.0 ? 1.41 + 0.19 * load : 0.36 + 0.885 * load;
-    const bool wide = fmt == QG_FMT_B8 || fmt == QG_FMT_B6;
-    const double direct = 5.3 + std::max(g.K / 128u * 1.04 * (wide ? 1.39 : 1.0) * rounds, used * (double)g.N * (double)g.row_bytes / 3.5e6);
-    if (!(g.M <= 8u * experts ? c.us < 1.3 * direct : load <= (g.M <= 10u * experts ? 0.8 : 0.6) && c.us < 0.9 * direct)) return false;
-    if (swiglu) c = qmr_choose(fmt, g, experts, true);   // fits where the plain form does
+    for (int r = 0; r < 3; ++r)
+        if (!(c.us[r] < 0.95 * qmr_direct_us(fmt, g, loads[r]))) return false;
+    if (swiglu) c = qmr_choose(fmt, g, loads, true);   // fits where the plain form does
     const uint32_t s = qmr_steps(fmt, g.K);
     qmr_params p;
     p.bank = g.bank;

@@ -450,6 +450,31 @@ def test_grouped_gemm_of_few_rows_an_expert(dev, fmt, counts, k, inter, xdt, com
     test_grouped_gemm_spans(dev, fmt, counts, k, inter, xdt, compact)
 
 
+@pytest.mark.parametrize("fmt", ["hq4_g32_m5", "hq8_g32", "hq6_g32", "hq4_g64"])
+@pytest.mark.parametrize("counts,k,inter", [([40, 20, 0, 33, 17], 1536, 1024), ([33, 20, 0, 32, 11], 640, 2048)], ids=["two-steps", "one-step"])
+def test_grouped_row_tiles_of_two_fragments(dev, fmt, counts, k, inter):
+    """About twenty rows an expert: 32 rows share a row tile, and an expert of one fragment, of part of a second and of a second tile."""
+    test_grouped_gemm_spans(dev, fmt, counts, k, inter, "f16", True)
+
+
+def test_grouped_calls_slow_on_few_experts_leave_the_row_tiles(dev):
+    """297 tokens x top-4 of 256 experts, 1280 x 512: with every token on the same experts the row tiles took 1.3 of the direct-operand kernel's
+    time, on routes falling as 1 / rank 1.2.  A list of more than 768 places is that kernel's: the same bits say that it has the call."""
+    fmt, e, n, k, top = "hq4_g32_m5", 256, 1280, 512, 4
+    blocks, _ = H.make_bank(fmt, n, k, seed=3)
+    ids = np.tile(np.arange(top), (297, 1)).astype(np.int32)
+    pairs, g, x = ids.size, _group(dev, ids, e, top), H.make_x(ids.size, k, 5).astype(np.float16)
+    b, bank, xb, y = g["bufs"], dev.put(np.tile(blocks.reshape(-1), e)), dev.put(x), dev.alloc(pairs * n * 4)
+    view, got = H.view_of(dev, bank, fmt, e * n, k), []
+    assert g["max_tiles"] <= 768
+    for capacity in (g["max_tiles"], 769):
+        qwhip.check(dev.lib.qwhip_moe_grouped_gemm(dev.stream.handle, C.byref(view), e, xb.ptr, qwhip.F16, 0, None, b["off"].ptr, b["te"].ptr,
+                                                   b["tr"].ptr, b["tc"].ptr, capacity, pairs, y.ptr, qwhip.F32, 0))
+        dev.stream.sync()
+        got.append(y.download(np.float32, (pairs, n)))
+    assert np.array_equal(got[0], got[1])
+
+
 # lists of one entry, of one wave's 64 and one more, of seven waves' with several chunks in the last; one expert with every row
 _LISTS = [[5], [1] * 64, [2] * 65, [int(c) for c in np.random.default_rng(1).integers(0, 4, 448)] + [70, 33], [0] * 20 + [96] + [0] * 19]
 
