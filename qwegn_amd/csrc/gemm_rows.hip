@@ -230,7 +230,8 @@ hipError_t qwr_launch(hipStream_t st, const qwr_params& p, const qwr_config& c, 
 // barrier and the sums, and for every step on a SIMD its unpacking and its products; more ranges pay their planes, at 5 TB/s, and the
 // summing launch; and no faster than the bank streams (7.4 TB/s, in quadrature).  Fitted to 4700 measured forms of 660 problems, 17 .. 64
 // rows on 220 banks of 12 containers (n 1024 .. 36000, k 1024 .. 17408): 7.6 % of root mean square error.  Of the other kernels' times on
-// these problems (choose_direct) the form chosen takes 0.63 up to 32 rows, 0.67 up to 48, 0.77 up to 64, none of them slower; on banks of
+// these problems (choose_direct) the form chosen takes 0.63 up to 32 rows, 0.67 up to 48, 0.77 up to 64, none of them slower; of 836 others, half
+// of them gate|up, five are slower by more than 3 %, up to 13 % (64 x 33792 x 1536 gate|up HQ4_G128 23.7 us, 26.7).  On banks of
 // many rows with 64 activation rows the tiles keep the lead (64 x 34816 x 5120 HQ4_G32_M5 62 us, 53 there).
 bool qw_gemm_rows_choose(int fmt, uint32_t m, uint32_t n, uint32_t k, uint64_t row_bytes, uint64_t plane_room, uint32_t ranges, double limit,
                          uint32_t* steps, uint32_t* chosen) {
