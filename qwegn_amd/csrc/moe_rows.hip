@@ -299,8 +299,8 @@ struct qmr_config {
     uint32_t waves, mf, units, wgs, flush, lds;   // waves = 0: none fits
     double us[3];                                 // by kind of route
 };
-// The launch with the lowest price, us, over the three kinds of routes (the product): fragments of rows, and workgroups for the bands of row
-// tiles of all chunks together (find).  A launch 3.9; then rounds of workgroups, one's activations and row tiles, a tile costing 0.36 (gate|up
+// The launch with the lowest price, us, over the three kinds of routes (product of the even one's square, the second's and the fourth root of the
+// third's): fragments of rows, and workgroups for the bands of row tiles of all chunks together (find).  A launch 3.9; then rounds of workgroups, one's activations and row tiles, a tile costing 0.36 (gate|up
 // 0.42) and every step's unpacking and products on a SIMD; no faster than 4.75 TB/s of the experts that have rows.  The chunks as they are and a
 // tenth more, in the mean of both: one more than the workgroups hold is another round of them.  Fitted to 19000 measured launches: up to 12
 // forms of 800 calls (16 .. 256 experts, 0.1 .. 24 rows each, 12 containers) on each kind of routes, 11 % of root mean square error.
@@ -327,8 +327,9 @@ qmr_config qmr_choose(int fmt, const qw_gemm_params& p, const qmr_load (&loads)[
                     us[r] += 0.5 * std::max(loads[r].stream, 3.9 + std::max(1.0, std::ceil(load / side - 0.01)) * (0.25 * s * mf + run * tile));
                 }
             }
-            if (us[0] * us[1] * us[2] >= lowest) continue;
-            lowest = us[0] * us[1] * us[2];
+            const double all = us[0] * us[0] * us[1] * std::sqrt(std::sqrt(us[2]));
+            if (all >= lowest) continue;
+            lowest = all;
             best.waves = waves, best.mf = mf, best.units = units, best.wgs = 256u * i;
             for (int r = 0; r < 3; ++r) best.us[r] = us[r];
             best.flush = gated ? 1u : max(1u, min(min(4u, run), (QMR_LDS / min(per_cu, i) - image) / part));
@@ -357,12 +358,12 @@ hipError_t qmr_launch(hipStream_t st, const qmr_params& p, const qmr_config& c, 
 
 }  // namespace
 
-// Up to 24 rows an expert, where the price is under the direct-operand kernel's, 0.95 of it, on each kind of routes.  Over 1400 calls (16 .. 256
-// experts, 0.1 .. 24 rows each, 12 containers, cold banks), of that kernel's time where this one takes them: even routes 0.67, 1 / rank 0.66, all
-// tokens on the same experts 0.52; down projections 3 % slower at most, of 545 gate|up calls 15 by more than 3 %, up to 1.33.  (The price of even
-// routes alone, which decided before, let through calls up to 2.1 times as slow on the same experts and 1.9 times on 1 / rank, each chunk of 16
-// rows unpacking the expert again: 966 rows x top-2 of 256 experts, 1792 x 512, 20.6 us, now 11.0.  Refused with them are some even calls that
-// it served better: 43 rows x top-8 of 64 experts, 3328 x 896, 30 -> 42 us.)
+// Up to 24 rows an expert, where the price is under the direct-operand kernel's, 0.95 of it, on each kind of routes.  Over 2000 calls (16 .. 256
+// experts, 0.1 .. 24 rows each, 12 containers, cold banks), of that kernel's time where this one takes them: even routes 0.68, 1 / rank 0.65, all
+// tokens on the same experts 0.54; of 704 down projections 5 slower by more than 3 %, up to 1.18, of 802 gate|up calls 23, up to 1.27.  (The price
+// of even routes alone, which decided before, let through calls up to 2.1 times as slow on the same experts and 1.9 times on 1 / rank, each chunk of
+// 16 rows unpacking the expert again: 966 rows x top-2 of 256 experts, 1792 x 512, 20.6 us, now 11.0.  Refused with them are some even calls
+// that it served better: 150 rows x top-8 of 256 experts, 1792 x 384, 45 -> 62 us.)
 // Both doors take the kernel by the plain door's price: one arithmetic.
 bool qw_grouped_rows(hipStream_t st, int fmt, const qw_gemm_params& g, uint32_t max_tiles, uint32_t experts, uint32_t xdt, uint32_t ydt, bool swiglu,
                      hipError_t* err) {
